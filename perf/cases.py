@@ -306,17 +306,21 @@ def run(state):
             m = int((start + count).max())
             tets = torch.empty((m, 4), dtype=torch.int32, device="cuda")
             ctx.copy(tets.data_ptr(), dt, m * 16)
-        # the cloud of each row; rows between clouds (a repaired cloud's rows
-        # come after the others, its old ones stay) are void
+        # the cloud of each row; rows before, between and after the clouds' own
+        # (a repaired cloud's rows come after the others, its old ones stay)
+        # are void
         order = np.argsort(start, kind="stable")
-        span = np.diff(np.append(start[order], len(tets)))
+        begin = start[order]
+        begin[0] = 0  # the first cloud's old rows, when it was repaired
+        span = np.diff(np.append(begin, len(tets)))
         gaps = int(span.sum() - count.sum())
         order, span = torch.from_numpy(order).cuda(), torch.from_numpy(span).cuda()
         cloud = torch.repeat_interleave(order, span, output_size=len(tets))
         void = None
         if gaps:
-            end = torch.from_numpy(start + count).cuda()
-            void = torch.arange(len(tets), device="cuda") >= end[cloud]
+            row = torch.arange(len(tets), device="cuda")
+            first, end = torch.from_numpy(start).cuda(), torch.from_numpy(start + count).cuda()
+            void = (row < first[cloud]) | (row >= end[cloud])
         mesh = _packed(tets, bits, rows, int(count.sum()), cloud, void)
         mesh["tets_per_cloud"] = torch.from_numpy(count)
         return mesh
