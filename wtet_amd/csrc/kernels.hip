@@ -11,6 +11,7 @@
 #include "kernels.h"
 #include "prep.h"
 #include "sort.h"
+#include "wave.h"
 
 namespace wtet {
 
@@ -20,20 +21,6 @@ __global__ void k_fill_u32(uint32_t* p, uint32_t v, uint64_t n);
 // helpers
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ uint32_t gid() { return blockIdx.x * blockDim.x + threadIdx.x; }
-
-// Adds this thread's local counters to the global u64 counters (one atomic
-// per counter per wavefront).  Must be reached by every lane of the wave.
-__device__ __forceinline__ void flush_stats(const PredStats& ls, uint64_t* st) {
-  if (!st) return;
-  unsigned long long* g = reinterpret_cast<unsigned long long*>(st);
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    uint32_t v = ls.c[k];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    if (__lane_id() == 0 && v) atomicAdd(g + k, (unsigned long long)v);
-  }
-}
 
 // exclusive rank of `flag` within the block; *total = block count.
 // Every thread of the block must call it.
@@ -236,16 +223,6 @@ hipError_t sort_pairs_u32(uint32_t* keys, uint32_t* vals, uint32_t* keys_tmp, ui
   return radix_sort_u32(keys, vals, keys_tmp, vals_tmp, n, end_bit, temp, temp_bytes, s);
 }
 
-// sorted position j of cloud c: kept unless it is a redundant duplicate;
-// the uninserted list holds (vertex j + 4c, start super tet 5c)
-__device__ __forceinline__ bool keep_point(const float4* pts, const uint64_t* keys, uint32_t n,
-                                           const Clouds& K, uint32_t j, uint32_t* c,
-                                           uint32_t* capped) {
-  if (j >= n) return false;
-  *c = cloud_of_key(K, keys[j]);
-  return !redundant_dup(pts + 4u * *c, keys, n, j, capped);
-}
-
 __global__ void k_uninit_count(const float4* pts, const uint64_t* keys, uint32_t n, Clouds K,
                                uint32_t* blk, uint32_t* ctr) {
   uint32_t j = gid();
@@ -317,45 +294,8 @@ hipError_t launch_stratify(uint32_t* uvert, uint32_t* utet, uint32_t U, const Cl
 // ---------------------------------------------------------------------------
 // insertion rounds
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ uint64_t shfl_u64(uint64_t v, int src) {
-  uint32_t lo = __shfl((uint32_t)v, src), hi = __shfl((uint32_t)(v >> 32), src);
-  return ((uint64_t)hi << 32) | lo;
-}
-__device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m) {
-  uint32_t lo = __shfl_xor((uint32_t)v, m), hi = __shfl_xor((uint32_t)(v >> 32), m);
-  return ((uint64_t)hi << 32) | lo;
-}
-
-// Lanes voting for the same tet as the wave's first pending lane combine
-// their keys with a wave min first (a few passes), so early rounds -- when
-// most points still share a few tets -- issue one atomic per wave instead of
-// one per point; the remaining lanes vote directly.
 __global__ void __launch_bounds__(kBlock) k_vote(Mesh M, const uint32_t* uvert, const uint32_t* utet) {
-  const uint32_t U = M.ctr[C_ULEN];
-  uint32_t i = gid();
-  uint64_t key = kVoteNone;
-  uint32_t t = 0;
-  if (i < U) {
-    t = utet[i];
-    key = vote_key(M, uvert, utet, i);
-  }
-  bool pending = key != kVoteNone;
-  for (int pass = 0; pass < 4; ++pass) {
-    uint64_t act = __ballot(pending);
-    if (!act) break;
-    int leader = __ffsll((unsigned long long)act) - 1;
-    uint32_t lt = __shfl(t, leader);
-    bool mine = pending && t == lt;
-    uint64_t k = mine ? key : kVoteNone;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      uint64_t o = shfl_xor_u64(k, off);
-      k = o < k ? o : k;
-    }
-    if (__lane_id() == leader) at_min_u64(&M.tvote[lt], k);
-    if (mine) pending = false;
-  }
-  if (pending) at_min_u64(&M.tvote[t], key);
+  vote_wave(M, uvert, utet, gid(), M.ctr[C_ULEN]);
 }
 
 __global__ void __launch_bounds__(kBlock) k_pick_count(Mesh M, const uint32_t* utet, uint32_t* blk, int ring) {
@@ -379,8 +319,8 @@ __global__ void __launch_bounds__(kBlock) k_pick_scatter(Mesh M, const uint32_t*
   uint32_t t = utet[i], v = uvert[i];
   if (w) {
     wlist[r] = make_uint2(t, v);
-    M.tsplit[t] = make_uint2(round, M.ctr[C_BASE] + 3u * r);
-    M.tpoint[t] = v;
+    TSPLIT(M, t) = make_uint2(round, M.ctr[C_BASE] + 3u * r);
+    TPOINT(M, t) = v;
   } else {
     uvert2[i - r] = v;
     utet2[i - r] = t;
@@ -405,7 +345,7 @@ void launch_vote(const Mesh& M, const uint32_t* uvert, const uint32_t* utet, uin
 // round (list positions change); split resets the votes of winning tets
 __global__ void k_clear_votes(Mesh M, const uint32_t* utet2, const uint32_t* ctr) {
   uint32_t i = gid();
-  if (i < ctr[C_SURV]) M.tvote[utet2[i]] = kVoteNone;
+  if (i < ctr[C_SURV]) TVOTE(M, utet2[i]) = kVoteNone;
 }
 
 void launch_pick(const Mesh& M, const uint32_t* uvert, const uint32_t* utet, uint32_t U,
@@ -570,77 +510,39 @@ __global__ void k_iter_step(uint32_t* ctr, unsigned long long* sums) {
   iter_begin(ctr);
 }
 
-template <int FORM>
+// The filters of the flip check on every list entry, one thread per tet; the
+// entries they leave go to L.slow.  98 VGPRs, 4 waves per SIMD (at 96 and 5
+// waves, with two registers spilled, it took the same time).  1M uniform
+// points: 6.68 ms of event time a triangulation with insphere_f32 and
+// insphere_f64 per face and three orient3d after each (158 VGPRs), 5.60 ms
+// with one set of cofactors per tet; 100k points 2.79 -> 2.05 ms.
 __global__ void __launch_bounds__(kBlock) k_flip_check(Mesh M, FlipLists L, uint64_t* st) {
   if (!M.ctr[C_RUN]) return;
   uint32_t it = M.ctr[C_IT];
   const uint32_t* cur = L.act[M.ctr[C_PAR] & 1u];
   uint32_t stride = gridDim.x * blockDim.x;
   PredStats ls = {};
-  // LEAN defers what its filters leave to k_flip_check_deferred; FULL runs
-  // the full predicates on every entry
   uint32_t A = M.ctr[C_A];
-  for (uint32_t j = gid(); j < A; j += stride) {
-    bool defer = flip_check_body_t<FORM == LEAN>(M, cur, L.prop, j, it, &ls);
-    if (defer) L.slow[append_slot(&M.ctr[C_SLOW_T])] = j;
-  }
+  for (uint32_t j = gid(); j < A; j += stride)
+    if (flip_check_lean(M, cur, L.prop, j, it, &ls))
+      L.slow[append_slot(&M.ctr[C_SLOW_T])] = j;
   flush_stats(ls, st);
 }
 
-// The full check of the tets the lean check deferred, four lanes per tet,
-// one per face: each lane runs its face's staged insphere and, where the
-// face's apex lies inside, the three orient3d that classify the flip; the
-// lowest face that proposes is the tet's proposal, as flip_check_body_t's
-// loop over the faces would choose it.  A tet's faces then reach the exact
-// and SoS stages together rather than one after another in divergent
-// passes.  A tet's lanes are consecutive in one wave (k = 4 * entry + face,
-// and a wave's first k is a multiple of 64).
-__global__ void __launch_bounds__(kBlock) k_flip_check_deferred(Mesh M, FlipLists L, uint64_t* st) {
+// The full predicates, four lanes per tet (flip_check_faces), on the entries
+// the filters left or, with ALL, on every entry of the list (exact mode: one
+// thread per tet and its faces in turn took 159 us a launch at 10,000 points,
+// four lanes 41 us).  A wave's first k is a multiple of 64, so a tet's four
+// lanes share a wave.
+template <bool ALL>
+__global__ void __launch_bounds__(kBlock) k_flip_check_faces(Mesh M, FlipLists L, uint64_t* st) {
   if (!M.ctr[C_RUN]) return;
   const uint32_t it = M.ctr[C_IT];
   const uint32_t* cur = L.act[M.ctr[C_PAR] & 1u];
-  const uint32_t n4 = 4u * M.ctr[C_SLOW_T], stride = gridDim.x * blockDim.x;
+  const uint32_t n4 = 4u * M.ctr[ALL ? C_A : C_SLOW_T], stride = gridDim.x * blockDim.x;
   PredStats ls = {};
-  for (uint32_t k = gid(); k < n4; k += stride) {
-    const uint32_t j = L.slow[k >> 2];
-    const int f = (int)(k & 3u);
-    const uint32_t t = cur[j];
-    const uint32_t info = INFO(M, t);
-    const uint4 tv = TV(M, t);
-    const uint4 tov = TOV(M, t);
-    const bool live = (info & kAlive) && tv.x != M.inf && tv.y != M.inf && tv.z != M.inf &&
-                      tv.w != M.inf;
-    bool qual = false;
-    uint32_t kind = 0u, bad = 0u, third = kInvalid;
-    if (live) {
-      float P[4][3], Q[4][3];
-      uint32_t R[4], RQ[4];
-      for (int q = 0; q < 4; ++q) load_pt(M, get4(tv, q), P[q], &R[q]);
-      for (int q = 0; q < 4; ++q) load_pt(M, get4(tov, q), Q[q], &RQ[q]);
-      qual = flip_face_full(M, t, tov, P, R, Q, RQ, f, &ls, &kind, &bad, &third);
-    }
-    const uint64_t qb = __ballot(qual);
-    const uint32_t g0 = __lane_id() & ~3u;
-    const uint32_t grp = (uint32_t)(qb >> g0) & 0xFu;
-    const uint32_t cf = grp ? (uint32_t)__builtin_ctz(grp) : 0u;
-    const uint32_t pk = (uint32_t)f | kind << 2 | bad << 3;
-    const uint32_t pk_c = (uint32_t)__shfl((int)pk, (int)(g0 + cf));
-    const uint32_t third_c = (uint32_t)__shfl((int)third, (int)(g0 + cf));
-    if (f == 0) {
-      // each entry is in the list once and only its lanes touch its info
-      INFO(M, t) = info & ~kQueued;
-      if (grp) {
-        uint32_t nt = opp_tet(*opp_word(M, t, cf));
-        uint64_t key = flip_key(it, t);
-        at_min_u64(&M.fvote[t], key);
-        at_min_u64(&M.fvote[nt], key);
-        if ((pk_c >> 2) & 1u) at_min_u64(&M.fvote[third_c], key);
-        L.prop[j] = make_uint4(t, pk_c, nt, third_c);
-      } else {
-        L.prop[j].x = kInvalid;
-      }
-    }
-  }
+  for (uint32_t k = gid(); k < n4; k += stride)
+    flip_check_faces(M, cur, L.prop, ALL ? k >> 2 : L.slow[k >> 2], (int)(k & 3u), it, &ls);
   flush_stats(ls, st);
 }
 
@@ -733,7 +635,7 @@ __global__ void __launch_bounds__(kBlock) k_flip_update(Mesh M, FlipLists L) {
 // other threads of the block change are read with atomic loads.
 __global__ void __launch_bounds__(kBlock) k_flip_small(Mesh M, FlipLists L, uint64_t* st,
                                                        unsigned long long* sums, int k, uint32_t limit) {
-  __shared__ uint32_t run;
+  __shared__ uint32_t run, nslow;
   PredStats ls = {};
   uint32_t* ctr = M.ctr;
   auto ld = [&](int i) { return __atomic_load_n(&ctr[i], __ATOMIC_RELAXED); };
@@ -757,14 +659,22 @@ __global__ void __launch_bounds__(kBlock) k_flip_small(Mesh M, FlipLists L, uint
       }
       __atomic_store_n(&ctr[C_RUN], go, __ATOMIC_RELAXED);
       run = go;
+      nslow = 0u;
     }
     __syncthreads();
     if (!run) break;
     uint32_t A = ld(C_A), it = ld(C_IT), par = ld(C_PAR) & 1u;
     const uint32_t* cur = L.act[par];
     uint32_t* nxt = L.act[par ^ 1u];
-    for (uint32_t j = threadIdx.x; j < A; j += blockDim.x)
-      (void)flip_check_body_t<false>(M, cur, L.prop, j, it, &ls);
+    uint32_t ns = A;
+    if (M.mode == PRED_FILTERED) {
+      for (uint32_t j = threadIdx.x; j < A; j += blockDim.x)
+        if (flip_check_lean(M, cur, L.prop, j, it, &ls)) L.slow[append_slot(&nslow)] = j;
+      __syncthreads();
+      ns = nslow;
+    }
+    for (uint32_t q = threadIdx.x; q < 4u * ns; q += blockDim.x)
+      flip_check_faces(M, cur, L.prop, M.mode == PRED_FILTERED ? L.slow[q >> 2] : q >> 2, (int)(q & 3u), it, &ls);
     __syncthreads();
     for (uint32_t j = threadIdx.x; j < A; j += blockDim.x)
       flip_decide_exec_body(M, L.prop, j, it, round, L.out, nxt);
@@ -811,12 +721,12 @@ void launch_iter_step(uint32_t* ctr, uint64_t* sums, hipStream_t s) {
   k_iter_step<<<1, 64, 0, s>>>(ctr, reinterpret_cast<unsigned long long*>(sums));
 }
 void launch_flip_check(const Mesh& M, const FlipLists& L, uint32_t grid, uint64_t* st, hipStream_t s) {
-  if (M.mode == PRED_FILTERED) k_flip_check<LEAN><<<grid, kBlock, 0, s>>>(M, L, st);
-  else k_flip_check<FULL><<<grid, kBlock, 0, s>>>(M, L, st);
+  if (M.mode == PRED_FILTERED) k_flip_check<<<grid, kBlock, 0, s>>>(M, L, st);
+  else k_flip_check_faces<true><<<std::min(4u * grid, 4096u), kBlock, 0, s>>>(M, L, st);
 }
 void launch_flip_check_deferred(const Mesh& M, const FlipLists& L, uint32_t grid, uint64_t* st,
                                 hipStream_t s) {
-  if (M.mode == PRED_FILTERED) k_flip_check_deferred<<<grid, kBlock, 0, s>>>(M, L, st);
+  if (M.mode == PRED_FILTERED) k_flip_check_faces<false><<<grid, kBlock, 0, s>>>(M, L, st);
 }
 // grid: blocks of kBlock threads, as the other list kernels; the same
 // threads in blocks of kDecBlock
@@ -861,8 +771,8 @@ void launch_relocate(const Mesh& M, const uint32_t* uvert, uint32_t* utet, uint3
 
 // LEAN: every slot, FP32 filter, undecided tets to slow[ctr[C_SLOW_T]];
 // SLOW: the full predicates on those; FULL: the full predicates on every slot
-template <int FORM>
-__global__ void __launch_bounds__(kBlock) k_audit(Mesh M, uint32_t T, uint32_t* rec, uint32_t cap,
+template <int FORM, class MS>
+__global__ void __launch_bounds__(kBlock) k_audit(MS M, uint32_t T, uint32_t* rec, uint32_t cap,
                                                   uint64_t* st, uint32_t* slow) {
   PredStats ls = {};
   if (FORM == SLOW) {
@@ -876,8 +786,9 @@ __global__ void __launch_bounds__(kBlock) k_audit(Mesh M, uint32_t T, uint32_t* 
   flush_stats(ls, st);
 }
 
-void launch_audit(const Mesh& M, uint32_t T, uint32_t* rec, uint32_t cap, uint64_t* st,
-                  uint32_t* slow, hipStream_t s) {
+template <class MS>
+static void audit_t(const MS& M, uint32_t T, uint32_t* rec, uint32_t cap, uint64_t* st, uint32_t* slow,
+                    hipStream_t s) {
   if (!T) return;
   if (M.mode == PRED_FILTERED) {
     k_set_ctr<<<1, 64, 0, s>>>(M.ctr, C_SLOW_T, 0u, -1, 0u);
@@ -888,10 +799,16 @@ void launch_audit(const Mesh& M, uint32_t T, uint32_t* rec, uint32_t cap, uint64
   }
 }
 
+void launch_audit(const Mesh& M, uint32_t T, uint32_t* rec, uint32_t cap, uint64_t* st, uint32_t* slow,
+                  hipStream_t s) {
+  audit_t(M, T, rec, cap, st, slow, s);
+}
+
 // ---------------------------------------------------------------------------
 // output
 // ---------------------------------------------------------------------------
-__global__ void k_alive_count(Mesh M, uint32_t T, uint32_t* blk) {
+template <class MS>
+__global__ void k_alive_count(MS M, uint32_t T, uint32_t* blk) {
   uint32_t t = gid();
   bool a = t < T && (INFO(M, t) & kAlive);
   uint32_t tot;
@@ -935,7 +852,8 @@ __global__ void k_cstart_tail(uint32_t* cstart, uint32_t C, const uint32_t* ctr)
   if (threadIdx.x == 0) cstart[C] = ctr[C_ALIVE];
 }
 
-__global__ void k_output_rows(Mesh M, uint32_t T, const uint32_t* olist, const uint32_t* okey,
+template <class MS>
+__global__ void k_output_rows(MS M, uint32_t T, const uint32_t* olist, const uint32_t* okey,
                               const uint32_t* cstart, const uint32_t* slot2pos, const uint32_t* vrank,
                               Clouds K, uint32_t* out_tets, uint32_t* out_adj) {
   uint32_t j = gid();

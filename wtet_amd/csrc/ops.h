@@ -78,7 +78,8 @@ struct __attribute__((aligned(64))) FlipMsg {
 
 // message of a destroyed tet: new neighbour pointers e (kInvalid where
 // unused), all opposite the vertex v
-WT_HD void set_msg(FlipMsg* m, uint4 e, uint32_t v) {
+template <class MSG>
+WT_HD void set_msg(MSG* m, uint4 e, uint32_t v) {
   m->lo = make_uint4(e.x, v, e.y, v);
   m->hi = make_uint4(e.z, v, e.w, v);
 }
@@ -103,32 +104,45 @@ struct Mesh {
 };
 
 WT_HD uint4& TV(const Mesh& M, uint32_t t) { return M.tet[t]; }
-WT_HD uint4 TN(const Mesh& M, uint32_t t) {
-  uint4 a = M.adj[t].lo, b = M.adj[t].hi;
+WT_HD AdjRec& ADJ(const Mesh& M, uint32_t t) { return M.adj[t]; }
+WT_HD uint32_t& INFO(const Mesh& M, uint32_t t) { return M.tinfo[t]; }
+WT_HD uint32_t& TFWD(const Mesh& M, uint32_t t) { return M.tfwd[t]; }
+WT_HD uint64_t& TVOTE(const Mesh& M, uint32_t t) { return M.tvote[t]; }
+WT_HD uint64_t& FVOTE(const Mesh& M, uint32_t t) { return M.fvote[t]; }
+WT_HD uint2& TSPLIT(const Mesh& M, uint32_t t) { return M.tsplit[t]; }
+WT_HD uint32_t& TPOINT(const Mesh& M, uint32_t t) { return M.tpoint[t]; }
+WT_HD FlipMsg& TMSG(const Mesh& M, uint32_t t) { return M.tmsg[t]; }
+
+template <class MS>
+WT_HD uint4 TN(const MS& M, uint32_t t) {
+  uint4 a = ADJ(M, t).lo, b = ADJ(M, t).hi;
   return make_uint4(a.x, a.z, b.x, b.z);
 }
-WT_HD uint4 TOV(const Mesh& M, uint32_t t) {
-  uint4 a = M.adj[t].lo, b = M.adj[t].hi;
+template <class MS>
+WT_HD uint4 TOV(const MS& M, uint32_t t) {
+  uint4 a = ADJ(M, t).lo, b = ADJ(M, t).hi;
   return make_uint4(a.y, a.w, b.y, b.w);
 }
 // both halves of slot t's record: neighbours n and opposite vertices ov
-WT_HD void set_adj(const Mesh& M, uint32_t t, uint4 n, uint4 ov) {
-  M.adj[t].lo = make_uint4(n.x, ov.x, n.y, ov.y);
-  M.adj[t].hi = make_uint4(n.z, ov.z, n.w, ov.w);
+template <class MS>
+WT_HD void set_adj(const MS& M, uint32_t t, uint4 n, uint4 ov) {
+  ADJ(M, t).lo = make_uint4(n.x, ov.x, n.y, ov.y);
+  ADJ(M, t).hi = make_uint4(n.z, ov.z, n.w, ov.w);
 }
-WT_HD uint32_t& INFO(const Mesh& M, uint32_t t) { return M.tinfo[t]; }
 // the stamp shares its slot's message line: the adjacency update reads a
 // flipped neighbour's stamp and message together
-WT_HD uint64_t& FSTAMP(const Mesh& M, uint32_t t) { return M.tmsg[t].stamp; }
+template <class MS>
+WT_HD uint64_t& FSTAMP(const MS& M, uint32_t t) { return TMSG(M, t).stamp; }
 WT_HD uint64_t flip_stamp(uint32_t round, uint32_t it) { return (uint64_t)round << 32 | it; }
-WT_HD uint32_t& TFWD(const Mesh& M, uint32_t t) { return M.tfwd[t]; }
 
-WT_HD float3 P3(const Mesh& M, uint32_t v) {
+template <class MS>
+WT_HD float3 P3(const MS& M, uint32_t v) {
   float4 p = M.pts[v];
   return make_float3(p.x, p.y, p.z);
 }
 
-WT_HD void load_pt(const Mesh& M, uint32_t v, float* out, uint32_t* rank) {
+template <class MS>
+WT_HD void load_pt(const MS& M, uint32_t v, float* out, uint32_t* rank) {
   float4 p = M.pts[v];
   out[0] = p.x;
   out[1] = p.y;
@@ -137,7 +151,8 @@ WT_HD void load_pt(const Mesh& M, uint32_t v, float* out, uint32_t* rank) {
 }
 
 // orient3d_sos on four vertex ids
-WT_HD int o3(const Mesh& M, uint32_t a, uint32_t b, uint32_t c, uint32_t d, PredStats* st) {
+template <class MS>
+WT_HD int o3(const MS& M, uint32_t a, uint32_t b, uint32_t c, uint32_t d, PredStats* st) {
   float A[3], B[3], C[3], D[3];
   uint32_t ra, rb, rc, rd;
   load_pt(M, a, A, &ra);
@@ -151,43 +166,23 @@ WT_HD int o3(const Mesh& M, uint32_t a, uint32_t b, uint32_t c, uint32_t d, Pred
 // alone and returns 2 when it cannot decide; the body then stops with no
 // side effect and reports the element as deferred, and a second kernel
 // runs the full staged predicates on the deferred elements only.
-template <bool FAST>
-WT_HD int o3s(const Mesh& M, const float* a, const float* b, const float* c, const float* d,
+template <bool FAST, class MS>
+WT_HD int o3s(const MS& M, const float* a, const float* b, const float* c, const float* d,
               uint32_t ra, uint32_t rb, uint32_t rc, uint32_t rd, PredStats* st) {
   if (FAST) return orient3d_sos_fast(a, b, c, d, st);
   return orient3d_sos(a, b, c, d, ra, rb, rc, rd, M.mode, st);
 }
 
-template <bool FAST>
-WT_HD int o4s(const Mesh& M, const float* a, const float* b, const float* c, const float* d,
+template <bool FAST, class MS>
+WT_HD int o4s(const MS& M, const float* a, const float* b, const float* c, const float* d,
               const float* e, uint32_t ra, uint32_t rb, uint32_t rc, uint32_t rd, uint32_t re,
               PredStats* st) {
   if (FAST) return orient4d_fast(a, b, c, d, e, st);
   return orient4d(a, b, c, d, e, ra, rb, rc, rd, re, M.mode, st);
 }
 
-// The flip check's insphere.  The lean form adds the FP64 filter, which
-// settles nearly every face the FP32 filter leaves on non-degenerate input:
-// few tets then wait for the deferred full check.  Measured at 1M uniform
-// points: the lean check 6.46 -> 6.79 ms (158 VGPRs, occupancy 5 -> 3), the
-// deferred check 2.76 -> 1.92 ms, device phase 27.35 -> 26.70 ms; calling
-// the FP64 stage out of line (128 VGPRs) made the lean check 7.40 ms.
-template <bool FAST>
-WT_HD int o4s_check(const Mesh& M, const float* a, const float* b, const float* c, const float* d,
-                    const float* e, uint32_t ra, uint32_t rb, uint32_t rc, uint32_t rd, uint32_t re,
-                    PredStats* st) {
-  if (FAST) {
-    int s = orient4d_fast(a, b, c, d, e, st);
-    if (s != 2) return s;
-    s = insphere_f64(a, b, c, d, e);
-    if (s != 2) stat_inc(st, 5);
-    return s;
-  }
-  return orient4d(a, b, c, d, e, ra, rb, rc, rd, re, M.mode, st);
-}
-
-template <bool FAST>
-WT_HD int o3v(const Mesh& M, uint32_t a, uint32_t b, uint32_t c, uint32_t d, PredStats* st) {
+template <bool FAST, class MS>
+WT_HD int o3v(const MS& M, uint32_t a, uint32_t b, uint32_t c, uint32_t d, PredStats* st) {
   float A[3], B[3], C[3], D[3];
   uint32_t ra, rb, rc, rd;
   load_pt(M, a, A, &ra);
@@ -197,17 +192,20 @@ WT_HD int o3v(const Mesh& M, uint32_t a, uint32_t b, uint32_t c, uint32_t d, Pre
   return o3s<FAST>(M, A, B, C, D, ra, rb, rc, rd, st);
 }
 
-WT_HD uint32_t* opp_word(const Mesh& M, uint32_t t, uint32_t f) {
-  return reinterpret_cast<uint32_t*>(&M.adj[t]) + 2 * f;
+template <class MS>
+WT_HD uint32_t* opp_word(const MS& M, uint32_t t, uint32_t f) {
+  return reinterpret_cast<uint32_t*>(&ADJ(M, t)) + 2 * f;
 }
 
-WT_HD uint32_t* oppv_word(const Mesh& M, uint32_t t, uint32_t f) {
-  return reinterpret_cast<uint32_t*>(&M.adj[t]) + 2 * f + 1;
+template <class MS>
+WT_HD uint32_t* oppv_word(const MS& M, uint32_t t, uint32_t f) {
+  return reinterpret_cast<uint32_t*>(&ADJ(M, t)) + 2 * f + 1;
 }
 
 // face f of slot t: neighbour pointer and opposite vertex in one store
-WT_HD void set_face(const Mesh& M, uint32_t t, uint32_t f, uint32_t n, uint32_t ov) {
-  reinterpret_cast<uint2*>(&M.adj[t])[f] = make_uint2(n, ov);
+template <class MS>
+WT_HD void set_face(const MS& M, uint32_t t, uint32_t f, uint32_t n, uint32_t ov) {
+  reinterpret_cast<uint2*>(&ADJ(M, t))[f] = make_uint2(n, ov);
 }
 
 // ---------------------------------------------------------------------------
@@ -217,7 +215,8 @@ WT_HD void set_face(const Mesh& M, uint32_t t, uint32_t f, uint32_t n, uint32_t 
 // lowest list position.  src/shaders/vote.wgsl:89-281 (two passes there).
 // ---------------------------------------------------------------------------
 // returns kVoteNone when the point must not vote
-WT_HD uint64_t vote_key(const Mesh& M, const uint32_t* uvert, const uint32_t* utet, uint32_t i) {
+template <class MS>
+WT_HD uint64_t vote_key(const MS& M, const uint32_t* uvert, const uint32_t* utet, uint32_t i) {
   // The key is computed before the infinity test (every id, infinity
   // included, is a loadable point), so that the point's own id and
   // coordinates load beside its tet's vertices: two round trips.
@@ -240,9 +239,10 @@ WT_HD uint64_t vote_key(const Mesh& M, const uint32_t* uvert, const uint32_t* ut
   return bad ? kVoteNone : key;
 }
 
-WT_HD void vote_body(const Mesh& M, const uint32_t* uvert, const uint32_t* utet, uint32_t i) {
+template <class MS>
+WT_HD void vote_body(const MS& M, const uint32_t* uvert, const uint32_t* utet, uint32_t i) {
   uint64_t key = vote_key(M, uvert, utet, i);
-  if (key != kVoteNone) at_min_u64(&M.tvote[utet[i]], key);
+  if (key != kVoteNone) at_min_u64(&TVOTE(M, utet[i]), key);
 }
 
 // Point i is inserted this round when it holds its tet's vote and no tet
@@ -251,20 +251,21 @@ WT_HD void vote_body(const Mesh& M, const uint32_t* uvert, const uint32_t* utet,
 // is what leaves concurrent flipping unable to finish (faces that are
 // neither 2-3 nor 3-2 flippable); the deferred points win a later round.
 // Reads votes only, so every thread sees the same decision.
-WT_HD bool is_winner(const Mesh& M, const uint32_t* utet, uint32_t i, int ring) {
+template <class MS>
+WT_HD bool is_winner(const MS& M, const uint32_t* utet, uint32_t i, int ring) {
   uint32_t t = utet[i];
-  uint64_t kt = M.tvote[t];
+  uint64_t kt = TVOTE(M, t);
   if ((uint32_t)(kt & 0xFFFFFFFFull) != i) return false;
   if (ring <= 0) return true;
   uint4 to = TN(M, t);
   for (int f = 0; f < 4; ++f) {
     uint32_t nt = opp_tet(get4(to, f));
-    if (M.tvote[nt] < kt) return false;
+    if (TVOTE(M, nt) < kt) return false;
     if (ring > 1) {
       uint4 no = TN(M, nt);
       for (int g = 0; g < 4; ++g) {
         uint32_t n2 = opp_tet(get4(no, g));
-        if (n2 != t && M.tvote[n2] < kt) return false;
+        if (n2 != t && TVOTE(M, n2) < kt) return false;
       }
     }
   }
@@ -284,10 +285,11 @@ WT_HD uint32_t child_slot(uint32_t t, uint32_t base, uint32_t j) {
 // active list (bit j for child j; slot t only if no earlier list holds it).
 // The neighbours' split records are loaded before any store: this kernel
 // writes those of fresh slots only, never a neighbour's.
-WT_HD uint32_t split_body(const Mesh& M, const uint2* wlist, uint32_t k, uint32_t round,
+template <class MS>
+WT_HD uint32_t split_body(const MS& M, const uint2* wlist, uint32_t k, uint32_t round,
                           uint32_t c[4]) {
   uint32_t t = wlist[k].x, p = wlist[k].y;
-  uint32_t base = M.tsplit[t].y;
+  uint32_t base = TSPLIT(M, t).y;
   uint4 tv = TV(M, t);
   uint4 to = TN(M, t);
   uint4 tov = TOV(M, t);
@@ -296,8 +298,8 @@ WT_HD uint32_t split_body(const Mesh& M, const uint2* wlist, uint32_t k, uint32_
   uint32_t np[4];
   for (int j = 0; j < 4; ++j) {
     uint32_t nt = opp_tet(get4(to, j));
-    ns[j] = M.tsplit[nt];
-    np[j] = M.tpoint[nt];  // read for every neighbour, used where it splits
+    ns[j] = TSPLIT(M, nt);
+    np[j] = TPOINT(M, nt);  // read for every neighbour, used where it splits
   }
   for (int j = 0; j < 4; ++j) {
     uint4 nv = tv;
@@ -322,11 +324,11 @@ WT_HD uint32_t split_body(const Mesh& M, const uint2* wlist, uint32_t k, uint32_
     }
     TV(M, c[j]) = nv;
     set_adj(M, c[j], no, nov);
-    M.tvote[c[j]] = kVoteNone;
+    TVOTE(M, c[j]) = kVoteNone;
     if (j > 0) {  // fresh slot: initialise every per-slot field
       INFO(M, c[j]) = kAlive | kQueued;
-      M.fvote[c[j]] = kVoteNone;
-      M.tsplit[c[j]] = make_uint2(0u, 0u);
+      FVOTE(M, c[j]) = kVoteNone;
+      TSPLIT(M, c[j]) = make_uint2(0u, 0u);
       FSTAMP(M, c[j]) = 0ull;
     }
   }
@@ -338,12 +340,12 @@ WT_HD uint32_t split_body(const Mesh& M, const uint2* wlist, uint32_t k, uint32_
 // move an uninserted point of a split tet into its child
 // (src/shaders/split_points.wgsl:222-335): three orient3d_sos tests.
 // ---------------------------------------------------------------------------
-template <bool FAST>
-WT_HD bool split_points_body_t(const Mesh& M, const uint32_t* uvert, uint32_t* utet, uint32_t i,
+template <bool FAST, class MS>
+WT_HD bool split_points_body_t(const MS& M, const uint32_t* uvert, uint32_t* utet, uint32_t i,
                                uint32_t round, PredStats* st) {
   uint32_t t = utet[i];
   uint32_t q = uvert[i];
-  uint2 sp = M.tsplit[t];
+  uint2 sp = TSPLIT(M, t);
   if (sp.x != round) return false;
   uint32_t base = sp.y;
   uint4 c0 = TV(M, t);      // (p, v1, v2, v3)
@@ -384,7 +386,8 @@ WT_HD bool split_points_body_t(const Mesh& M, const uint32_t* uvert, uint32_t* u
   return false;
 }
 
-WT_HD void split_points_body(const Mesh& M, const uint32_t* uvert, uint32_t* utet, uint32_t i,
+template <class MS>
+WT_HD void split_points_body(const MS& M, const uint32_t* uvert, uint32_t* utet, uint32_t i,
                              uint32_t round, PredStats* st) {
   (void)split_points_body_t<false>(M, uvert, utet, i, round, st);
 }
@@ -399,9 +402,83 @@ WT_HD uint64_t flip_key(uint32_t it, uint32_t t) {
   return ((uint64_t)(0xFFFFFFFFu - it) << 32) | t;
 }
 
-template <bool FAST>
-WT_HD bool flip_check_body_t(const Mesh& M, const uint32_t* act, uint4* prop, uint32_t j,
-                             uint32_t it, PredStats* st) {
+// xyz of point k (0..3, chosen at run time) of a tet's four, by selects
+WT_HD void pick_xyz(const float (*P)[3], int k, float* out) {
+  for (int c = 0; c < 3; ++c) out[c] = pick4(k, P[0][c], P[1][c], P[2][c], P[3][c]);
+}
+
+// The proposal of tet t across face f (its kind, offending edge and third
+// tet as flip_check_lean finds them): votes for the tets it involves.
+template <class MS>
+WT_HD uint4 flip_propose(const MS& M, uint32_t t, uint32_t f, uint32_t kind, uint32_t bad, uint32_t third,
+                         uint32_t it) {
+  uint32_t nt = opp_tet(*opp_word(M, t, f));
+  uint64_t key = flip_key(it, t);
+  at_min_u64(&FVOTE(M, t), key);
+  at_min_u64(&FVOTE(M, nt), key);
+  if (kind == 1u) at_min_u64(&FVOTE(M, third), key);
+  return make_uint4(t, f | kind << 2 | bad << 3, nt, third);
+}
+
+// The insphere filters take one of the tet's vertices as origin: a real point
+// (coordinates in [0, 1]; a super vertex has |x| >= 100), from which every
+// difference is as short as the tet allows.  origin_of: which of the four;
+// swap_origin exchanges it with P[0] (and back), which flips the determinant's
+// sign.
+WT_HD bool near_coord(float x) { return x >= -2.0f && x <= 2.0f; }
+WT_HD int origin_of(const float (*P)[3]) {
+  int k = near_coord(P[2][0]) ? 2 : 3;
+  k = near_coord(P[1][0]) ? 1 : k;
+  return near_coord(P[0][0]) ? 0 : k;
+}
+WT_HD void swap_origin(float (*P)[3], int k) {
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const float v = P[0][c];
+    P[0][c] = pick4(k, P[0][c], P[1][c], P[2][c], P[3][c]);
+    P[1][c] = k == 1 ? v : P[1][c];
+    P[2][c] = k == 2 ? v : P[2][c];
+    P[3][c] = k == 3 ? v : P[3][c];
+  }
+}
+
+// What the filters say about one face whose apex o lies inside the
+// circumsphere: kFaceNo (no flip), kFaceFlip (*kind, *bad set; *pthird is the
+// tet's vertex opposite the third tet of a 3-2 flip) or kFaceUndecided.
+enum FaceCheck : int { kFaceNo = 0, kFaceFlip = 1, kFaceUndecided = 2 };
+WT_HD int face_classify(const float* x, const float* y, const float* z, const float* a, const float* o,
+                        const int* pos, const uint4& tov, uint32_t ov, uint32_t* kind, uint32_t* bad,
+                        int* pthird, PredStats* st) {
+  // differences are taken from o, or, where o is a super vertex, from a:
+  // exchanging the two negates every determinant
+  const bool far = !near_coord(o[0]);
+  float p[3], q[3];
+  for (int k = 0; k < 3; ++k) p[k] = far ? o[k] : a[k], q[k] = far ? a[k] : o[k];
+  int s[3];
+  orient3d_edges_f32(x, y, z, p, q, s);
+  if (far)
+    for (int k = 0; k < 3; ++k) s[k] = s[k] == 2 ? 2 : -s[k];
+  if (s[0] == 2 || s[1] == 2 || s[2] == 2) return kFaceUndecided;
+  for (int k = 0; k < 3; ++k) stat_inc(st, 0);
+  // edge k: the line a-o should pass on the face side (raw sign > 0)
+  int nbad = (s[0] < 0) + (s[1] < 0) + (s[2] < 0);
+  int b = s[0] < 0 ? 0 : (s[1] < 0 ? 1 : 2);
+  *kind = nbad == 1 ? 1u : 0u;
+  *bad = nbad == 1 ? (uint32_t)b : 0u;
+  *pthird = b == 0 ? pos[2] : (b == 1 ? pos[0] : pos[1]);
+  if (nbad == 0) return kFaceFlip;
+  // 3-2 needs the edge to have degree 3: the tet across t's face opposite the
+  // third vertex must have o as its apex
+  return nbad == 1 && get4(tov, *pthird) == ov ? kFaceFlip : kFaceNo;
+}
+
+// Lean check of list entry j, one thread per tet: FP32 filters, and the FP64
+// filter for the faces whose insphere they leave.  The first face (in order)
+// that can flip is proposed; true (no side effect but the queued bit) when a
+// face before it is undecided, and the entry needs the full predicates.
+template <class MS>
+WT_HD bool flip_check_lean(const MS& M, const uint32_t* act, uint4* prop, uint32_t j, uint32_t it,
+                           PredStats* st) {
   uint32_t t = act[j];
   // Two memory round trips: the slot's info, vertices and opposite vertices
   // together (all in the slot's own records), then all eight points (the
@@ -416,50 +493,58 @@ WT_HD bool flip_check_body_t(const Mesh& M, const uint32_t* act, uint4* prop, ui
   if (!(info & kAlive)) return false;
   if (tv.x == M.inf || tv.y == M.inf || tv.z == M.inf || tv.w == M.inf) return false;
   float P[4][3], Q[4][3];
-  uint32_t R[4], RQ[4];
-  for (int k = 0; k < 4; ++k) load_pt(M, get4(tv, k), P[k], &R[k]);
-  for (int k = 0; k < 4; ++k) load_pt(M, get4(tov, k), Q[k], &RQ[k]);
-  for (int f = 0; f < 4; ++f) {
-    uint32_t o = get4(tov, f);
-    if (o == M.inf) continue;
-    const float* O = Q[f];
-    uint32_t ro = RQ[f];
-    int ins = o4s_check<FAST>(M, P[0], P[1], P[2], P[3], O, R[0], R[1], R[2], R[3], ro, st);
-    if (ins == 2) return true;
-    if (ins > 0) continue;
-    // o lies inside the circumsphere: classify the flip
-    int px = face_vi(f, 0), py = face_vi(f, 1), pz = face_vi(f, 2);
-    int pos[3] = {px, py, pz};
-    int bad = -1, nbad = 0;
-    for (int k = 0; k < 3; ++k) {
-      int u = pos[k], w = pos[(k + 1) % 3];
-      // edge (u, w): the line a-o should pass on the face side -> raw > 0
-      int s = o3s<FAST>(M, P[u], P[w], P[f], O, R[u], R[w], R[f], ro, st);
-      if (s == 2) return true;
-      if (s > 0) {
-        bad = k;
-        ++nbad;
-      }
+  uint32_t r;
+  for (int k = 0; k < 4; ++k) load_pt(M, get4(tv, k), P[k], &r);
+  for (int k = 0; k < 4; ++k) load_pt(M, get4(tov, k), Q[k], &r);
+  // bit f: the apex across face f lies inside, or the filters cannot tell
+  uint32_t in = 0u, und = 0u;
+  const int org = origin_of(P);
+  if (org) swap_origin(P, org);
+  const int inside = org ? 1 : -1;
+  {
+    const InsphereTet<float> q = insphere_tet<float>(P[0], P[1], P[2], P[3]);
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+      if (get4(tov, f) == M.inf) continue;
+      int s = insphere_query_f32(q, P[0], Q[f]);
+      if (s == 2) und |= 1u << f;
+      else stat_inc(st, 4);
+      if (s == inside) in |= 1u << f;
     }
-    uint32_t kind, third = kInvalid;
-    if (nbad == 0) {
-      kind = 0;
-    } else if (nbad == 1) {
-      // 3-2 needs the edge to have degree 3: the tet across t's face
-      // opposite the third vertex must have o as its apex
-      int pthird = pos[(bad + 2) % 3];
-      if (get4(tov, pthird) != o) continue;
-      kind = 1;
-      third = opp_tet(*opp_word(M, t, (uint32_t)pthird));
-    } else {
-      continue;
+  }
+  if (und) {
+    const InsphereTet<double> q = insphere_tet<double>(P[0], P[1], P[2], P[3]);
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+      if (!((und >> f) & 1u)) continue;
+      int s = insphere_query_f64(q, P[0], Q[f]);
+      if (s == 2) continue;
+      stat_inc(st, 5);
+      und &= ~(1u << f);
+      if (s == inside) in |= 1u << f;
     }
-    uint32_t nt = opp_tet(*opp_word(M, t, (uint32_t)f));
-    uint64_t key = flip_key(it, t);
-    at_min_u64(&M.fvote[t], key);
-    at_min_u64(&M.fvote[nt], key);
-    if (kind == 1) at_min_u64(&M.fvote[third], key);
-    prop[j] = make_uint4(t, (uint32_t)f | kind << 2 | (uint32_t)(kind ? bad : 0) << 3, nt, third);
+  }
+  if (org) swap_origin(P, org);
+  // the faces left, in order: most lanes have at most one or two
+  uint32_t todo = in | und;
+  while (todo) {
+    const int f = ctz32(todo);
+    if ((und >> f) & 1u) return true;
+    todo &= todo - 1u;
+    float A[3], O[3], X[3], Y[3], Z[3];
+    const int pos[3] = {face_vi(f, 0), face_vi(f, 1), face_vi(f, 2)};
+    pick_xyz(P, f, A);
+    pick_xyz(Q, f, O);
+    pick_xyz(P, pos[0], X);
+    pick_xyz(P, pos[1], Y);
+    pick_xyz(P, pos[2], Z);
+    uint32_t kind, bad;
+    int pthird;
+    const int v = face_classify(X, Y, Z, A, O, pos, tov, get4(tov, f), &kind, &bad, &pthird, st);
+    if (v == kFaceUndecided) return true;
+    if (v == kFaceNo) continue;
+    const uint32_t third = kind ? opp_tet(*opp_word(M, t, (uint32_t)pthird)) : kInvalid;
+    prop[j] = flip_propose(M, t, (uint32_t)f, kind, bad, third, it);
     return false;
   }
   return false;
@@ -468,15 +553,16 @@ WT_HD bool flip_check_body_t(const Mesh& M, const uint32_t* act, uint4* prop, ui
 // point k (0..3, chosen at run time) of a tet's four: selects instead of an
 // indexed local array, which would live in scratch memory
 WT_HD void pick_pt(const float (*P)[3], const uint32_t* R, int k, float* out, uint32_t* r) {
-  for (int c = 0; c < 3; ++c) out[c] = k == 0 ? P[0][c] : (k == 1 ? P[1][c] : (k == 2 ? P[2][c] : P[3][c]));
-  *r = k == 0 ? R[0] : (k == 1 ? R[1] : (k == 2 ? R[2] : R[3]));
+  pick_xyz(P, k, out);
+  *r = pick4(k, R[0], R[1], R[2], R[3]);
 }
 
-// One face f (chosen at run time) of flip_check_body_t's loop with the full
+// One face f (chosen at run time) with the full
 // predicates: true when the face proposes a flip, with its kind, the
-// offending edge (3-2) and the third tet (3-2) as that loop sets them.  P, R:
+// offending edge (3-2) and the third tet (3-2).  P, R:
 // the tet's points and ranks; Q, RQ: the vertices across its faces.
-WT_HD bool flip_face_full(const Mesh& M, uint32_t t, const uint4& tov, const float (*P)[3],
+template <class MS>
+WT_HD bool flip_face_full(const MS& M, uint32_t t, const uint4& tov, const float (*P)[3],
                           const uint32_t* R, const float (*Q)[3], const uint32_t* RQ, int f,
                           PredStats* st, uint32_t* kind, uint32_t* bad, uint32_t* third) {
   uint32_t o = get4(tov, f);
@@ -484,7 +570,7 @@ WT_HD bool flip_face_full(const Mesh& M, uint32_t t, const uint4& tov, const flo
   float O[3];
   uint32_t ro;
   pick_pt(Q, RQ, f, O, &ro);
-  int ins = o4s_check<false>(M, P[0], P[1], P[2], P[3], O, R[0], R[1], R[2], R[3], ro, st);
+  int ins = o4s<false>(M, P[0], P[1], P[2], P[3], O, R[0], R[1], R[2], R[3], ro, st);
   if (ins > 0) return false;
   // o lies inside the circumsphere: classify the flip
   float A[3], V[3][3];
@@ -507,7 +593,7 @@ WT_HD bool flip_face_full(const Mesh& M, uint32_t t, const uint4& tov, const flo
     return true;
   }
   if (nbad > 1) return false;
-  // 3-2 needs the edge to have degree 3 (see flip_check_body_t)
+  // 3-2 needs the edge to have degree 3 (see face_classify)
   int pthird = b == 0 ? pos[2] : (b == 1 ? pos[0] : pos[1]);
   if (get4(tov, pthird) != o) return false;
   *kind = 1u;
@@ -534,7 +620,8 @@ struct FlipTets {
   uint4 tv, to, tov, nv, no, nov, mv, mo, mov;
 };
 
-WT_HD void flip_load(const Mesh& M, const uint4& pr, FlipTets& F) {
+template <class MS>
+WT_HD void flip_load(const MS& M, const uint4& pr, FlipTets& F) {
   // a 2-3 flip has no third tet: its slot is replaced by t's, so every load
   // is of a valid slot and none depends on a branch
   uint32_t m = ((pr.y >> 2) & 1u) ? pr.w : pr.x;
@@ -543,7 +630,8 @@ WT_HD void flip_load(const Mesh& M, const uint4& pr, FlipTets& F) {
   F.mv = TV(M, m), F.mo = TN(M, m), F.mov = TOV(M, m);
 }
 
-WT_HD void flip_exec_loaded(const Mesh& M, const uint4 pr, const FlipTets& F, uint32_t it,
+template <class MS>
+WT_HD void flip_exec_loaded(const MS& M, const uint4 pr, const FlipTets& F, uint32_t it,
                             uint32_t round, uint32_t s, uint4* outk) {
   uint32_t t = pr.x, f = pr.y & 3u, kind = (pr.y >> 2) & 1u, edge = (pr.y >> 3) & 3u;
   uint32_t n = pr.z;
@@ -575,13 +663,13 @@ WT_HD void flip_exec_loaded(const Mesh& M, const uint4 pr, const FlipTets& F, ui
     set4(mn, qz, enc_opp(Txy, 3));
     set4(mn, qx, enc_opp(Tyz, 3));
     set4(mn, qy, enc_opp(Tzx, 3));
-    set_msg(&M.tmsg[t], mt, o);
-    set_msg(&M.tmsg[n], mn, a);
+    set_msg(&TMSG(M, t), mt, o);
+    set_msg(&TMSG(M, n), mn, a);
     FSTAMP(M, t) = flip_stamp(round, it);
     FSTAMP(M, n) = flip_stamp(round, it);
-    M.tvote[s] = kVoteNone;
-    M.fvote[s] = kVoteNone;
-    M.tsplit[s] = make_uint2(0u, 0u);
+    TVOTE(M, s) = kVoteNone;
+    FVOTE(M, s) = kVoteNone;
+    TSPLIT(M, s) = make_uint2(0u, 0u);
     FSTAMP(M, s) = 0ull;
     INFO(M, s) = kAlive | kQueued;  // fresh slot: queued by the caller
     outk[0] = make_uint4(Txy, Tyz, Tzx, 0u);
@@ -611,9 +699,9 @@ WT_HD void flip_exec_loaded(const Mesh& M, const uint4 pr, const FlipTets& F, ui
     uint4 mm = make_uint4(kInvalid, kInvalid, kInvalid, kInvalid);
     set4(mm, my, enc_opp(A, 1));
     set4(mm, mx, enc_opp(B, 0));
-    set_msg(&M.tmsg[t], mt, o);
-    set_msg(&M.tmsg[n], mn, a);
-    set_msg(&M.tmsg[m], mm, z);
+    set_msg(&TMSG(M, t), mt, o);
+    set_msg(&TMSG(M, n), mn, a);
+    set_msg(&TMSG(M, m), mm, z);
     FSTAMP(M, t) = flip_stamp(round, it);
     FSTAMP(M, n) = flip_stamp(round, it);
     FSTAMP(M, m) = flip_stamp(round, it);
@@ -624,7 +712,8 @@ WT_HD void flip_exec_loaded(const Mesh& M, const uint4 pr, const FlipTets& F, ui
   }
 }
 
-WT_HD void flip_exec_body(const Mesh& M, const uint4 pr, uint32_t it, uint32_t round,
+template <class MS>
+WT_HD void flip_exec_body(const MS& M, const uint4 pr, uint32_t it, uint32_t round,
                           uint32_t s, uint4* outk) {
   FlipTets F;
   flip_load(M, pr, F);
@@ -640,14 +729,15 @@ WT_HD void flip_exec_body(const Mesh& M, const uint4 pr, uint32_t it, uint32_t r
 // or a loser's own tet.  qid[0..*nq) are the tets to append to the next
 // active list (kQueued is set here, so each tet is appended once); for a
 // 2-3 winner the fresh slot is appended by the caller after qid.
-WT_HD bool flip_decide_body(const Mesh& M, const uint4& pr, uint32_t it, uint32_t qid[2],
+template <class MS>
+WT_HD bool flip_decide_body(const MS& M, const uint4& pr, uint32_t it, uint32_t qid[2],
                             uint32_t* nq, uint32_t* nslot) {
   *nq = 0;
   *nslot = 0;
   if (pr.x == kInvalid) return false;
   uint64_t key = flip_key(it, pr.x);
-  bool win = M.fvote[pr.x] == key && M.fvote[pr.z] == key;
-  if (((pr.y >> 2) & 1u) && M.fvote[pr.w] != key) win = false;
+  bool win = FVOTE(M, pr.x) == key && FVOTE(M, pr.z) == key;
+  if (((pr.y >> 2) & 1u) && FVOTE(M, pr.w) != key) win = false;
   if (win) {
     uint32_t reuse[2] = {pr.x, pr.z};
     for (int k = 0; k < 2; ++k) {
@@ -665,14 +755,15 @@ WT_HD bool flip_decide_body(const Mesh& M, const uint4& pr, uint32_t it, uint32_
 // flip_decide_body for the list kernel: a winner also loads its flip's
 // tets (into F), issued after its queue claims so that the loads and the
 // claims' round trips overlap.  Same decisions and queue entries.
-WT_HD bool flip_decide_load(const Mesh& M, const uint4& pr, uint32_t it, uint32_t qid[2],
+template <class MS>
+WT_HD bool flip_decide_load(const MS& M, const uint4& pr, uint32_t it, uint32_t qid[2],
                             uint32_t* nq, uint32_t* nslot, FlipTets& F) {
   *nq = 0;
   *nslot = 0;
   if (pr.x == kInvalid) return false;
   uint64_t key = flip_key(it, pr.x);
-  bool win = M.fvote[pr.x] == key && M.fvote[pr.z] == key;
-  if (((pr.y >> 2) & 1u) && M.fvote[pr.w] != key) win = false;
+  bool win = FVOTE(M, pr.x) == key && FVOTE(M, pr.z) == key;
+  if (((pr.y >> 2) & 1u) && FVOTE(M, pr.w) != key) win = false;
   if (win) {
     uint32_t o0 = at_or_u32(&INFO(M, pr.x), kAlive | kQueued);
     uint32_t o1 = at_or_u32(&INFO(M, pr.z), kAlive | kQueued);
@@ -689,7 +780,8 @@ WT_HD bool flip_decide_load(const Mesh& M, const uint4& pr, uint32_t it, uint32_
 
 // Sequential form (one proposal at a time, host callers): counters advance
 // with one atomic each.
-WT_HD void flip_decide_exec_body(const Mesh& M, const uint4* prop, uint32_t j, uint32_t it,
+template <class MS>
+WT_HD void flip_decide_exec_body(const MS& M, const uint4* prop, uint32_t j, uint32_t it,
                                  uint32_t round, uint4* out, uint32_t* act_next) {
   uint4 pr = prop[j];
   uint32_t qid[2], nq, nslot;
@@ -711,7 +803,8 @@ WT_HD void flip_decide_exec_body(const Mesh& M, const uint4* prop, uint32_t j, u
 // stores a word that one of these loads reads (a flipped tet's external face
 // is rewritten only by its own flip, after the read; an unflipped
 // neighbour's face is never read; tags and messages are read-only here).
-WT_HD void flip_update_body(const Mesh& M, const uint4* out, uint32_t k, uint32_t it) {
+template <class MS>
+WT_HD void flip_update_body(const MS& M, const uint4* out, uint32_t k, uint32_t it) {
   uint4 r = out[2 * (size_t)k];
   uint4 w = out[2 * (size_t)k + 1];  // o, a, z
   // 2-3: new tets (x, y, o, a), external faces 2 (apex o) and 3 (apex a);
@@ -729,7 +822,7 @@ WT_HD void flip_update_body(const Mesh& M, const uint4* out, uint32_t k, uint32_
   // every neighbour is a valid slot: its message is loaded unconditionally
   // (stale where it did not flip, then unused), so no branch splits the loads
   for (int i = 0; i < 6; ++i)
-    msg[i] = reinterpret_cast<const uint2*>(&M.tmsg[opp_tet(ptr[i])])[opp_face(ptr[i])];
+    msg[i] = reinterpret_cast<const uint2*>(&TMSG(M, opp_tet(ptr[i])))[opp_face(ptr[i])];
   // one 8-byte store per face, its slot and value chosen without a branch
   for (int i = 0; i < 6; ++i) {
     bool fl = fq[i] == it;
@@ -746,8 +839,8 @@ WT_HD void flip_update_body(const Mesh& M, const uint4* out, uint32_t k, uint32_
 constexpr uint32_t kWalkLimit = 1u << 16;
 
 // *state: 0 arrived, 1 step limit, 2 deferred (FAST filter undecided)
-template <bool FAST>
-WT_HD uint32_t walk_to_t(const Mesh& M, uint32_t t, uint32_t q, uint32_t seed, PredStats* st,
+template <bool FAST, class MS>
+WT_HD uint32_t walk_to_t(const MS& M, uint32_t t, uint32_t q, uint32_t seed, PredStats* st,
                          int* state) {
   float Q[3];
   uint32_t rq;
@@ -787,8 +880,8 @@ WT_HD uint32_t walk_to_t(const Mesh& M, uint32_t t, uint32_t q, uint32_t seed, P
   return t;
 }
 
-template <bool FAST>
-WT_HD bool relocate_body_t(const Mesh& M, const uint32_t* uvert, uint32_t* utet, uint32_t i,
+template <bool FAST, class MS>
+WT_HD bool relocate_body_t(const MS& M, const uint32_t* uvert, uint32_t* utet, uint32_t i,
                            uint32_t round, PredStats* st) {
   uint32_t t = utet[i];
   if ((uint32_t)(FSTAMP(M, t) >> 32) != round) return false;
@@ -801,7 +894,8 @@ WT_HD bool relocate_body_t(const Mesh& M, const uint32_t* uvert, uint32_t* utet,
   return false;
 }
 
-WT_HD void relocate_body(const Mesh& M, const uint32_t* uvert, uint32_t* utet, uint32_t i,
+template <class MS>
+WT_HD void relocate_body(const MS& M, const uint32_t* uvert, uint32_t* utet, uint32_t i,
                          uint32_t round, PredStats* st) {
   (void)relocate_body_t<false>(M, uvert, utet, i, round, st);
 }
@@ -813,8 +907,8 @@ WT_HD void relocate_body(const Mesh& M, const uint32_t* uvert, uint32_t* utet, u
 // returns true (nothing recorded) when a face is undecided, for the full
 // pass to redo the tet.
 // ---------------------------------------------------------------------------
-template <bool FAST>
-WT_HD bool audit_body_t(const Mesh& M, uint32_t t, uint32_t* rec, uint32_t cap, PredStats* st) {
+template <bool FAST, class MS>
+WT_HD bool audit_body_t(const MS& M, uint32_t t, uint32_t* rec, uint32_t cap, PredStats* st) {
   if (!(INFO(M, t) & kAlive)) return false;
   uint4 tv = TV(M, t);
   if (tv.x == M.inf || tv.y == M.inf || tv.z == M.inf || tv.w == M.inf) return false;
@@ -845,7 +939,8 @@ WT_HD bool audit_body_t(const Mesh& M, uint32_t t, uint32_t* rec, uint32_t cap, 
   return false;
 }
 
-WT_HD void audit_body(const Mesh& M, uint32_t t, uint32_t* rec, uint32_t cap, PredStats* st) {
+template <class MS>
+WT_HD void audit_body(const MS& M, uint32_t t, uint32_t* rec, uint32_t cap, PredStats* st) {
   (void)audit_body_t<false>(M, t, rec, cap, st);
 }
 

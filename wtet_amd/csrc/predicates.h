@@ -612,6 +612,135 @@ WT_HD int insphere_f64(const float* a, const float* b, const float* c, const flo
 }
 
 // ---------------------------------------------------------------------------
+// The filters of the flip check: one tet against the vertices across its four
+// faces, and one face's three edge tests.  Shared work is done once -- the
+// insphere determinant is expanded along the query's row, so its cofactors
+// depend on the tet alone (about 70 operations and then 20 per face, where
+// insphere_f32 takes about 200 per face) -- and sums are fused multiply-adds,
+// which only drop roundings.  For coordinates of at most 2^9 in magnitude
+// (the normalized domain with the super vertices).
+//
+// Error bounds, u = 2^-24 (f32) or 2^-53 (f64), counting the roundings on the
+// longest path from an input to the result: a coordinate difference 1; a 2x2
+// minor 2 leaves + product + fused add = 4; a lift 2 leaves + 3 = 5; a cofactor
+// with lifts 5 + 4 + (product + two fused adds) = 12; the determinant leaf +
+// 12 + (product + three fused adds) = 17.  Each term of the expansion is then
+// off by at most a factor (1 + u)^17, so the determinant by 17.01 u times the
+// permanent (the same sum over absolute values), which is computed to a
+// factor (1 - 20 u); 18 u covers both.  The edge test: minor 4, leaf 1,
+// product and two fused adds 3 = 8, bound 9 u.
+// ---------------------------------------------------------------------------
+WT_HD float flt_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+WT_HD double flt_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+WT_HD float flt_abs(float a) { return __builtin_fabsf(a); }
+WT_HD double flt_abs(double a) { return __builtin_fabs(a); }
+
+// u_i v_j - u_j v_i and |u_i v_j| + |u_j v_i|
+template <typename T>
+WT_HD void minor2(T ui, T vj, T uj, T vi, T* m, T* p) {
+  T t = ui * vj;
+  *m = flt_fma(-uj, vi, t);
+  *p = flt_fma(flt_abs(uj), flt_abs(vi), flt_abs(t));
+}
+
+template <typename T>
+WT_HD T dot3(T a, T x, T b, T y, T c, T z) {
+  return flt_fma(c, z, flt_fma(b, y, a * x));
+}
+
+// cofactors of the query row (x, y, z, lift) relative to the tet's vertex o,
+// and their permanents
+template <typename T>
+struct InsphereTet {
+  T k[4], p[4];
+};
+
+// o: the tet's vertex taken as origin; b, c, d its others
+template <typename T>
+WT_HD InsphereTet<T> insphere_tet(const float* o, const float* b, const float* c, const float* d) {
+  T R[3][3], L[3];
+  const float* V[3] = {b, c, d};
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) R[r][k] = (T)V[r][k] - (T)o[k];
+    L[r] = dot3(R[r][0], R[r][0], R[r][1], R[r][1], R[r][2], R[r][2]);
+  }
+  InsphereTet<T> q;
+  // minors of rows (c, d), (d, b), (b, c) in columns (i, j)
+  T m[3], w[3];
+#define WT_MINORS(i, j)                                            \
+  minor2(R[1][i], R[2][j], R[1][j], R[2][i], &m[0], &w[0]);        \
+  minor2(R[2][i], R[0][j], R[2][j], R[0][i], &m[1], &w[1]);        \
+  minor2(R[0][i], R[1][j], R[0][j], R[1][i], &m[2], &w[2]);
+  WT_MINORS(1, 2)
+  q.k[0] = -dot3(L[0], m[0], L[1], m[1], L[2], m[2]);
+  q.p[0] = dot3(L[0], w[0], L[1], w[1], L[2], w[2]);
+  WT_MINORS(0, 2)
+  q.k[1] = dot3(L[0], m[0], L[1], m[1], L[2], m[2]);
+  q.p[1] = dot3(L[0], w[0], L[1], w[1], L[2], w[2]);
+  WT_MINORS(0, 1)
+  q.k[2] = -dot3(L[0], m[0], L[1], m[1], L[2], m[2]);
+  q.p[2] = dot3(L[0], w[0], L[1], w[1], L[2], w[2]);
+  q.k[3] = dot3(R[0][2], m[0], R[1][2], m[1], R[2][2], m[2]);
+  q.p[3] = dot3(flt_abs(R[0][2]), w[0], flt_abs(R[1][2]), w[1], flt_abs(R[2][2]), w[2]);
+#undef WT_MINORS
+  return q;
+}
+
+template <typename T>
+WT_HD void insphere_query(const InsphereTet<T>& q, const float* o, const float* e, T* det, T* perm) {
+  T x = (T)e[0] - (T)o[0], y = (T)e[1] - (T)o[1], z = (T)e[2] - (T)o[2];
+  T l = dot3(x, x, y, y, z, z);
+  *det = flt_fma(l, q.k[3], dot3(x, q.k[0], y, q.k[1], z, q.k[2]));
+  *perm = flt_fma(l, q.p[3], dot3(flt_abs(x), q.p[0], flt_abs(y), q.p[1], flt_abs(z), q.p[2]));
+}
+
+// insphere(o, b, c, d, e) from the tet's cofactors, 2 when undecided
+WT_HD int insphere_query_f32(const InsphereTet<float>& q, const float* o, const float* e) {
+  float det, perm;
+  insphere_query(q, o, e, &det, &perm);
+  const float kB = 1.0729e-06f;                // 18 * 2^-24, rounded up
+  if (!(perm >= 8.271806e-25f)) return 2;      // 2^-80: keep f32 underflow out
+  float eb = kB * perm + 7.7e-34f;             // + 2^-110
+  return det > eb ? 1 : (-det > eb ? -1 : 2);
+}
+WT_HD int insphere_query_f64(const InsphereTet<double>& q, const float* o, const float* e) {
+  double det, perm;
+  insphere_query(q, o, e, &det, &perm);
+  double eb = 2.0e-15 * perm;  // 18 * 2^-53, rounded up
+  return det > eb ? 1 : (-det > eb ? -1 : 2);
+}
+
+// orient3d of (x, y, a, o), (y, z, a, o) and (z, x, a, o), raw signs, 2 where
+// undecided
+WT_HD void orient3d_edges_f32(const float* x, const float* y, const float* z, const float* a,
+                              const float* o, int* s) {
+  float R[3][3], A[3];
+  const float* V[3] = {x, y, z};
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    A[k] = a[k] - o[k];
+#pragma unroll
+    for (int r = 0; r < 3; ++r) R[r][k] = V[r][k] - o[k];
+  }
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    const float *u = R[r], *w = R[(r + 1) % 3];
+    float m0, m1, m2, p0, p1, p2;
+    minor2(u[1], w[2], u[2], w[1], &m0, &p0);
+    minor2(u[2], w[0], u[0], w[2], &m1, &p1);
+    minor2(u[0], w[1], u[1], w[0], &m2, &p2);
+    float det = dot3(A[0], m0, A[1], m1, A[2], m2);
+    float perm = dot3(flt_abs(A[0]), p0, flt_abs(A[1]), p1, flt_abs(A[2]), p2);
+    const float kB = 5.3645e-07f;  // 9 * 2^-24, rounded up
+    float eb = kB * perm + 1.0e-36f;
+    // 2^-90: keep f32 underflow out
+    s[r] = !(perm >= 8.0e-28f) ? 2 : (det > eb ? 1 : (-det > eb ? -1 : 2));
+  }
+}
+
+// ---------------------------------------------------------------------------
 // FP64 adaptive stage for insphere: the same determinant in double-double
 // arithmetic (error-free products by fused multiply-add, Knuth's two-sum;
 // T. J. Dekker, Numer. Math. 18, 1971; Y. Hida, X. S. Li, D. H. Bailey,
