@@ -58,8 +58,8 @@ struct wtet_ctx {
   DevBuf uvert[2], utet[2], wlist, act[2], prop, fout, blk, slot2idx, rec;
   // output grouping for many clouds
   DevBuf ord[2], ord_tmp, cstart;
-  // learned presizing
-  DevBuf presize_params, feat_acc, feat, pred;
+  // learned presizing (mlp: the arena of the training calls)
+  DevBuf presize_params, feat_acc, feat, pred, mlp;
   bool presize_loaded = false;
   std::vector<float> h_pred;
   // device-driven flip iterations: sums (checked tets, flips, iterations),
@@ -136,7 +136,7 @@ struct wtet_ctx {
                    &tmsg,   &uvert[0], &uvert[1], &utet[0], &utet[1],
                    &wlist,  &act[0], &act[1], &prop,  &fout,   &blk,      &slot2idx, &rec,
                    &ord[0], &ord[1], &ord_tmp, &cstart, &ctr,  &gstats,   &patch,
-                   &presize_params, &feat_acc, &feat, &pred, &isums, &slow_t, &slow_p,
+                   &presize_params, &feat_acc, &feat, &pred, &mlp, &isums, &slow_t, &slow_p,
                    &nbr_mark, &nbr_list, &nbr_misc, &nbr_pack, &nbr_seed};
     all.assign(std::begin(l), std::end(l));
   }
@@ -2247,44 +2247,43 @@ static void predict_impl(void* a_) {
 }
 
 // device buffers of one training / gradient call
-struct MlpBufs {
-  DevBuf params, grad, m, v, xraw, yraw, idx, x, y, h1, h2, out, d3, d2, d1, loss;
-  std::vector<DevBuf*> all() {
-    return {&params, &grad, &m, &v, &xraw, &yraw, &idx, &x, &y, &h1, &h2, &out, &d3, &d2, &d1, &loss};
-  }
-  ~MlpBufs() {
-    for (DevBuf* b : all())
-      if (b->p) (void)hipFree(b->p);
-  }
+// Device memory of one training call, in the context's arena (kept between
+// calls; a call's data does not outlive it)
+struct MlpDev {
+  MlpWork w;
+  float *params, *grad, *m, *v, *feat, *tgt, *loss;
+  uint32_t* idx;
 };
 
-static MlpWork mlp_alloc(wtet_ctx* c, MlpBufs& B, uint32_t rows, uint32_t batch) {
-  ensure(c, B.params, kParamCount * 4);
-  ensure(c, B.grad, kParamCount * 4);
-  ensure(c, B.xraw, (size_t)rows * kFeat * 4);
-  ensure(c, B.yraw, (size_t)rows * kOut * 4);
-  ensure(c, B.idx, (size_t)std::max(rows, batch) * 4);
-  ensure(c, B.x, (size_t)batch * kFeat * 4);
-  ensure(c, B.y, (size_t)batch * kOut * 4);
-  ensure(c, B.h1, (size_t)batch * kHidden * 4);
-  ensure(c, B.h2, (size_t)batch * kHidden * 4);
-  ensure(c, B.out, (size_t)batch * kOut * 4);
-  ensure(c, B.d3, (size_t)batch * kOut * 4);
-  ensure(c, B.d2, (size_t)batch * kHidden * 4);
-  ensure(c, B.d1, (size_t)batch * kHidden * 4);
-  ensure(c, B.loss, 64);
-  MlpWork w;
-  w.x = P<float>(B.x);
-  w.y = P<float>(B.y);
-  w.h1 = P<float>(B.h1);
-  w.h2 = P<float>(B.h2);
-  w.out = P<float>(B.out);
-  w.d3 = P<float>(B.d3);
-  w.d2 = P<float>(B.d2);
-  w.d1 = P<float>(B.d1);
-  w.grad = P<float>(B.grad);
-  w.loss = P<float>(B.loss);
-  return w;
+// batch: rows of a minibatch; losses: loss slots
+static MlpDev mlp_alloc(wtet_ctx* c, uint32_t rows, uint32_t batch, uint32_t losses) {
+  MlpDev d;
+  for (int pass = 0; pass < 2; ++pass) {  // the size, then the pointers
+    char* base = pass ? P<char>(c->mlp) : nullptr;
+    size_t at = 0;
+    auto take = [&](auto*& p, size_t count) {
+      p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(base + at);
+      at += (count * 4 + 255) & ~(size_t)255;
+    };
+    take(d.params, kParamCount);
+    take(d.grad, kParamCount);
+    take(d.m, kParamCount);
+    take(d.v, kParamCount);
+    take(d.feat, (size_t)rows * kFeat);
+    take(d.tgt, (size_t)rows * kOut);
+    take(d.idx, rows);
+    take(d.loss, losses);
+    take(d.w.x, (size_t)batch * kFeat);
+    take(d.w.h1, (size_t)batch * kHidden);
+    take(d.w.h2, (size_t)batch * kHidden);
+    take(d.w.d3, (size_t)batch * kOut);
+    take(d.w.d2, (size_t)batch * kHidden);
+    take(d.w.d1, (size_t)batch * kHidden);
+    take(d.w.part, (size_t)mlp_slices(batch) * kTrainCount);
+    take(d.w.lpart, mlp_row_tiles(batch));
+    if (!pass) ensure(c, c->mlp, at);
+  }
+  return d;
 }
 
 struct GradArgs {
@@ -2302,24 +2301,16 @@ static void grad_impl(void* a_) {
   wtet_ctx* c = a.c;
   HIP_CHECK(hipSetDevice(c->device));
   hipStream_t s = c->stream;
-  MlpBufs B;
-  MlpWork w = mlp_alloc(c, B, a.rows, a.rows);
-  std::vector<uint32_t> idx(a.rows);
-  for (uint32_t i = 0; i < a.rows; ++i) idx[i] = i;
-  HIP_CHECK(hipMemcpyAsync(B.params.p, a.params, kParamCount * 4, hipMemcpyHostToDevice, s));
-  HIP_CHECK(hipMemcpyAsync(B.xraw.p, a.feat, (size_t)a.rows * kFeat * 4, hipMemcpyHostToDevice, s));
-  HIP_CHECK(hipMemcpyAsync(B.yraw.p, a.tgt, (size_t)a.rows * kOut * 4, hipMemcpyHostToDevice, s));
-  HIP_CHECK(hipMemcpyAsync(B.idx.p, idx.data(), (size_t)a.rows * 4, hipMemcpyHostToDevice, s));
-  launch_fill_u32(P<uint32_t>(B.grad), 0u, kParamCount, s);
-  const float* Pp = P<float>(B.params);
-  launch_gather_standardize(P<float>(B.xraw), P<uint32_t>(B.idx), a.rows, kFeat, Pp + kOffFeatMean,
-                            Pp + kOffFeatStd, w.x, s);
-  launch_gather_standardize(P<float>(B.yraw), P<uint32_t>(B.idx), a.rows, kOut, Pp + kOffTgtMean,
-                            Pp + kOffTgtStd, w.y, s);
-  launch_mlp_forward_backward(Pp, w, a.rows, s);
+  const MlpDev d = mlp_alloc(c, a.rows, a.rows, 1);
+  HIP_CHECK(hipMemcpyAsync(d.params, a.params, kParamCount * 4, hipMemcpyHostToDevice, s));
+  HIP_CHECK(hipMemcpyAsync(d.feat, a.feat, (size_t)a.rows * kFeat * 4, hipMemcpyHostToDevice, s));
+  HIP_CHECK(hipMemcpyAsync(d.tgt, a.tgt, (size_t)a.rows * kOut * 4, hipMemcpyHostToDevice, s));
+  launch_fill_u32(reinterpret_cast<uint32_t*>(d.grad), 0u, kParamCount, s);
+  launch_mlp_forward_backward(d.params, d.feat, d.tgt, nullptr, d.w, a.rows, s);
+  launch_mlp_gradient(d.w, a.rows, d.grad, d.loss, s);
   HIP_CHECK(hipGetLastError());
-  HIP_CHECK(hipMemcpyAsync(a.grad, B.grad.p, kParamCount * 4, hipMemcpyDeviceToHost, s));
-  HIP_CHECK(hipMemcpyAsync(a.loss, B.loss.p, 4, hipMemcpyDeviceToHost, s));
+  HIP_CHECK(hipMemcpyAsync(a.grad, d.grad, kParamCount * 4, hipMemcpyDeviceToHost, s));
+  HIP_CHECK(hipMemcpyAsync(a.loss, d.loss, 4, hipMemcpyDeviceToHost, s));
   HIP_CHECK(hipStreamSynchronize(s));
 }
 
@@ -2339,17 +2330,13 @@ static void train_impl(void* a_) {
   wtet_ctx* c = a.c;
   HIP_CHECK(hipSetDevice(c->device));
   hipStream_t s = c->stream;
-  MlpBufs B;
-  MlpWork w = mlp_alloc(c, B, a.rows, a.batch);
-  ensure(c, B.m, kParamCount * 4);
-  ensure(c, B.v, kParamCount * 4);
-  HIP_CHECK(hipMemcpyAsync(B.params.p, a.params, kParamCount * 4, hipMemcpyHostToDevice, s));
-  HIP_CHECK(hipMemcpyAsync(B.xraw.p, a.feat, (size_t)a.rows * kFeat * 4, hipMemcpyHostToDevice, s));
-  HIP_CHECK(hipMemcpyAsync(B.yraw.p, a.tgt, (size_t)a.rows * kOut * 4, hipMemcpyHostToDevice, s));
-  launch_fill_u32(P<uint32_t>(B.m), 0u, kParamCount, s);
-  launch_fill_u32(P<uint32_t>(B.v), 0u, kParamCount, s);
-  launch_fill_u32(P<uint32_t>(B.grad), 0u, kParamCount, s);
-  float* Pp = P<float>(B.params);
+  const uint32_t nb = a.rows / a.batch;
+  const MlpDev d = mlp_alloc(c, a.rows, a.batch, std::max<uint32_t>(nb, 1));
+  HIP_CHECK(hipMemcpyAsync(d.params, a.params, kParamCount * 4, hipMemcpyHostToDevice, s));
+  HIP_CHECK(hipMemcpyAsync(d.feat, a.feat, (size_t)a.rows * kFeat * 4, hipMemcpyHostToDevice, s));
+  HIP_CHECK(hipMemcpyAsync(d.tgt, a.tgt, (size_t)a.rows * kOut * 4, hipMemcpyHostToDevice, s));
+  launch_fill_u32(reinterpret_cast<uint32_t*>(d.m), 0u, kParamCount, s);
+  launch_fill_u32(reinterpret_cast<uint32_t*>(d.v), 0u, kParamCount, s);
   std::vector<uint32_t> perm(a.rows);
   std::vector<float> losses;
   uint64_t rng = a.seed * 0x9E3779B97F4A7C15ull + 1;
@@ -2359,34 +2346,27 @@ static void train_impl(void* a_) {
     rng ^= rng << 17;
     return rng;
   };
-  uint32_t nb = a.rows / a.batch;
-  ensure(c, B.loss, (size_t)std::max<uint32_t>(nb, 1) * 4 + 64);
   uint32_t step = 0;
   for (uint32_t e = 0; e < a.epochs; ++e) {
     for (uint32_t i = 0; i < a.rows; ++i) perm[i] = i;
     for (uint32_t i = a.rows - 1; i > 0; --i) std::swap(perm[i], perm[next() % (i + 1)]);
-    HIP_CHECK(hipMemcpyAsync(B.idx.p, perm.data(), (size_t)a.rows * 4, hipMemcpyHostToDevice, s));
+    HIP_CHECK(hipMemcpyAsync(d.idx, perm.data(), (size_t)a.rows * 4, hipMemcpyHostToDevice, s));
     for (uint32_t b = 0; b < nb; ++b) {
-      const uint32_t* bi = P<uint32_t>(B.idx) + (size_t)b * a.batch;
-      launch_gather_standardize(P<float>(B.xraw), bi, a.batch, kFeat, Pp + kOffFeatMean,
-                                Pp + kOffFeatStd, w.x, s);
-      launch_gather_standardize(P<float>(B.yraw), bi, a.batch, kOut, Pp + kOffTgtMean,
-                                Pp + kOffTgtStd, w.y, s);
-      w.loss = P<float>(B.loss) + b;  // one slot per minibatch of this epoch
-      launch_mlp_forward_backward(Pp, w, a.batch, s);
-      launch_adam(Pp, w.grad, P<float>(B.m), P<float>(B.v), a.lr, 0.9f, 0.999f, 1e-8f, ++step, s);
+      launch_mlp_forward_backward(d.params, d.feat, d.tgt, d.idx + (size_t)b * a.batch, d.w, a.batch, s);
+      // one loss slot per minibatch of this epoch
+      launch_mlp_adam(d.w, a.batch, d.params, d.m, d.v, a.lr, 0.9f, 0.999f, 1e-8f, ++step, d.loss + b, s);
     }
     HIP_CHECK(hipGetLastError());
     if (a.curve && nb) {
       losses.resize(nb);
-      HIP_CHECK(hipMemcpyAsync(losses.data(), B.loss.p, (size_t)nb * 4, hipMemcpyDeviceToHost, s));
+      HIP_CHECK(hipMemcpyAsync(losses.data(), d.loss, (size_t)nb * 4, hipMemcpyDeviceToHost, s));
       HIP_CHECK(hipStreamSynchronize(s));
       double sum = 0;
       for (float l : losses) sum += l;
       a.curve[e] = (float)(sum / nb);
     }
   }
-  HIP_CHECK(hipMemcpyAsync(a.params, B.params.p, kParamCount * 4, hipMemcpyDeviceToHost, s));
+  HIP_CHECK(hipMemcpyAsync(a.params, d.params, kParamCount * 4, hipMemcpyDeviceToHost, s));
   HIP_CHECK(hipStreamSynchronize(s));
 }
 

@@ -51,26 +51,35 @@ void launch_features(const float* xyz, uint32_t n, const uint32_t* off, uint32_t
 void launch_mlp_predict(const float* params, const float* feat, uint32_t C, float* pred,
                         hipStream_t s);
 
-// Training pieces (minibatch of B rows, standardized inputs and targets).
+// Training on a minibatch of B rows (mlp.hip): one kernel for what is local to
+// a row (standardization, forward pass, loss, deltas), one for the weight
+// gradients as partial sums over slices of kGradSlice rows, and one that adds
+// the slices up.
+constexpr int kRowTile = 16;      // rows a workgroup takes through the network
+constexpr uint32_t kGradSlice = 256;
+constexpr size_t kTrainCount = kTrainEnd - kTrainBegin;
+
 struct MlpWork {
-  float* x;    // B * kFeat (standardized features)
-  float* y;    // B * kOut  (standardized targets)
-  float* h1;   // B * kHidden (post-ReLU)
-  float* h2;   // B * kHidden
-  float* out;  // B * kOut
-  float* d3;   // B * kOut
-  float* d2;   // B * kHidden
-  float* d1;   // B * kHidden
-  float* grad; // kParamCount (only the trainable range is written)
-  float* loss; // 1
+  float* x;     // B * kFeat (standardized features)
+  float* h1;    // B * kHidden (post-ReLU)
+  float* h2;    // B * kHidden
+  float* d3;    // B * kOut
+  float* d2;    // B * kHidden
+  float* d1;    // B * kHidden
+  float* part;  // mlp_slices(B) * kTrainCount: gradient slices
+  float* lpart; // mlp_row_tiles(B): squared error of each row tile
 };
-// forward + MSE loss + backward into w.grad (trainable range)
-void launch_mlp_forward_backward(const float* params, const MlpWork& w, uint32_t B, hipStream_t s);
-// Adam step on the trainable range
-void launch_adam(float* params, const float* grad, float* m, float* v, float lr, float b1,
-                 float b2, float eps, uint32_t step, hipStream_t s);
-// standardize rows: x = (raw - mean) / std, gathering rows idx[0..B)
-void launch_gather_standardize(const float* raw, const uint32_t* idx, uint32_t B, int width,
-                               const float* mean, const float* stdv, float* out, hipStream_t s);
+inline uint32_t mlp_row_tiles(uint32_t B) { return (B + kRowTile - 1) / kRowTile; }
+inline uint32_t mlp_slices(uint32_t B) { return (B + kGradSlice - 1) / kGradSlice; }
+
+// rows idx[0..B) (null: 0..B-1) of the raw features and targets: forward pass,
+// MSE loss and backward pass into w.part and w.lpart
+void launch_mlp_forward_backward(const float* params, const float* feat, const float* tgt, const uint32_t* idx,
+                                 const MlpWork& w, uint32_t B, hipStream_t s);
+// the gradient (trainable range of grad) and the loss
+void launch_mlp_gradient(const MlpWork& w, uint32_t B, float* grad, float* loss, hipStream_t s);
+// the loss, and an Adam step on the trainable range with the gradient
+void launch_mlp_adam(const MlpWork& w, uint32_t B, float* params, float* m, float* v, float lr, float b1,
+                     float b2, float eps, uint32_t step, float* loss, hipStream_t s);
 
 }  // namespace wtet
