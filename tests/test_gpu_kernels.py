@@ -37,3 +37,23 @@ def test_gradient_row_tiles_and_slices(ctx, rows):
     assert loss == pytest.approx(lref, rel=1e-4)
     scale = np.abs(gref).max()
     assert np.abs(g - gref).max() <= 1e-4 * scale, np.abs(g - gref).max() / scale
+
+
+# one workgroup up to 4,096 pairs, tiles of 1,024 below 192 * 4,096 pairs, of 4,096 from there
+@pytest.mark.parametrize("n", [4095, 4096, 4097, 5120, 5121, 192 * 4096 - 1, 192 * 4096, 193 * 4096 + 1])
+@pytest.mark.parametrize("bits", [32, 64])
+def test_sort_tile_sizes(ctx, n, bits):
+    """Stable order of few distinct keys and of random ones, whole and partial bit ranges."""
+    rng = np.random.default_rng(n + bits)
+    dt = np.uint64 if bits == 64 else np.uint32
+    for keys, end in ((rng.integers(0, 7, n).astype(dt), 3), (rng.integers(0, 1 << (bits - 1), n).astype(dt), bits - 3)):
+        d = [ctx.upload(a) for a in (keys, np.arange(n, dtype=np.uint32), np.zeros_like(keys), np.zeros(n, np.uint32))]
+        try:
+            ctx.sort_pairs(d[0], d[1], d[2], d[3], n, bits, end)
+            got = ctx.download(d[3], (n,), np.uint32)
+            gk = ctx.download(d[2], (n,), dt)
+        finally:
+            for p in d:
+                ctx.free(p)
+        order = np.argsort(keys & dt((1 << end) - 1), kind="stable")
+        assert np.array_equal(got, order.astype(np.uint32)) and np.array_equal(gk, keys[order])

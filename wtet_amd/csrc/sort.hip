@@ -1,17 +1,25 @@
 // Stable LSD radix sort of (key, value) pairs, 8-bit digits (sort.h).
 //
-// Per pass, over tiles of 2048 pairs (256 threads x 8):
-//  * k_radix_up: each tile's digit counts, from wave64 ballots (the lanes
-//    with this lane's digit) so that one LDS atomic per distinct digit per
-//    wave is issued, stored digit-major (counts[d * tiles + tile]);
+// Per pass, over tiles of pairs:
+//  * k_radix_up: each tile's digit counts (LDS atomics), digit-major
+//    (counts[d * tiles + tile]);
 //  * k_radix_scan: one workgroup per digit turns its row into global
 //    offsets: the pairs of smaller digits (from the all-pass histogram that
 //    k_radix_hist builds once, before the first pass) plus the exclusive
 //    prefix over earlier tiles;
-//  * k_radix_down: each tile ranks its pairs stably (slab by slab in index
-//    order: the wave's ballot rank, the earlier waves' counts, the earlier
-//    slabs' counts) and scatters them to their offsets.
-// Equal digits keep their order in every pass, so the whole sort is stable.
+//  * k_radix_down: each tile ranks its pairs stably, sorts them by digit in
+//    LDS and writes each digit's run to its place.
+// Ranks need no workgroup barrier: a wave owns a contiguous part of the tile
+// and its own row of digit counters, and ranks 64 pairs at a time with wave
+// ballots.  At most kSmallTile pairs are sorted by one workgroup in one
+// launch (k_radix_small).  Equal digits keep their order in every pass, so
+// the whole sort is stable.
+//
+// What bounds it: pass for pass 32 bytes a pair (key read twice, value read
+// once, both written).  4M pairs of 63-bit keys: 720 us with per-slab
+// barriers and a scatter straight from registers (8 passes of 56 + 15 us,
+// histogram 86 us), 359 us now (27 + 8, 31).  4,000
+// pairs: 26 launches of about 4 us each before, 51 us in one now.
 #include "sort.h"
 
 #include <algorithm>
@@ -20,17 +28,24 @@ namespace wtet {
 
 namespace {
 
-constexpr int kSortThreads = 256;
-constexpr int kSortItems = 8;
-constexpr uint32_t kTile = kSortThreads * kSortItems;
+constexpr int kSortThreads = 256;  // histogram, upsweep and scan
 constexpr int kDigitBits = 8;
 constexpr int kRadix = 1 << kDigitBits;
 constexpr int kMaxPasses = 8;
 constexpr int kWaves = kSortThreads / 64;
 static_assert(kSortThreads == kRadix, "one thread per digit in the per-digit steps");
 
+// Tiles: 4,096 pairs (runs of 16 a digit on average, 128 bytes of 64-bit
+// keys) where that gives most CUs one, 1,024 below.  63-bit keys, 1,024
+// against 4,096 a tile: 300k pairs 142 and 156 us, 500k 154 and 163, 1M 202
+// and 180.
+constexpr uint32_t kBigTile = 4096, kLittleTile = 1024;
+constexpr uint32_t kBigFrom = 192 * kBigTile;
+constexpr uint32_t kSmallTile = 4096;
+
 inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
-inline uint32_t tiles_of(uint32_t n) { return (n + kTile - 1) / kTile; }
+inline uint32_t tile_of(uint32_t n) { return n >= kBigFrom ? kBigTile : kLittleTile; }
+inline uint32_t tiles_of(uint32_t n) { return (n + tile_of(n) - 1) / tile_of(n); }
 __host__ __device__ inline int passes_of(int end_bit) { return (end_bit + kDigitBits - 1) / kDigitBits; }
 
 __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
@@ -77,20 +92,12 @@ __global__ void __launch_bounds__(kSortThreads) k_radix_hist(const K* keys, uint
   const int P = passes_of(end_bit);
   for (int i = threadIdx.x; i < P * kRadix; i += kSortThreads) lh[i] = 0u;
   __syncthreads();
-  const uint32_t lane = lane_id();
-  // the loop bound depends on the block only, so every lane of a wave takes
-  // part in each ballot
-  for (uint32_t base = blockIdx.x * kSortThreads; base < n; base += gridDim.x * kSortThreads) {
-    uint32_t i = base + threadIdx.x;
-    bool valid = i < n;
-    K key = valid ? keys[i] : (K)0;
+  for (uint32_t i = blockIdx.x * kSortThreads + threadIdx.x; i < n; i += gridDim.x * kSortThreads) {
+    const K key = keys[i];
     for (int p = 0; p < P; ++p) {
       int shift = p * kDigitBits;
       int bits = min(kDigitBits, end_bit - shift);
-      uint32_t d = digit_of(key, shift, (1u << bits) - 1u);
-      uint64_t peers = peer_mask(d, valid);
-      if (valid && (uint32_t)__builtin_ctzll(peers) == lane)
-        atomicAdd(&lh[p * kRadix + d], (uint32_t)__popcll(peers));
+      atomicAdd(&lh[p * kRadix + digit_of(key, shift, (1u << bits) - 1u)], 1u);
     }
   }
   __syncthreads();
@@ -98,29 +105,24 @@ __global__ void __launch_bounds__(kSortThreads) k_radix_hist(const K* keys, uint
     if (lh[i]) atomicAdd(&ghist[i], lh[i]);
 }
 
-template <typename K>
+template <typename K, int ITEMS>
 __global__ void __launch_bounds__(kSortThreads) k_radix_up(const K* keys, uint32_t n, int shift,
                                                            uint32_t mask, uint32_t tiles,
                                                            uint32_t* counts) {
   __shared__ uint32_t cnt[kRadix];
-  const uint32_t t = threadIdx.x, lane = lane_id();
-  const uint32_t base = blockIdx.x * kTile;
+  const uint32_t t = threadIdx.x;
+  const uint32_t base = blockIdx.x * (kSortThreads * ITEMS);
   cnt[t] = 0u;
-  K kk[kSortItems];
+  K kk[ITEMS];
 #pragma unroll
-  for (int k = 0; k < kSortItems; ++k) {
+  for (int k = 0; k < ITEMS; ++k) {
     uint32_t i = base + (uint32_t)k * kSortThreads + t;
     kk[k] = i < n ? keys[i] : (K)0;
   }
   __syncthreads();
 #pragma unroll
-  for (int k = 0; k < kSortItems; ++k) {
-    uint32_t i = base + (uint32_t)k * kSortThreads + t;
-    bool valid = i < n;
-    uint32_t d = valid ? digit_of(kk[k], shift, mask) : 0u;
-    uint64_t peers = peer_mask(d, valid);
-    if (valid && (uint32_t)__builtin_ctzll(peers) == lane) atomicAdd(&cnt[d], (uint32_t)__popcll(peers));
-  }
+  for (int k = 0; k < ITEMS; ++k)
+    if (base + (uint32_t)k * kSortThreads + t < n) atomicAdd(&cnt[digit_of(kk[k], shift, mask)], 1u);
   __syncthreads();
   counts[(size_t)t * tiles + blockIdx.x] = cnt[t];
 }
@@ -167,58 +169,133 @@ __global__ void __launch_bounds__(kSortThreads) k_radix_scan(const uint32_t* his
   }
 }
 
-template <typename K>
-__global__ void __launch_bounds__(kSortThreads) k_radix_down(const K* kin, const uint32_t* vin, K* kout,
-                                                             uint32_t* vout, uint32_t n, int shift,
-                                                             uint32_t mask, uint32_t tiles,
-                                                             const uint32_t* offs) {
-  __shared__ uint32_t goff[kRadix];
-  __shared__ uint32_t run[kRadix];
-  __shared__ uint32_t wc[kWaves][kRadix];
-  const uint32_t t = threadIdx.x, lane = lane_id(), wave = t >> 6;
-  const uint32_t base = blockIdx.x * kTile;
-  goff[t] = offs[(size_t)t * tiles + blockIdx.x];
-  run[t] = 0u;
-  K kk[kSortItems];
-  uint32_t vv[kSortItems];
-#pragma unroll
-  for (int k = 0; k < kSortItems; ++k) {
-    uint32_t i = base + (uint32_t)k * kSortThreads + t;
-    bool valid = i < n;
-    kk[k] = valid ? kin[i] : (K)0;
-    vv[k] = valid ? vin[i] : 0u;
-  }
-  const uint64_t lt = (1ull << lane) - 1ull;
-#pragma unroll
-  for (int k = 0; k < kSortItems; ++k) {
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) wc[w][t] = 0u;
+// A tile of T * I pairs in registers -- wave w holds pairs [64 I w, 64 I (w + 1)),
+// 64 at a time -- sorted by one digit into LDS.
+template <typename K, int T, int I>
+struct TileSort {
+  static constexpr int kW = T / 64;
+  K key[T * I];
+  uint32_t val[T * I];
+  uint32_t wc[kW][kRadix];  // per wave: pairs of a digit so far, then its offset in the digit
+  uint32_t dstart[kRadix];  // first pair of a digit in the tile
+  uint32_t ws[4];
+
+  __device__ void sort(const K* kk, const uint32_t* vv, uint32_t count, int shift, uint32_t mask) {
+    const uint32_t t = threadIdx.x, lane = lane_id(), wave = t >> 6;
+    const uint64_t lt = (1ull << lane) - 1ull;
+    for (uint32_t i = t; i < (uint32_t)kW * kRadix; i += T) (&wc[0][0])[i] = 0u;
     __syncthreads();
-    uint32_t i = base + (uint32_t)k * kSortThreads + t;
-    bool valid = i < n;
-    uint32_t d = valid ? digit_of(kk[k], shift, mask) : 0u;
-    uint64_t peers = peer_mask(d, valid);
-    uint32_t wr = (uint32_t)__popcll(peers & lt);
-    if (valid && (uint32_t)__builtin_ctzll(peers) == lane) wc[wave][d] = (uint32_t)__popcll(peers);
-    __syncthreads();
-    // thread t: digit t's slab counts -> the offsets of each wave's run
-    {
-      uint32_t x = run[t];
+    uint32_t rank[I];
 #pragma unroll
-      for (int w = 0; w < kWaves; ++w) {
-        uint32_t y = wc[w][t];
-        wc[w][t] = x;
-        x += y;
+    for (int k = 0; k < I; ++k) {
+      const bool valid = wave * 64u * I + (uint32_t)k * 64u + lane < count;
+      const uint32_t d = valid ? digit_of(kk[k], shift, mask) : 0u;
+      const uint64_t peers = peer_mask(d, valid);
+      // the wave's own counters: its LDS operations complete in order
+      const uint32_t pre = __hip_atomic_load(&wc[wave][d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      rank[k] = pre + (uint32_t)__popcll(peers & lt);
+      if (valid && (uint32_t)__builtin_ctzll(peers) == lane)
+        __hip_atomic_store(&wc[wave][d], pre + (uint32_t)__popcll(peers), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_WORKGROUP);
+      __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    // thread d: each wave's offset within digit d, and the digit's first place
+    uint32_t total = 0, incl = 0;
+    if (t < (uint32_t)kRadix) {
+#pragma unroll
+      for (int w = 0; w < kW; ++w) {
+        const uint32_t y = wc[w][t];
+        wc[w][t] = total;
+        total += y;
       }
-      run[t] = x;
+      incl = wave_incl_scan(total);
+      if (lane == 63) ws[wave] = incl;
     }
     __syncthreads();
-    if (valid) {
-      uint32_t pos = goff[d] + wc[wave][d] + wr;
-      kout[pos] = kk[k];
-      vout[pos] = vv[k];
+    if (t < (uint32_t)kRadix) {
+      uint32_t before = 0;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) before += (uint32_t)w < wave ? ws[w] : 0u;
+      dstart[t] = before + incl - total;
     }
-    __syncthreads();  // wc is cleared by the next slab
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < I; ++k) {
+      if (wave * 64u * I + (uint32_t)k * 64u + lane >= count) continue;
+      const uint32_t d = digit_of(kk[k], shift, mask);
+      const uint32_t p = dstart[d] + wc[wave][d] + rank[k];
+      key[p] = kk[k];
+      val[p] = vv[k];
+    }
+    __syncthreads();
+  }
+};
+
+template <typename K, int T, int I>
+__global__ void __launch_bounds__(T) k_radix_down(const K* kin, const uint32_t* vin, K* kout, uint32_t* vout,
+                                                  uint32_t n, int shift, uint32_t mask, uint32_t tiles,
+                                                  const uint32_t* offs) {
+  __shared__ TileSort<K, T, I> sh;
+  __shared__ uint32_t goff[kRadix];
+  const uint32_t t = threadIdx.x, lane = lane_id(), wave = t >> 6;
+  const uint32_t base = blockIdx.x * (uint32_t)(T * I), count = min(n - base, (uint32_t)(T * I));
+  K kk[I];
+  uint32_t vv[I];
+#pragma unroll
+  for (int k = 0; k < I; ++k) {
+    const uint32_t i = wave * 64u * I + (uint32_t)k * 64u + lane;
+    kk[k] = i < count ? kin[base + i] : (K)0;
+    vv[k] = i < count ? vin[base + i] : 0u;
+  }
+  if (t < (uint32_t)kRadix) goff[t] = offs[(size_t)t * tiles + blockIdx.x];
+  sh.sort(kk, vv, count, shift, mask);
+#pragma unroll
+  for (int k = 0; k < I; ++k) {
+    const uint32_t p = (uint32_t)k * T + t;
+    if (p >= count) continue;
+    const K key = sh.key[p];
+    const uint32_t d = digit_of(key, shift, mask);
+    const uint32_t pos = goff[d] + (p - sh.dstart[d]);
+    kout[pos] = key;
+    vout[pos] = sh.val[p];
+  }
+}
+
+// every pass of at most kSmallTile pairs in one workgroup
+template <typename K>
+__global__ void __launch_bounds__(512) k_radix_small(const K* kin, const uint32_t* vin, K* kout, uint32_t* vout,
+                                                     uint32_t n, int end_bit) {
+  constexpr int T = 512, I = (int)kSmallTile / T;
+  __shared__ TileSort<K, T, I> sh;
+  const uint32_t lane = lane_id(), wave = threadIdx.x >> 6;
+  K kk[I];
+  uint32_t vv[I];
+#pragma unroll
+  for (int k = 0; k < I; ++k) {
+    const uint32_t i = wave * 64u * I + (uint32_t)k * 64u + lane;
+    kk[k] = i < n ? kin[i] : (K)0;
+    vv[k] = i < n ? vin[i] : 0u;
+  }
+  for (int shift = 0; shift < end_bit; shift += kDigitBits) {
+    sh.sort(kk, vv, n, shift, (1u << min(kDigitBits, end_bit - shift)) - 1u);
+#pragma unroll
+    for (int k = 0; k < I; ++k) {
+      const uint32_t i = wave * 64u * I + (uint32_t)k * 64u + lane;
+      if (i < n) {
+        kk[k] = sh.key[i];
+        vv[k] = sh.val[i];
+      }
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int k = 0; k < I; ++k) {
+    const uint32_t i = wave * 64u * I + (uint32_t)k * 64u + lane;
+    if (i < n) {
+      kout[i] = kk[k];
+      vout[i] = vv[k];
+    }
   }
 }
 
@@ -242,7 +319,12 @@ hipError_t sort_t(const K* kin, const uint32_t* vin, K* kout, uint32_t* vout, ui
     if (e != hipSuccess) return e;
     return hipMemcpyAsync(vout, vin, (size_t)n * 4, hipMemcpyDeviceToDevice, s);
   }
+  if (n <= kSmallTile) {
+    k_radix_small<K><<<1, 512, 0, s>>>(kin, vin, kout, vout, n, end_bit);
+    return hipGetLastError();
+  }
   const uint32_t tiles = tiles_of(n);
+  const bool big = tile_of(n) == kBigTile;
   char* tp = static_cast<char*>(temp);
   uint32_t* hist = reinterpret_cast<uint32_t*>(tp);
   tp += align256((size_t)kMaxPasses * kRadix * 4);
@@ -252,7 +334,7 @@ hipError_t sort_t(const K* kin, const uint32_t* vin, K* kout, uint32_t* vout, ui
   tp += align256((size_t)n * sizeof(K));
   uint32_t* valt = reinterpret_cast<uint32_t*>(tp);
   k_radix_zero<<<(P * kRadix + 255) / 256, 256, 0, s>>>(hist, (uint32_t)(P * kRadix));
-  uint32_t hgrid = std::min<uint32_t>(1024u, (n + kSortThreads - 1) / kSortThreads);
+  uint32_t hgrid = std::min<uint32_t>(256u, (n + kSortThreads - 1) / kSortThreads);
   k_radix_hist<K><<<hgrid, kSortThreads, 0, s>>>(kin, n, end_bit, hist);
   const K* ksrc = kin;
   const uint32_t* vsrc = vin;
@@ -264,9 +346,11 @@ hipError_t sort_t(const K* kin, const uint32_t* vin, K* kout, uint32_t* vout, ui
     int shift = p * kDigitBits;
     int bits = std::min(kDigitBits, end_bit - shift);
     uint32_t mask = (1u << bits) - 1u;
-    k_radix_up<K><<<tiles, kSortThreads, 0, s>>>(ksrc, n, shift, mask, tiles, counts);
+    if (big) k_radix_up<K, kBigTile / kSortThreads><<<tiles, kSortThreads, 0, s>>>(ksrc, n, shift, mask, tiles, counts);
+    else k_radix_up<K, kLittleTile / kSortThreads><<<tiles, kSortThreads, 0, s>>>(ksrc, n, shift, mask, tiles, counts);
     k_radix_scan<<<kRadix, kSortThreads, 0, s>>>(hist + p * kRadix, tiles, counts);
-    k_radix_down<K><<<tiles, kSortThreads, 0, s>>>(ksrc, vsrc, kd, vd, n, shift, mask, tiles, counts);
+    if (big) k_radix_down<K, 512, kBigTile / 512><<<tiles, 512, 0, s>>>(ksrc, vsrc, kd, vd, n, shift, mask, tiles, counts);
+    else k_radix_down<K, 256, kLittleTile / 256><<<tiles, 256, 0, s>>>(ksrc, vsrc, kd, vd, n, shift, mask, tiles, counts);
     ksrc = kd;
     vsrc = vd;
   }
