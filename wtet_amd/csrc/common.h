@@ -90,6 +90,24 @@ WT_HD uint32_t at_and_u32(uint32_t* p, uint32_t v) {
 #endif
 }
 
+// the same at workgroup scope, for data that one workgroup owns while it
+// runs: performed in the XCD's L2, not at the memory side
+WT_HD void wg_min_u64(uint64_t* p, uint64_t v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  (void)__hip_atomic_fetch_min((unsigned long long*)p, (unsigned long long)v, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WORKGROUP);
+#else
+  (void)__atomic_fetch_min(p, v, __ATOMIC_RELAXED);
+#endif
+}
+WT_HD uint32_t wg_or_u32(uint32_t* p, uint32_t v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __hip_atomic_fetch_or(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+#else
+  return __atomic_fetch_or(p, v, __ATOMIC_RELAXED);
+#endif
+}
+
 // Append to a list with one atomic per wavefront: the active lanes that call
 // this together get consecutive slots.
 WT_HD uint32_t append_slot(uint32_t* counter) {

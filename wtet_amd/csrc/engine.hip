@@ -370,7 +370,7 @@ Mesh mesh_of(wtet_ctx* c, uint32_t inf, int mode) {
 }
 
 void read_ctr(wtet_ctx* c) {
-  HIP_CHECK(hipMemcpyAsync(c->h_ctr, c->ctr.p, C_COUNT * 4, hipMemcpyDeviceToHost, c->stream));
+  HIP_CHECK(hipMemcpyAsync(c->h_ctr, c->ctr.p, C_HEAD * 4, hipMemcpyDeviceToHost, c->stream));
   HIP_CHECK(hipStreamSynchronize(c->stream));
 }
 
@@ -394,20 +394,26 @@ FlipLists lists_of(wtet_ctx* c) {
   return L;
 }
 
+// The iterations of a batch of k, between launch_batch_begin and _end.
+// sparse: the full check of deferred tets runs in the first iteration only;
+// later ones leave such tets in the active list.
 void enqueue_flip_iterations(wtet_ctx* c, const Mesh& M, const FlipLists& L, uint64_t* st, int k,
-                             uint32_t grid, uint32_t dgrid) {
+                             uint32_t grid, uint32_t dgrid, bool sparse) {
   hipStream_t s = c->stream;
-  uint64_t* sums = P<uint64_t>(c->isums);
-  launch_iter_begin(M.ctr, s);
   for (int i = 0; i < k; ++i) {
-    timed(c, K_FLIP_CHECK, [&] { launch_flip_check(M, L, grid, st, s); });
-    timed(c, K_FLIP_CHECK_DEFERRED, [&] { launch_flip_check_deferred(M, L, dgrid, st, s); });
-    timed(c, K_FLIP_EXEC, [&] { launch_flip_decide_exec(M, L, grid, s); });
-    timed(c, K_FLIP_UPDATE, [&] { launch_flip_update(M, L, grid, s); });
-    if (i + 1 < k) launch_iter_step(M.ctr, sums, s);
-    else launch_iter_end(M.ctr, sums, s);
+    const bool requeue = sparse && i > 0;
+    timed(c, K_FLIP_CHECK, [&] { launch_flip_check(M, L, i, requeue, grid, st, s); });
+    if (!requeue) timed(c, K_FLIP_CHECK_DEFERRED, [&] { launch_flip_check_deferred(M, L, i, dgrid, st, s); });
+    timed(c, K_FLIP_EXEC, [&] { launch_flip_decide_exec(M, L, i, grid, s); });
+    timed(c, K_FLIP_UPDATE, [&] { launch_flip_update(M, L, i, grid, s); });
   }
 }
+
+// Deferred tets per iteration (as the previous round had them) up to which
+// the full check runs once a round.  Its launch takes 4 to 5 us however few
+// tets it finds, 160 to 280 times a triangulation; points in general position
+// defer a handful a round.
+constexpr uint64_t kSparseDeferred = 64;
 
 // persistent grid for a list of about `a` entries: a power of two of
 // workgroups in [lo, 4096]
@@ -518,14 +524,18 @@ void run_flip_batch(wtet_ctx* c, uint32_t inf, int mode, uint64_t* st, int k, ui
   }
   uint32_t grid = grid_for(c, a_hint, 16);
   uint32_t dgrid = deferred_grid(c, d_hint, grid);
+  auto enqueue = [&] {
+    launch_batch_begin(M.ctr, k, c->stream);
+    enqueue_flip_iterations(c, M, L, st, k, grid, dgrid, false);
+    launch_batch_end(M.ctr, P<uint64_t>(c->isums), k, c->stream);
+  };
   if (!c->use_graphs || c->profiling) {
     if (c->evused > 4096) collect_times(c);
-    enqueue_flip_iterations(c, M, L, st, k, grid, dgrid);
+    enqueue();
     HIP_CHECK(hipGetLastError());
     return;
   }
-  launch_cached_graph(c, c->graphs, buffer_key(c, M, L, st), {(uint64_t)dgrid, (uint64_t)grid, (uint64_t)k},
-                      [&] { enqueue_flip_iterations(c, M, L, st, k, grid, dgrid); });
+  launch_cached_graph(c, c->graphs, buffer_key(c, M, L, st), {(uint64_t)dgrid, (uint64_t)grid, (uint64_t)k}, enqueue);
 }
 
 // tet slots after growth by `need`; the flip iterations read the capacity
@@ -737,7 +747,8 @@ void after_pick(wtet_ctx* c, Run& R, uint32_t U) {
   uint32_t W = c->h_ctr[C_WIN];
   if (c->h_ctr[C_BADTET]) throw Fail{WTET_ERR_INTERNAL, "a point was located outside the super tet"};
   if (W == 0) throw Fail{WTET_ERR_INTERNAL, "no insertion possible in a round"};
-  uint64_t need = (uint64_t)c->h_ctr[C_TETS] + 64 + (c->h_ctr[C_STOP] ? c->h_ctr[C_A] : 0u);
+  // the winners' slots, which the split takes
+  uint64_t need = (uint64_t)c->h_ctr[C_TETS] + 3ull * W + 64 + (c->h_ctr[C_STOP] ? c->h_ctr[C_LIST] : 0u);
   if (need > c->cap_tets || c->h_ctr[C_STOP]) grow_for(c, need);
   R.K.sumU += U;
   R.K.rounds++;
@@ -755,7 +766,7 @@ uint32_t dev_vote(wtet_ctx* c, Run& R) {
   if (R.round > (1u << 16)) throw Fail{WTET_ERR_NOT_CONVERGED, "insertion did not finish"};
   Mesh M = mesh_of(c, R.V, R.mode);
   const uint32_t U = R.U, cur = R.cur, round = R.round;
-  launch_set_ctr(M.ctr, C_ULEN, U, C_ROUND, round, s);
+  launch_set_ctr(M.ctr, C_SURV, U, C_ROUND, round - 1u, s);  // the pick begins the round
   timed(c, K_VOTE, [&] { launch_vote(M, P<uint32_t>(c->uvert[cur]), P<uint32_t>(c->utet[cur]), U, s); });
   timed(c, K_PICK, [&] {
     launch_pick(M, P<uint32_t>(c->uvert[cur]), P<uint32_t>(c->utet[cur]), U, P<uint2>(c->wlist),
@@ -780,7 +791,7 @@ void dev_split_points(wtet_ctx* c, Run& R) {
   Mesh M = mesh_of(c, R.V, R.mode);
   timed(c, K_SPLIT_POINTS, [&] {
     launch_split_points(M, P<uint32_t>(c->uvert[R.cur]), P<uint32_t>(c->utet[R.cur]), R.U, R.st,
-                        P<uint32_t>(c->slow_p), c->stream);
+                        P<uint32_t>(c->slow_p), 0, c->stream);
   });
   HIP_CHECK(hipGetLastError());
 }
@@ -792,16 +803,17 @@ void dev_round_flips(wtet_ctx* c, Run& R) {
   uint64_t dsum = c->h_ctr[C_SLOW_SUM];
   uint64_t dper = (2 * (dsum - R.dsum_prev) + R.max_fi - 1) / (uint64_t)R.max_fi;
   R.dsum_prev = dsum;
-  run_flip_batch(c, R.V, R.mode, R.st, R.max_fi, (uint64_t)c->h_ctr[C_A] + 4ull * R.W, dper);
+  run_flip_batch(c, R.V, R.mode, R.st, R.max_fi, (uint64_t)c->h_ctr[C_LIST] + 4ull * R.W, dper);
 }
 
 // uninserted points of flipped tets to their new tets (relocate_points_fast.wgsl)
 void dev_relocate(wtet_ctx* c, Run& R) {
   if (R.U == 0) return;
   Mesh M = mesh_of(c, R.V, R.mode);
+  launch_set_ctr(M.ctr, C_SLOW_R, 0u, -1, 0u, c->stream);  // a caller may relocate again before the next split
   timed(c, K_RELOCATE, [&] {
     launch_relocate(M, P<uint32_t>(c->uvert[R.cur]), P<uint32_t>(c->utet[R.cur]), R.U, R.st,
-                    P<uint32_t>(c->slow_p), c->stream);
+                    P<uint32_t>(c->slow_p), nullptr, 0, c->stream);
   });
   HIP_CHECK(hipGetLastError());
 }
@@ -824,7 +836,7 @@ void run_round(wtet_ctx* c, Run& R, bool last) {
   uint64_t dsum = c->h_ctr[C_SLOW_SUM];
   uint64_t dper = (2 * (dsum - R.dsum_prev) + R.max_fi - 1) / (uint64_t)R.max_fi;
   R.dsum_prev = dsum;
-  const uint64_t a_hint = (uint64_t)c->h_ctr[C_A] + 4ull * W;
+  const uint64_t a_hint = (uint64_t)c->h_ctr[C_LIST] + 4ull * W;
   const int variant = !R.flipping ? 0 : (a_hint <= kSmallList ? 1 : 2);
   const uint32_t grid = variant == 2 ? grid_for(c, a_hint, 16) : 0u;
   const uint32_t dgrid = variant == 2 ? deferred_grid(c, dper, grid) : 0u;
@@ -833,20 +845,26 @@ void run_round(wtet_ctx* c, Run& R, bool last) {
   uint32_t* ut = P<uint32_t>(c->utet[cur]);
   uint32_t* slow_p = P<uint32_t>(c->slow_p);
   uint64_t* sums = P<uint64_t>(c->isums);
+  const bool sparse = dper <= kSparseDeferred;
   auto enqueue = [&] {
+    // the batch of iterations begins and ends in the point kernels beside
+    // it, unless there are no points left
+    const int beside = variant == 2 && U > 0 ? k : 0;
     timed(c, K_SPLIT, [&] { launch_split(M, P<uint2>(c->wlist), W, L, s); });
-    timed(c, K_SPLIT_POINTS, [&] { launch_split_points(M, uv, ut, U, R.st, slow_p, s); });
+    timed(c, K_SPLIT_POINTS, [&] { launch_split_points(M, uv, ut, U, R.st, slow_p, beside, s); });
     if (variant == 0) {
-      launch_set_ctr(M.ctr, C_A, 0u, -1, 0u, s);
+      launch_set_ctr(M.ctr, C_LIST, 0u, -1, 0u, s);
     } else {
-      if (variant == 1)
+      if (variant == 1) {
         timed(c, K_FLIP_SMALL, [&] { launch_flip_small(M, L, R.st, sums, k, kSmallLimit, s); });
-      else
-        enqueue_flip_iterations(c, M, L, R.st, k, grid, dgrid);
-      timed(c, K_RELOCATE, [&] { launch_relocate(M, uv, ut, U, R.st, slow_p, s); });
+      } else {
+        if (!beside) launch_batch_begin(M.ctr, k, s);
+        enqueue_flip_iterations(c, M, L, R.st, k, grid, dgrid, sparse);
+        if (!beside) launch_batch_end(M.ctr, sums, k, s);
+      }
+      timed(c, K_RELOCATE, [&] { launch_relocate(M, uv, ut, U, R.st, slow_p, sums, beside, s); });
     }
     if (!last) {
-      launch_round_next(M.ctr, s);
       timed(c, K_VOTE, [&] { launch_vote(M, uv, ut, U, s); });
       timed(c, K_PICK, [&] {
         launch_pick(M, uv, ut, U, P<uint2>(c->wlist), P<uint32_t>(c->uvert[cur ^ 1]),
@@ -860,7 +878,7 @@ void run_round(wtet_ctx* c, Run& R, bool last) {
   } else {
     launch_cached_graph(c, c->round_graphs, buffer_key(c, M, L, R.st),
                         {(uint64_t)cur, (uint64_t)round_grid(W), (uint64_t)round_grid(U), (uint64_t)(U > 0),
-                         (uint64_t)variant, (uint64_t)grid, (uint64_t)dgrid, (uint64_t)k, (uint64_t)last,
+                         (uint64_t)variant, (uint64_t)grid, (uint64_t)dgrid, (uint64_t)sparse, (uint64_t)k, (uint64_t)last,
                          (uint64_t)ring_next},
                         enqueue);
   }
@@ -872,9 +890,9 @@ void dev_finish_flips(wtet_ctx* c, Run& R) {
   for (uint32_t guard = 0;; ++guard) {
     if (guard > 20000) throw Fail{WTET_ERR_NOT_CONVERGED, "flipping did not terminate"};
     read_ctr(c);
-    if (c->h_ctr[C_STOP]) grow_for(c, (uint64_t)c->h_ctr[C_TETS] + c->h_ctr[C_A] + 64);
-    else if (c->h_ctr[C_A] == 0) break;
-    run_flip_batch(c, R.V, R.mode, R.st, 16, c->h_ctr[C_A], c->h_ctr[C_A] / 64);
+    if (c->h_ctr[C_STOP]) grow_for(c, (uint64_t)c->h_ctr[C_TETS] + c->h_ctr[C_LIST] + 64);
+    else if (c->h_ctr[C_LIST] == 0) break;
+    run_flip_batch(c, R.V, R.mode, R.st, 16, c->h_ctr[C_LIST], c->h_ctr[C_LIST] / 64);
   }
 }
 
@@ -2741,19 +2759,13 @@ void stage_info(wtet_ctx* c, const wtet_stage_session* S, wtet_stage_info* info)
   info->round = S->R.round;
   info->uninserted = S->R.U;
   info->winners = S->R.W;
-  info->tet_slots = c->h_ctr[C_TETS];
-  info->active = c->h_ctr[C_A];
+  // after a vote, with the slots its winners take at the split
+  info->tet_slots = c->h_ctr[C_TETS] + (S->phase == 2 ? 3u * S->R.W : 0u);
+  info->active = c->h_ctr[C_LIST];
   info->checked = S->checked;
   info->flips = S->flips;
   info->violations = S->violations;
   info->deferred = S->deferred;
-}
-
-// slots holding tets: between a vote and its split the slots the vote
-// reserved (from ctr[C_BASE]) are not written yet
-uint32_t written_slots(wtet_ctx* c, const wtet_stage_session* S) {
-  read_ctr(c);
-  return S->phase == 2 ? c->h_ctr[C_BASE] : c->h_ctr[C_TETS];
 }
 
 }  // namespace
@@ -2849,8 +2861,8 @@ wtet_status wtet_stage_flip(wtet_ctx* c, int predicate_mode, wtet_stage_info* in
     Run& R = S->R;
     int mode = predicate_mode < 0 ? R.mode : (predicate_mode == 1 ? PRED_EXACT_ONLY : PRED_FILTERED);
     read_ctr(c);
-    if (c->h_ctr[C_STOP]) grow_for(c, (uint64_t)c->h_ctr[C_TETS] + c->h_ctr[C_A] + 64);
-    uint32_t a = c->h_ctr[C_A];
+    if (c->h_ctr[C_STOP]) grow_for(c, (uint64_t)c->h_ctr[C_TETS] + c->h_ctr[C_LIST] + 64);
+    uint32_t a = c->h_ctr[C_LIST];
     uint64_t before[S_COUNT] = {}, after[S_COUNT] = {};
     HIP_CHECK(hipMemcpyAsync(before, c->isums.p, S_COUNT * 8, hipMemcpyDeviceToHost, c->stream));
     if (a > 0) run_flip_batch(c, R.V, mode, R.st, 1, a, a / 8 + 1);
@@ -2859,7 +2871,7 @@ wtet_status wtet_stage_flip(wtet_ctx* c, int predicate_mode, wtet_stage_info* in
     S->checked = (uint32_t)(after[0] - before[0]);
     S->flips = (uint32_t)(after[1] - before[1]);
     read_ctr(c);
-    S->deferred = a > 0 ? c->h_ctr[C_SLOW_T] : 0u;
+    S->deferred = a > 0 ? c->h_ctr[C_SLOW_LAST] : 0u;
     if (S->flips) {
       S->audit_valid = false;
       if (R.U > 0) S->stale = true;
@@ -2884,7 +2896,8 @@ wtet_status wtet_stage_gather(wtet_ctx* c, wtet_stage_info* info) {
   if (!c) return WTET_ERR_INVALID_ARGUMENT;
   return guarded(c, [&] {
     wtet_stage_session* S = session_of(c, 0, "gather");
-    uint32_t T = written_slots(c, S);
+    read_ctr(c);
+    uint32_t T = c->h_ctr[C_TETS];
     Mesh M = mesh_of(c, S->R.V, S->R.mode);
     launch_set_ctr(M.ctr, C_VIOL, 0u, C_FAILREC, 0u, c->stream);
     const uint32_t rec_cap = (uint32_t)std::min<size_t>(c->rec.bytes / 4, c->audit_records);
@@ -2907,7 +2920,8 @@ wtet_status wtet_stage_readback(wtet_ctx* c, wtet_result* out) {
   wtet_status st = guarded(c, [&] {
     wtet_stage_session* S = session_of(c, 0, "readback");
     hipStream_t s = c->stream;
-    uint32_t T = written_slots(c, S);
+    read_ctr(c);
+    uint32_t T = c->h_ctr[C_TETS];
     // the flip lists stay as they are: the rows go through ord[0]
     dev_compact(c, S->R, T, true, true);
     read_ctr(c);
@@ -2953,7 +2967,8 @@ wtet_status wtet_stage_locations(wtet_ctx* c, uint32_t cap, uint32_t* point_ids,
     *count = R.U;
     uint32_t k = std::min(cap, R.U);
     if (k == 0) return;
-    uint32_t T = written_slots(c, S);
+    read_ctr(c);
+    uint32_t T = c->h_ctr[C_TETS];
     dev_compact(c, R, T, false, true);  // slot -> row, as a readback numbers them
     std::vector<uint32_t> uv(k), ut(k), slot2row(T);
     std::vector<float4> pts((size_t)R.V + 1);

@@ -48,56 +48,58 @@ hipError_t launch_stratify(uint32_t* uvert, uint32_t* utet, uint32_t U, const Cl
                            size_t temp_bytes, hipStream_t s);
 
 // rounds.  The round kernels read their counts and the round number from
-// ctr (C_ULEN, C_WIN, C_SURV, C_ROUND); the count arguments only bound the
-// launch grids, a power of two of workgroups (round_grid), so a captured
-// round replays for any count up to its bound.
+// ctr (C_WIN, C_SURV, C_ROUND); the count arguments only bound the launch
+// grids, a power of two of workgroups (round_grid), so a captured round
+// replays for any count up to its bound.
 uint32_t round_grid(uint64_t bound);
 void launch_vote(const Mesh& M, const uint32_t* uvert, const uint32_t* utet, uint32_t U,
                  hipStream_t s);
+// begins the next round (C_ROUND) and counts its winners (C_WIN); they leave
+// C_SURV, and take their slots from C_TETS, at the split.
 // ring: insert only where no tet within `ring` face-steps has a smaller vote
 // (blk: round_grid(U) entries)
 void launch_pick(const Mesh& M, const uint32_t* uvert, const uint32_t* utet, uint32_t U,
                  uint2* wlist, uint32_t* uvert2, uint32_t* utet2, uint32_t* blk, int ring,
                  hipStream_t s);
-// the two active lists (current = act[ctr[C_PAR]]), flip proposals and the
-// executed flips of one iteration
+// the two active lists, flip proposals and the executed flips of one
+// iteration
 struct FlipLists {
   uint32_t* act[2];
   uint4* prop;
-  uint4* out;    // two uint4 per executed flip (flip_exec_body)
-  uint32_t* slow;  // entries the FP32-only check deferred (ctr[C_SLOW_T])
+  uint4* out;    // two uint4 per executed flip (flip_exec_loaded)
+  uint32_t* slow;  // entries the lean check deferred
 };
-// appends the children to the current active list after its ctr[C_A]
-// entries and updates ctr[C_A]
+// appends the children to the active list after its ctr[C_LIST] entries
 void launch_split(const Mesh& M, const uint2* wlist, uint32_t W, const FlipLists& L, hipStream_t s);
-// ctr[C_ULEN] = ctr[C_SURV], ctr[C_ROUND] += 1: the next round, on the device
-void launch_round_next(uint32_t* ctr, hipStream_t s);
 // filtered mode: an FP32-only kernel, then the full predicates on the points
-// it deferred (slow, U entries of scratch); exact mode: one full kernel
+// it deferred (slow, U entries of scratch); exact mode: one full kernel.
+// begin > 0: also launch_batch_begin(begin)
 void launch_split_points(const Mesh& M, const uint32_t* uvert, uint32_t* utet, uint32_t U,
-                         uint64_t* st, uint32_t* slow, hipStream_t s);
-// one flip iteration = begin, check, decide+execute, update, end; counts,
-// tag, round and parity are read from ctr (device-driven, graph-capturable);
-// grid = persistent blocks of the three list kernels
-void launch_iter_begin(uint32_t* ctr, hipStream_t s);
-// filtered mode: the FP32-only check (deferring undecided tets), then the
-// full check of the deferred tets; exact mode: the full check, nothing deferred
-void launch_flip_check(const Mesh& M, const FlipLists& L, uint32_t grid, uint64_t* st,
+                         uint64_t* st, uint32_t* slow, int begin, hipStream_t s);
+// a batch of k <= kMaxBatch flip iterations = begin; check, (deferred check,)
+// decide+execute, update for i = 0..k-1; end.  Counts, tags, round and
+// parity are read from ctr (device-driven, graph-capturable); grid =
+// persistent blocks of the list kernels
+void launch_batch_begin(uint32_t* ctr, int k, hipStream_t s);
+// filtered mode: the FP32-only check, deferring undecided tets to the full
+// check that follows or, with requeue, to a later iteration (none follows);
+// exact mode: the full check, nothing deferred
+void launch_flip_check(const Mesh& M, const FlipLists& L, int i, bool requeue, uint32_t grid, uint64_t* st,
                        hipStream_t s);
-void launch_flip_check_deferred(const Mesh& M, const FlipLists& L, uint32_t grid, uint64_t* st,
+void launch_flip_check_deferred(const Mesh& M, const FlipLists& L, int i, uint32_t grid, uint64_t* st,
                                 hipStream_t s);
-void launch_flip_decide_exec(const Mesh& M, const FlipLists& L, uint32_t grid, hipStream_t s);
-void launch_flip_update(const Mesh& M, const FlipLists& L, uint32_t grid, hipStream_t s);
-// up to k iterations of a list of at most `limit` entries in one workgroup
-// (no deferral: the full predicates inline); sums as launch_iter_end
+void launch_flip_decide_exec(const Mesh& M, const FlipLists& L, int i, uint32_t grid, hipStream_t s);
+void launch_flip_update(const Mesh& M, const FlipLists& L, int i, uint32_t grid, hipStream_t s);
+// sums (IterSum) += what the batch did; the list it left in C_LIST
+void launch_batch_end(uint32_t* ctr, uint64_t* sums, int k, hipStream_t s);
+// a batch of up to k iterations of a list of at most `limit` entries in one
+// workgroup, begin and end included
 void launch_flip_small(const Mesh& M, const FlipLists& L, uint64_t* st, uint64_t* sums, int k,
                        uint32_t limit, hipStream_t s);
-// sums[0] += checked tets, sums[1] += flips, sums[2] += iterations
-void launch_iter_end(uint32_t* ctr, uint64_t* sums, hipStream_t s);
-// end of one iteration followed by the begin of the next
-void launch_iter_step(uint32_t* ctr, uint64_t* sums, hipStream_t s);
+// end > 0: also launch_batch_end(end).  ctr[C_SLOW_R] is 0 before (the split
+// clears it)
 void launch_relocate(const Mesh& M, const uint32_t* uvert, uint32_t* utet, uint32_t U,
-                     uint64_t* st, uint32_t* slow, hipStream_t s);
+                     uint64_t* st, uint32_t* slow, uint64_t* sums, int end, hipStream_t s);
 // filtered mode: an FP32-only pass, then the full predicates on the tets it
 // could not decide (slow: T entries of scratch); exact mode: one full pass
 void launch_audit(const Mesh& M, uint32_t T, uint32_t* rec, uint32_t cap, uint64_t* st,

@@ -43,7 +43,7 @@ __device__ __forceinline__ uint32_t block_rank(bool flag, uint32_t* total) {
 }
 
 // in-place exclusive scan of blk[0..nb) by one 1024-thread block
-// mode 0: insertion round -> ctr[C_WIN] = total, reserve 3*total slots
+// mode 0: insertion round -> ctr[C_WIN] = total
 // mode 1: output          -> ctr[C_ALIVE] = total
 // mode 2: point list      -> ctr[C_NPTS] = total
 __global__ void __launch_bounds__(1024) k_scan_blocks(uint32_t* blk, uint32_t nb, uint32_t* ctr,
@@ -72,9 +72,6 @@ __global__ void __launch_bounds__(1024) k_scan_blocks(uint32_t* blk, uint32_t nb
     uint32_t total = part[1023];
     if (mode == 0) {
       ctr[C_WIN] = total;
-      ctr[C_SURV] = ctr[C_ULEN] - total;
-      ctr[C_BASE] = ctr[C_TETS];
-      ctr[C_TETS] += 3u * total;
     } else if (mode == 1) {
       ctr[C_ALIVE] = total;
     } else {
@@ -295,31 +292,54 @@ hipError_t launch_stratify(uint32_t* uvert, uint32_t* utet, uint32_t U, const Cl
 // insertion rounds
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(kBlock) k_vote(Mesh M, const uint32_t* uvert, const uint32_t* utet) {
-  vote_wave(M, uvert, utet, gid(), M.ctr[C_ULEN]);
+  vote_wave(M, uvert, utet, gid(), M.ctr[C_SURV]);
 }
 
+// Counts the winners of each block of points.  Begins the round in the
+// counters: no other thread of this kernel reads them.
 __global__ void __launch_bounds__(kBlock) k_pick_count(Mesh M, const uint32_t* utet, uint32_t* blk, int ring) {
-  const uint32_t U = M.ctr[C_ULEN];
+  const uint32_t U = M.ctr[C_SURV];
   uint32_t i = gid();
+  if (i == 0) {
+    M.ctr[C_ROUND] += 1u;
+    M.ctr[C_SLOW_P] = 0u;
+  }
   bool w = i < U && is_winner(M, utet, i, ring);
   uint32_t tot;
   block_rank(w, &tot);
   if (threadIdx.x == 0) blk[blockIdx.x] = tot;
 }
 
+// SCANNED: blk holds each block's first winner; otherwise the blocks' counts,
+// which every block adds up to its own (and the last one to C_WIN): a launch
+// less, for grids whose counts are few enough to read in each block.
+template <bool SCANNED>
 __global__ void __launch_bounds__(kBlock) k_pick_scatter(Mesh M, const uint32_t* uvert, const uint32_t* utet,
                                uint2* wlist, uint32_t* uvert2, uint32_t* utet2, const uint32_t* blk,
                                int ring) {
-  const uint32_t U = M.ctr[C_ULEN], round = M.ctr[C_ROUND];
+  const uint32_t U = M.ctr[C_SURV], round = M.ctr[C_ROUND];
   uint32_t i = gid();
+  uint32_t first = 0;
+  if (SCANNED) {
+    first = blk[blockIdx.x];
+  } else {
+    __shared__ uint32_t part[kBlock / 64];
+    for (uint32_t b = threadIdx.x; b < blockIdx.x; b += kBlock) first += blk[b];
+    for (int off = 32; off > 0; off >>= 1) first += __shfl_xor(first, off);
+    if (__lane_id() == 0) part[threadIdx.x >> 6] = first;
+    __syncthreads();
+    first = 0;
+    for (int w = 0; w < kBlock / 64; ++w) first += part[w];
+  }
   bool w = i < U && is_winner(M, utet, i, ring);
   uint32_t tot;
-  uint32_t r = blk[blockIdx.x] + block_rank(w, &tot);
+  uint32_t r = first + block_rank(w, &tot);
+  if (!SCANNED && blockIdx.x == gridDim.x - 1u && threadIdx.x == 0) M.ctr[C_WIN] = first + tot;
   if (i >= U) return;
   uint32_t t = utet[i], v = uvert[i];
   if (w) {
     wlist[r] = make_uint2(t, v);
-    TSPLIT(M, t) = make_uint2(round, M.ctr[C_BASE] + 3u * r);
+    TSPLIT(M, t) = make_uint2(round, M.ctr[C_TETS] + 3u * r);
     TPOINT(M, t) = v;
   } else {
     uvert2[i - r] = v;
@@ -341,12 +361,9 @@ void launch_vote(const Mesh& M, const uint32_t* uvert, const uint32_t* utet, uin
   k_vote<<<round_grid(U), kBlock, 0, s>>>(M, uvert, utet);
 }
 
-// votes of tets whose winner was deferred must not survive into the next
-// round (list positions change); split resets the votes of winning tets
-__global__ void k_clear_votes(Mesh M, const uint32_t* utet2, const uint32_t* ctr) {
-  uint32_t i = gid();
-  if (i < ctr[C_SURV]) TVOTE(M, utet2[i]) = kVoteNone;
-}
+// Up to this many blocks every block of the scatter adds up the counts before
+// its own (4,096 words from L2: 1M points); above, one block scans them.
+constexpr uint32_t kScatterScan = 4096;
 
 void launch_pick(const Mesh& M, const uint32_t* uvert, const uint32_t* utet, uint32_t U,
                  uint2* wlist, uint32_t* uvert2, uint32_t* utet2, uint32_t* blk, int ring,
@@ -355,9 +372,12 @@ void launch_pick(const Mesh& M, const uint32_t* uvert, const uint32_t* utet, uin
   // the whole grid
   uint32_t nb = round_grid(U);
   k_pick_count<<<nb, kBlock, 0, s>>>(M, utet, blk, ring);
-  k_scan_blocks<<<1, 1024, 0, s>>>(blk, nb, M.ctr, 0);
-  k_pick_scatter<<<nb, kBlock, 0, s>>>(M, uvert, utet, wlist, uvert2, utet2, blk, ring);
-  if (ring > 0) k_clear_votes<<<nb, kBlock, 0, s>>>(M, utet2, M.ctr);
+  if (nb <= kScatterScan) {
+    k_pick_scatter<false><<<nb, kBlock, 0, s>>>(M, uvert, utet, wlist, uvert2, utet2, blk, ring);
+  } else {
+    k_scan_blocks<<<1, 1024, 0, s>>>(blk, nb, M.ctr, 0);
+    k_pick_scatter<true><<<nb, kBlock, 0, s>>>(M, uvert, utet, wlist, uvert2, utet2, blk, ring);
+  }
 }
 
 // The children join the active list with one counter atomic per wave, in
@@ -366,9 +386,16 @@ void launch_pick(const Mesh& M, const uint32_t* uvert, const uint32_t* utet, uin
 // that follow are numbered in list order, and lower slot ids win flip
 // votes.  On co-spherical inputs a tet-major order left about four times
 // as many faces stuck (1M points on a sphere: 3,150 against 866).
+// Also takes the winners' slots and points off the counters, which no thread
+// of this kernel reads.
 __global__ void __launch_bounds__(kBlock) k_split(Mesh M, const uint2* wlist, FlipLists L) {
   const uint32_t W = M.ctr[C_WIN], round = M.ctr[C_ROUND];
   uint32_t k = gid();
+  if (k == 0) {
+    M.ctr[C_TETS] += 3u * W;
+    M.ctr[C_SURV] -= W;
+    M.ctr[C_SLOW_R] = 0u;
+  }
   uint32_t c[4], m = 0u;
   if (k < W) m = split_body(M, wlist, k, round, c);
   uint64_t lt = (1ull << __lane_id()) - 1ull;
@@ -377,37 +404,82 @@ __global__ void __launch_bounds__(kBlock) k_split(Mesh M, const uint2* wlist, Fl
   uint32_t tot = n0 + 3u * nv;
   if (tot == 0u) return;
   uint32_t base = 0u;
-  if (__lane_id() == 0) base = atomicAdd(&M.ctr[C_ACT_NEXT], tot);
+  if (__lane_id() == 0) base = atomicAdd(&M.ctr[C_LIST], tot);
   base = __shfl(base, 0);
-  uint32_t* act_next = L.act[M.ctr[C_PAR] & 1u];
-  if (m & 1u) act_next[base + __popcll(b0 & lt)] = c[0];
+  uint32_t* act = L.act[M.ctr[C_PAR] & 1u];
+  if (m & 1u) act[base + __popcll(b0 & lt)] = c[0];
   if (m) {
     uint32_t r = __popcll(bv & lt);
-    for (uint32_t j = 1; j < 4; ++j) act_next[base + n0 + (j - 1u) * nv + r] = c[j];
+    for (uint32_t j = 1; j < 4; ++j) act[base + n0 + (j - 1u) * nv + r] = c[j];
   }
-}
-
-// ctr[dst] = ctr[src]
-__global__ void k_ctr_copy(uint32_t* ctr, int dst, int src) {
-  if (threadIdx.x == 0) ctr[dst] = ctr[src];
 }
 
 void launch_split(const Mesh& M, const uint2* wlist, uint32_t W, const FlipLists& L, hipStream_t s) {
-  // the children are appended after the active entries carried over
-  k_ctr_copy<<<1, 64, 0, s>>>(M.ctr, C_ACT_NEXT, C_A);
   k_split<<<round_grid(W), kBlock, 0, s>>>(M, wlist, L);
-  k_ctr_copy<<<1, 64, 0, s>>>(M.ctr, C_A, C_ACT_NEXT);
 }
 
-// the next round's uninserted count and number, on the device
-__global__ void k_round_next(uint32_t* ctr) {
-  if (threadIdx.x == 0) {
-    ctr[C_ULEN] = ctr[C_SURV];
-    ctr[C_ROUND] += 1u;
+// ---------------------------------------------------------------------------
+// Batches of flip iterations, driven from the device: every count, the
+// iteration tags, the round and the list parity are read from ctr, so a batch
+// runs (and can be captured in a graph) without the host.  Iteration i of a
+// batch has counters of its own (C_ITA + 32 i, ..): no kernel stands between
+// two iterations to reset them, and one wave adds them up at the end.
+// Measured with a one-thread kernel between iterations instead: 3 to 4 us
+// each and the gap, 160 to 270 times a triangulation.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ uint32_t* it_ctr(uint32_t* ctr, int which, int i) { return &ctr[which + 32 * i]; }
+
+// the counters of a batch of k iterations; by one workgroup
+__device__ __forceinline__ void batch_begin(uint32_t* ctr, int k) {
+  for (int i = threadIdx.x; i < 4 * (k + 1); i += blockDim.x) {
+    const int which = i / (k + 1), slot = i - which * (k + 1);
+    *it_ctr(ctr, C_ITA + 65 * 32 * which, slot) = which == 0 && slot == 0 ? ctr[C_LIST] : 0u;
   }
+  if (threadIdx.x == 0) ctr[C_TETS_IT] = ctr[C_TETS];
 }
 
-void launch_round_next(uint32_t* ctr, hipStream_t s) { k_round_next<<<1, 64, 0, s>>>(ctr); }
+__device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+  return v;
+}
+
+// by one whole wave.  sums (IterSum): checked tets, flips, iterations, 2-3
+// flips (a 2-3 flip takes one fresh slot, a 3-2 none)
+__device__ __forceinline__ void batch_end(uint32_t* ctr, unsigned long long* sums, int k) {
+  const int i = __lane_id();
+  const bool run = i < k && *it_ctr(ctr, C_ITR, i) != 0u;
+  const uint32_t a = run ? *it_ctr(ctr, C_ITA, i) : 0u, f = run ? *it_ctr(ctr, C_ITF, i) : 0u,
+                 d = run ? *it_ctr(ctr, C_ITS, i) : 0u;
+  const int n = __popcll(__ballot(run));  // iterations run: the first n
+  uint64_t sa = a;
+  uint32_t peak = a;
+  for (int off = 32; off > 0; off >>= 1) {
+    sa += (uint64_t)__shfl_xor((uint32_t)sa, off) | (uint64_t)__shfl_xor((uint32_t)(sa >> 32), off) << 32;
+    peak = max(peak, (uint32_t)__shfl_xor(peak, off));
+  }
+  const uint32_t sf = wave_sum_u32(f), sd = wave_sum_u32(d), last = __shfl(d, n > 0 ? n - 1 : 0);
+  if (i != 0) return;
+  const uint32_t left = *it_ctr(ctr, C_ITA, n);
+  sums[S_CHECKED] += sa;
+  sums[S_FLIPS] += sf;
+  sums[S_ITERS] += (unsigned long long)n;
+  sums[S_FLIPS23] += ctr[C_TETS] - ctr[C_TETS_IT];
+  ctr[C_SLOW_SUM] += sd;
+  ctr[C_SLOW_LAST] = last;
+  if (peak > ctr[C_PEAKA]) ctr[C_PEAKA] = peak;
+  if (n < k && left > 0u) ctr[C_STOP] = 1u;  // the tet slots could not hold the next one
+  ctr[C_LIST] = left;
+  ctr[C_IT] += (uint32_t)k;
+  ctr[C_PAR] ^= (uint32_t)n & 1u;
+}
+
+__global__ void __launch_bounds__(kBlock) k_batch_begin(uint32_t* ctr, int k) { batch_begin(ctr, k); }
+__global__ void k_batch_end(uint32_t* ctr, unsigned long long* sums, int k) { batch_end(ctr, sums, k); }
+
+void launch_batch_begin(uint32_t* ctr, int k, hipStream_t s) { k_batch_begin<<<1, kBlock, 0, s>>>(ctr, k); }
+void launch_batch_end(uint32_t* ctr, uint64_t* sums, int k, hipStream_t s) {
+  k_batch_end<<<1, 64, 0, s>>>(ctr, reinterpret_cast<unsigned long long*>(sums), k);
+}
 
 // Point kernels in three forms: LEAN runs the FP32 filter alone and defers
 // the points it cannot decide to `slow` (ctr[C_SLOW_P]); SLOW runs the full
@@ -422,9 +494,12 @@ enum KForm : int { LEAN = 0, FULL = 1, SLOW = 2 };
 static uint32_t slow_grid(uint32_t g) { return std::min(g / 4u + 16u, 1024u); }
 
 // The survivors of the round's pick (ctr[C_SURV]) in the round ctr[C_ROUND].
+// Each clears the vote of its tet first: votes of tets whose winner was
+// deferred must not survive into the next round (a split clears its own).
+// begin > 0: the last form's first workgroup begins the batch of iterations.
 template <int FORM>
-__global__ void __launch_bounds__(kBlock) k_split_points(Mesh M, const uint32_t* uvert,
-                                                         uint32_t* utet, uint64_t* st, uint32_t* slow) {
+__global__ void __launch_bounds__(kBlock) k_split_points(Mesh M, const uint32_t* uvert, uint32_t* utet,
+                                                         uint64_t* st, uint32_t* slow, int begin) {
   const uint32_t U = M.ctr[C_SURV], round = M.ctr[C_ROUND];
   PredStats ls = {};
   if (FORM == SLOW) {
@@ -434,81 +509,43 @@ __global__ void __launch_bounds__(kBlock) k_split_points(Mesh M, const uint32_t*
   } else {
     uint32_t i = gid();
     bool defer = false;
-    if (i < U) defer = split_points_body_t<FORM == LEAN>(M, uvert, utet, i, round, &ls);
+    if (i < U) {
+      TVOTE(M, utet[i]) = kVoteNone;
+      defer = split_points_body_t<FORM == LEAN>(M, uvert, utet, i, round, &ls);
+    }
     if (defer) slow[append_slot(&M.ctr[C_SLOW_P])] = i;
   }
   flush_stats(ls, st);
+  if (FORM != LEAN && begin > 0 && blockIdx.x == 0) batch_begin(M.ctr, begin);
 }
 
 void launch_split_points(const Mesh& M, const uint32_t* uvert, uint32_t* utet, uint32_t U,
-                         uint64_t* st, uint32_t* slow, hipStream_t s) {
+                         uint64_t* st, uint32_t* slow, int begin, hipStream_t s) {
   if (!U) return;
   uint32_t g = round_grid(U);
   if (M.mode == PRED_FILTERED) {
-    launch_set_ctr(M.ctr, C_SLOW_P, 0u, -1, 0u, s);
-    k_split_points<LEAN><<<g, kBlock, 0, s>>>(M, uvert, utet, st, slow);
-    k_split_points<SLOW><<<slow_grid(g), kBlock, 0, s>>>(M, uvert, utet, st, slow);
+    k_split_points<LEAN><<<g, kBlock, 0, s>>>(M, uvert, utet, st, slow, 0);
+    k_split_points<SLOW><<<slow_grid(g), kBlock, 0, s>>>(M, uvert, utet, st, slow, begin);
   } else {
-    k_split_points<FULL><<<g, kBlock, 0, s>>>(M, uvert, utet, st, slow);
+    k_split_points<FULL><<<g, kBlock, 0, s>>>(M, uvert, utet, st, slow, begin);
   }
 }
 
 // ---------------------------------------------------------------------------
-// flips
+// flips: iteration i of a batch.  The kernels are persistent: a fixed grid
+// strides over the current list.
 // ---------------------------------------------------------------------------
-// ---------------------------------------------------------------------------
-// flip iterations, driven from the device: every count, the iteration tag,
-// the round and the list parity are read from ctr, so a sequence of
-// iterations runs (and can be captured in a graph) without the host.  The
-// kernels are persistent: a fixed grid strides over the current list.
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ void iter_begin(uint32_t* ctr) {
-  uint32_t A = ctr[C_A];
-  uint32_t run = 0u;
-  if (!ctr[C_STOP] && A > 0u) {
-    // worst case every proposal wins a 2-3 flip and takes a fresh slot
-    if ((uint64_t)ctr[C_TETS] + A + 64u > (uint64_t)ctr[C_CAP]) ctr[C_STOP] = 1u;
-    else run = 1u;
-  }
-  ctr[C_RUN] = run;
-  if (run) {
-    ctr[C_IT] += 1u;
-    ctr[C_ACT_NEXT] = 0u;
-    ctr[C_FLIPS] = 0u;
-    ctr[C_SLOW_T] = 0u;
-    ctr[C_TETS_IT] = ctr[C_TETS];
-    if (A > ctr[C_PEAKA]) ctr[C_PEAKA] = A;
-  }
+// The first kernel of an iteration decides whether it runs (C_TETS changes in
+// decide_exec only) and says so to the others.
+__device__ __forceinline__ bool iter_runs(uint32_t* ctr, int i) {
+  const uint32_t A = *it_ctr(ctr, C_ITA, i);
+  // worst case every proposal wins a 2-3 flip and takes a fresh slot
+  if (A == 0u || ctr[C_STOP] || (uint64_t)ctr[C_TETS] + A + 64u > (uint64_t)ctr[C_CAP]) return false;
+  if (gid() == 0) *it_ctr(ctr, C_ITR, i) = 1u;
+  return true;
 }
-
-__global__ void k_iter_begin(uint32_t* ctr) {
-  if (threadIdx.x == 0) iter_begin(ctr);
-}
-
-// sums (IterSum): checked tets, flips, iterations, 2-3 flips (a 2-3 flip
-// takes one fresh slot, a 3-2 none), then the checked tets and flips of the
-// iterations k_flip_small ran.
-__device__ __forceinline__ void iter_end(uint32_t* ctr, unsigned long long* sums) {
-  if (!ctr[C_RUN]) return;
-  sums[S_CHECKED] += ctr[C_A];
-  sums[S_FLIPS] += ctr[C_FLIPS];
-  sums[S_ITERS] += 1ull;
-  sums[S_FLIPS23] += ctr[C_TETS] - ctr[C_TETS_IT];
-  ctr[C_SLOW_SUM] += ctr[C_SLOW_T];
-  ctr[C_A] = ctr[C_ACT_NEXT];
-  ctr[C_PAR] ^= 1u;
-}
-
-__global__ void k_iter_end(uint32_t* ctr, unsigned long long* sums) {
-  if (threadIdx.x == 0) iter_end(ctr, sums);
-}
-
-// end of one iteration and begin of the next in one launch
-__global__ void k_iter_step(uint32_t* ctr, unsigned long long* sums) {
-  if (threadIdx.x) return;
-  iter_end(ctr, sums);
-  iter_begin(ctr);
-}
+__device__ __forceinline__ uint32_t iter_tag(const uint32_t* ctr, int i) { return ctr[C_IT] + (uint32_t)i + 1u; }
+__device__ __forceinline__ uint32_t iter_par(const uint32_t* ctr, int i) { return (ctr[C_PAR] + (uint32_t)i) & 1u; }
 
 // The filters of the flip check on every list entry, one thread per tet; the
 // entries they leave go to L.slow.  98 VGPRs, 4 waves per SIMD (at 96 and 5
@@ -516,16 +553,21 @@ __global__ void k_iter_step(uint32_t* ctr, unsigned long long* sums) {
 // points: 6.68 ms of event time a triangulation with insphere_f32 and
 // insphere_f64 per face and three orient3d after each (158 VGPRs), 5.60 ms
 // with one set of cofactors per tet; 100k points 2.79 -> 2.05 ms.
-__global__ void __launch_bounds__(kBlock) k_flip_check(Mesh M, FlipLists L, uint64_t* st) {
-  if (!M.ctr[C_RUN]) return;
-  uint32_t it = M.ctr[C_IT];
-  const uint32_t* cur = L.act[M.ctr[C_PAR] & 1u];
+// requeue: no kernel of this iteration runs the full predicates; an entry that
+// needs them stays in the active list.
+__global__ void __launch_bounds__(kBlock) k_flip_check(Mesh M, FlipLists L, int i, int requeue, uint64_t* st) {
+  if (!iter_runs(M.ctr, i)) return;
+  const uint32_t it = iter_tag(M.ctr, i);
+  const uint32_t* cur = L.act[iter_par(M.ctr, i)];
   uint32_t stride = gridDim.x * blockDim.x;
   PredStats ls = {};
-  uint32_t A = M.ctr[C_A];
+  uint32_t A = *it_ctr(M.ctr, C_ITA, i);
   for (uint32_t j = gid(); j < A; j += stride)
-    if (flip_check_lean(M, cur, L.prop, j, it, &ls))
-      L.slow[append_slot(&M.ctr[C_SLOW_T])] = j;
+    if (flip_check_lean(M, cur, L.prop, j, it, &ls)) {
+      const uint32_t k = append_slot(it_ctr(M.ctr, C_ITS, i));
+      if (requeue) L.prop[j] = requeue_proposal(cur[j]);
+      else L.slow[k] = j;
+    }
   flush_stats(ls, st);
 }
 
@@ -535,11 +577,11 @@ __global__ void __launch_bounds__(kBlock) k_flip_check(Mesh M, FlipLists L, uint
 // four lanes 41 us).  A wave's first k is a multiple of 64, so a tet's four
 // lanes share a wave.
 template <bool ALL>
-__global__ void __launch_bounds__(kBlock) k_flip_check_faces(Mesh M, FlipLists L, uint64_t* st) {
-  if (!M.ctr[C_RUN]) return;
-  const uint32_t it = M.ctr[C_IT];
-  const uint32_t* cur = L.act[M.ctr[C_PAR] & 1u];
-  const uint32_t n4 = 4u * M.ctr[ALL ? C_A : C_SLOW_T], stride = gridDim.x * blockDim.x;
+__global__ void __launch_bounds__(kBlock) k_flip_check_faces(Mesh M, FlipLists L, int i, uint64_t* st) {
+  if (ALL ? !iter_runs(M.ctr, i) : !*it_ctr(M.ctr, C_ITR, i)) return;
+  const uint32_t it = iter_tag(M.ctr, i);
+  const uint32_t* cur = L.act[iter_par(M.ctr, i)];
+  const uint32_t n4 = 4u * *it_ctr(M.ctr, ALL ? C_ITA : C_ITS, i), stride = gridDim.x * blockDim.x;
   PredStats ls = {};
   for (uint32_t k = gid(); k < n4; k += stride)
     flip_check_faces(M, cur, L.prop, ALL ? k >> 2 : L.slow[k >> 2], (int)(k & 3u), it, &ls);
@@ -584,18 +626,18 @@ __device__ __forceinline__ uint32_t block_prefix3(uint32_t a, uint32_t b, uint32
 constexpr uint32_t kDecBlock = 512;
 static_assert(kDecBlock <= 512, "block_prefix3 packs totals of at most 512 threads");
 
-__global__ void __launch_bounds__(kDecBlock) k_flip_decide_exec(Mesh M, FlipLists L) {
+__global__ void __launch_bounds__(kDecBlock) k_flip_decide_exec(Mesh M, FlipLists L, int i) {
   constexpr uint32_t kBS = kDecBlock;
   __shared__ uint32_t wsum[kBS / 64];
   __shared__ uint32_t base[3];
-  if (!M.ctr[C_RUN]) return;
-  uint32_t A = M.ctr[C_A], it = M.ctr[C_IT], round = M.ctr[C_ROUND];
-  uint32_t* act_next = L.act[(M.ctr[C_PAR] & 1u) ^ 1u];
+  if (!*it_ctr(M.ctr, C_ITR, i)) return;
+  const uint32_t A = *it_ctr(M.ctr, C_ITA, i), it = iter_tag(M.ctr, i), round = M.ctr[C_ROUND];
+  uint32_t* act_next = L.act[iter_par(M.ctr, i) ^ 1u];
   for (uint32_t b0 = blockIdx.x * kBS; b0 < A; b0 += gridDim.x * kBS) {
     uint32_t j = b0 + threadIdx.x;
     uint4 pr = make_uint4(kInvalid, 0u, 0u, 0u);
     if (j < A) pr = L.prop[j];
-    uint32_t qid[2], nq = 0, nslot = 0;
+    uint32_t qid[2], nq, nslot;
     FlipTets F;
     bool win = flip_decide_load(M, pr, it, qid, &nq, &nslot, F);
     uint32_t nqa = nq + nslot;  // the fresh slot is queued too
@@ -604,13 +646,14 @@ __global__ void __launch_bounds__(kDecBlock) k_flip_decide_exec(Mesh M, FlipList
     uint32_t rf = r & 1023u, rs = (r >> 10) & 1023u, rq = r >> 20;
     uint32_t tf = tot & 1023u, ts = (tot >> 10) & 1023u, tq = tot >> 20;
     if (threadIdx.x == 0) {
-      base[0] = tf ? atomicAdd(&M.ctr[C_FLIPS], tf) : 0u;
+      base[0] = tf ? atomicAdd(it_ctr(M.ctr, C_ITF, i), tf) : 0u;
       base[1] = ts ? atomicAdd(&M.ctr[C_TETS], ts) : 0u;
-      base[2] = tq ? atomicAdd(&M.ctr[C_ACT_NEXT], tq) : 0u;
+      base[2] = tq ? atomicAdd(it_ctr(M.ctr, C_ITA, i + 1), tq) : 0u;
     }
     __syncthreads();
     uint32_t q = base[2] + rq;
-    for (uint32_t k = 0; k < nq; ++k) act_next[q + k] = qid[k];
+    if (nq > 0u) act_next[q] = qid[0];
+    if (nq > 1u) act_next[q + 1u] = qid[1];
     if (win) {
       uint32_t sl = nslot ? base[1] + rs : kInvalid;
       if (nslot) act_next[q + nq] = sl;
@@ -620,86 +663,68 @@ __global__ void __launch_bounds__(kDecBlock) k_flip_decide_exec(Mesh M, FlipList
   }
 }
 
-__global__ void __launch_bounds__(kBlock) k_flip_update(Mesh M, FlipLists L) {
-  if (!M.ctr[C_RUN]) return;
-  uint32_t F = M.ctr[C_FLIPS], it = M.ctr[C_IT];
+__global__ void __launch_bounds__(kBlock) k_flip_update(Mesh M, FlipLists L, int i) {
+  if (!*it_ctr(M.ctr, C_ITR, i)) return;
+  const uint32_t F = *it_ctr(M.ctr, C_ITF, i), it = iter_tag(M.ctr, i);
   uint32_t stride = gridDim.x * blockDim.x;
   for (uint32_t k = gid(); k < F; k += stride) flip_update_body(M, L.out, k, it);
 }
 
-// Up to k flip iterations of a short list in one workgroup: the phases of
-// an iteration (check with the full predicates, decide + execute, adjacency
-// update, end) are separated by workgroup barriers instead of launches.
-// Stops at the first iteration whose list is empty or longer than `limit`;
-// a longer list stays for the next batch of iterations.  Counters that
-// other threads of the block change are read with atomic loads.
-__global__ void __launch_bounds__(kBlock) k_flip_small(Mesh M, FlipLists L, uint64_t* st,
-                                                       unsigned long long* sums, int k, uint32_t limit) {
-  __shared__ uint32_t run, nslow;
-  PredStats ls = {};
+// Up to k flip iterations of a short list in one workgroup
+// (wg_flip_iteration), a whole batch.  Stops at the first iteration whose
+// list is empty or longer than `limit`; a longer list stays for the next
+// batch.  Event time at 100k points: 1.28 ms a triangulation with counters and
+// atomics at the memory side (and the full predicates inline), 0.37 ms with
+// LDS counters and atomics at workgroup scope.
+constexpr int kFlipSmallBlock = 512;
+
+__global__ void __launch_bounds__(kFlipSmallBlock) k_flip_small(WgMesh M, FlipLists L, uint64_t* st,
+                                                                unsigned long long* sums, int k, uint32_t limit) {
+  __shared__ WgCounters c;
   uint32_t* ctr = M.ctr;
-  auto ld = [&](int i) { return __atomic_load_n(&ctr[i], __ATOMIC_RELAXED); };
-  const uint32_t round = ld(C_ROUND);
-  for (int i = 0; i < k; ++i) {
-    if (threadIdx.x == 0) {
-      uint32_t A = ld(C_A);
-      uint32_t go = 0u;
-      if (A > 0u && A <= limit && !ld(C_STOP)) {
-        if ((uint64_t)ld(C_TETS) + A + 64u > (uint64_t)ld(C_CAP)) {
-          __atomic_store_n(&ctr[C_STOP], 1u, __ATOMIC_RELAXED);
-        } else {
-          go = 1u;
-          __atomic_store_n(&ctr[C_IT], ld(C_IT) + 1u, __ATOMIC_RELAXED);
-          __atomic_store_n(&ctr[C_ACT_NEXT], 0u, __ATOMIC_RELAXED);
-          __atomic_store_n(&ctr[C_FLIPS], 0u, __ATOMIC_RELAXED);
-          __atomic_store_n(&ctr[C_SLOW_T], 0u, __ATOMIC_RELAXED);
-          __atomic_store_n(&ctr[C_TETS_IT], ld(C_TETS), __ATOMIC_RELAXED);
-          if (A > ld(C_PEAKA)) __atomic_store_n(&ctr[C_PEAKA], A, __ATOMIC_RELAXED);
-        }
-      }
-      __atomic_store_n(&ctr[C_RUN], go, __ATOMIC_RELAXED);
-      run = go;
-      nslow = 0u;
+  const uint32_t round = ctr[C_ROUND], tets0 = ctr[C_TETS], cap = ctr[C_CAP], it0 = ctr[C_IT];
+  uint32_t A = ctr[C_LIST], par = ctr[C_PAR] & 1u, tets = tets0, sa = 0, sf = 0, peak = 0, slow = 0, last = 0;
+  bool stop = ctr[C_STOP] != 0u;
+  int n = 0;
+  if (threadIdx.x == 0) c.slots = tets0;
+  for (; n < k && !stop && A > 0u && A <= limit; ++n) {
+    if ((uint64_t)tets + A + 64u > (uint64_t)cap) {
+      stop = true;
+      break;
     }
-    __syncthreads();
-    if (!run) break;
-    uint32_t A = ld(C_A), it = ld(C_IT), par = ld(C_PAR) & 1u;
-    const uint32_t* cur = L.act[par];
-    uint32_t* nxt = L.act[par ^ 1u];
-    uint32_t ns = A;
-    if (M.mode == PRED_FILTERED) {
-      for (uint32_t j = threadIdx.x; j < A; j += blockDim.x)
-        if (flip_check_lean(M, cur, L.prop, j, it, &ls)) L.slow[append_slot(&nslow)] = j;
-      __syncthreads();
-      ns = nslow;
-    }
-    for (uint32_t q = threadIdx.x; q < 4u * ns; q += blockDim.x)
-      flip_check_faces(M, cur, L.prop, M.mode == PRED_FILTERED ? L.slow[q >> 2] : q >> 2, (int)(q & 3u), it, &ls);
-    __syncthreads();
-    for (uint32_t j = threadIdx.x; j < A; j += blockDim.x)
-      flip_decide_exec_body(M, L.prop, j, it, round, L.out, nxt);
-    __syncthreads();
-    uint32_t F = ld(C_FLIPS);
-    for (uint32_t f = threadIdx.x; f < F; f += blockDim.x) flip_update_body(M, L.out, f, it);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      sums[S_CHECKED] += A;
-      sums[S_FLIPS] += F;
-      sums[S_ITERS] += 1ull;
-      sums[S_FLIPS23] += ld(C_TETS) - ld(C_TETS_IT);
-      sums[S_SMALL_CHECKED] += A;
-      sums[S_SMALL_FLIPS] += F;
-      __atomic_store_n(&ctr[C_A], ld(C_ACT_NEXT), __ATOMIC_RELAXED);
-      __atomic_store_n(&ctr[C_PAR], par ^ 1u, __ATOMIC_RELAXED);
-    }
-    __syncthreads();
+    wg_flip_iteration<WgMesh, kFlipSmallBlock>(M, c, par ? L.act[1] : L.act[0], par ? L.act[0] : L.act[1], L.prop,
+                                               L.slow, L.out, A, it0 + (uint32_t)n + 1u, round, st);
+    sa += A;
+    sf += c.flips;
+    slow += c.slow;
+    last = c.slow;
+    peak = max(peak, A);
+    A = c.act_next;
+    tets = c.slots;
+    par ^= 1u;
+    __syncthreads();  // the counters are read before the next iteration resets them
   }
-  flush_stats(ls, st);
+  if (threadIdx.x == 0) {
+    sums[S_CHECKED] += sa;
+    sums[S_FLIPS] += sf;
+    sums[S_ITERS] += (unsigned long long)n;
+    sums[S_FLIPS23] += tets - tets0;
+    sums[S_SMALL_CHECKED] += sa;
+    sums[S_SMALL_FLIPS] += sf;
+    ctr[C_TETS] = tets;
+    ctr[C_SLOW_SUM] += slow;
+    ctr[C_SLOW_LAST] = last;
+    if (peak > ctr[C_PEAKA]) ctr[C_PEAKA] = peak;
+    if (stop) ctr[C_STOP] = 1u;
+    ctr[C_LIST] = A;
+    ctr[C_IT] = it0 + (uint32_t)k;
+    ctr[C_PAR] = par;
+  }
 }
 
 void launch_flip_small(const Mesh& M, const FlipLists& L, uint64_t* st, uint64_t* sums, int k,
                        uint32_t limit, hipStream_t s) {
-  k_flip_small<<<1, kBlock, 0, s>>>(M, L, st, reinterpret_cast<unsigned long long*>(sums), k, limit);
+  k_flip_small<<<1, kFlipSmallBlock, 0, s>>>(WgMesh{M}, L, st, reinterpret_cast<unsigned long long*>(sums), k, limit);
 }
 
 __global__ void k_set_ctr(uint32_t* ctr, int idx, uint32_t v, int idx2, uint32_t v2) {
@@ -713,59 +738,56 @@ void launch_set_ctr(uint32_t* ctr, int idx, uint32_t v, int idx2, uint32_t v2, h
   k_set_ctr<<<1, 64, 0, s>>>(ctr, idx, v, idx2, v2);
 }
 
-void launch_iter_begin(uint32_t* ctr, hipStream_t s) { k_iter_begin<<<1, 64, 0, s>>>(ctr); }
-void launch_iter_end(uint32_t* ctr, uint64_t* sums, hipStream_t s) {
-  k_iter_end<<<1, 64, 0, s>>>(ctr, reinterpret_cast<unsigned long long*>(sums));
+void launch_flip_check(const Mesh& M, const FlipLists& L, int i, bool requeue, uint32_t grid, uint64_t* st,
+                       hipStream_t s) {
+  if (M.mode == PRED_FILTERED) k_flip_check<<<grid, kBlock, 0, s>>>(M, L, i, requeue ? 1 : 0, st);
+  else k_flip_check_faces<true><<<std::min(4u * grid, 4096u), kBlock, 0, s>>>(M, L, i, st);
 }
-void launch_iter_step(uint32_t* ctr, uint64_t* sums, hipStream_t s) {
-  k_iter_step<<<1, 64, 0, s>>>(ctr, reinterpret_cast<unsigned long long*>(sums));
-}
-void launch_flip_check(const Mesh& M, const FlipLists& L, uint32_t grid, uint64_t* st, hipStream_t s) {
-  if (M.mode == PRED_FILTERED) k_flip_check<<<grid, kBlock, 0, s>>>(M, L, st);
-  else k_flip_check_faces<true><<<std::min(4u * grid, 4096u), kBlock, 0, s>>>(M, L, st);
-}
-void launch_flip_check_deferred(const Mesh& M, const FlipLists& L, uint32_t grid, uint64_t* st,
+void launch_flip_check_deferred(const Mesh& M, const FlipLists& L, int i, uint32_t grid, uint64_t* st,
                                 hipStream_t s) {
-  if (M.mode == PRED_FILTERED) k_flip_check_faces<false><<<grid, kBlock, 0, s>>>(M, L, st);
+  if (M.mode == PRED_FILTERED) k_flip_check_faces<false><<<grid, kBlock, 0, s>>>(M, L, i, st);
 }
 // grid: blocks of kBlock threads, as the other list kernels; the same
 // threads in blocks of kDecBlock
-void launch_flip_decide_exec(const Mesh& M, const FlipLists& L, uint32_t grid, hipStream_t s) {
-  k_flip_decide_exec<<<std::max<uint32_t>(grid * kBlock / kDecBlock, 1u), kDecBlock, 0, s>>>(M, L);
+void launch_flip_decide_exec(const Mesh& M, const FlipLists& L, int i, uint32_t grid, hipStream_t s) {
+  k_flip_decide_exec<<<std::max<uint32_t>(grid * kBlock / kDecBlock, 1u), kDecBlock, 0, s>>>(M, L, i);
 }
-void launch_flip_update(const Mesh& M, const FlipLists& L, uint32_t grid, hipStream_t s) {
-  k_flip_update<<<grid, kBlock, 0, s>>>(M, L);
+void launch_flip_update(const Mesh& M, const FlipLists& L, int i, uint32_t grid, hipStream_t s) {
+  k_flip_update<<<grid, kBlock, 0, s>>>(M, L, i);
 }
 
-// The uninserted points after the round's pick (ctr[C_SURV]), round ctr[C_ROUND].
+// The uninserted points after the round's pick (ctr[C_SURV]), round
+// ctr[C_ROUND].  end > 0: the last form's first workgroup ends the batch of
+// `end` iterations, which none of these kernels reads the counters of.
 template <int FORM>
 __global__ void __launch_bounds__(kBlock) k_relocate(Mesh M, const uint32_t* uvert, uint32_t* utet,
-                                                     uint64_t* st, uint32_t* slow) {
+                                                     uint64_t* st, uint32_t* slow, unsigned long long* sums, int end) {
   const uint32_t U = M.ctr[C_SURV], round = M.ctr[C_ROUND];
   PredStats ls = {};
   if (FORM == SLOW) {
-    uint32_t n = M.ctr[C_SLOW_P], stride = gridDim.x * blockDim.x;
+    uint32_t n = M.ctr[C_SLOW_R], stride = gridDim.x * blockDim.x;
     for (uint32_t k = gid(); k < n; k += stride)
       (void)relocate_body_t<false>(M, uvert, utet, slow[k], round, &ls);
   } else {
     uint32_t i = gid();
     bool defer = false;
     if (i < U) defer = relocate_body_t<FORM == LEAN>(M, uvert, utet, i, round, &ls);
-    if (defer) slow[append_slot(&M.ctr[C_SLOW_P])] = i;
+    if (defer) slow[append_slot(&M.ctr[C_SLOW_R])] = i;
   }
   flush_stats(ls, st);
+  if (FORM != LEAN && end > 0 && blockIdx.x == 0 && threadIdx.x < 64) batch_end(M.ctr, sums, end);
 }
 
 void launch_relocate(const Mesh& M, const uint32_t* uvert, uint32_t* utet, uint32_t U,
-                     uint64_t* st, uint32_t* slow, hipStream_t s) {
+                     uint64_t* st, uint32_t* slow, uint64_t* sums, int end, hipStream_t s) {
   if (!U) return;
   uint32_t g = round_grid(U);
+  unsigned long long* sm = reinterpret_cast<unsigned long long*>(sums);
   if (M.mode == PRED_FILTERED) {
-    launch_set_ctr(M.ctr, C_SLOW_P, 0u, -1, 0u, s);
-    k_relocate<LEAN><<<g, kBlock, 0, s>>>(M, uvert, utet, st, slow);
-    k_relocate<SLOW><<<slow_grid(g), kBlock, 0, s>>>(M, uvert, utet, st, slow);
+    k_relocate<LEAN><<<g, kBlock, 0, s>>>(M, uvert, utet, st, slow, sm, 0);
+    k_relocate<SLOW><<<slow_grid(g), kBlock, 0, s>>>(M, uvert, utet, st, slow, sm, end);
   } else {
-    k_relocate<FULL><<<g, kBlock, 0, s>>>(M, uvert, utet, st, slow);
+    k_relocate<FULL><<<g, kBlock, 0, s>>>(M, uvert, utet, st, slow, sm, end);
   }
 }
 

@@ -15,36 +15,42 @@ namespace wtet {
 // device-side counters (Mesh::ctr)
 enum Ctr : int {
   // read by every thread of the flip kernels, written between kernels: the
-  // first line.  Counters that take atomics at volume sit 1 KB apart, away
-  // from it and from each other.
-  C_A = 0,         // length of the current active list
-  C_IT = 1,        // flip iteration tag (fvote keys, flip stamps)
-  C_PAR = 2,       // which of the two active lists is current
-  C_RUN = 3,       // 1 while this iteration runs
-  C_STOP = 4,      // set when an iteration could overflow the tet slots
-  C_ROUND = 5,     // insertion round (flip stamps)
-  C_CAP = 6,       // tet slot capacity
-  C_PEAKA = 7,     // longest active list seen
-  C_TETS_IT = 8,   // C_TETS when the current flip iteration began
-  C_SLOW_SUM = 9,  // tets deferred by the lean flip check, summed over iterations
-  C_WALK_FAIL = 10, // relocation walks that hit the step limit
-  C_WIN = 11,      // insertions this round
-  C_BASE = 12,     // first slot reserved for this round's splits
-  C_ALIVE = 13,    // alive tets (output compaction)
-  C_BADTET = 14,   // points found in a tet touching infinity (must stay 0)
-  C_NPTS = 15,     // points to insert (input minus exact duplicates)
-  C_DUPSCAN = 16,  // duplicate scans that hit their length cap
-  C_ULEN = 17,     // uninserted list length at the start of the round
-  C_SURV = 18,     // points left after this round's insertions
-  C_TETS = 256,      // next free tet slot
-  C_ACT_NEXT = 512,  // length of the next active list
-  C_FLIPS = 768,     // winning flips this iteration
-  C_SLOW_T = 1024,   // tets deferred by the lean flip check this iteration
-  C_SLOW_P = 1280,   // points deferred by the lean point kernels
-  C_VIOL = 1536,     // non-Delaunay faces found by the audit
-  C_FAILREC = 1537,  // recorded violation entries
-  C_COUNT = 1792
+  // first line.  Counters that take atomics at volume sit 1 KB or more apart,
+  // away from it and from each other.
+  C_IT = 0,         // flip iterations before this batch (fvote keys, flip stamps)
+  C_PAR = 1,        // which of the two active lists the batch begins with
+  C_STOP = 2,       // set when an iteration could overflow the tet slots
+  C_ROUND = 3,      // insertion round (flip stamps)
+  C_CAP = 4,        // tet slot capacity
+  C_PEAKA = 5,      // longest active list seen
+  C_TETS_IT = 6,    // C_TETS when the batch of iterations began
+  C_SLOW_SUM = 7,   // tets deferred by the lean flip check, summed over iterations
+  C_SLOW_LAST = 8,  // tets deferred in the last iteration
+  C_WALK_FAIL = 9,  // relocation walks that hit the step limit
+  C_WIN = 10,       // insertions this round
+  C_ALIVE = 11,     // alive tets (output compaction)
+  C_BADTET = 12,    // points found in a tet touching infinity (must stay 0)
+  C_NPTS = 13,      // points to insert (input minus exact duplicates)
+  C_DUPSCAN = 14,   // duplicate scans that hit their length cap
+  C_SURV = 15,      // uninserted points (the pick's winners leave at the split)
+  C_TETS = 256,     // next free tet slot (the winners' at the split)
+  C_LIST = 512,     // length of the active list between batches of iterations
+  C_SLOW_P = 768,   // points deferred by the lean point split
+  C_SLOW_R = 1024,  // points deferred by the lean relocation
+  C_SLOW_T = 1280,  // tets deferred by the lean audit
+  C_VIOL = 1536,    // non-Delaunay faces found by the audit
+  C_FAILREC = 1537, // recorded violation entries
+  C_HEAD = 1792,    // the counters the host reads
+  // one slot per iteration of a batch, a 128-byte line apart, and a zero
+  // slot after the last: list length, executed flips, deferred tets, and
+  // whether the iteration ran
+  C_ITA = C_HEAD,
+  C_ITF = C_ITA + 65 * 32,
+  C_ITS = C_ITF + 65 * 32,
+  C_ITR = C_ITS + 65 * 32,
+  C_COUNT = C_ITR + 65 * 32
 };
+constexpr int kMaxBatch = 64;  // flip iterations in a batch
 
 // per-call sums over flip iterations (u64, device)
 enum IterSum : int {
@@ -112,6 +118,17 @@ WT_HD uint64_t& FVOTE(const Mesh& M, uint32_t t) { return M.fvote[t]; }
 WT_HD uint2& TSPLIT(const Mesh& M, uint32_t t) { return M.tsplit[t]; }
 WT_HD uint32_t& TPOINT(const Mesh& M, uint32_t t) { return M.tpoint[t]; }
 WT_HD FlipMsg& TMSG(const Mesh& M, uint32_t t) { return M.tmsg[t]; }
+
+// The same mesh while one workgroup alone changes it: its atomics need the
+// workgroup's scope only and complete in the XCD's L2 instead of at the
+// memory side.
+struct WgMesh : Mesh {};
+
+// atomics at the scope the mesh is shared at
+WT_HD void mesh_min(const Mesh&, uint64_t* p, uint64_t v) { at_min_u64(p, v); }
+WT_HD uint32_t mesh_or(const Mesh&, uint32_t* p, uint32_t v) { return at_or_u32(p, v); }
+WT_HD void mesh_min(const WgMesh&, uint64_t* p, uint64_t v) { wg_min_u64(p, v); }
+WT_HD uint32_t mesh_or(const WgMesh&, uint32_t* p, uint32_t v) { return wg_or_u32(p, v); }
 
 template <class MS>
 WT_HD uint4 TN(const MS& M, uint32_t t) {
@@ -242,7 +259,7 @@ WT_HD uint64_t vote_key(const MS& M, const uint32_t* uvert, const uint32_t* utet
 template <class MS>
 WT_HD void vote_body(const MS& M, const uint32_t* uvert, const uint32_t* utet, uint32_t i) {
   uint64_t key = vote_key(M, uvert, utet, i);
-  if (key != kVoteNone) at_min_u64(&TVOTE(M, utet[i]), key);
+  if (key != kVoteNone) mesh_min(M, &TVOTE(M, utet[i]), key);
 }
 
 // Point i is inserted this round when it holds its tet's vote and no tet
@@ -332,7 +349,7 @@ WT_HD uint32_t split_body(const MS& M, const uint2* wlist, uint32_t k, uint32_t 
       FSTAMP(M, c[j]) = 0ull;
     }
   }
-  uint32_t old = at_or_u32(&INFO(M, t), kQueued);
+  uint32_t old = mesh_or(M, &INFO(M, t), kQueued);
   return (old & kQueued) ? 0xEu : 0xFu;
 }
 
@@ -414,9 +431,9 @@ WT_HD uint4 flip_propose(const MS& M, uint32_t t, uint32_t f, uint32_t kind, uin
                          uint32_t it) {
   uint32_t nt = opp_tet(*opp_word(M, t, f));
   uint64_t key = flip_key(it, t);
-  at_min_u64(&FVOTE(M, t), key);
-  at_min_u64(&FVOTE(M, nt), key);
-  if (kind == 1u) at_min_u64(&FVOTE(M, third), key);
+  mesh_min(M, &FVOTE(M, t), key);
+  mesh_min(M, &FVOTE(M, nt), key);
+  if (kind == 1u) mesh_min(M, &FVOTE(M, third), key);
   return make_uint4(t, f | kind << 2 | bad << 3, nt, third);
 }
 
@@ -609,7 +626,7 @@ WT_HD bool flip_face_full(const MS& M, uint32_t t, const uint4& tov, const float
 // External faces keep the old neighbour pointer; flip_update_body fixes
 // them once every flip of the iteration is written.
 // s: the fresh slot of a 2-3 flip.  The caller queues the new tets (the
-// reused slots were claimed by flip_decide_body).
+// reused slots were claimed by flip_decide_load).
 // outk[0]: x,y,z = slots of the new tets (z unused for 3-2), w = kind;
 // outk[1]: the flip's vertices o, a and (3-2) z, for the adjacency update
 // ---------------------------------------------------------------------------
@@ -712,87 +729,47 @@ WT_HD void flip_exec_loaded(const MS& M, const uint4 pr, const FlipTets& F, uint
   }
 }
 
-template <class MS>
-WT_HD void flip_exec_body(const MS& M, const uint4 pr, uint32_t it, uint32_t round,
-                          uint32_t s, uint4* outk) {
-  FlipTets F;
-  flip_load(M, pr, F);
-  flip_exec_loaded(M, pr, F, it, round, s, outk);
-}
-
 // A proposal wins when it holds the vote of every tet it involves; the
 // winner executes at once (its tets belong to no other winner), losers go
 // back to the active list (src/shaders/mark_rejected_flips.wgsl:61-178 and
 // src/shaders/flip.wgsl:531-845, one pass here).
-// Decide proposal j and claim the queue entries it needs: a winner's two
-// reused slots (and, for a 2-3 flip, the fresh slot, counted in *nslot),
-// or a loser's own tet.  qid[0..*nq) are the tets to append to the next
-// active list (kQueued is set here, so each tet is appended once); for a
-// 2-3 winner the fresh slot is appended by the caller after qid.
-template <class MS>
-WT_HD bool flip_decide_body(const MS& M, const uint4& pr, uint32_t it, uint32_t qid[2],
-                            uint32_t* nq, uint32_t* nslot) {
-  *nq = 0;
-  *nslot = 0;
-  if (pr.x == kInvalid) return false;
-  uint64_t key = flip_key(it, pr.x);
-  bool win = FVOTE(M, pr.x) == key && FVOTE(M, pr.z) == key;
-  if (((pr.y >> 2) & 1u) && FVOTE(M, pr.w) != key) win = false;
-  if (win) {
-    uint32_t reuse[2] = {pr.x, pr.z};
-    for (int k = 0; k < 2; ++k) {
-      uint32_t old = at_or_u32(&INFO(M, reuse[k]), kAlive | kQueued);
-      if (!(old & kQueued)) qid[(*nq)++] = reuse[k];
-    }
-    if (((pr.y >> 2) & 1u) == 0u) *nslot = 1;
-  } else {
-    uint32_t old = at_or_u32(&INFO(M, pr.x), kQueued);
-    if (!(old & kQueued)) qid[(*nq)++] = pr.x;
-  }
-  return win;
-}
-
-// flip_decide_body for the list kernel: a winner also loads its flip's
-// tets (into F), issued after its queue claims so that the loads and the
-// claims' round trips overlap.  Same decisions and queue entries.
+// Decide proposal pr and claim the queue entries it needs: a winner's two
+// reused slots (and, for a 2-3 flip, the fresh slot, counted in *nslot), or a
+// loser's own tet.  qid[0..*nq) are the tets to append to the next active
+// list (kQueued is set here, so each tet is appended once); for a 2-3 winner
+// the fresh slot is appended by the caller after qid.  A winner also loads
+// its flip's tets (into F), issued after its queue claims so that the loads
+// and the claims' round trips overlap.
 template <class MS>
 WT_HD bool flip_decide_load(const MS& M, const uint4& pr, uint32_t it, uint32_t qid[2],
                             uint32_t* nq, uint32_t* nslot, FlipTets& F) {
   *nq = 0;
   *nslot = 0;
+  qid[0] = qid[1] = kInvalid;
   if (pr.x == kInvalid) return false;
   uint64_t key = flip_key(it, pr.x);
   bool win = FVOTE(M, pr.x) == key && FVOTE(M, pr.z) == key;
   if (((pr.y >> 2) & 1u) && FVOTE(M, pr.w) != key) win = false;
   if (win) {
-    uint32_t o0 = at_or_u32(&INFO(M, pr.x), kAlive | kQueued);
-    uint32_t o1 = at_or_u32(&INFO(M, pr.z), kAlive | kQueued);
+    uint32_t o0 = mesh_or(M, &INFO(M, pr.x), kAlive | kQueued);
+    uint32_t o1 = mesh_or(M, &INFO(M, pr.z), kAlive | kQueued);
     flip_load(M, pr, F);
-    if (!(o0 & kQueued)) qid[(*nq)++] = pr.x;
-    if (!(o1 & kQueued)) qid[(*nq)++] = pr.z;
+    const bool q0 = !(o0 & kQueued), q1 = !(o1 & kQueued);
+    qid[0] = q0 ? pr.x : pr.z;
+    qid[1] = pr.z;
+    *nq = (uint32_t)q0 + (uint32_t)q1;
     if (((pr.y >> 2) & 1u) == 0u) *nslot = 1;
   } else {
-    uint32_t old = at_or_u32(&INFO(M, pr.x), kQueued);
-    if (!(old & kQueued)) qid[(*nq)++] = pr.x;
+    uint32_t old = mesh_or(M, &INFO(M, pr.x), kQueued);
+    qid[0] = pr.x;
+    *nq = (old & kQueued) ? 0u : 1u;
   }
   return win;
 }
 
-// Sequential form (one proposal at a time, host callers): counters advance
-// with one atomic each.
-template <class MS>
-WT_HD void flip_decide_exec_body(const MS& M, const uint4* prop, uint32_t j, uint32_t it,
-                                 uint32_t round, uint4* out, uint32_t* act_next) {
-  uint4 pr = prop[j];
-  uint32_t qid[2], nq, nslot;
-  bool win = flip_decide_body(M, pr, it, qid, &nq, &nslot);
-  for (uint32_t k = 0; k < nq; ++k) act_next[at_add_u32(&M.ctr[C_ACT_NEXT], 1u)] = qid[k];
-  if (!win) return;
-  uint32_t s = nslot ? at_add_u32(&M.ctr[C_TETS], 1u) : kInvalid;
-  uint32_t f = at_add_u32(&M.ctr[C_FLIPS], 1u);
-  flip_exec_body(M, pr, it, round, s, &out[2 * (size_t)f]);
-  if (nslot) act_next[at_add_u32(&M.ctr[C_ACT_NEXT], 1u)] = s;
-}
+// The proposal of a tet that no kernel of this iteration decides: nobody
+// votes for it, so it loses and stays in the active list.
+WT_HD uint4 requeue_proposal(uint32_t t) { return make_uint4(t, 0u, t, kInvalid); }
 
 // src/shaders/update_opp.wgsl:73-220.  The flip's six external faces
 // (tet T, face e, T's vertex vT opposite e): a face whose neighbour q

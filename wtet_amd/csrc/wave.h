@@ -1,4 +1,5 @@
-// Device helpers that work on a whole wavefront, for the kernels of kernels.hip.
+// Device helpers that work on a whole wavefront, and the flip iteration of one
+// workgroup.
 #pragma once
 
 #include "ops.h"
@@ -106,6 +107,106 @@ __device__ __forceinline__ void flip_check_faces(const MS& M, const uint32_t* ac
     if (grp) prop[j] = flip_propose(M, t, cf, (pk_c >> 2) & 1u, pk_c >> 3, third_c, it);
     else prop[j].x = kInvalid;
   }
+}
+
+// ---------------------------------------------------------------------------
+// A flip iteration in one workgroup: barriers in place of launches, counters
+// in LDS, atomics at workgroup scope.
+// ---------------------------------------------------------------------------
+struct WgCounters {
+  uint32_t act_next;  // length of the next active list
+  uint32_t slots;     // next free tet slot
+  uint32_t flips;     // flips of this iteration
+  uint32_t slow;      // entries deferred to the full predicates
+};
+
+__device__ __forceinline__ uint32_t lds_add(uint32_t* counter, uint32_t v) {
+  return __hip_atomic_fetch_add(counter, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// the active lanes that call this together get consecutive entries of an LDS
+// counter
+__device__ __forceinline__ uint32_t lds_slot(uint32_t* counter) {
+  const uint64_t mask = __ballot(1);
+  const int lane = __lane_id(), leader = __ffsll((unsigned long long)mask) - 1;
+  uint32_t base = 0;
+  if (lane == leader) base = lds_add(counter, (uint32_t)__popcll(mask));
+  return __shfl(base, leader) + __popcll(mask & ((1ull << lane) - 1ull));
+}
+
+// The full predicates on the entries list[0..n) (null: 0..n-1), out of line:
+// their registers and stack stay out of the phases that run for every entry.
+template <class MS, int BS>
+__device__ __noinline__ void wg_slow_check(MS M, const uint32_t* act, uint4* prop, const uint32_t* list, uint32_t n,
+                                           uint32_t it, uint64_t* st) {
+  PredStats ls = {};
+  for (uint32_t k = threadIdx.x; k < 4u * n; k += BS)
+    flip_check_faces(M, act, prop, list ? list[k >> 2] : k >> 2, (int)(k & 3u), it, &ls);
+  flush_stats(ls, st);
+}
+
+// Checks, decides and executes the A entries of act (tag it); the entries of
+// the next iteration go to next.  Every thread of the workgroup of BS threads
+// calls it.  On return c.act_next, c.slots, c.flips and c.slow hold the
+// results and every thread may read them; c.slots counts on from its value
+// before the call.  prop, slow_t: A entries of scratch; out: two per flip.
+template <class MS, int BS>
+__device__ __forceinline__ void wg_flip_iteration(const MS& M, WgCounters& c, const uint32_t* act, uint32_t* next,
+                                                  uint4* prop, uint32_t* slow_t, uint4* out, uint32_t A,
+                                                  uint32_t it, uint32_t round, uint64_t* st) {
+  const uint32_t tid = threadIdx.x;
+  const uint64_t lt = (1ull << __lane_id()) - 1ull;
+  const bool filtered = M.mode == PRED_FILTERED;
+  if (tid == 0) {
+    c.act_next = 0u;
+    c.flips = 0u;
+    c.slow = 0u;
+  }
+  __syncthreads();
+  uint32_t ns = A;
+  if (filtered) {
+    PredStats ls = {};
+    for (uint32_t j = tid; j < A; j += BS)
+      if (flip_check_lean(M, act, prop, j, it, &ls)) slow_t[lds_slot(&c.slow)] = j;
+    flush_stats(ls, st);
+    __syncthreads();
+    ns = c.slow;
+  }
+  if (ns) {
+    wg_slow_check<MS, BS>(M, act, prop, filtered ? slow_t : nullptr, ns, it, st);
+    __syncthreads();
+  }
+  // a wave claims its flips, fresh slots and queue entries with one LDS
+  // atomic each
+  for (uint32_t b = 0; b < A; b += BS) {
+    const uint32_t j = b + tid;
+    uint4 pr = make_uint4(kInvalid, 0u, 0u, 0u);
+    if (j < A) pr = prop[j];
+    uint32_t qid[2], nq, nslot;
+    FlipTets F;
+    const bool win = flip_decide_load(M, pr, it, qid, &nq, &nslot, F);
+    const uint32_t nqa = nq + nslot;
+    const uint64_t bw = __ballot(win), bs = __ballot(nslot), q0 = __ballot(nqa & 1u), q1 = __ballot(nqa & 2u);
+    uint32_t cf = 0, cs = 0, cq = 0;
+    if (__lane_id() == 0) {
+      if (bw) cf = lds_add(&c.flips, __popcll(bw));
+      if (bs) cs = lds_add(&c.slots, __popcll(bs));
+      if (q0 | q1) cq = lds_add(&c.act_next, __popcll(q0) + 2u * __popcll(q1));
+    }
+    cf = __shfl(cf, 0) + __popcll(bw & lt);
+    cs = __shfl(cs, 0) + __popcll(bs & lt);
+    cq = __shfl(cq, 0) + __popcll(q0 & lt) + 2u * __popcll(q1 & lt);
+    if (nq > 0u) next[cq] = qid[0];
+    if (nq > 1u) next[cq + 1u] = qid[1];
+    if (win) {
+      if (nslot) next[cq + nq] = cs;
+      flip_exec_loaded(M, pr, F, it, round, nslot ? cs : kInvalid, &out[2 * (size_t)cf]);
+    }
+  }
+  __syncthreads();
+  const uint32_t nf = c.flips;
+  for (uint32_t k = tid; k < nf; k += BS) flip_update_body(M, out, k, it);
+  __syncthreads();
 }
 
 }  // namespace wtet
