@@ -273,7 +273,7 @@ wtet_status wtet_set_audit_records(wtet_ctx *ctx, uint32_t records);
  * graph is captured the second time its key comes up: the first time its
  * kernels are launched directly.  The list kernels are persistent grid-stride kernels
  * whose grid is sized per round from the host's bound on the first list,
- * for `items` entries per thread (default 2; powers of two from 16 to 4096
+ * for `items` entries per thread (default 1; powers of two from 16 to 4096
  * workgroups, one graph per size).  No counterpart in the reference, which
  * reads counters back every iteration (src/phase1.rs:16-1431). */
 wtet_status wtet_set_flip_graphs(wtet_ctx *ctx, int on);

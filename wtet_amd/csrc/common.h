@@ -11,10 +11,11 @@ namespace wtet {
 constexpr uint32_t kInvalid = 0xFFFFFFFFu;
 constexpr uint64_t kVoteNone = 0xFFFFFFFFFFFFFFFFull;
 
-// tinfo bits
-constexpr uint32_t kAlive = 1u;   // slot holds a live tet
-constexpr uint32_t kQueued = 2u;  // tet id is in the next active list
-constexpr uint32_t kDead = 4u;    // slot freed by a 3-2 flip; tfwd holds a live neighbour
+// A slot's queue tag (Mesh::tqueue): the flip iteration whose list last took
+// the tet, so that a list takes each tet once; kFreed for a slot that a 3-2
+// flip freed (its record then holds kInvalid as first vertex and a live
+// neighbour to go on to).
+constexpr uint32_t kFreed = 0xFFFFFFFFu;
 
 // Face f of a tet is the face opposite vertex f.  kFace[f] lists its three
 // vertex positions ordered so that (face..., v_f) is an even permutation of
@@ -75,18 +76,11 @@ WT_HD uint32_t at_add_u32(uint32_t* p, uint32_t v) {
   return __atomic_fetch_add(p, v, __ATOMIC_RELAXED);
 #endif
 }
-WT_HD uint32_t at_or_u32(uint32_t* p, uint32_t v) {
+WT_HD uint32_t at_max_u32(uint32_t* p, uint32_t v) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  return atomicOr(p, v);
+  return atomicMax(p, v);
 #else
-  return __atomic_fetch_or(p, v, __ATOMIC_RELAXED);
-#endif
-}
-WT_HD uint32_t at_and_u32(uint32_t* p, uint32_t v) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return atomicAnd(p, v);
-#else
-  return __atomic_fetch_and(p, v, __ATOMIC_RELAXED);
+  return __atomic_fetch_max(p, v, __ATOMIC_RELAXED);
 #endif
 }
 
@@ -100,11 +94,11 @@ WT_HD void wg_min_u64(uint64_t* p, uint64_t v) {
   (void)__atomic_fetch_min(p, v, __ATOMIC_RELAXED);
 #endif
 }
-WT_HD uint32_t wg_or_u32(uint32_t* p, uint32_t v) {
+WT_HD uint32_t wg_max_u32(uint32_t* p, uint32_t v) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  return __hip_atomic_fetch_or(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  return __hip_atomic_fetch_max(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 #else
-  return __atomic_fetch_or(p, v, __ATOMIC_RELAXED);
+  return __atomic_fetch_max(p, v, __ATOMIC_RELAXED);
 #endif
 }
 

@@ -53,9 +53,9 @@ struct wtet_ctx {
   // point preparation
   DevBuf xyz_in, xyzn, keys, ids, keys2, ids2, sort_tmp, mm6, pts, doff;
   // mesh (per tet slot)
-  DevBuf tet, adj_t, tinfo, tfwd, tvote, fvote, tsplit, tpoint, tmsg;
+  DevBuf rec, tmsg, tqueue, tvote, fvote;
   // lists
-  DevBuf uvert[2], utet[2], wlist, act[2], prop, fout, blk, slot2idx, rec;
+  DevBuf uvert[2], utet[2], wlist, act[2], prop, fout, blk, slot2idx, viol;
   // output grouping for many clouds
   DevBuf ord[2], ord_tmp, cstart;
   // learned presizing (mlp: the arena of the training calls)
@@ -67,7 +67,11 @@ struct wtet_ctx {
   DevBuf isums, slow_t, slow_p;
   // neighbourhood of the host repair (sparse download)
   DevBuf nbr_mark, nbr_list, nbr_misc, nbr_pack, nbr_seed;
-  uint32_t items = 2;  // list entries per thread the persistent grids are sized for
+  // list entries per thread the persistent grids are sized for.  Every entry
+  // costs its thread the same chain of round trips, so two in turn double it
+  // (device ms at 1 / 2 / 4 entries: 100k points 6.7 / 7.3 / 8.7, 1M 19.2 /
+  // 20.0 / 21.2, 1,024 clouds 39.0 / 39.9 / 41.6)
+  uint32_t items = 1;
   uint32_t audit_records = 1u << 20;  // violation records the first audit of a call keeps
   bool use_graphs = true;
   struct GraphEntry {
@@ -132,9 +136,8 @@ struct wtet_ctx {
 
   wtet_ctx() {
     DevBuf* l[] = {&xyz_in, &xyzn,   &keys,   &ids,   &keys2,  &ids2,     &sort_tmp, &mm6,
-                   &pts,    &doff,   &tet,    &adj_t,  &tinfo,  &tfwd,  &tvote,    &fvote,    &tsplit,  &tpoint,
-                   &tmsg,   &uvert[0], &uvert[1], &utet[0], &utet[1],
-                   &wlist,  &act[0], &act[1], &prop,  &fout,   &blk,      &slot2idx, &rec,
+                   &pts,    &doff,   &rec,    &tmsg,   &tqueue, &tvote,  &fvote,    &uvert[0], &uvert[1], &utet[0], &utet[1],
+                   &wlist,  &act[0], &act[1], &prop,  &fout,   &blk,      &slot2idx, &viol,
                    &ord[0], &ord[1], &ord_tmp, &cstart, &ctr,  &gstats,   &patch,
                    &presize_params, &feat_acc, &feat, &pred, &mlp, &isums, &slow_t, &slow_p,
                    &nbr_mark, &nbr_list, &nbr_misc, &nbr_pack, &nbr_seed};
@@ -289,24 +292,20 @@ void pin_ahead(wtet_ctx* c, size_t rows) {
 void ensure_tets(wtet_ctx* c, uint64_t cap, bool keep) {
   if (cap <= c->cap_tets) return;
   if (cap >= (1ull << 30)) throw Fail{WTET_ERR_OUT_OF_MEMORY, "more than 2^30 tet slots required"};
-  ensure(c, c->tet, cap * 16, keep);
-  ensure(c, c->adj_t, cap * sizeof(AdjRec), keep);
-  ensure(c, c->tinfo, cap * 4, keep);
-  ensure(c, c->tfwd, cap * 4, keep);
+  ensure(c, c->rec, cap * sizeof(TetRec), keep);
+  ensure(c, c->tmsg, cap * sizeof(FlipMsg), keep);
+  ensure(c, c->tqueue, cap * 4, keep);
   ensure(c, c->tvote, cap * 8, keep);
   ensure(c, c->fvote, cap * 8, keep);
-  ensure(c, c->tsplit, cap * 8, keep);
-  ensure(c, c->tpoint, cap * 4, keep);
-  ensure(c, c->tmsg, cap * sizeof(FlipMsg), keep);
   ensure(c, c->act[0], cap * 4, keep);
   ensure(c, c->act[1], cap * 4, keep);
   ensure(c, c->slow_t, cap * 4, false);
   ensure(c, c->prop, cap * 16, false);
-  ensure(c, c->fout, cap * 32, false);  // two uint4 per flip; also the output adjacency
+  ensure(c, c->fout, cap * 32, false);  // 64 bytes per flip of two or more tets; also the output adjacency
   ensure(c, c->slot2idx, cap * 4, false);
   ensure(c, c->blk, (cap / kBlock + 2) * 4, false);
   if (keep) c->stats.grow_events++;
-  c->cap_tets = std::min<uint64_t>(c->tet.bytes / 16, (1ull << 30) - 1);
+  c->cap_tets = std::min<uint64_t>(c->rec.bytes / sizeof(TetRec), (1ull << 30) - 1);
 }
 
 enum KernelKind : int {
@@ -354,15 +353,11 @@ void collect_times(wtet_ctx* c) {
 Mesh mesh_of(wtet_ctx* c, uint32_t inf, int mode) {
   Mesh M;
   M.pts = P<float4>(c->pts);
-  M.tet = P<uint4>(c->tet);
-  M.adj = P<AdjRec>(c->adj_t);
-  M.tinfo = P<uint32_t>(c->tinfo);
-  M.tfwd = P<uint32_t>(c->tfwd);
+  M.rec = P<TetRec>(c->rec);
+  M.tmsg = P<FlipMsg>(c->tmsg);
+  M.tqueue = P<uint32_t>(c->tqueue);
   M.tvote = P<uint64_t>(c->tvote);
   M.fvote = P<uint64_t>(c->fvote);
-  M.tsplit = P<uint2>(c->tsplit);
-  M.tpoint = P<uint32_t>(c->tpoint);
-  M.tmsg = P<FlipMsg>(c->tmsg);
   M.ctr = P<uint32_t>(c->ctr);
   M.inf = inf;
   M.mode = mode;
@@ -451,10 +446,9 @@ constexpr uint32_t kSmallLimit = 2048;
 // The device buffers a captured sequence reads: a graph of another buffer
 // set is stale.
 std::vector<uint64_t> buffer_key(wtet_ctx* c, const Mesh& M, const FlipLists& L, uint64_t* st) {
-  return {(uint64_t)(uintptr_t)M.pts,    (uint64_t)(uintptr_t)M.tet,    (uint64_t)(uintptr_t)M.tvote,
-          (uint64_t)(uintptr_t)M.adj,    (uint64_t)(uintptr_t)M.tinfo,  (uint64_t)(uintptr_t)M.tfwd,
-          (uint64_t)(uintptr_t)M.fvote,  (uint64_t)(uintptr_t)M.tsplit, (uint64_t)(uintptr_t)M.tmsg,
-          (uint64_t)(uintptr_t)M.tpoint, (uint64_t)(uintptr_t)M.ctr,
+  return {(uint64_t)(uintptr_t)M.pts,    (uint64_t)(uintptr_t)M.rec,    (uint64_t)(uintptr_t)M.tmsg,
+          (uint64_t)(uintptr_t)M.tqueue, (uint64_t)(uintptr_t)M.tvote,  (uint64_t)(uintptr_t)M.fvote,
+          (uint64_t)(uintptr_t)M.ctr,
           (uint64_t)M.inf,               (uint64_t)M.mode,              (uint64_t)(uintptr_t)L.act[0],
           (uint64_t)(uintptr_t)L.act[1], (uint64_t)(uintptr_t)L.prop,   (uint64_t)(uintptr_t)L.out,
           (uint64_t)(uintptr_t)L.slow,   (uint64_t)(uintptr_t)st,       (uint64_t)(uintptr_t)c->isums.p,
@@ -640,7 +634,7 @@ void dev_prepare(wtet_ctx* c, Run& R, const float* d_xyz) {
   ensure(c, c->ctr, C_COUNT * 4);
   ensure(c, c->gstats, 64);
   ensure(c, c->isums, S_COUNT * 8);
-  ensure(c, c->rec, (size_t)c->audit_records * 4);
+  ensure(c, c->viol, (size_t)c->audit_records * 4);
   ensure(c, c->blk, ((size_t)round_grid(n) + 2) * 4);
   if (R.learned) {
     if (!c->presize_loaded) throw Fail{WTET_ERR_INVALID_ARGUMENT, "presize_mode 1 needs a model (wtet_set_presize_model)"};
@@ -939,12 +933,12 @@ void dev_compact(wtet_ctx* c, Run& R, uint32_t T, bool out, bool keep_lists) {
 // first pass counted (C_FAILREC); leaves the counters in h_ctr.
 void reaudit(wtet_ctx* c, Run& R, uint32_t T) {
   uint32_t need = c->h_ctr[C_FAILREC];
-  ensure(c, c->rec, ((size_t)need + need / 8 + 1024) * 4);
+  ensure(c, c->viol, ((size_t)need + need / 8 + 1024) * 4);
   Mesh M = mesh_of(c, R.V, R.mode);
   launch_set_ctr(M.ctr, C_VIOL, 0u, C_FAILREC, 0u, c->stream);
-  const uint32_t rec_cap = (uint32_t)std::min<size_t>(c->rec.bytes / 4, 0xFFFFFFFFu);
+  const uint32_t rec_cap = (uint32_t)std::min<size_t>(c->viol.bytes / 4, 0xFFFFFFFFu);
   timed(c, K_AUDIT, [&] {
-    launch_audit(M, T, P<uint32_t>(c->rec), rec_cap, nullptr, P<uint32_t>(c->slow_t), c->stream);
+    launch_audit(M, T, P<uint32_t>(c->viol), rec_cap, nullptr, P<uint32_t>(c->slow_t), c->stream);
   });
   HIP_CHECK(hipGetLastError());
   read_ctr(c);
@@ -973,8 +967,8 @@ void dev_output(wtet_ctx* c, Run& R, std::vector<uint32_t>& viol_rec, uint32_t& 
   uint32_t T = c->h_ctr[C_TETS];
   Mesh M = mesh_of(c, R.V, R.mode);
   launch_set_ctr(M.ctr, C_VIOL, 0u, C_FAILREC, 0u, s);
-  const uint32_t rec_cap = (uint32_t)std::min<size_t>(c->rec.bytes / 4, c->audit_records);
-  timed(c, K_AUDIT, [&] { launch_audit(M, T, P<uint32_t>(c->rec), rec_cap, R.st, P<uint32_t>(c->slow_t), s); });
+  const uint32_t rec_cap = (uint32_t)std::min<size_t>(c->viol.bytes / 4, c->audit_records);
+  timed(c, K_AUDIT, [&] { launch_audit(M, T, P<uint32_t>(c->viol), rec_cap, R.st, P<uint32_t>(c->slow_t), s); });
   dev_compact(c, R, T, true, false);
   HIP_CHECK(hipEventRecord(c->ev1, s));
   cstart.resize((size_t)C + 1);
@@ -1013,8 +1007,8 @@ void dev_output(wtet_ctx* c, Run& R, std::vector<uint32_t>& viol_rec, uint32_t& 
   viol_rec.resize(nrec);
   if (nrec) {
     // records are slot-based; map them to rows on the device
-    launch_map_records(P<uint32_t>(c->rec), nrec, P<uint32_t>(c->slot2idx), s);
-    HIP_CHECK(hipMemcpyAsync(viol_rec.data(), c->rec.p, (size_t)nrec * 4, hipMemcpyDeviceToHost, s));
+    launch_map_records(P<uint32_t>(c->viol), nrec, P<uint32_t>(c->slot2idx), s);
+    HIP_CHECK(hipMemcpyAsync(viol_rec.data(), c->viol.p, (size_t)nrec * 4, hipMemcpyDeviceToHost, s));
   }
   if (R.cfg.collect_stats)
     HIP_CHECK(hipMemcpyAsync(c->stats.pred, c->gstats.p, 64, hipMemcpyDeviceToHost, s));
@@ -1121,7 +1115,7 @@ struct DelaunayArgs {
 // Rows the host repair will read, for a resident result: those within a
 // few face-steps of the recorded faces and the tail rows that fill holes,
 // with their neighbours.  They land in the pinned staging at their own row;
-// present[] marks them.  rec (rows) is on the device in c->rec.
+// present[] marks them.  rec (rows) is on the device in c->viol.
 constexpr int kRepairRingsMax = 16;
 constexpr uint32_t kRepairTail = 4096;
 
@@ -1190,7 +1184,7 @@ void stage_neighbourhood(wtet_ctx* c, uint32_t nrec, uint32_t M, int rings) {
   ensure(c, c->nbr_list, (size_t)M * 4 + 16);
   ensure(c, c->nbr_misc, 4 * (kRepairRingsMax + 4));
   uint32_t* cnt = P<uint32_t>(c->nbr_misc);
-  launch_neighbourhood(P<uint32_t>(c->rec), nrec, M, tail, rings, P<uint32_t>(c->fout),
+  launch_neighbourhood(P<uint32_t>(c->viol), nrec, M, tail, rings, P<uint32_t>(c->fout),
                        P<uint32_t>(c->nbr_mark), P<uint32_t>(c->nbr_list), cnt, cnt + 1, false, s);
   HIP_CHECK(hipGetLastError());
   uint32_t n = listed_rows(c, M);
@@ -2900,9 +2894,9 @@ wtet_status wtet_stage_gather(wtet_ctx* c, wtet_stage_info* info) {
     uint32_t T = c->h_ctr[C_TETS];
     Mesh M = mesh_of(c, S->R.V, S->R.mode);
     launch_set_ctr(M.ctr, C_VIOL, 0u, C_FAILREC, 0u, c->stream);
-    const uint32_t rec_cap = (uint32_t)std::min<size_t>(c->rec.bytes / 4, c->audit_records);
+    const uint32_t rec_cap = (uint32_t)std::min<size_t>(c->viol.bytes / 4, c->audit_records);
     timed(c, K_AUDIT, [&] {
-      launch_audit(M, T, P<uint32_t>(c->rec), rec_cap, S->R.st, P<uint32_t>(c->slow_t), c->stream);
+      launch_audit(M, T, P<uint32_t>(c->viol), rec_cap, S->R.st, P<uint32_t>(c->slow_t), c->stream);
     });
     HIP_CHECK(hipGetLastError());
     read_ctr(c);
@@ -2934,7 +2928,7 @@ wtet_status wtet_stage_readback(wtet_ctx* c, wtet_result* out) {
       std::vector<uint32_t> slot2row(T);
       rec.resize(S->nrec);
       HIP_CHECK(hipMemcpyAsync(slot2row.data(), c->slot2idx.p, (size_t)T * 4, hipMemcpyDeviceToHost, s));
-      HIP_CHECK(hipMemcpyAsync(rec.data(), c->rec.p, (size_t)S->nrec * 4, hipMemcpyDeviceToHost, s));
+      HIP_CHECK(hipMemcpyAsync(rec.data(), c->viol.p, (size_t)S->nrec * 4, hipMemcpyDeviceToHost, s));
       HIP_CHECK(hipStreamSynchronize(s));
       for (uint32_t& r : rec) r = (slot2row[r >> 2] << 2) | (r & 3u);
     }

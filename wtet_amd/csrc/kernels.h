@@ -66,7 +66,7 @@ void launch_pick(const Mesh& M, const uint32_t* uvert, const uint32_t* utet, uin
 struct FlipLists {
   uint32_t* act[2];
   uint4* prop;
-  uint4* out;    // two uint4 per executed flip (flip_exec_loaded)
+  uint4* out;    // four uint4 per executed flip (flip_exec_loaded)
   uint32_t* slow;  // entries the lean check deferred
 };
 // appends the children to the active list after its ctr[C_LIST] entries

@@ -389,15 +389,16 @@ void launch_pick(const Mesh& M, const uint32_t* uvert, const uint32_t* utet, uin
 // Also takes the winners' slots and points off the counters, which no thread
 // of this kernel reads.
 __global__ void __launch_bounds__(kBlock) k_split(Mesh M, const uint2* wlist, FlipLists L) {
-  const uint32_t W = M.ctr[C_WIN], round = M.ctr[C_ROUND];
+  const uint32_t W = M.ctr[C_WIN], round = M.ctr[C_ROUND], it = M.ctr[C_IT];
   uint32_t k = gid();
   if (k == 0) {
+    M.ctr[C_IT0] = it;
     M.ctr[C_TETS] += 3u * W;
     M.ctr[C_SURV] -= W;
     M.ctr[C_SLOW_R] = 0u;
   }
   uint32_t c[4], m = 0u;
-  if (k < W) m = split_body(M, wlist, k, round, c);
+  if (k < W) m = split_body(M, wlist, k, round, it + 1u, c);
   uint64_t lt = (1ull << __lane_id()) - 1ull;
   uint64_t b0 = __ballot(m & 1u), bv = __ballot(m != 0u);
   uint32_t n0 = __popcll(b0), nv = __popcll(bv);
@@ -469,7 +470,7 @@ __device__ __forceinline__ void batch_end(uint32_t* ctr, unsigned long long* sum
   if (peak > ctr[C_PEAKA]) ctr[C_PEAKA] = peak;
   if (n < k && left > 0u) ctr[C_STOP] = 1u;  // the tet slots could not hold the next one
   ctr[C_LIST] = left;
-  ctr[C_IT] += (uint32_t)k;
+  ctr[C_IT] += (uint32_t)n;  // the list left is that of the next iteration
   ctr[C_PAR] ^= (uint32_t)n & 1u;
 }
 
@@ -619,6 +620,11 @@ __device__ __forceinline__ uint32_t block_prefix3(uint32_t a, uint32_t b, uint32
 // next active entries) -- the counters share a cache line, so per-wave
 // atomics from every wave would serialize -- and every winner executes its
 // own flip from registers.
+// A tet's plain-stored fields are one 64-byte record (TetRec) and the update
+// finds the external neighbours in the flip's own record.  Event time at 1M
+// points against an array per field: flip_check 5.58 -> 4.28 ms (it reads one
+// line of a tet instead of three, and no queued bit to clear), decide_exec 6.81
+// -> 5.83 ms, flip_update 4.83 -> 4.39 ms.
 // Blocks of 512 threads: each tile of proposals claims its flips, fresh
 // slots and queue entries with one atomic per counter, and those
 // same-address atomics complete one at a time at the memory side; 512
@@ -631,7 +637,7 @@ __global__ void __launch_bounds__(kDecBlock) k_flip_decide_exec(Mesh M, FlipList
   __shared__ uint32_t wsum[kBS / 64];
   __shared__ uint32_t base[3];
   if (!*it_ctr(M.ctr, C_ITR, i)) return;
-  const uint32_t A = *it_ctr(M.ctr, C_ITA, i), it = iter_tag(M.ctr, i), round = M.ctr[C_ROUND];
+  const uint32_t A = *it_ctr(M.ctr, C_ITA, i), it = iter_tag(M.ctr, i);
   uint32_t* act_next = L.act[iter_par(M.ctr, i) ^ 1u];
   for (uint32_t b0 = blockIdx.x * kBS; b0 < A; b0 += gridDim.x * kBS) {
     uint32_t j = b0 + threadIdx.x;
@@ -657,7 +663,7 @@ __global__ void __launch_bounds__(kDecBlock) k_flip_decide_exec(Mesh M, FlipList
     if (win) {
       uint32_t sl = nslot ? base[1] + rs : kInvalid;
       if (nslot) act_next[q + nq] = sl;
-      flip_exec_loaded(M, pr, F, it, round, sl, &L.out[2 * (size_t)(base[0] + rf)]);
+      flip_exec_loaded(M, pr, F, it, sl, &L.out[4 * (size_t)(base[0] + rf)]);
     }
     // the next tile's prefix sums synchronize before base is rewritten
   }
@@ -682,7 +688,7 @@ __global__ void __launch_bounds__(kFlipSmallBlock) k_flip_small(WgMesh M, FlipLi
                                                                 unsigned long long* sums, int k, uint32_t limit) {
   __shared__ WgCounters c;
   uint32_t* ctr = M.ctr;
-  const uint32_t round = ctr[C_ROUND], tets0 = ctr[C_TETS], cap = ctr[C_CAP], it0 = ctr[C_IT];
+  const uint32_t tets0 = ctr[C_TETS], cap = ctr[C_CAP], it0 = ctr[C_IT];
   uint32_t A = ctr[C_LIST], par = ctr[C_PAR] & 1u, tets = tets0, sa = 0, sf = 0, peak = 0, slow = 0, last = 0;
   bool stop = ctr[C_STOP] != 0u;
   int n = 0;
@@ -693,7 +699,7 @@ __global__ void __launch_bounds__(kFlipSmallBlock) k_flip_small(WgMesh M, FlipLi
       break;
     }
     wg_flip_iteration<WgMesh, kFlipSmallBlock>(M, c, par ? L.act[1] : L.act[0], par ? L.act[0] : L.act[1], L.prop,
-                                               L.slow, L.out, A, it0 + (uint32_t)n + 1u, round, st);
+                                               L.slow, L.out, A, it0 + (uint32_t)n + 1u, st);
     sa += A;
     sf += c.flips;
     slow += c.slow;
@@ -717,7 +723,7 @@ __global__ void __launch_bounds__(kFlipSmallBlock) k_flip_small(WgMesh M, FlipLi
     if (peak > ctr[C_PEAKA]) ctr[C_PEAKA] = peak;
     if (stop) ctr[C_STOP] = 1u;
     ctr[C_LIST] = A;
-    ctr[C_IT] = it0 + (uint32_t)k;
+    ctr[C_IT] = it0 + (uint32_t)n;
     ctr[C_PAR] = par;
   }
 }
@@ -756,22 +762,22 @@ void launch_flip_update(const Mesh& M, const FlipLists& L, int i, uint32_t grid,
   k_flip_update<<<grid, kBlock, 0, s>>>(M, L, i);
 }
 
-// The uninserted points after the round's pick (ctr[C_SURV]), round
-// ctr[C_ROUND].  end > 0: the last form's first workgroup ends the batch of
+// The uninserted points after the round's pick (ctr[C_SURV]) whose tet a flip
+// since the split (ctr[C_IT0]) took apart.  end > 0: the last form's first workgroup ends the batch of
 // `end` iterations, which none of these kernels reads the counters of.
 template <int FORM>
 __global__ void __launch_bounds__(kBlock) k_relocate(Mesh M, const uint32_t* uvert, uint32_t* utet,
                                                      uint64_t* st, uint32_t* slow, unsigned long long* sums, int end) {
-  const uint32_t U = M.ctr[C_SURV], round = M.ctr[C_ROUND];
+  const uint32_t U = M.ctr[C_SURV], it0 = M.ctr[C_IT0];
   PredStats ls = {};
   if (FORM == SLOW) {
     uint32_t n = M.ctr[C_SLOW_R], stride = gridDim.x * blockDim.x;
     for (uint32_t k = gid(); k < n; k += stride)
-      (void)relocate_body_t<false>(M, uvert, utet, slow[k], round, &ls);
+      (void)relocate_body_t<false>(M, uvert, utet, slow[k], it0, &ls);
   } else {
     uint32_t i = gid();
     bool defer = false;
-    if (i < U) defer = relocate_body_t<FORM == LEAN>(M, uvert, utet, i, round, &ls);
+    if (i < U) defer = relocate_body_t<FORM == LEAN>(M, uvert, utet, i, it0, &ls);
     if (defer) slow[append_slot(&M.ctr[C_SLOW_R])] = i;
   }
   flush_stats(ls, st);
@@ -832,7 +838,7 @@ void launch_audit(const Mesh& M, uint32_t T, uint32_t* rec, uint32_t cap, uint64
 template <class MS>
 __global__ void k_alive_count(MS M, uint32_t T, uint32_t* blk) {
   uint32_t t = gid();
-  bool a = t < T && (INFO(M, t) & kAlive);
+  bool a = t < T && slot_alive(M, t);
   uint32_t tot;
   block_rank(a, &tot);
   if (threadIdx.x == 0) blk[blockIdx.x] = tot;
@@ -842,7 +848,7 @@ __global__ void k_alive_count(MS M, uint32_t T, uint32_t* blk) {
 __global__ void k_alive_scatter(Mesh M, uint32_t T, const uint32_t* blk, uint32_t* olist,
                                 uint32_t* slot2pos) {
   uint32_t t = gid();
-  bool a = t < T && (INFO(M, t) & kAlive);
+  bool a = t < T && slot_alive(M, t);
   uint32_t tot;
   uint32_t r = blk[blockIdx.x] + block_rank(a, &tot);
   if (t < T) {
@@ -855,7 +861,7 @@ __global__ void k_alive_scatter(Mesh M, uint32_t T, const uint32_t* blk, uint32_
 __global__ void k_slot_keys(Mesh M, uint32_t T, Clouds K, uint32_t* okey, uint32_t* oslot) {
   uint32_t t = gid();
   if (t >= T) return;
-  okey[t] = (INFO(M, t) & kAlive) ? cloud_of_tet(M, t, K) : K.C;
+  okey[t] = slot_alive(M, t) ? cloud_of_tet(M, t, K) : K.C;
   oslot[t] = t;
 }
 

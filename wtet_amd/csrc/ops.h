@@ -17,10 +17,10 @@ enum Ctr : int {
   // read by every thread of the flip kernels, written between kernels: the
   // first line.  Counters that take atomics at volume sit 1 KB or more apart,
   // away from it and from each other.
-  C_IT = 0,         // flip iterations before this batch (fvote keys, flip stamps)
+  C_IT = 0,         // flip iterations before this batch (fvote keys, stamps, queue tags)
   C_PAR = 1,        // which of the two active lists the batch begins with
   C_STOP = 2,       // set when an iteration could overflow the tet slots
-  C_ROUND = 3,      // insertion round (flip stamps)
+  C_ROUND = 3,      // insertion round (split records)
   C_CAP = 4,        // tet slot capacity
   C_PEAKA = 5,      // longest active list seen
   C_TETS_IT = 6,    // C_TETS when the batch of iterations began
@@ -32,6 +32,7 @@ enum Ctr : int {
   C_BADTET = 12,    // points found in a tet touching infinity (must stay 0)
   C_NPTS = 13,      // points to insert (input minus exact duplicates)
   C_DUPSCAN = 14,   // duplicate scans that hit their length cap
+  C_IT0 = 16,       // flip iterations before this round
   C_SURV = 15,      // uninserted points (the pick's winners leave at the split)
   C_TETS = 256,     // next free tet slot (the winners' at the split)
   C_LIST = 512,     // length of the active list between batches of iterations
@@ -72,52 +73,64 @@ struct __attribute__((aligned(32))) AdjRec {
   uint4 hi;  // faces 2, 3
 };
 
+// One tet slot's record, a 64-byte half line: everything about it that plain
+// stores write and that the kernels read at random.  What atomics write (the
+// votes, the queue tag) is in arrays of its own: atomics complete at the
+// memory side, and a plain store beside them would leave the line dirty in
+// an XCD's L2.  Measured against an array per field (the check then read
+// three lines of a tet, a flip wrote three of each new tet): see
+// k_flip_decide_exec.
+struct __attribute__((aligned(64))) TetRec {
+  AdjRec adj;      // neighbours and the vertices across the faces
+  uint4 v;         // vertex ids; x = kInvalid when a 3-2 flip freed the slot
+  uint2 split;     // (round, first new slot) for a tet split this round
+  uint32_t point;  // the point inserted into a tet split this round; in a freed
+                   // slot a live neighbour
+  uint32_t stamp;  // tag of the last flip iteration that took the tet apart
+};
+
 // Where the faces of a tet destroyed by a flip went: for each external face
 // f, w[2f] = (new tet << 2) | face and w[2f + 1] = the new tet's vertex
 // opposite it (one 8-byte load per face in flip_update_body).
-struct __attribute__((aligned(64))) FlipMsg {
-  uint4 lo;        // faces 0, 1
-  uint4 hi;        // faces 2, 3
-  uint64_t stamp;  // the last flip that wrote the slot: round << 32 | flip iteration
-  uint64_t pad[3];
+struct __attribute__((aligned(32))) FlipMsg {
+  uint4 lo;  // faces 0, 1
+  uint4 hi;  // faces 2, 3
 };
 
 // message of a destroyed tet: new neighbour pointers e (kInvalid where
 // unused), all opposite the vertex v
-template <class MSG>
-WT_HD void set_msg(MSG* m, uint4 e, uint32_t v) {
+WT_HD void set_msg(FlipMsg* m, uint4 e, uint32_t v) {
   m->lo = make_uint4(e.x, v, e.y, v);
   m->hi = make_uint4(e.z, v, e.w, v);
 }
 
 static_assert(sizeof(AdjRec) == 32, "adjacency record layout");
-static_assert(sizeof(FlipMsg) == 64, "flip message layout: one 64-byte line per slot");
+static_assert(sizeof(TetRec) == 64, "half a line per slot");
+static_assert(sizeof(FlipMsg) == 32, "flip message layout");
 
 struct Mesh {
   const float4* pts;  // n + 5 points (n real, 4 super, 1 infinity)
-  uint4* tet;         // vertex ids
-  AdjRec* adj;        // neighbours and the vertices across the faces
-  uint32_t* tinfo;    // kAlive | kQueued | kDead
-  uint32_t* tfwd;     // live neighbour of a slot freed by a 3-2 flip
-  uint64_t* tvote;    // insertion vote (min key)
-  uint64_t* fvote;    // flip vote (min key, iteration-tagged)
-  uint2* tsplit;      // (round, first new slot) for tets split this round
-  uint32_t* tpoint;   // the point inserted into a tet split this round
-  FlipMsg* tmsg;      // per slot destroyed by a flip this iteration
-  uint32_t* ctr;      // Ctr counters
-  uint32_t inf;       // id of the infinity vertex
-  int mode;           // PredMode
+  TetRec* rec;
+  FlipMsg* tmsg;     // per slot destroyed by a flip this iteration
+  uint32_t* tqueue;  // queue tag, kFreed
+  uint64_t* tvote;   // insertion vote (min key)
+  uint64_t* fvote;   // flip vote (min key, iteration-tagged)
+  uint32_t* ctr;     // Ctr counters
+  uint32_t inf;      // id of the infinity vertex
+  int mode;          // PredMode
 };
 
-WT_HD uint4& TV(const Mesh& M, uint32_t t) { return M.tet[t]; }
-WT_HD AdjRec& ADJ(const Mesh& M, uint32_t t) { return M.adj[t]; }
-WT_HD uint32_t& INFO(const Mesh& M, uint32_t t) { return M.tinfo[t]; }
-WT_HD uint32_t& TFWD(const Mesh& M, uint32_t t) { return M.tfwd[t]; }
+WT_HD uint4& TV(const Mesh& M, uint32_t t) { return M.rec[t].v; }
+WT_HD AdjRec& ADJ(const Mesh& M, uint32_t t) { return M.rec[t].adj; }
+WT_HD uint2& TSPLIT(const Mesh& M, uint32_t t) { return M.rec[t].split; }
+WT_HD uint32_t& TPOINT(const Mesh& M, uint32_t t) { return M.rec[t].point; }
+WT_HD uint32_t& TFWD(const Mesh& M, uint32_t t) { return M.rec[t].point; }
+WT_HD uint32_t& FSTAMP(const Mesh& M, uint32_t t) { return M.rec[t].stamp; }
+WT_HD FlipMsg& TMSG(const Mesh& M, uint32_t t) { return M.tmsg[t]; }
+WT_HD uint32_t& TQUEUE(const Mesh& M, uint32_t t) { return M.tqueue[t]; }
 WT_HD uint64_t& TVOTE(const Mesh& M, uint32_t t) { return M.tvote[t]; }
 WT_HD uint64_t& FVOTE(const Mesh& M, uint32_t t) { return M.fvote[t]; }
-WT_HD uint2& TSPLIT(const Mesh& M, uint32_t t) { return M.tsplit[t]; }
-WT_HD uint32_t& TPOINT(const Mesh& M, uint32_t t) { return M.tpoint[t]; }
-WT_HD FlipMsg& TMSG(const Mesh& M, uint32_t t) { return M.tmsg[t]; }
+WT_HD bool slot_alive(const Mesh& M, uint32_t t) { return M.tqueue[t] != kFreed; }
 
 // The same mesh while one workgroup alone changes it: its atomics need the
 // workgroup's scope only and complete in the XCD's L2 instead of at the
@@ -126,9 +139,9 @@ struct WgMesh : Mesh {};
 
 // atomics at the scope the mesh is shared at
 WT_HD void mesh_min(const Mesh&, uint64_t* p, uint64_t v) { at_min_u64(p, v); }
-WT_HD uint32_t mesh_or(const Mesh&, uint32_t* p, uint32_t v) { return at_or_u32(p, v); }
+WT_HD uint32_t mesh_max(const Mesh&, uint32_t* p, uint32_t v) { return at_max_u32(p, v); }
 WT_HD void mesh_min(const WgMesh&, uint64_t* p, uint64_t v) { wg_min_u64(p, v); }
-WT_HD uint32_t mesh_or(const WgMesh&, uint32_t* p, uint32_t v) { return wg_or_u32(p, v); }
+WT_HD uint32_t mesh_max(const WgMesh&, uint32_t* p, uint32_t v) { return wg_max_u32(p, v); }
 
 template <class MS>
 WT_HD uint4 TN(const MS& M, uint32_t t) {
@@ -146,12 +159,6 @@ WT_HD void set_adj(const MS& M, uint32_t t, uint4 n, uint4 ov) {
   ADJ(M, t).lo = make_uint4(n.x, ov.x, n.y, ov.y);
   ADJ(M, t).hi = make_uint4(n.z, ov.z, n.w, ov.w);
 }
-// the stamp shares its slot's message line: the adjacency update reads a
-// flipped neighbour's stamp and message together
-template <class MS>
-WT_HD uint64_t& FSTAMP(const MS& M, uint32_t t) { return TMSG(M, t).stamp; }
-WT_HD uint64_t flip_stamp(uint32_t round, uint32_t it) { return (uint64_t)round << 32 | it; }
-
 template <class MS>
 WT_HD float3 P3(const MS& M, uint32_t v) {
   float4 p = M.pts[v];
@@ -299,11 +306,12 @@ WT_HD uint32_t child_slot(uint32_t t, uint32_t base, uint32_t j) {
 }
 
 // c[0..3] receives the children's slots; returns which of them join the
-// active list (bit j for child j; slot t only if no earlier list holds it).
+// active list of iteration `it` (bit j for child j; slot t only if the list
+// does not hold it yet).
 // The neighbours' split records are loaded before any store: this kernel
 // writes those of fresh slots only, never a neighbour's.
 template <class MS>
-WT_HD uint32_t split_body(const MS& M, const uint2* wlist, uint32_t k, uint32_t round,
+WT_HD uint32_t split_body(const MS& M, const uint2* wlist, uint32_t k, uint32_t round, uint32_t it,
                           uint32_t c[4]) {
   uint32_t t = wlist[k].x, p = wlist[k].y;
   uint32_t base = TSPLIT(M, t).y;
@@ -343,14 +351,13 @@ WT_HD uint32_t split_body(const MS& M, const uint2* wlist, uint32_t k, uint32_t 
     set_adj(M, c[j], no, nov);
     TVOTE(M, c[j]) = kVoteNone;
     if (j > 0) {  // fresh slot: initialise every per-slot field
-      INFO(M, c[j]) = kAlive | kQueued;
+      TQUEUE(M, c[j]) = it;
       FVOTE(M, c[j]) = kVoteNone;
       TSPLIT(M, c[j]) = make_uint2(0u, 0u);
-      FSTAMP(M, c[j]) = 0ull;
+      FSTAMP(M, c[j]) = 0u;
     }
   }
-  uint32_t old = mesh_or(M, &INFO(M, t), kQueued);
-  return (old & kQueued) ? 0xEu : 0xFu;
+  return mesh_max(M, &TQUEUE(M, t), it) == it ? 0xEu : 0xFu;
 }
 
 // ---------------------------------------------------------------------------
@@ -491,23 +498,19 @@ WT_HD int face_classify(const float* x, const float* y, const float* z, const fl
 
 // Lean check of list entry j, one thread per tet: FP32 filters, and the FP64
 // filter for the faces whose insphere they leave.  The first face (in order)
-// that can flip is proposed; true (no side effect but the queued bit) when a
+// that can flip is proposed; true (with no vote cast) when a
 // face before it is undecided, and the entry needs the full predicates.
 template <class MS>
 WT_HD bool flip_check_lean(const MS& M, const uint32_t* act, uint4* prop, uint32_t j, uint32_t it,
                            PredStats* st) {
   uint32_t t = act[j];
-  // Two memory round trips: the slot's info, vertices and opposite vertices
-  // together (all in the slot's own records), then all eight points (the
-  // point array includes the infinity vertex, so every id is loadable).
-  uint32_t info = INFO(M, t);
+  // Two memory round trips: the slot's record (vertices and opposite
+  // vertices), then all eight points (the point array includes the infinity
+  // vertex, so every id is loadable).
   uint4 tv = TV(M, t);
   uint4 tov = TOV(M, t);
-  // each tet is on the list once and no other thread of this kernel writes
-  // its info word: a plain read-modify-write clears the queued bit
-  INFO(M, t) = info & ~kQueued;
   prop[j].x = kInvalid;
-  if (!(info & kAlive)) return false;
+  if (tv.x == kInvalid) return false;  // freed since it was queued
   if (tv.x == M.inf || tv.y == M.inf || tv.z == M.inf || tv.w == M.inf) return false;
   float P[4][3], Q[4][3];
   uint32_t r;
@@ -627,8 +630,10 @@ WT_HD bool flip_face_full(const MS& M, uint32_t t, const uint4& tov, const float
 // them once every flip of the iteration is written.
 // s: the fresh slot of a 2-3 flip.  The caller queues the new tets (the
 // reused slots were claimed by flip_decide_load).
-// outk[0]: x,y,z = slots of the new tets (z unused for 3-2), w = kind;
-// outk[1]: the flip's vertices o, a and (3-2) z, for the adjacency update
+// outk, the flip's record for the adjacency update (64 bytes: the update
+// reads it in order instead of the new tets' own records): slots of the new
+// tets (the third unused for 3-2) and the kind; the vertices o, a and (3-2)
+// z; the six external neighbour pointers in flip_update_body's order
 // ---------------------------------------------------------------------------
 // The records a flip reads: vertices, neighbours and opposite vertices of
 // its two (2-3) or three (3-2) tets.  Loading them is split from the flip so
@@ -649,7 +654,7 @@ WT_HD void flip_load(const MS& M, const uint4& pr, FlipTets& F) {
 
 template <class MS>
 WT_HD void flip_exec_loaded(const MS& M, const uint4 pr, const FlipTets& F, uint32_t it,
-                            uint32_t round, uint32_t s, uint4* outk) {
+                            uint32_t s, uint4* outk) {
   uint32_t t = pr.x, f = pr.y & 3u, kind = (pr.y >> 2) & 1u, edge = (pr.y >> 3) & 3u;
   uint32_t n = pr.z;
   const uint4 tv = F.tv, to = F.to, tov = F.tov;
@@ -682,15 +687,17 @@ WT_HD void flip_exec_loaded(const MS& M, const uint4 pr, const FlipTets& F, uint
     set4(mn, qy, enc_opp(Tzx, 3));
     set_msg(&TMSG(M, t), mt, o);
     set_msg(&TMSG(M, n), mn, a);
-    FSTAMP(M, t) = flip_stamp(round, it);
-    FSTAMP(M, n) = flip_stamp(round, it);
+    FSTAMP(M, t) = it;
+    FSTAMP(M, n) = it;
     TVOTE(M, s) = kVoteNone;
     FVOTE(M, s) = kVoteNone;
     TSPLIT(M, s) = make_uint2(0u, 0u);
-    FSTAMP(M, s) = 0ull;
-    INFO(M, s) = kAlive | kQueued;  // fresh slot: queued by the caller
+    FSTAMP(M, s) = 0u;
+    TQUEUE(M, s) = it + 1u;  // fresh slot: queued by the caller
     outk[0] = make_uint4(Txy, Tyz, Tzx, 0u);
-    outk[1] = make_uint4(o, a, 0u, 0u);
+    outk[1] = make_uint4(o, a, 0u, get4(to, pos[2]));
+    outk[2] = make_uint4(get4(no, qz), get4(to, pos[0]), get4(no, qx), get4(to, pos[1]));
+    outk[3].x = get4(no, qy);
   } else {
     // rotate the face triple so the offending edge is (x, y), third z
     uint32_t x = get4(tv, pos[edge]), y = get4(tv, pos[(edge + 1) % 3]),
@@ -719,13 +726,16 @@ WT_HD void flip_exec_loaded(const MS& M, const uint4 pr, const FlipTets& F, uint
     set_msg(&TMSG(M, t), mt, o);
     set_msg(&TMSG(M, n), mn, a);
     set_msg(&TMSG(M, m), mm, z);
-    FSTAMP(M, t) = flip_stamp(round, it);
-    FSTAMP(M, n) = flip_stamp(round, it);
-    FSTAMP(M, m) = flip_stamp(round, it);
-    INFO(M, m) = kDead;
+    FSTAMP(M, t) = it;
+    FSTAMP(M, n) = it;
+    FSTAMP(M, m) = it;
+    TQUEUE(M, m) = kFreed;
+    TV(M, m).x = kInvalid;
     TFWD(M, m) = A;
     outk[0] = make_uint4(A, B, kInvalid, 1u);
-    outk[1] = make_uint4(o, a, z, 0u);
+    outk[1] = make_uint4(o, a, z, get4(no, qy));
+    outk[2] = make_uint4(get4(mo, my), get4(to, py), get4(mo, mx), get4(no, qx));
+    outk[3].x = get4(to, px);
   }
 }
 
@@ -736,7 +746,8 @@ WT_HD void flip_exec_loaded(const MS& M, const uint4 pr, const FlipTets& F, uint
 // Decide proposal pr and claim the queue entries it needs: a winner's two
 // reused slots (and, for a 2-3 flip, the fresh slot, counted in *nslot), or a
 // loser's own tet.  qid[0..*nq) are the tets to append to the next active
-// list (kQueued is set here, so each tet is appended once); for a 2-3 winner
+// list, that of iteration it + 1 (their queue tag is set here, so each tet is
+// appended once); for a 2-3 winner
 // the fresh slot is appended by the caller after qid.  A winner also loads
 // its flip's tets (into F), issued after its queue claims so that the loads
 // and the claims' round trips overlap.
@@ -751,18 +762,17 @@ WT_HD bool flip_decide_load(const MS& M, const uint4& pr, uint32_t it, uint32_t 
   bool win = FVOTE(M, pr.x) == key && FVOTE(M, pr.z) == key;
   if (((pr.y >> 2) & 1u) && FVOTE(M, pr.w) != key) win = false;
   if (win) {
-    uint32_t o0 = mesh_or(M, &INFO(M, pr.x), kAlive | kQueued);
-    uint32_t o1 = mesh_or(M, &INFO(M, pr.z), kAlive | kQueued);
+    uint32_t o0 = mesh_max(M, &TQUEUE(M, pr.x), it + 1u);
+    uint32_t o1 = mesh_max(M, &TQUEUE(M, pr.z), it + 1u);
     flip_load(M, pr, F);
-    const bool q0 = !(o0 & kQueued), q1 = !(o1 & kQueued);
+    const bool q0 = o0 != it + 1u, q1 = o1 != it + 1u;
     qid[0] = q0 ? pr.x : pr.z;
     qid[1] = pr.z;
     *nq = (uint32_t)q0 + (uint32_t)q1;
     if (((pr.y >> 2) & 1u) == 0u) *nslot = 1;
   } else {
-    uint32_t old = mesh_or(M, &INFO(M, pr.x), kQueued);
     qid[0] = pr.x;
-    *nq = (old & kQueued) ? 0u : 1u;
+    *nq = mesh_max(M, &TQUEUE(M, pr.x), it + 1u) != it + 1u ? 1u : 0u;
   }
   return win;
 }
@@ -775,15 +785,16 @@ WT_HD uint4 requeue_proposal(uint32_t t) { return make_uint4(t, 0u, t, kInvalid)
 // (tet T, face e, T's vertex vT opposite e): a face whose neighbour q
 // flipped too takes the tet and vertex that q's flip left in its message;
 // otherwise q's face points back at T.  Every load comes before the first
-// store (the flip record, the pointers, then tags and messages: three round
-// trips): no thread of this kernel
-// stores a word that one of these loads reads (a flipped tet's external face
-// is rewritten only by its own flip, after the read; an unflipped
-// neighbour's face is never read; tags and messages are read-only here).
+// store (the flip record, the stamps in the records that most faces then
+// write, and the messages of the few neighbours that flipped): no
+// thread of this kernel
+// stores a word that one of these loads reads (stamps and messages are
+// read-only here).
 template <class MS>
 WT_HD void flip_update_body(const MS& M, const uint4* out, uint32_t k, uint32_t it) {
-  uint4 r = out[2 * (size_t)k];
-  uint4 w = out[2 * (size_t)k + 1];  // o, a, z
+  uint4 r = out[4 * (size_t)k];
+  uint4 w = out[4 * (size_t)k + 1];  // o, a, z
+  uint4 p = out[4 * (size_t)k + 2];
   // 2-3: new tets (x, y, o, a), external faces 2 (apex o) and 3 (apex a);
   // 3-2: A = (a, z, o, x), B = (z, a, o, y), external faces 0, 1, 2.
   // Selected without a branch, so the record is read in one round trip.
@@ -792,14 +803,13 @@ WT_HD void flip_update_body(const MS& M, const uint4* out, uint32_t k, uint32_t 
   uint32_t E[6] = {k32 ? 0u : 2u, k32 ? 1u : 3u, 2u, k32 ? 0u : 3u, k32 ? 1u : 2u, k32 ? 2u : 3u};
   uint32_t V[6] = {k32 ? w.y : w.x, k32 ? w.z : w.y, w.x, k32 ? w.z : w.y, k32 ? w.y : w.x,
                    k32 ? w.x : w.y};
-  uint32_t ptr[6], fq[6];
+  uint32_t ptr[6] = {w.w, p.x, p.y, p.z, p.w, out[4 * (size_t)k + 3].x}, fq[6];
   uint2 msg[6];
-  for (int i = 0; i < 6; ++i) ptr[i] = *opp_word(M, T[i], E[i]);
-  for (int i = 0; i < 6; ++i) fq[i] = (uint32_t)FSTAMP(M, opp_tet(ptr[i]));
-  // every neighbour is a valid slot: its message is loaded unconditionally
-  // (stale where it did not flip, then unused), so no branch splits the loads
-  for (int i = 0; i < 6; ++i)
-    msg[i] = reinterpret_cast<const uint2*>(&TMSG(M, opp_tet(ptr[i])))[opp_face(ptr[i])];
+  for (int i = 0; i < 6; ++i) fq[i] = FSTAMP(M, opp_tet(ptr[i]));
+  for (int i = 0; i < 6; ++i) {
+    msg[i] = make_uint2(0u, 0u);
+    if (fq[i] == it) msg[i] = reinterpret_cast<const uint2*>(&TMSG(M, opp_tet(ptr[i])))[opp_face(ptr[i])];
+  }
   // one 8-byte store per face, its slot and value chosen without a branch
   for (int i = 0; i < 6; ++i) {
     bool fl = fq[i] == it;
@@ -858,23 +868,18 @@ WT_HD uint32_t walk_to_t(const MS& M, uint32_t t, uint32_t q, uint32_t seed, Pre
 }
 
 template <bool FAST, class MS>
+// it0: flip iterations before this round
 WT_HD bool relocate_body_t(const MS& M, const uint32_t* uvert, uint32_t* utet, uint32_t i,
-                           uint32_t round, PredStats* st) {
+                           uint32_t it0, PredStats* st) {
   uint32_t t = utet[i];
-  if ((uint32_t)(FSTAMP(M, t) >> 32) != round) return false;
-  for (int guard = 0; guard < 64 && (INFO(M, t) & kDead); ++guard) t = TFWD(M, t);
+  if (FSTAMP(M, t) <= it0) return false;
+  for (int guard = 0; guard < 64 && TV(M, t).x == kInvalid; ++guard) t = TFWD(M, t);
   int state = 0;
   t = walk_to_t<FAST>(M, t, uvert[i], i * 0x85EBCA6Bu, st, &state);
   if (state == 2) return true;  // the full walk restarts from utet[i]
   if (state == 1) at_add_u32(&M.ctr[C_WALK_FAIL], 1u);
   utet[i] = t;
   return false;
-}
-
-template <class MS>
-WT_HD void relocate_body(const MS& M, const uint32_t* uvert, uint32_t* utet, uint32_t i,
-                         uint32_t round, PredStats* st) {
-  (void)relocate_body_t<false>(M, uvert, utet, i, round, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -886,7 +891,7 @@ WT_HD void relocate_body(const MS& M, const uint32_t* uvert, uint32_t* utet, uin
 // ---------------------------------------------------------------------------
 template <bool FAST, class MS>
 WT_HD bool audit_body_t(const MS& M, uint32_t t, uint32_t* rec, uint32_t cap, PredStats* st) {
-  if (!(INFO(M, t) & kAlive)) return false;
+  if (!slot_alive(M, t)) return false;
   uint4 tv = TV(M, t);
   if (tv.x == M.inf || tv.y == M.inf || tv.z == M.inf || tv.w == M.inf) return false;
   uint4 to = TN(M, t);

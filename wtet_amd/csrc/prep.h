@@ -289,11 +289,11 @@ WT_HD void start_tet_at(const MS& M, const StartTets& S, uint32_t c, uint32_t t,
   }
   TV(M, g) = tv;
   set_adj(M, g, to, tov);
-  INFO(M, g) = kAlive;
+  TQUEUE(M, g) = 0u;
   TVOTE(M, g) = kVoteNone;
   FVOTE(M, g) = kVoteNone;
   TSPLIT(M, g) = make_uint2(0u, 0u);
-  FSTAMP(M, g) = 0ull;
+  FSTAMP(M, g) = 0u;
 }
 
 // g in [0, 5C): start tet g % 5 of cloud g / 5, in slot g

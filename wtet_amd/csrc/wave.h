@@ -81,10 +81,9 @@ template <class MS>
 __device__ __forceinline__ void flip_check_faces(const MS& M, const uint32_t* act, uint4* prop, uint32_t j,
                                                  int f, uint32_t it, PredStats* st) {
   const uint32_t t = act[j];
-  const uint32_t info = INFO(M, t);
   const uint4 tv = TV(M, t);
   const uint4 tov = TOV(M, t);
-  const bool live = (info & kAlive) && tv.x != M.inf && tv.y != M.inf && tv.z != M.inf && tv.w != M.inf;
+  const bool live = tv.x != kInvalid && tv.x != M.inf && tv.y != M.inf && tv.z != M.inf && tv.w != M.inf;
   bool qual = false;
   uint32_t kind = 0u, bad = 0u, third = kInvalid;
   if (live) {
@@ -102,8 +101,6 @@ __device__ __forceinline__ void flip_check_faces(const MS& M, const uint32_t* ac
   const uint32_t pk_c = (uint32_t)__shfl((int)pk, (int)(g0 + cf));
   const uint32_t third_c = (uint32_t)__shfl((int)third, (int)(g0 + cf));
   if (f == 0) {
-    // each entry is in the list once and only its lanes touch its info
-    INFO(M, t) = info & ~kQueued;
     if (grp) prop[j] = flip_propose(M, t, cf, (pk_c >> 2) & 1u, pk_c >> 3, third_c, it);
     else prop[j].x = kInvalid;
   }
@@ -149,11 +146,12 @@ __device__ __noinline__ void wg_slow_check(MS M, const uint32_t* act, uint4* pro
 // the next iteration go to next.  Every thread of the workgroup of BS threads
 // calls it.  On return c.act_next, c.slots, c.flips and c.slow hold the
 // results and every thread may read them; c.slots counts on from its value
-// before the call.  prop, slow_t: A entries of scratch; out: two per flip.
+// before the call.  prop, slow_t: A entries of scratch; out: four per flip
+// (at most half as many as the mesh has tets).
 template <class MS, int BS>
 __device__ __forceinline__ void wg_flip_iteration(const MS& M, WgCounters& c, const uint32_t* act, uint32_t* next,
                                                   uint4* prop, uint32_t* slow_t, uint4* out, uint32_t A,
-                                                  uint32_t it, uint32_t round, uint64_t* st) {
+                                                  uint32_t it, uint64_t* st) {
   const uint32_t tid = threadIdx.x;
   const uint64_t lt = (1ull << __lane_id()) - 1ull;
   const bool filtered = M.mode == PRED_FILTERED;
@@ -200,7 +198,7 @@ __device__ __forceinline__ void wg_flip_iteration(const MS& M, WgCounters& c, co
     if (nq > 1u) next[cq + 1u] = qid[1];
     if (win) {
       if (nslot) next[cq + nq] = cs;
-      flip_exec_loaded(M, pr, F, it, round, nslot ? cs : kInvalid, &out[2 * (size_t)cf]);
+      flip_exec_loaded(M, pr, F, it, nslot ? cs : kInvalid, &out[4 * (size_t)cf]);
     }
   }
   __syncthreads();
