@@ -57,3 +57,14 @@ def test_sort_tile_sizes(ctx, n, bits):
                 ctx.free(p)
         order = np.argsort(keys & dt((1 << end) - 1), kind="stable")
         assert np.array_equal(got, order.astype(np.uint32)) and np.array_equal(gk, keys[order])
+
+
+def test_exact_rounds_of_all_small_sizes(ctx, oracle):
+    """A captured round is replayed for every number of points that shares
+    its grids: exact mode, sizes falling and rising, against the oracle."""
+    pts = np.random.default_rng(11).random((340, 3)).astype(np.float32)
+    cfg = wtet_amd.Config(predicate_mode="exact")
+    for n in list(range(330, 20, -9)) + list(range(20, 330, 7)):
+        got = oracle.canonical_real(ctx.delaunay(pts[:n], cfg).tets, n)
+        want = oracle.canonical_real(oracle.delaunay(oracle.normalize_points(pts[:n])[0]), n)
+        assert np.array_equal(got, want), n

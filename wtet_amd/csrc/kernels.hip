@@ -771,13 +771,15 @@ __global__ void __launch_bounds__(kBlock) k_relocate(Mesh M, const uint32_t* uve
   const uint32_t U = M.ctr[C_SURV], it0 = M.ctr[C_IT0];
   PredStats ls = {};
   if (FORM == SLOW) {
-    uint32_t n = M.ctr[C_SLOW_R], stride = gridDim.x * blockDim.x;
-    for (uint32_t k = gid(); k < n; k += stride)
-      (void)relocate_body_t<false>(M, uvert, utet, slow[k], it0, &ls);
+    uint32_t n = 4u * M.ctr[C_SLOW_R], stride = gridDim.x * blockDim.x;
+    for (uint32_t k = gid(); k < n; k += stride) relocate_faces(M, uvert, utet, slow[k >> 2], (int)(k & 3u), it0, &ls);
+  } else if (FORM == FULL) {
+    uint32_t k = gid();
+    if (k < 4u * U) relocate_faces(M, uvert, utet, k >> 2, (int)(k & 3u), it0, &ls);
   } else {
     uint32_t i = gid();
     bool defer = false;
-    if (i < U) defer = relocate_body_t<FORM == LEAN>(M, uvert, utet, i, it0, &ls);
+    if (i < U) defer = relocate_body_t<true>(M, uvert, utet, i, it0, &ls);
     if (defer) slow[append_slot(&M.ctr[C_SLOW_R])] = i;
   }
   flush_stats(ls, st);
@@ -793,7 +795,10 @@ void launch_relocate(const Mesh& M, const uint32_t* uvert, uint32_t* utet, uint3
     k_relocate<LEAN><<<g, kBlock, 0, s>>>(M, uvert, utet, st, slow, sm, 0);
     k_relocate<SLOW><<<slow_grid(g), kBlock, 0, s>>>(M, uvert, utet, st, slow, sm, end);
   } else {
-    k_relocate<FULL><<<g, kBlock, 0, s>>>(M, uvert, utet, st, slow, sm, end);
+    // four lanes per point; 4 g, as every grid, follows from the rounded bound
+    // that a captured round is kept by (the rounded grid of 4 U does not: one
+    // block for 64 points, four for 65)
+    k_relocate<FULL><<<4u * g, kBlock, 0, s>>>(M, uvert, utet, st, slow, sm, end);
   }
 }
 

@@ -577,51 +577,46 @@ WT_HD void pick_pt(const float (*P)[3], const uint32_t* R, int k, float* out, ui
   *r = pick4(k, R[0], R[1], R[2], R[3]);
 }
 
-// One face f (chosen at run time) with the full
-// predicates: true when the face proposes a flip, with its kind, the
-// offending edge (3-2) and the third tet (3-2).  P, R:
-// the tet's points and ranks; Q, RQ: the vertices across its faces.
+// A face whose apex o across it is tested: its three vertices v, the tet's
+// vertex a opposite it, and o, with their ranks.
+struct FaceEdges {
+  float v[3][3], a[3], o[3];
+  uint32_t rv[3], ra, ro;
+};
+
+// The apex across face f of a tet lies inside its circumsphere (full
+// predicates).  P, R: the tet's points and ranks; Q, RQ: the vertices across
+// its faces.
 template <class MS>
-WT_HD bool flip_face_full(const MS& M, uint32_t t, const uint4& tov, const float (*P)[3],
-                          const uint32_t* R, const float (*Q)[3], const uint32_t* RQ, int f,
-                          PredStats* st, uint32_t* kind, uint32_t* bad, uint32_t* third) {
-  uint32_t o = get4(tov, f);
-  if (o == M.inf) return false;
-  float O[3];
-  uint32_t ro;
-  pick_pt(Q, RQ, f, O, &ro);
-  int ins = o4s<false>(M, P[0], P[1], P[2], P[3], O, R[0], R[1], R[2], R[3], ro, st);
-  if (ins > 0) return false;
-  // o lies inside the circumsphere: classify the flip
-  float A[3], V[3][3];
-  uint32_t ra, RV[3];
-  pick_pt(P, R, f, A, &ra);
-  int pos[3] = {face_vi(f, 0), face_vi(f, 1), face_vi(f, 2)};
-  for (int k = 0; k < 3; ++k) pick_pt(P, R, pos[k], V[k], &RV[k]);
-  int b = -1, nbad = 0;
-  for (int k = 0; k < 3; ++k) {
-    int w = (k + 1) % 3;
-    if (o3s<false>(M, V[k], V[w], A, O, RV[k], RV[w], ra, ro, st) > 0) {
-      b = k;
-      ++nbad;
-    }
-  }
-  if (nbad == 0) {
-    *kind = 0u;
-    *bad = 0u;
-    *third = kInvalid;
-    return true;
-  }
-  if (nbad > 1) return false;
+WT_HD bool flip_face_inside(const MS& M, const uint4& tov, const float (*P)[3], const uint32_t* R,
+                            const float (*Q)[3], const uint32_t* RQ, int f, PredStats* st, FaceEdges* E) {
+  if (get4(tov, f) == M.inf) return false;
+  pick_pt(Q, RQ, f, E->o, &E->ro);
+  pick_pt(P, R, f, E->a, &E->ra);
+  for (int k = 0; k < 3; ++k) pick_pt(P, R, face_vi(f, k), E->v[k], &E->rv[k]);
+  return o4s<false>(M, P[0], P[1], P[2], P[3], E->o, R[0], R[1], R[2], R[3], E->ro, st) <= 0;
+}
+
+// The flip of face f whose apex lies inside, from bits k: the segment a-o
+// passes beyond edge (v[k], v[k + 1]).  False when no flip fits.  kind (1:
+// 3-2), the offending edge and the third tet (3-2)
+template <class MS>
+WT_HD bool flip_face_kind(const MS& M, uint32_t t, const uint4& tov, int f, uint32_t beyond, uint32_t* kind,
+                          uint32_t* bad, uint32_t* third) {
+  *kind = 0u;
+  *bad = 0u;
+  *third = kInvalid;
+  if (beyond == 0u) return true;
+  if (beyond & (beyond - 1u)) return false;
   // 3-2 needs the edge to have degree 3 (see face_classify)
-  int pthird = b == 0 ? pos[2] : (b == 1 ? pos[0] : pos[1]);
-  if (get4(tov, pthird) != o) return false;
+  const int b = (int)ctz32(beyond);
+  const int pthird = face_vi(f, b == 0 ? 2 : b - 1);
+  if (get4(tov, pthird) != get4(tov, f)) return false;
   *kind = 1u;
   *bad = (uint32_t)b;
   *third = opp_tet(*opp_word(M, t, (uint32_t)pthird));
   return true;
 }
-
 
 // ---------------------------------------------------------------------------
 // execute a winning flip (src/shaders/flip.wgsl:531-845).  New tets reuse
@@ -867,15 +862,23 @@ WT_HD uint32_t walk_to_t(const MS& M, uint32_t t, uint32_t q, uint32_t seed, Pre
   return t;
 }
 
+// the live slot that a point of slot t walks from; false when no flip of
+// this round replaced t.  it0: flip iterations before this round
+template <class MS>
+WT_HD bool walk_start(const MS& M, uint32_t it0, uint32_t* t) {
+  if (FSTAMP(M, *t) <= it0) return false;
+  for (int guard = 0; guard < 64 && TV(M, *t).x == kInvalid; ++guard) *t = TFWD(M, *t);
+  return true;
+}
+WT_HD uint32_t walk_seed(uint32_t i) { return i * 0x85EBCA6Bu; }
+
 template <bool FAST, class MS>
-// it0: flip iterations before this round
 WT_HD bool relocate_body_t(const MS& M, const uint32_t* uvert, uint32_t* utet, uint32_t i,
                            uint32_t it0, PredStats* st) {
   uint32_t t = utet[i];
-  if (FSTAMP(M, t) <= it0) return false;
-  for (int guard = 0; guard < 64 && TV(M, t).x == kInvalid; ++guard) t = TFWD(M, t);
+  if (!walk_start(M, it0, &t)) return false;
   int state = 0;
-  t = walk_to_t<FAST>(M, t, uvert[i], i * 0x85EBCA6Bu, st, &state);
+  t = walk_to_t<FAST>(M, t, uvert[i], walk_seed(i), st, &state);
   if (state == 2) return true;  // the full walk restarts from utet[i]
   if (state == 1) at_add_u32(&M.ctr[C_WALK_FAIL], 1u);
   utet[i] = t;

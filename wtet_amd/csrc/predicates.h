@@ -10,11 +10,12 @@
 //      exact in f64);
 //   3. exact stage: every coordinate is an integer multiple of 2^E, where E
 //      is the lowest set-bit exponent over the coordinates involved, so the
-//      determinant is evaluated exactly in fixed-width two's-complement
-//      integers (32-bit limbs): one limb per coordinate difference when the
-//      differences to the last point are exact in f64 and span <= 30 bits,
-//      else 64-bit limb pairs per coordinate when the coordinates span
-//      <= 60 bits, 192-bit limbs otherwise.
+//      determinant is evaluated exactly in integers: native 64- and 128-bit
+//      products of the coordinate differences when the differences to the
+//      last point are exact in f64 and span <= 30 or <= 41 bits, else
+//      fixed-width two's-complement integers of 32-bit limbs: 64-bit limb
+//      pairs per coordinate when the coordinates span <= 60 bits, 192-bit
+//      limbs otherwise.
 // When the exact determinant is zero, Simulation of Simplicity decides, with
 // the cascades of the reference (src/predicates.rs:106-208 for orient3d,
 // :478-675 for insphere): Edelsbrunner-Muecke perturbations ranked by point
@@ -212,40 +213,19 @@ WT_HD BI<D> to_fixed(float v, int E) {
 }
 
 // ---------------------------------------------------------------------------
-// Short differences.  orient3d and insphere depend only on the differences
-// of their points to the last one.  Each difference of two f32 coordinates
-// is computed in f64 and kept when exact (checked with Knuth's two-sum
-// error term); when every one is exact and their set bits span at most
-// kRelSpan bits, they are integers below 2^30 in units of their lowest set
-// bit, and the determinant runs on single 32-bit limbs.  Nearby points have
-// short differences even where the coordinates themselves span many bits
+// Differences.  orient3d and insphere depend only on the differences of their
+// points to the last one.  Each difference of two f32 coordinates is computed
+// in f64 and kept when exact (checked with Knuth's two-sum error term); when
+// every one is exact and their set bits span at most kRelSpan bits, they are
+// integers below 2^30 in units of their lowest set bit, and the determinant
+// runs on native 32- and 64-bit products; up to kMidSpan bits, the largest
+// whose 3x3 determinants fit 128 bits, on 64- and 128-bit ones.  Nearby points
+// have short differences even where the coordinates themselves span many bits
 // (a 128^3 lattice: coordinates span up to 31 bits, neighbour differences
-// 24), and the limb products fall about fourfold.
+// 24); differences to a super vertex (coordinates -100 and 400) span 38 there.
 // ---------------------------------------------------------------------------
 constexpr int kRelSpan = 30;
-
-struct F64Parts {
-  uint64_t m;  // significand (0 for zero)
-  int e;       // value = +-m * 2^e
-  bool neg;
-};
-
-WT_HD F64Parts f64_parts(double v) {
-  uint64_t u;
-  __builtin_memcpy(&u, &v, 8);
-  F64Parts p;
-  p.neg = (u >> 63) != 0u;
-  uint32_t be = (uint32_t)((u >> 52) & 0x7FFu);
-  uint64_t fr = u & ((1ull << 52) - 1ull);
-  if (be == 0u) {
-    p.m = fr;
-    p.e = -1074;
-  } else {
-    p.m = fr | (1ull << 52);
-    p.e = (int)be - 1075;
-  }
-  return p;
-}
+constexpr int kMidSpan = 41;
 
 // a - b in f64; false when the rounded difference is not the exact one
 WT_HD bool exact_sub(double a, double b, double* d) {
@@ -256,41 +236,189 @@ WT_HD bool exact_sub(double a, double b, double* d) {
   return err == 0.0;
 }
 
-// the R points before the last as differences to it, 1-limb integers in
-// units of 2^E (E the lowest set bit over them); false when the tier does
-// not apply (a difference not exact in f64, or a span over kRelSpan)
+// the R points before the last as differences v to it; false when one is not
+// exact.  top: the largest magnitude
 template <int R>
-WT_HD bool rel_fixed1(const float* P, BI<1> (*d)[3]) {
-  double v[R][3];
-  int L = 100000, H = -100000;
+WT_HD bool rel_diff(const float* P, double (*v)[3], double* top) {
+  bool ok = true;
+  double t = 0.0;
 #pragma unroll
   for (int r = 0; r < R; ++r)
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      if (!exact_sub((double)P[r * 3 + k], (double)P[R * 3 + k], &v[r][k])) return false;
-      F64Parts p = f64_parts(v[r][k]);
-      if (p.m == 0u) continue;
-      int l = p.e + __builtin_ctzll(p.m);
-      int h = p.e + 63 - __builtin_clzll(p.m);
-      L = l < L ? l : L;
-      H = h > H ? h : H;
+      ok = exact_sub((double)P[r * 3 + k], (double)P[R * 3 + k], &v[r][k]) && ok;
+      t = __builtin_fmax(t, __builtin_fabs(v[r][k]));
     }
-  if (L != 100000 && H - L + 1 > kRelSpan) return false;
+  *top = t;
+  return ok;
+}
+
+// the differences as integers below 2^bits in a common unit: the largest is
+// scaled into [2^(bits-1), 2^bits), and the span fits when every scaled one is
+// whole (else false)
+template <int R, typename T>
+WT_HD bool rel_scale(const double (*v)[3], double top, int bits, T (*d)[3]) {
+  // differences of f32 values are 0 or at least 2^-149: top is normal
+  uint64_t u;
+  __builtin_memcpy(&u, &top, 8);
+  u = (uint64_t)(1022 + bits + 1023 - (int)(u >> 52)) << 52;
+  double scale;
+  __builtin_memcpy(&scale, &u, 8);
+  if (top == 0.0) scale = 1.0;
+  bool ok = true;
 #pragma unroll
   for (int r = 0; r < R; ++r)
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      F64Parts p = f64_parts(v[r][k]);
-      BI<1> x;
-      x.w[0] = 0u;
-      if (p.m != 0u) {
-        int tz = __builtin_ctzll(p.m);
-        x.w[0] = (uint32_t)((p.m >> tz) << (p.e + tz - L));  // < 2^30
-        if (p.neg) x = bi_neg(x);
+      double x = v[r][k] * scale;
+      d[r][k] = (T)x;
+      ok = ok && (double)d[r][k] == x;
+    }
+  return ok;
+}
+
+template <int R>
+WT_HD bool rel_int(const float* P, int32_t (*d)[3]) {
+  double v[R][3], top;
+  const bool ok = rel_diff<R>(P, v, &top);
+  return rel_scale<R>(v, top, kRelSpan, d) && ok;
+}
+
+WT_HD int64_t mul_wide(int32_t a, int32_t b) { return (int64_t)a * b; }
+WT_HD __int128 mul_wide(int64_t a, int64_t b) { return (__int128)a * b; }
+WT_HD int sign_int(__int128 v) { return v < 0 ? -1 : (v != 0 ? 1 : 0); }
+
+// u_i w_j - u_j w_i
+template <typename T>
+WT_HD auto minor_int(const T* a, const T* b, int u, int w) -> decltype(mul_wide(a[0], b[0])) {
+  return mul_wide(a[u], b[w]) - mul_wide(a[w], b[u]);
+}
+template <typename T>
+WT_HD auto lift_int(const T* a) -> decltype(mul_wide(a[0], a[0])) {
+  return mul_wide(a[0], a[0]) + mul_wide(a[1], a[1]) + mul_wide(a[2], a[2]);
+}
+
+// hi * 2^32 + lo
+struct I96 {
+  int64_t hi;
+  uint32_t lo;
+};
+WT_HD int sign_int(const I96& v) { return v.hi < 0 ? -1 : ((v.hi | (int64_t)v.lo) != 0 ? 1 : 0); }
+
+// x a + y b + z c; |x|, |y|, |z| < 2^30, |a|, |b|, |c| < 2^62
+WT_HD I96 sum3(int32_t x, int64_t a, int32_t y, int64_t b, int32_t z, int64_t c) {
+  // 30- by 32-bit products fit 64 bits; their low words add up separately
+  int64_t p = (int64_t)x * (int64_t)(uint32_t)a, q = (int64_t)y * (int64_t)(uint32_t)b,
+          r = (int64_t)z * (int64_t)(uint32_t)c;
+  uint64_t l = (uint64_t)(uint32_t)p + (uint32_t)q + (uint32_t)r;
+  int64_t h = mul_wide(x, (int32_t)(a >> 32)) + mul_wide(y, (int32_t)(b >> 32)) + mul_wide(z, (int32_t)(c >> 32));
+  h += (p >> 32) + (q >> 32) + (r >> 32) + (int64_t)(l >> 32);
+  return {h, (uint32_t)l};
+}
+// |x|, |y|, |z| < 2^41, |a|, |b|, |c| < 2^83
+WT_HD __int128 sum3(int64_t x, __int128 a, int64_t y, __int128 b, int64_t z, __int128 c) {
+  return a * x + b * y + c * z;
+}
+
+// det of rows a, b, c
+template <typename T>
+WT_HD auto det3_int(const T* a, const T* b, const T* c) -> decltype(sum3(a[0], minor_int(a, b, 0, 1), a[0],
+                                                                         minor_int(a, b, 0, 1), a[0],
+                                                                         minor_int(a, b, 0, 1))) {
+  return sum3(a[2], minor_int(b, c, 0, 1), b[2], minor_int(c, a, 0, 1), c[2], minor_int(a, b, 0, 1));
+}
+
+WT_HD void words_of(int64_t v, uint32_t* w) { w[0] = (uint32_t)v, w[1] = (uint32_t)(v >> 32); }
+WT_HD void words_of(const I96& v, uint32_t* w) {
+  w[0] = v.lo;
+  words_of(v.hi, w + 1);
+}
+WT_HD void words_of(__int128 v, uint32_t* w) {
+  words_of((int64_t)v, w);
+  words_of((int64_t)(v >> 64), w + 2);
+}
+
+// acc += l v (sgn >= 0) or acc -= l v, in columns of 32 bits: l >= 0 of NL
+// words, v of NV words (the last signed).  A column takes a few words of
+// either sign, far below its 64 bits.
+template <int NL, int NV>
+WT_HD void mac_columns(int64_t* acc, const uint32_t* l, const uint32_t* v, int sgn) {
+  int64_t col[NL + NV];
+#pragma unroll
+  for (int k = 0; k < NL + NV; ++k) col[k] = 0;
+#pragma unroll
+  for (int i = 0; i < NL; ++i)
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      if (j + 1 < NV) {
+        const uint64_t p = (uint64_t)l[i] * v[j];
+        col[i + j] += (int64_t)(uint32_t)p;
+        col[i + j + 1] += (int64_t)(p >> 32);
+      } else {
+        const int64_t p = (int64_t)(uint64_t)l[i] * (int32_t)v[j];
+        col[i + j] += (int64_t)(uint32_t)p;
+        col[i + j + 1] += p >> 32;
       }
-      d[r][k] = x;
     }
-  return true;
+#pragma unroll
+  for (int k = 0; k < NL + NV; ++k) acc[k] += sgn < 0 ? -col[k] : col[k];
+}
+
+template <int N>
+WT_HD int sign_columns(int64_t* acc) {
+  uint32_t low = (uint32_t)acc[0];
+#pragma unroll
+  for (int k = 0; k + 1 < N; ++k) {
+    acc[k + 1] += acc[k] >> 32;
+    if (k + 2 < N) low |= (uint32_t)acc[k + 1];
+  }
+  return acc[N - 1] < 0 ? -1 : ((acc[N - 1] != 0 || low != 0u) ? 1 : 0);
+}
+
+// Shewchuk's insphere on the differences d (rows a-e .. d-e); NL words hold a
+// lift, NV a 3x3 determinant
+template <int NL, int NV, typename T>
+WT_HD int insphere_int(const T (*d)[3]) {
+  const auto ab = minor_int(d[0], d[1], 0, 1), bc = minor_int(d[1], d[2], 0, 1), cd = minor_int(d[2], d[3], 0, 1),
+             da = minor_int(d[3], d[0], 0, 1), ac = minor_int(d[0], d[2], 0, 1), bd = minor_int(d[1], d[3], 0, 1);
+  const T z0 = d[0][2], z1 = d[1][2], z2 = d[2][2], z3 = d[3][2];
+  int64_t acc[NL + NV];
+#pragma unroll
+  for (int k = 0; k < NL + NV; ++k) acc[k] = 0;
+  uint32_t l[4], v[4];
+#define WT_TERM(row, det, sgn)   \
+  words_of(lift_int(d[row]), l); \
+  words_of(det, v);              \
+  mac_columns<NL, NV>(acc, l, v, sgn);
+  WT_TERM(3, sum3(z0, bc, (T)-z1, ac, z2, ab), 1)
+  WT_TERM(2, sum3(z3, ab, z0, bd, z1, da), -1)
+  WT_TERM(1, sum3(z2, da, z3, ac, z0, cd), 1)
+  WT_TERM(0, sum3(z1, cd, (T)-z2, bd, z3, bc), -1)
+#undef WT_TERM
+  return sign_columns<NL + NV>(acc);
+}
+
+// det [[u v |p|^2 1]] over 4 COPLANAR points from the differences d of three
+// of them to the fourth (rows a, b, c).  Translating the points by t changes
+// the lifted determinant by -2 t_w det[[p0 p1 p2 1]] (t_w the coordinate left
+// out of the first two columns), which vanishes when the four points are
+// coplanar; the sign is then the absolute form's.
+WT_HD int lifted_int(const int32_t* a, const int32_t* b, const int32_t* c, int u, int w) {
+  const __int128 det = (__int128)lift_int(a) * minor_int(b, c, u, w) + (__int128)lift_int(b) * minor_int(c, a, u, w) +
+                       (__int128)lift_int(c) * minor_int(a, b, u, w);
+  return sign_int(det);
+}
+WT_HD int lifted_int(const int64_t* a, const int64_t* b, const int64_t* c, int u, int w) {
+  const int64_t* p[3] = {a, b, c};
+  int64_t acc[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    uint32_t l[4], v[4];
+    words_of(lift_int(p[k]), l);  // < 2^84
+    words_of(minor_int(p[(k + 1) % 3], p[(k + 2) % 3], u, w), v);  // |.| < 2^83
+    mac_columns<3, 3>(acc, l, v, 1);
+  }
+  return sign_columns<6>(acc);
 }
 
 // ---------------------------------------------------------------------------
@@ -317,39 +445,9 @@ WT_HD int exact_orient3d_T(const float* P, int E) {
   return orient3d_core<D>(d);
 }
 
-// Shewchuk's insphere on the differences d (rows a-e .. d-e)
-template <int D>
-WT_HD int insphere_core(const BI<D> (*d)[3]) {
-  BI<D> x[4], y[4], z[4];
-  BI<2 * D> l[4];
-  for (int r = 0; r < 4; ++r) {
-    x[r] = d[r][0];
-    y[r] = d[r][1];
-    z[r] = d[r][2];
-    l[r] = bi_add(bi_add(bi_mul(x[r], x[r]), bi_mul(y[r], y[r])), bi_mul(z[r], z[r]));
-  }
-  // 2x2 minors on (x, y)
-  BI<2 * D> ab = bi_sub(bi_mul(x[0], y[1]), bi_mul(x[1], y[0]));
-  BI<2 * D> bc = bi_sub(bi_mul(x[1], y[2]), bi_mul(x[2], y[1]));
-  BI<2 * D> cd = bi_sub(bi_mul(x[2], y[3]), bi_mul(x[3], y[2]));
-  BI<2 * D> da = bi_sub(bi_mul(x[3], y[0]), bi_mul(x[0], y[3]));
-  BI<2 * D> ac = bi_sub(bi_mul(x[0], y[2]), bi_mul(x[2], y[0]));
-  BI<2 * D> bd = bi_sub(bi_mul(x[1], y[3]), bi_mul(x[3], y[1]));
-  // 3x3 minors with z
-  BI<3 * D> abc = bi_add(bi_sub(bi_mul(z[0], bc), bi_mul(z[1], ac)), bi_mul(z[2], ab));
-  BI<3 * D> bcd = bi_add(bi_sub(bi_mul(z[1], cd), bi_mul(z[2], bd)), bi_mul(z[3], bc));
-  BI<3 * D> cda = bi_add(bi_add(bi_mul(z[2], da), bi_mul(z[3], ac)), bi_mul(z[0], cd));
-  BI<3 * D> dab = bi_add(bi_add(bi_mul(z[3], ab), bi_mul(z[0], bd)), bi_mul(z[1], da));
-  BI<5 * D> det = bi_add(bi_sub(bi_mul(l[3], abc), bi_mul(l[2], dab)),
-                         bi_sub(bi_mul(l[1], cda), bi_mul(l[0], bcd)));
-  return bi_sign(det);
-}
-
 template <int D>
 WT_HD int exact_insphere_T(const float* P, int E) {
-  // P: 5 points; Shewchuk's insphere with a..d relative to e.  The same
-  // expression as insphere_core, written out on its own: built through the
-  // core's array argument, the wide forms spilled more.
+  // P: 5 points; Shewchuk's insphere with a..d relative to e
   BI<D> x[4], y[4], z[4];
   BI<2 * D> l[4];
   for (int r = 0; r < 4; ++r) {
@@ -398,22 +496,6 @@ WT_HD int exact_orient3d_lifted_T(const float* P, int E) {
   return bi_sign(det);
 }
 
-// det [[p0 p1 |p|^2 1]] over 4 COPLANAR points from their differences to
-// the last one: det[[u_i - u_3, v_i - v_3, |p_i - p_3|^2]].  Translating
-// the points by t changes the lifted determinant by -2 t_w det[[p0 p1 p2 1]]
-// (t_w the coordinate left out of the first two columns), which vanishes
-// when the four points are coplanar; the sign is then the absolute form's.
-WT_HD int orient3d_lifted_rel1(const BI<1> (*d)[3]) {
-  BI<2> w[3];
-  for (int r = 0; r < 3; ++r)
-    w[r] = bi_add(bi_add(bi_mul(d[r][0], d[r][0]), bi_mul(d[r][1], d[r][1])), bi_mul(d[r][2], d[r][2]));
-  BI<2> bc = bi_sub(bi_mul(d[1][0], d[2][1]), bi_mul(d[2][0], d[1][1]));
-  BI<2> ca = bi_sub(bi_mul(d[2][0], d[0][1]), bi_mul(d[0][0], d[2][1]));
-  BI<2> ab = bi_sub(bi_mul(d[0][0], d[1][1]), bi_mul(d[1][0], d[0][1]));
-  BI<4> det = bi_add(bi_add(bi_mul(w[0], bc), bi_mul(w[1], ca)), bi_mul(w[2], ab));
-  return bi_sign(det);
-}
-
 // det [[p0 |p|^2 1]] over 3 points
 template <int D>
 WT_HD int exact_orient2d_lifted_T(const float* P, int E) {
@@ -451,46 +533,51 @@ constexpr int kNarrowSpan = 60;
   if (hi_ - lo_ + 1 <= kNarrowSpan) return fn<2>(P, lo_); \
   return fn<6>(P, lo_);
 
-// The short-difference tier as small leaf functions (few registers, so a
-// call saves none: no scratch traffic on the path degenerate inputs take
-// millions of times), returning 2 when the tier does not apply; the wide
+// The difference tiers as leaf functions with their points passed by
+// value (in registers: no scratch traffic on the path degenerate inputs take
+// millions of times), returning 2 when neither applies; the wide
 // forms are separate calls for the rest.
-WT_HDN int exact_orient3d_short(const float* P) {
-  BI<1> d[3][3];
-  return rel_fixed1<3>(P, d) ? orient3d_core<1>(d) : 2;
+#define WT_P12(P) P[0], P[1], P[2], P[3], P[4], P[5], P[6], P[7], P[8], P[9], P[10], P[11]
+#define WT_P15(P) WT_P12(P), P[12], P[13], P[14]
+#define WT_ARGS12                                                                                                  \
+  float p0, float p1, float p2, float p3, float p4, float p5, float p6, float p7, float p8, float p9, float p10, \
+      float p11
+#define WT_LIST12 p0, p1, p2, p3, p4, p5, p6, p7, p8, p9, p10, p11
+WT_HDN int exact_orient3d_rel(WT_ARGS12) {
+  const float P[12] = {WT_LIST12};
+  double v[3][3], top;
+  if (!rel_diff<3>(P, v, &top)) return 2;
+  int32_t d[3][3];
+  if (rel_scale<3>(v, top, kRelSpan, d)) return sign_int(det3_int(d[0], d[1], d[2]));
+  int64_t m[3][3];
+  return rel_scale<3>(v, top, kMidSpan, m) ? sign_int(det3_int(m[0], m[1], m[2])) : 2;
 }
-WT_HDN int exact_insphere_short(const float* P) {
-  BI<1> d[4][3];
-  return rel_fixed1<4>(P, d) ? insphere_core<1>(d) : 2;
+WT_HDN int exact_insphere_rel(WT_ARGS12, float p12, float p13, float p14) {
+  const float P[15] = {WT_LIST12, p12, p13, p14};
+  double v[4][3], top;
+  if (!rel_diff<4>(P, v, &top)) return 2;
+  int32_t d[4][3];
+  if (rel_scale<4>(v, top, kRelSpan, d)) return insphere_int<2, 3>(d);
+  int64_t m[4][3];
+  return rel_scale<4>(v, top, kMidSpan, m) ? insphere_int<3, 4>(m) : 2;
 }
 WT_HDN int exact_orient3d_wide(const float* P) { WT_EXACT_DISPATCH(exact_orient3d_T, P, 12) }
 WT_HDN int exact_insphere_wide(const float* P) { WT_EXACT_DISPATCH(exact_insphere_T, P, 15) }
-// The short tier cannot apply with a super vertex among the points (its
-// coordinates are -100 or 400, the differences to it span more than 30
-// bits): such calls go to the wide forms at once, without a failed try.
-WT_HD bool near_unit(const float* P, int k) {
-  bool ok = true;
-  for (int i = 0; i < k; ++i) ok = ok && P[i] > -4.0f && P[i] < 4.0f;
-  return ok;
-}
 WT_HD int exact_orient3d(const float* P) {
-  int s = near_unit(P, 12) ? exact_orient3d_short(P) : 2;
+  int s = exact_orient3d_rel(WT_P12(P));
   return s != 2 ? s : exact_orient3d_wide(P);
-}
-WT_HD int exact_insphere(const float* P) {
-  int s = near_unit(P, 15) ? exact_insphere_short(P) : 2;
-  return s != 2 ? s : exact_insphere_wide(P);
 }
 // the lifted orient3d of four points known to be coplanar (the SoS cascade
 // reaches a lifted 4-point step only after the plain orient3d of the same
 // four points vanished): short differences when they apply
-WT_HDN int exact_orient3d_lifted_coplanar_short(const float* P) {
-  BI<1> d[3][3];
-  return rel_fixed1<3>(P, d) ? orient3d_lifted_rel1(d) : 2;
+WT_HDN int exact_orient3d_lifted_coplanar_short(WT_ARGS12) {
+  const float P[12] = {WT_LIST12};
+  int32_t d[3][3];
+  return rel_int<3>(P, d) ? lifted_int(d[0], d[1], d[2], 0, 1) : 2;
 }
 WT_HDN int exact_orient3d_lifted_wide(const float* P) { WT_EXACT_DISPATCH(exact_orient3d_lifted_T, P, 12) }
 WT_HD int exact_orient3d_lifted_coplanar(const float* P) {
-  int s = near_unit(P, 12) ? exact_orient3d_lifted_coplanar_short(P) : 2;
+  int s = exact_orient3d_lifted_coplanar_short(WT_P12(P));
   return s != 2 ? s : exact_orient3d_lifted_wide(P);
 }
 WT_HDN int exact_orient2d_lifted(const float* P) { WT_EXACT_DISPATCH(exact_orient2d_lifted_T, P, 9) }
@@ -872,25 +959,21 @@ WT_HD int orient3d_raw(const float* a, const float* b, const float* c, const flo
     }
   }
   float P[12] = {a[0], a[1], a[2], b[0], b[1], b[2], c[0], c[1], c[2], d[0], d[1], d[2]};
-  // the short tier pays where the filters have left the near-degenerate
-  // cases (a lattice's co-planar and co-spherical sets); on every call of
-  // the exact-only mode the wide form alone is faster
-  int s = mode == PRED_FILTERED ? exact_orient3d(P) : exact_orient3d_wide(P);
+  int s = exact_orient3d(P);
   stat_inc(st, s != 0 ? 2 : 3);
   return s;
 }
 
 WT_HD int insphere_raw(const float* a, const float* b, const float* c, const float* d,
                        const float* e, int mode, PredStats* st) {
+  double perm = 0.0;
   if (mode == PRED_FILTERED) {
     int s = insphere_f32(a, b, c, d, e);
     if (s != 2) {
       stat_inc(st, 4);
       return s;
     }
-    double perm = 0.0;
     s = insphere_f64(a, b, c, d, e, &perm);
-    if (s == 2) s = insphere_dd(a, b, c, d, e, perm);
     if (s != 2) {
       stat_inc(st, 5);
       return s;
@@ -898,7 +981,20 @@ WT_HD int insphere_raw(const float* a, const float* b, const float* c, const flo
   }
   float P[15] = {a[0], a[1], a[2], b[0], b[1], b[2], c[0], c[1], c[2],
                  d[0], d[1], d[2], e[0], e[1], e[2]};
-  int s = mode == PRED_FILTERED ? exact_insphere(P) : exact_insphere_wide(P);
+  // the integers come before the double-double stage: they settle the zeros
+  // too, which it has to leave (a launch on 16,384 co-spherical sets: 14 us
+  // with the double-double first, 9 us)
+  int s = exact_insphere_rel(WT_P15(P));
+  if (s == 2) {
+    if (mode == PRED_FILTERED) {
+      s = insphere_dd(a, b, c, d, e, perm);
+      if (s != 2) {
+        stat_inc(st, 5);
+        return s;
+      }
+    }
+    s = exact_insphere_wide(P);
+  }
   stat_inc(st, s != 0 ? 6 : 7);
   return s;
 }
@@ -908,51 +1004,49 @@ WT_HD int insphere_raw(const float* a, const float* b, const float* c, const flo
 // ---------------------------------------------------------------------------
 WT_HD int sgn_diff(float a, float b) { return (a > b) - (a < b); }
 
-// src/predicates.rs:106-208 after the exact determinant vanished
-WT_HDN int orient3d_sos_only(const float* a, const float* b, const float* c, const float* d,
-                             uint32_t ia, uint32_t ib, uint32_t ic, uint32_t id) {
-  uint32_t v[4] = {ia, ib, ic, id};
-  const float* p[4] = {a, b, c, d};
+// a point with its rank, and the compare-exchange of a sorting network that
+// keeps the parity of the permutation
+struct Ranked {
+  float x, y, z;
+  uint32_t id;
+};
+WT_HD void sort2(Ranked& a, Ranked& b, int& parity) {
+  const bool g = b.id < a.id;
+  const Ranked t = a;
+  a.x = g ? b.x : a.x, a.y = g ? b.y : a.y, a.z = g ? b.z : a.z, a.id = g ? b.id : a.id;
+  b.x = g ? t.x : b.x, b.y = g ? t.y : b.y, b.z = g ? t.z : b.z, b.id = g ? t.id : b.id;
+  parity = g ? -parity : parity;
+}
+
+// src/predicates.rs:106-208 after the exact determinant vanished.  The depths
+// of the cascade in order, on points sorted in registers: a sort through
+// arrays indexed at run time and a loop over the depths kept them in scratch
+// memory.  Four distinct points that are not collinear end within the first
+// three.
+WT_HDN int orient3d_sos_only(WT_ARGS12, uint32_t ia, uint32_t ib, uint32_t ic, uint32_t id) {
+  Ranked a = {p0, p1, p2, ia}, b = {p3, p4, p5, ib}, c = {p6, p7, p8, ic}, d = {p9, p10, p11, id};
   int parity = 1;
-  for (int i = 0; i < 3; ++i) {
-    int mi = i;
-    for (int j = i + 1; j < 4; ++j)
-      if (v[j] < v[mi]) mi = j;
-    if (mi != i) {
-      uint32_t tv = v[i];
-      v[i] = v[mi];
-      v[mi] = tv;
-      const float* tp = p[i];
-      p[i] = p[mi];
-      p[mi] = tp;
-      parity = -parity;
-    }
-  }
-  // (point, point, point, axis u, axis w) for the orient2d depths
-  int depth = 0, r = 0;
-  for (; depth < 13; ++depth) {
-    int P0 = -1, P1 = 0, P2 = 0, U = 0, W = 0;
-    switch (depth) {
-      case 0: P0 = 1; P1 = 2; P2 = 3; U = 0; W = 1; break;
-      case 1: P0 = 1; P1 = 2; P2 = 3; U = 0; W = 2; break;
-      case 2: P0 = 1; P1 = 2; P2 = 3; U = 1; W = 2; break;
-      case 3: P0 = 0; P1 = 2; P2 = 3; U = 0; W = 1; break;
-      case 4: r = sgn_diff(p[2][0], p[3][0]); break;
-      case 5: r = sgn_diff(p[2][1], p[3][1]); break;
-      case 6: P0 = 0; P1 = 2; P2 = 3; U = 0; W = 2; break;
-      case 7: r = sgn_diff(p[2][2], p[3][2]); break;
-      case 8: P0 = 0; P1 = 2; P2 = 3; U = 1; W = 2; break;
-      case 9: P0 = 0; P1 = 1; P2 = 3; U = 0; W = 1; break;
-      case 10: r = sgn_diff(p[1][0], p[3][0]); break;
-      case 11: r = sgn_diff(p[1][1], p[3][1]); break;
-      default: r = sgn_diff(p[0][0], p[3][0]); break;
-    }
-    if (P0 >= 0)
-      r = dsign(orient2d_plain(p[P0][U], p[P0][W], p[P1][U], p[P1][W], p[P2][U], p[P2][W]));
-    if (r != 0) break;
-  }
-  if (depth == 13) r = 1;
-  if (depth == 1 || depth == 3 || depth == 5 || depth == 8 || depth == 10) r = -r;
+  sort2(a, b, parity);
+  sort2(c, d, parity);
+  sort2(a, c, parity);
+  sort2(b, d, parity);
+  sort2(b, c, parity);
+#define WT_O2(p, q, r, u, w) dsign(orient2d_plain(p.u, p.w, q.u, q.w, r.u, r.w))
+  int r = WT_O2(b, c, d, x, y);
+  if (r == 0) r = -WT_O2(b, c, d, x, z);
+  if (r == 0) r = WT_O2(b, c, d, y, z);
+  if (r == 0) r = -WT_O2(a, c, d, x, y);
+  if (r == 0) r = sgn_diff(c.x, d.x);
+  if (r == 0) r = -sgn_diff(c.y, d.y);
+  if (r == 0) r = WT_O2(a, c, d, x, z);
+  if (r == 0) r = sgn_diff(c.z, d.z);
+  if (r == 0) r = -WT_O2(a, c, d, y, z);
+  if (r == 0) r = WT_O2(a, b, d, x, y);
+  if (r == 0) r = -sgn_diff(b.x, d.x);
+  if (r == 0) r = sgn_diff(b.y, d.y);
+  if (r == 0) r = sgn_diff(a.x, d.x);
+  if (r == 0) r = 1;
+#undef WT_O2
   r *= parity;
   return r < 0 ? 1 : -1;
 }
@@ -962,7 +1056,7 @@ WT_HD int orient3d_sos(const float* a, const float* b, const float* c, const flo
                        PredStats* st) {
   int s = orient3d_raw(a, b, c, d, mode, st);
   if (s != 0) return s < 0 ? 1 : -1;
-  return orient3d_sos_only(a, b, c, d, ia, ib, ic, id);
+  return orient3d_sos_only(a[0], a[1], a[2], b[0], b[1], b[2], c[0], c[1], c[2], d[0], d[1], d[2], ia, ib, ic, id);
 }
 
 // FP32 filter stage alone, for the lean kernels: the staged functions
@@ -1035,6 +1129,60 @@ WT_HD void perm_coords(const float* p, int perm, float* q) {
   q[2] = p[i2];
 }
 
+// depths 1-4 of orient4d's cascade from the differences v of points 1-3 to
+// point 4
+template <typename T>
+WT_HD int sos4_plane(const T (*v)[3]) {
+  int r = -sign_int(det3_int(v[0], v[1], v[2]));
+  if (r == 0) r = lifted_int(v[0], v[1], v[2], 0, 1);
+  if (r == 0) r = -lifted_int(v[0], v[1], v[2], 0, 2);
+  if (r == 0) r = lifted_int(v[0], v[1], v[2], 1, 2);
+  return r;
+}
+
+// The cascade's depths 1-5, 0 when they do not decide here.  Five distinct
+// cospherical points end here: depth 1 is zero only with points 1-4 coplanar;
+// depths 2-4 too only with those on a circle, three of which are not
+// collinear, and point 0 then lies off their plane (or the five are
+// coplanar), so depth 5 decides.  The depths share their differences and
+// minors, and nothing lies in scratch memory: a wave's insphere with the
+// cascade took 170 us through orient4d_sos_only, and the deferred flip checks of
+// a 48^3 lattice 97 us a launch with it, 38 us here.
+WT_HDN int orient4d_sos_short(WT_ARGS12, float p12, float p13, float p14, uint32_t ia, uint32_t ib, uint32_t ic,
+                              uint32_t id, uint32_t ie) {
+  Ranked a = {p0, p1, p2, ia}, b = {p3, p4, p5, ib}, c = {p6, p7, p8, ic}, d = {p9, p10, p11, id},
+         e = {p12, p13, p14, ie};
+  int parity = 1;
+  sort2(a, b, parity);
+  sort2(d, e, parity);
+  sort2(c, e, parity);
+  sort2(c, d, parity);
+  sort2(b, e, parity);
+  sort2(a, d, parity);
+  sort2(a, c, parity);
+  sort2(b, d, parity);
+  sort2(b, c, parity);
+  int r = 0;
+#pragma unroll 1
+  for (int pass = 0; pass < 2 && r == 0; ++pass) {
+    // points 1-4, then 0, 2, 3, 4 (depth 5)
+    const float P[12] = {pass ? a.x : b.x, pass ? a.y : b.y, pass ? a.z : b.z, c.x, c.y, c.z, d.x, d.y, d.z, e.x, e.y, e.z};
+    r = orient3d_f32(P, P + 3, P + 6, P + 9);
+    if (r != 2) {
+      r = pass ? r : -r;
+      continue;
+    }
+    double v[3][3], top;
+    if (!rel_diff<3>(P, v, &top)) return 0;
+    int32_t s[3][3];
+    int64_t m[3][3];
+    if (rel_scale<3>(v, top, kRelSpan, s)) r = pass ? sign_int(det3_int(s[0], s[1], s[2])) : sos4_plane(s);
+    else if (rel_scale<3>(v, top, kMidSpan, m)) r = pass ? sign_int(det3_int(m[0], m[1], m[2])) : sos4_plane(m);
+    else return 0;
+  }
+  return r * parity;
+}
+
 // src/predicates.rs:478-675 after the exact insphere vanished
 WT_HDN int orient4d_sos_only(const float* a, const float* b, const float* c, const float* d,
                              const float* e, uint32_t ia, uint32_t ib, uint32_t ic,
@@ -1085,7 +1233,9 @@ WT_HD int orient4d(const float* a, const float* b, const float* c, const float* 
                    uint32_t ie, int mode, PredStats* st) {
   int s = insphere_raw(a, b, c, d, e, mode, st);
   if (s != 0) return s;
-  return orient4d_sos_only(a, b, c, d, e, ia, ib, ic, id, ie);
+  s = orient4d_sos_short(a[0], a[1], a[2], b[0], b[1], b[2], c[0], c[1], c[2], d[0], d[1], d[2], e[0], e[1], e[2], ia,
+                         ib, ic, id, ie);
+  return s != 0 ? s : orient4d_sos_only(a, b, c, d, e, ia, ib, ic, id, ie);
 }
 
 WT_HD int orient4d_fast(const float* a, const float* b, const float* c, const float* d,

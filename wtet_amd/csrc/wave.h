@@ -69,12 +69,70 @@ __device__ __forceinline__ bool keep_point(const float4* pts, const uint64_t* ke
   return !redundant_dup(pts + 4u * *c, keys, n, j, capped);
 }
 
+// The tests of the three edges of every lane's face (inside: the lane has
+// one), spread over the wave's active lanes (lanes 0..n-1): job j is edge j % 3
+// of the (j / 3)th such lane.  Each lane gets its bits: edge k has the segment
+// a-o beyond it.  One after another on the lanes that have a face, the three
+// tests kept most of the wave idle for three times as long: 16 tets rarely
+// have more than 21 such faces.
+template <class MS>
+__device__ __forceinline__ uint32_t face_edges_wave(const MS& M, bool inside, const FaceEdges& E, PredStats* st) {
+  const uint64_t mask = __ballot(inside);
+  const uint32_t n = (uint32_t)__popcll(__ballot(1)), lane = __lane_id();
+  const uint32_t jobs = 3u * (uint32_t)__popcll(mask);
+  const uint32_t mine = 3u * (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
+  uint32_t beyond = 0u;
+  for (uint32_t b = 0; b < jobs; b += n) {
+    const uint32_t j = b + lane, k = j % 3u;
+    // the lane of the job's face: the (j / 3)th set bit of the mask
+    uint32_t want = j < jobs ? j / 3u : 0u, src = 0u;
+#pragma unroll
+    for (uint32_t w = 32u; w > 0u; w >>= 1) {
+      const uint32_t low = (uint32_t)__popcll(mask >> src & ((1ull << w) - 1ull));
+      if (want >= low) {
+        want -= low;
+        src += w;
+      }
+    }
+    FaceEdges F;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      F.a[q] = __shfl(E.a[q], (int)src);
+      F.o[q] = __shfl(E.o[q], (int)src);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) F.v[i][q] = __shfl(E.v[i][q], (int)src);
+      F.rv[q] = (uint32_t)__shfl((int)E.rv[q], (int)src);
+    }
+    F.ra = (uint32_t)__shfl((int)E.ra, (int)src);
+    F.ro = (uint32_t)__shfl((int)E.ro, (int)src);
+    bool out = false;
+    if (j < jobs) {
+      float X[3], Y[3];
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        X[q] = k == 0u ? F.v[0][q] : (k == 1u ? F.v[1][q] : F.v[2][q]);
+        Y[q] = k == 0u ? F.v[1][q] : (k == 1u ? F.v[2][q] : F.v[0][q]);
+      }
+      const uint32_t rx = k == 0u ? F.rv[0] : (k == 1u ? F.rv[1] : F.rv[2]);
+      const uint32_t ry = k == 0u ? F.rv[1] : (k == 1u ? F.rv[2] : F.rv[0]);
+      out = o3s<false>(M, X, Y, F.a, F.o, rx, ry, F.ra, F.ro, st) > 0;
+    }
+    const uint64_t res = __ballot(out);
+#pragma unroll
+    for (uint32_t q = 0; q < 3u; ++q) {
+      const uint32_t d = mine + q - b;  // wraps below b
+      if (d < n) beyond |= (uint32_t)(res >> d & 1u) << q;
+    }
+  }
+  return beyond;
+}
+
 // The full check of list entry j's face f, four lanes per tet, one per face
 // (f = this lane's index modulo 4; a tet's lanes are consecutive in the
-// wave and all take part): each lane runs its face's staged insphere and,
-// where the face's apex lies inside, the three orient3d that classify the
-// flip; the lowest face that proposes is the tet's proposal, as a loop over
-// the faces would choose it.  A tet's faces
+// wave and all take part; the wave's active lanes are its first): each lane
+// runs its face's staged insphere, the wave the edge tests of the faces whose
+// apex lies inside; the lowest face that proposes is the tet's proposal, as a
+// loop over the faces would choose it.  A tet's faces
 // then reach the exact and SoS stages together rather than one after another
 // in divergent passes.
 template <class MS>
@@ -84,15 +142,18 @@ __device__ __forceinline__ void flip_check_faces(const MS& M, const uint32_t* ac
   const uint4 tv = TV(M, t);
   const uint4 tov = TOV(M, t);
   const bool live = tv.x != kInvalid && tv.x != M.inf && tv.y != M.inf && tv.z != M.inf && tv.w != M.inf;
-  bool qual = false;
-  uint32_t kind = 0u, bad = 0u, third = kInvalid;
+  bool inside = false, qual = false;
+  FaceEdges E = {};
   if (live) {
     float P[4][3], Q[4][3];
     uint32_t R[4], RQ[4];
     for (int q = 0; q < 4; ++q) load_pt(M, get4(tv, q), P[q], &R[q]);
     for (int q = 0; q < 4; ++q) load_pt(M, get4(tov, q), Q[q], &RQ[q]);
-    qual = flip_face_full(M, t, tov, P, R, Q, RQ, f, st, &kind, &bad, &third);
+    inside = flip_face_inside(M, tov, P, R, Q, RQ, f, st, &E);
   }
+  uint32_t kind = 0u, bad = 0u, third = kInvalid;
+  const uint32_t beyond = face_edges_wave(M, inside, E, st);
+  if (inside) qual = flip_face_kind(M, t, tov, f, beyond, &kind, &bad, &third);
   const uint64_t qb = __ballot(qual);
   const uint32_t g0 = __lane_id() & ~3u;
   const uint32_t grp = (uint32_t)(qb >> g0) & 0xFu;
@@ -103,6 +164,43 @@ __device__ __forceinline__ void flip_check_faces(const MS& M, const uint32_t* ac
   if (f == 0) {
     if (grp) prop[j] = flip_propose(M, t, cf, (pk_c >> 2) & 1u, pk_c >> 3, third_c, it);
     else prop[j].x = kInvalid;
+  }
+}
+
+// The full walk of point i, four lanes per point, one per face (f = this
+// lane's index modulo 4; a point's lanes are consecutive in the wave and all
+// take part): the steps of walk_to_t, whose four exact face tests run side by
+// side instead of one after another.  A walk is a chain of those tests, so
+// a wave waits for one per step, not four (19 walks of 10,000 uniform points
+// in exact mode: 160 -> 43 us each).
+template <class MS>
+__device__ __forceinline__ void relocate_faces(const MS& M, const uint32_t* uvert, uint32_t* utet, uint32_t i, int f,
+                                               uint32_t it0, PredStats* st) {
+  uint32_t t = utet[i];
+  if (!walk_start(M, it0, &t)) return;
+  float Q[3];
+  uint32_t rq;
+  load_pt(M, uvert[i], Q, &rq);
+  const uint32_t seed = walk_seed(i), g0 = __lane_id() & ~3u;
+  bool there = false;
+  for (uint32_t step = 0; step < kWalkLimit && !there; ++step) {
+    const uint4 tv = TV(M, t);
+    const uint4 to = TN(M, t);
+    const uint32_t r0 = hash32(seed + step * 0x9E3779B9u) & 3u;
+    float A[3], B[3], C[3];
+    uint32_t ra, rb, rc;
+    load_pt(M, get4(tv, face_vi(f, 0)), A, &ra);
+    load_pt(M, get4(tv, face_vi(f, 1)), B, &rb);
+    load_pt(M, get4(tv, face_vi(f, 2)), C, &rc);
+    const bool beyond = o3s<false>(M, A, B, C, Q, ra, rb, rc, rq, st) < 0;
+    const uint32_t m = (uint32_t)(__ballot(beyond) >> g0) & 0xFu;
+    const uint32_t rot = ((m >> r0) | (m << (4u - r0))) & 0xFu;
+    there = m == 0u;
+    if (!there) t = opp_tet(get4(to, (int)(((uint32_t)ctz32(rot) + r0) & 3u)));
+  }
+  if (f == 0) {
+    if (!there) at_add_u32(&M.ctr[C_WALK_FAIL], 1u);
+    utet[i] = t;
   }
 }
 
