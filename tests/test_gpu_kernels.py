@@ -68,3 +68,32 @@ def test_exact_rounds_of_all_small_sizes(ctx, oracle):
         got = oracle.canonical_real(ctx.delaunay(pts[:n], cfg).tets, n)
         want = oracle.canonical_real(oracle.delaunay(oracle.normalize_points(pts[:n])[0]), n)
         assert np.array_equal(got, want), n
+
+
+# 2,048 points (512 in exact mode) end the one-workgroup rounds; lists of more
+# than 1,024 (128) entries leave them within a run, and so do too few slots
+@pytest.mark.parametrize("n", [4, 5, 64, 512, 513, 2047, 2048, 2049])
+@pytest.mark.parametrize("kw", [{}, {"predicate_mode": "exact"}, {"presize": "grow"},
+                                {"enable_hilbert_sorting": True, "collect_stats": True}])
+def test_rounds_in_one_workgroup(ctx, oracle, n, kw):
+    """The mesh of few points, and the same mesh cut short by the round limit
+    and finished by the host, against the oracle."""
+    rng = np.random.default_rng(n)
+    p = rng.random((n, 3)).astype(np.float32)
+    p[n // 2:] = p[n // 2:] * np.float32(0.05) + np.float32(0.4)
+    p[-1] = p[0] if n > 64 else p[-1]
+    want = oracle.canonical_real(oracle.delaunay(oracle.normalize_points(p)[0]), n)
+    for extra in ({}, {"max_insert_iterations": 7}):
+        r = ctx.delaunay(p, wtet_amd.Config(**kw, **extra))
+        assert np.array_equal(oracle.canonical_real(r.tets, n), want), (n, kw, extra)
+        assert r.stats["rounds"] <= extra.get("max_insert_iterations", 100)
+
+
+def test_batch_of_few_points_in_all(ctx, oracle):
+    """Clouds that share the one-workgroup rounds: 40 of 4 to 45 points."""
+    rng = np.random.default_rng(3)
+    clouds = [rng.random((4 + i, 3)).astype(np.float32) for i in range(40)]
+    r = ctx.delaunay_batch(clouds)
+    for c, p in zip(range(40), clouds):
+        want = oracle.canonical_real(oracle.delaunay(oracle.normalize_points(p)[0]), len(p))
+        assert np.array_equal(oracle.canonical_real(r[c].tets, len(p)), want), c

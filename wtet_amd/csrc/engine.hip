@@ -430,18 +430,33 @@ uint32_t deferred_grid(const wtet_ctx* c, uint64_t dper, uint32_t grid) {
   return std::min(grid_for(c, 16 * dper, 1), std::min(grid * 8, 4096u));
 }
 
-// k flip iterations without the host: replays a captured graph (one per
-// buffer set, grid and k; captured on first use), or launches directly when
-// profiling (per-kernel events) or when graphs are off.
-// a_hint: bound on the first list; d_hint: deferred tets per iteration
-// expected (from the previous round).  The deferred check runs the full
-// predicates, whose exact stage keeps a thread busy for microseconds, so its
-// grid follows the deferred count rather than the list.
-// Lists this short run in one workgroup (k_flip_small): launches, not
-// work, set the time of their iterations.  The list may grow a few times
-// within the batch; past kSmallLimit the rest is left to the next batch.
-constexpr uint64_t kSmallList = 512;
+// Lists this short run in one workgroup (k_flip_small, k_rounds_small):
+// launches, not work, set the time of their iterations.  The list may grow a
+// few times within the batch; past kSmallLimit the rest is left to the next
+// batch.  Device time by the longest list (uniform points):
+//             filters   128   256   512   1024
+//             1,000 ms  2.59  2.53  2.21  2.09
+//             8,000 ms  4.27  4.20  4.10  4.04
+//             exact     64    128   256   512   1024
+//             700 ms    3.31  3.30  3.36  3.70  4.41
+//             8,000 ms  6.60  6.50  6.49  6.96  7.65
+// The full predicates of the exact mode are work, four lanes per tet, and one
+// CU is slow at it.
+uint64_t small_list(int mode) { return mode == PRED_FILTERED ? 1024 : 128; }
 constexpr uint32_t kSmallLimit = 2048;
+
+// Rounds of at most this many points whose flip lists begin with at most
+// small_list entries run in one workgroup, as many as there are: no round's
+// nine launches and no read by the host.  Device time by the most points:
+//             filters   0     1,024  2,048  4,096
+//             64 ms     1.05  0.75   0.74   0.74
+//             1,000 ms  2.47  2.09   2.10   2.10
+//             1,500 ms  2.65  2.64   2.49   2.51
+//             3,000 ms  3.14  3.14   3.11   3.39
+//             exact     0     512    2,048
+//             300 ms    3.31  3.08   3.01
+//             1,500 ms  4.29  4.26   5.22
+uint32_t small_points(int mode) { return mode == PRED_FILTERED ? 2048 : 512; }
 
 // The device buffers a captured sequence reads: a graph of another buffer
 // set is stale.
@@ -505,11 +520,18 @@ void launch_cached_graph(wtet_ctx* c, std::vector<wtet_ctx::GraphEntry>& cache,
   HIP_CHECK(hipGraphLaunch(exec, c->stream));
 }
 
+// k flip iterations without the host: replays a captured graph (one per
+// buffer set, grid and k; captured on first use), or launches directly when
+// profiling (per-kernel events) or when graphs are off.
+// a_hint: bound on the first list; d_hint: deferred tets per iteration
+// expected (from the previous round).  The deferred check runs the full
+// predicates, whose exact stage keeps a thread busy for microseconds, so its
+// grid follows the deferred count rather than the list.
 void run_flip_batch(wtet_ctx* c, uint32_t inf, int mode, uint64_t* st, int k, uint64_t a_hint,
                     uint64_t d_hint) {
   Mesh M = mesh_of(c, inf, mode);
   FlipLists L = lists_of(c);
-  if (a_hint <= kSmallList) {
+  if (a_hint <= small_list(mode)) {
     timed(c, K_FLIP_SMALL, [&] {
       launch_flip_small(M, L, st, P<uint64_t>(c->isums), k, kSmallLimit, c->stream);
     });
@@ -831,7 +853,7 @@ void run_round(wtet_ctx* c, Run& R, bool last) {
   uint64_t dper = (2 * (dsum - R.dsum_prev) + R.max_fi - 1) / (uint64_t)R.max_fi;
   R.dsum_prev = dsum;
   const uint64_t a_hint = (uint64_t)c->h_ctr[C_LIST] + 4ull * W;
-  const int variant = !R.flipping ? 0 : (a_hint <= kSmallList ? 1 : 2);
+  const int variant = !R.flipping ? 0 : (a_hint <= small_list(R.mode) ? 1 : 2);
   const uint32_t grid = variant == 2 ? grid_for(c, a_hint, 16) : 0u;
   const uint32_t dgrid = variant == 2 ? deferred_grid(c, dper, grid) : 0u;
   const int k = R.max_fi;
@@ -877,6 +899,47 @@ void run_round(wtet_ctx* c, Run& R, bool last) {
                         enqueue);
   }
   HIP_CHECK(hipGetLastError());
+}
+
+// The next rounds in one launch, from the vote or (voted) from the split of
+// the last pick's winners.  True: the last round is over.  False: a pick is
+// done whose round needs run_round, or room for more tets, made here.
+bool run_rounds_small(wtet_ctx* c, Run& R, bool voted) {
+  Mesh M = mesh_of(c, R.V, R.mode);
+  if (!voted) launch_set_ctr(M.ctr, C_SURV, R.U, C_ROUND, R.round, c->stream);
+  SmallRun J;
+  for (int q = 0; q < 2; ++q) {
+    J.uvert[q] = P<uint32_t>(c->uvert[q]);
+    J.utet[q] = P<uint32_t>(c->utet[q]);
+  }
+  J.wlist = P<uint2>(c->wlist);
+  J.slow = P<uint32_t>(c->slow_p);
+  J.cur = (uint32_t)R.cur;
+  J.voted = voted ? 1 : 0;
+  J.k = R.max_fi;
+  J.ring = c->ring;
+  J.warmup = (uint32_t)R.warmup;
+  J.max_round = (uint32_t)R.cfg.max_insert_iterations;
+  J.list = (uint32_t)small_list(R.mode);
+  J.limit = kSmallLimit;
+  if (c->profiling && c->evused > 4096) collect_times(c);
+  timed(c, K_FLIP_SMALL, [&] { launch_rounds_small(M, lists_of(c), J, R.st, P<uint64_t>(c->isums), c->stream); });
+  HIP_CHECK(hipGetLastError());
+  read_ctr(c);
+  const uint32_t* h = c->h_ctr;
+  R.dsum_prev = h[C_SLOW_SUM];
+  R.round += (int)h[C_RUN_PICKS];
+  R.cur ^= (int)(h[C_RUN_PICKS] & 1u);
+  R.K.rounds += h[C_RUN_PICKS];
+  R.K.sumU += h[C_RUN_SUMU];
+  R.W = h[C_WIN];
+  R.U = h[C_SURV] - R.W;
+  if (h[C_BADTET]) throw Fail{WTET_ERR_INTERNAL, "a point was located outside the super tet"};
+  if (h[C_RUN_DONE]) return true;
+  if (R.W == 0) throw Fail{WTET_ERR_INTERNAL, "no insertion possible in a round"};
+  const uint64_t need = (uint64_t)h[C_TETS] + 3ull * R.W + 64 + (h[C_STOP] ? h[C_LIST] : 0u);
+  if (need > c->cap_tets || h[C_STOP]) grow_for(c, need);
+  return false;
 }
 
 // batches of flip iterations until the active list is empty
@@ -1035,10 +1098,18 @@ void run_device(wtet_ctx* c, const float* d_xyz, const std::vector<uint32_t>& of
   dev_prepare(c, R, d_xyz);
   // at most max_insert_iterations rounds (src/phase1.rs:26); the host phase
   // inserts what they leave.  The first round's vote and pick are launched
-  // one by one, every later round runs from a captured graph (run_round).
+  // one by one, every later round runs from a captured graph (run_round);
+  // rounds of few points run many to a launch (run_rounds_small).
   if (R.U > 0 && R.round < R.cfg.max_insert_iterations) {
-    dev_vote(c, R);
-    for (;;) {
+    bool over = false;
+    if (R.flipping && R.U <= small_points(R.mode)) over = run_rounds_small(c, R, false);
+    else dev_vote(c, R);
+    while (!over) {
+      if (R.flipping && R.U + R.W <= small_points(R.mode) &&
+          (uint64_t)c->h_ctr[C_LIST] + 4ull * R.W <= small_list(R.mode)) {
+        over = run_rounds_small(c, R, true);
+        continue;
+      }
       const bool last = R.U == 0 || R.round >= R.cfg.max_insert_iterations;
       const uint32_t U = R.U;
       run_round(c, R, last);

@@ -96,6 +96,24 @@ void launch_batch_end(uint32_t* ctr, uint64_t* sums, int k, hipStream_t s);
 // workgroup, begin and end included
 void launch_flip_small(const Mesh& M, const FlipLists& L, uint64_t* st, uint64_t* sums, int k,
                        uint32_t limit, hipStream_t s);
+// Insertion rounds of few points in one workgroup, from the vote (voted 0) or
+// from the split of the winners a pick left (voted 1), until the rounds are
+// over (ctr[C_RUN_DONE]) or, after a pick, the next one does not fit.
+struct SmallRun {
+  uint32_t* uvert[2];
+  uint32_t* utet[2];
+  uint2* wlist;
+  uint32_t* slow;    // one entry per point
+  uint32_t cur;      // the list that holds the points
+  int voted;
+  int k;             // flip iterations in a round
+  int ring;          // insertion ring after the warmup rounds
+  uint32_t warmup, max_round;
+  uint32_t list;     // longest flip list a round may begin with
+  uint32_t limit;    // and an iteration of it
+};
+void launch_rounds_small(const Mesh& M, const FlipLists& L, const SmallRun& J, uint64_t* st, uint64_t* sums,
+                         hipStream_t s);
 // end > 0: also launch_batch_end(end).  ctr[C_SLOW_R] is 0 before (the split
 // clears it)
 void launch_relocate(const Mesh& M, const uint32_t* uvert, uint32_t* utet, uint32_t U,

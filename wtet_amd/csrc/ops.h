@@ -33,6 +33,9 @@ enum Ctr : int {
   C_NPTS = 13,      // points to insert (input minus exact duplicates)
   C_DUPSCAN = 14,   // duplicate scans that hit their length cap
   C_IT0 = 16,       // flip iterations before this round
+  C_RUN_PICKS = 17, // of k_rounds_small: rounds it picked,
+  C_RUN_SUMU = 18,  // the points they chose from,
+  C_RUN_DONE = 19,  // and whether the last round is over
   C_SURV = 15,      // uninserted points (the pick's winners leave at the split)
   C_TETS = 256,     // next free tet slot (the winners' at the split)
   C_LIST = 512,     // length of the active list between batches of iterations
@@ -59,8 +62,8 @@ enum IterSum : int {
   S_FLIPS = 1,          // flips executed
   S_ITERS = 2,          // iterations
   S_FLIPS23 = 3,        // 2-3 flips (the rest are 3-2)
-  S_SMALL_CHECKED = 4,  // of S_CHECKED: in k_flip_small
-  S_SMALL_FLIPS = 5,    // of S_FLIPS: in k_flip_small
+  S_SMALL_CHECKED = 4,  // of S_CHECKED: in one-workgroup kernels
+  S_SMALL_FLIPS = 5,    // of S_FLIPS: in one-workgroup kernels
   S_COUNT = 8
 };
 

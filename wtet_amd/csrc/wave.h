@@ -53,10 +53,10 @@ __device__ __forceinline__ void vote_wave(const MS& M, const uint32_t* uvert, co
       uint64_t o = shfl_xor_u64(k, off);
       k = o < k ? o : k;
     }
-    if (__lane_id() == leader) at_min_u64(&TVOTE(M, lt), k);
+    if (__lane_id() == leader) mesh_min(M, &TVOTE(M, lt), k);
     if (mine) pending = false;
   }
-  if (pending) at_min_u64(&TVOTE(M, t), key);
+  if (pending) mesh_min(M, &TVOTE(M, t), key);
 }
 
 // sorted position j of cloud c: kept unless it is a redundant duplicate;
@@ -238,6 +238,41 @@ __device__ __noinline__ void wg_slow_check(MS M, const uint32_t* act, uint4* pro
   for (uint32_t k = threadIdx.x; k < 4u * n; k += BS)
     flip_check_faces(M, act, prop, list ? list[k >> 2] : k >> 2, (int)(k & 3u), it, &ls);
   flush_stats(ls, st);
+}
+
+// The full point split (walk: relocation) of the points list[0..n) (null:
+// 0..n-1), out of line for the same reason.  a: the round (walk: the flip
+// iterations before it).
+template <class MS, int BS>
+__device__ __noinline__ void wg_slow_points(MS M, const uint32_t* uvert, uint32_t* utet, const uint32_t* list,
+                                            uint32_t n, uint32_t a, bool walk, uint64_t* st) {
+  PredStats ls = {};
+  if (walk) {
+    for (uint32_t k = threadIdx.x; k < 4u * n; k += BS)
+      relocate_faces(M, uvert, utet, list ? list[k >> 2] : k >> 2, (int)(k & 3u), a, &ls);
+  } else {
+    for (uint32_t k = threadIdx.x; k < n; k += BS) (void)split_points_body_t<false>(M, uvert, utet, list ? list[k] : k, a, &ls);
+  }
+  flush_stats(ls, st);
+}
+
+// exclusive rank of `flag` within the workgroup of BS threads, *total its
+// count; every thread calls it; w: BS / 64 words of LDS
+template <int BS>
+__device__ __forceinline__ uint32_t wg_rank(bool flag, uint32_t* total, uint32_t* w) {
+  const uint64_t m = __ballot(flag);
+  const uint32_t wave = threadIdx.x >> 6;
+  if (__lane_id() == 0) w[wave] = __popcll(m);
+  __syncthreads();
+  uint32_t off = 0, tot = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < BS / 64; ++k) {
+    off += k < wave ? w[k] : 0u;
+    tot += w[k];
+  }
+  __syncthreads();
+  *total = tot;
+  return off + __popcll(m & ((1ull << __lane_id()) - 1ull));
 }
 
 // Checks, decides and executes the A entries of act (tag it); the entries of
