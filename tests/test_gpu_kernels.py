@@ -97,3 +97,15 @@ def test_batch_of_few_points_in_all(ctx, oracle):
     for c, p in zip(range(40), clouds):
         want = oracle.canonical_real(oracle.delaunay(oracle.normalize_points(p)[0]), len(p))
         assert np.array_equal(oracle.canonical_real(r[c].tets, len(p)), want), c
+
+
+@pytest.mark.parametrize("n", [700, 3000, 20000])
+@pytest.mark.parametrize("iters", [1, 2, 5])
+@pytest.mark.parametrize("mode", ["filtered", "exact"])
+def test_flip_lists_left_over_rounds(ctx, oracle, n, iters, mode):
+    """Few flip iterations a round: most of the list waits over the splits of
+    the next rounds, and each tet has to stand in it once."""
+    p = np.random.default_rng(n + iters).random((n, 3)).astype(np.float32)
+    r = ctx.delaunay(p, wtet_amd.Config(max_flip_iterations=iters, predicate_mode=mode))
+    want = oracle.canonical_real(oracle.delaunay(oracle.normalize_points(p)[0]), n)
+    assert np.array_equal(oracle.canonical_real(r.tets, n), want)

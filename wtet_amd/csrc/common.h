@@ -11,10 +11,16 @@ namespace wtet {
 constexpr uint32_t kInvalid = 0xFFFFFFFFu;
 constexpr uint64_t kVoteNone = 0xFFFFFFFFFFFFFFFFull;
 
-// A slot's queue tag (Mesh::tqueue): the flip iteration whose list last took
-// the tet, so that a list takes each tet once; kFreed for a slot that a 3-2
-// flip freed (its record then holds kInvalid as first vertex and a live
-// neighbour to go on to).
+// A slot's queue tag (Mesh::tqueue): the last flip iteration in which the tet,
+// as an entry of the list, proposed a flip (or, with kWaits, was left to a
+// later one).  Its own thread then appends it to the next list, won or lost,
+// so that a list takes each tet once with no atomic, and the tag stands for
+// the proposal's vote for the tet itself.  kListed | i while it waits in the
+// list that iteration i begins with, over an insertion round; kFreed for a
+// slot that a 3-2 flip freed (its record then holds kInvalid as first vertex
+// and a live neighbour to go on to).
+constexpr uint32_t kWaits = 0x40000000u;
+constexpr uint32_t kListed = 0x80000000u;
 constexpr uint32_t kFreed = 0xFFFFFFFFu;
 
 // Face f of a tet is the face opposite vertex f.  kFace[f] lists its three
@@ -76,13 +82,6 @@ WT_HD uint32_t at_add_u32(uint32_t* p, uint32_t v) {
   return __atomic_fetch_add(p, v, __ATOMIC_RELAXED);
 #endif
 }
-WT_HD uint32_t at_max_u32(uint32_t* p, uint32_t v) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return atomicMax(p, v);
-#else
-  return __atomic_fetch_max(p, v, __ATOMIC_RELAXED);
-#endif
-}
 
 // the same at workgroup scope, for data that one workgroup owns while it
 // runs: performed in the XCD's L2, not at the memory side
@@ -92,13 +91,6 @@ WT_HD void wg_min_u64(uint64_t* p, uint64_t v) {
                                __HIP_MEMORY_SCOPE_WORKGROUP);
 #else
   (void)__atomic_fetch_min(p, v, __ATOMIC_RELAXED);
-#endif
-}
-WT_HD uint32_t wg_max_u32(uint32_t* p, uint32_t v) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return __hip_atomic_fetch_max(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-#else
-  return __atomic_fetch_max(p, v, __ATOMIC_RELAXED);
 #endif
 }
 

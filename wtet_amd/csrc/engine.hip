@@ -787,7 +787,7 @@ uint32_t dev_vote(wtet_ctx* c, Run& R) {
   timed(c, K_PICK, [&] {
     launch_pick(M, P<uint32_t>(c->uvert[cur]), P<uint32_t>(c->utet[cur]), U, P<uint2>(c->wlist),
                 P<uint32_t>(c->uvert[cur ^ 1]), P<uint32_t>(c->utet[cur ^ 1]), P<uint32_t>(c->blk),
-                round <= R.warmup ? 0 : c->ring, s);
+                round <= R.warmup ? 0 : c->ring, lists_of(c), s);
   });
   HIP_CHECK(hipGetLastError());
   after_pick(c, R, U);
@@ -884,7 +884,7 @@ void run_round(wtet_ctx* c, Run& R, bool last) {
       timed(c, K_VOTE, [&] { launch_vote(M, uv, ut, U, s); });
       timed(c, K_PICK, [&] {
         launch_pick(M, uv, ut, U, P<uint2>(c->wlist), P<uint32_t>(c->uvert[cur ^ 1]),
-                    P<uint32_t>(c->utet[cur ^ 1]), P<uint32_t>(c->blk), ring_next, s);
+                    P<uint32_t>(c->utet[cur ^ 1]), P<uint32_t>(c->blk), ring_next, L, s);
       });
     }
   };

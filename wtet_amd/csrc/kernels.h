@@ -54,13 +54,6 @@ hipError_t launch_stratify(uint32_t* uvert, uint32_t* utet, uint32_t U, const Cl
 uint32_t round_grid(uint64_t bound);
 void launch_vote(const Mesh& M, const uint32_t* uvert, const uint32_t* utet, uint32_t U,
                  hipStream_t s);
-// begins the next round (C_ROUND) and counts its winners (C_WIN); they leave
-// C_SURV, and take their slots from C_TETS, at the split.
-// ring: insert only where no tet within `ring` face-steps has a smaller vote
-// (blk: round_grid(U) entries)
-void launch_pick(const Mesh& M, const uint32_t* uvert, const uint32_t* utet, uint32_t U,
-                 uint2* wlist, uint32_t* uvert2, uint32_t* utet2, uint32_t* blk, int ring,
-                 hipStream_t s);
 // the two active lists, flip proposals and the executed flips of one
 // iteration
 struct FlipLists {
@@ -69,6 +62,13 @@ struct FlipLists {
   uint4* out;    // four uint4 per executed flip (flip_exec_loaded)
   uint32_t* slow;  // entries the lean check deferred
 };
+// begins the next round (C_ROUND) and counts its winners (C_WIN); they leave
+// C_SURV, and take their slots from C_TETS, at the split.
+// ring: insert only where no tet within `ring` face-steps has a smaller vote
+// (blk: round_grid(U) entries)
+void launch_pick(const Mesh& M, const uint32_t* uvert, const uint32_t* utet, uint32_t U,
+                 uint2* wlist, uint32_t* uvert2, uint32_t* utet2, uint32_t* blk, int ring,
+                 const FlipLists& L, hipStream_t s);
 // appends the children to the active list after its ctr[C_LIST] entries
 void launch_split(const Mesh& M, const uint2* wlist, uint32_t W, const FlipLists& L, hipStream_t s);
 // filtered mode: an FP32-only kernel, then the full predicates on the points

@@ -295,10 +295,14 @@ __global__ void __launch_bounds__(kBlock) k_vote(Mesh M, const uint32_t* uvert, 
   vote_wave(M, uvert, utet, gid(), M.ctr[C_SURV]);
 }
 
-// Counts the winners of each block of points.  Begins the round in the
+// Counts the winners of each block of points, and marks the tets left in the
+// flip list.  Begins the round in the
 // counters: no other thread of this kernel reads them.
-__global__ void __launch_bounds__(kBlock) k_pick_count(Mesh M, const uint32_t* utet, uint32_t* blk, int ring) {
-  const uint32_t U = M.ctr[C_SURV];
+__global__ void __launch_bounds__(kBlock) k_pick_count(Mesh M, const uint32_t* utet, uint32_t* blk, int ring,
+                                                       FlipLists L) {
+  const uint32_t U = M.ctr[C_SURV], A = M.ctr[C_LIST], it = M.ctr[C_IT] + 1u;
+  const uint32_t* act = L.act[M.ctr[C_PAR] & 1u];
+  for (uint32_t j = gid(); j < A; j += gridDim.x * blockDim.x) mark_listed(M, act[j], it);
   uint32_t i = gid();
   if (i == 0) {
     M.ctr[C_ROUND] += 1u;
@@ -367,11 +371,11 @@ constexpr uint32_t kScatterScan = 4096;
 
 void launch_pick(const Mesh& M, const uint32_t* uvert, const uint32_t* utet, uint32_t U,
                  uint2* wlist, uint32_t* uvert2, uint32_t* utet2, uint32_t* blk, int ring,
-                 hipStream_t s) {
+                 const FlipLists& L, hipStream_t s) {
   // blocks past the count write zero block totals, so the scan may cover
   // the whole grid
   uint32_t nb = round_grid(U);
-  k_pick_count<<<nb, kBlock, 0, s>>>(M, utet, blk, ring);
+  k_pick_count<<<nb, kBlock, 0, s>>>(M, utet, blk, ring, L);
   if (nb <= kScatterScan) {
     k_pick_scatter<false><<<nb, kBlock, 0, s>>>(M, uvert, utet, wlist, uvert2, utet2, blk, ring);
   } else {
@@ -549,7 +553,7 @@ __device__ __forceinline__ uint32_t iter_tag(const uint32_t* ctr, int i) { retur
 __device__ __forceinline__ uint32_t iter_par(const uint32_t* ctr, int i) { return (ctr[C_PAR] + (uint32_t)i) & 1u; }
 
 // The filters of the flip check on every list entry, one thread per tet; the
-// entries they leave go to L.slow.  98 VGPRs, 4 waves per SIMD (at 96 and 5
+// entries they leave go to L.slow.  104 VGPRs, 4 waves per SIMD (at 96 and 5
 // waves, with two registers spilled, it took the same time).  1M uniform
 // points: 6.68 ms of event time a triangulation with insphere_f32 and
 // insphere_f64 per face and three orient3d after each (158 VGPRs), 5.60 ms
@@ -566,7 +570,7 @@ __global__ void __launch_bounds__(kBlock) k_flip_check(Mesh M, FlipLists L, int 
   for (uint32_t j = gid(); j < A; j += stride)
     if (flip_check_lean(M, cur, L.prop, j, it, &ls)) {
       const uint32_t k = append_slot(it_ctr(M.ctr, C_ITS, i));
-      if (requeue) L.prop[j] = requeue_proposal(cur[j]);
+      if (requeue) L.prop[j] = requeue_proposal(M, cur[j], it);
       else L.slow[k] = j;
     }
   flush_stats(ls, st);
@@ -615,7 +619,7 @@ __device__ __forceinline__ uint32_t block_prefix3(uint32_t a, uint32_t b, uint32
 }
 
 // Decide every proposal; a winner loads its flip's tets at once, so those
-// loads overlap its queue claims and the block's counter claims.  Then the
+// loads overlap the block's counter claims.  Then the
 // block claims list space with one atomic per counter (flips, fresh slots,
 // next active entries) -- the counters share a cache line, so per-wave
 // atomics from every wave would serialize -- and every winner executes its
@@ -624,7 +628,11 @@ __device__ __forceinline__ uint32_t block_prefix3(uint32_t a, uint32_t b, uint32
 // finds the external neighbours in the flip's own record.  Event time at 1M
 // points against an array per field: flip_check 5.58 -> 4.28 ms (it reads one
 // line of a tet instead of three, and no queued bit to clear), decide_exec 6.81
-// -> 5.83 ms, flip_update 4.83 -> 4.39 ms.
+// -> 5.83 ms, flip_update 4.83 -> 4.39 ms.  With plain tags instead of an
+// atomic maximum per queued tet and an atomic vote for the proposal's own:
+// decide_exec 5.83 -> 5.20 ms, flip_check 4.28 -> 4.17 ms (1,024 clouds: 9.52 ->
+// 8.69 and 11.6 -> 10.8).  Random lines bound both: this card serves 55 G/s
+// of 64-byte reads, 27 G/s of atomics.
 // Blocks of 512 threads: each tile of proposals claims its flips, fresh
 // slots and queue entries with one atomic per counter, and those
 // same-address atomics complete one at a time at the memory side; 512
@@ -761,6 +769,7 @@ __global__ void __launch_bounds__(kFlipSmallBlock) k_rounds_small(WgMesh M, Flip
       uint32_t* uv2 = cur ? J.uvert[0] : J.uvert[1];
       uint32_t* ut2 = cur ? J.utet[0] : J.utet[1];
       for (uint32_t b = 0; b < U; b += BS) vote_wave(M, uv, ut, b + tid, U);
+      for (uint32_t j = tid; j < A; j += BS) mark_listed(M, par ? L.act[1][j] : L.act[0][j], it + 1u);
       __syncthreads();
       ++round;
       const int ring = round <= J.warmup ? 0 : J.ring;

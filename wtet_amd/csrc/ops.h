@@ -78,9 +78,8 @@ struct __attribute__((aligned(32))) AdjRec {
 
 // One tet slot's record, a 64-byte half line: everything about it that plain
 // stores write and that the kernels read at random.  What atomics write (the
-// votes, the queue tag) is in arrays of its own: atomics complete at the
-// memory side, and a plain store beside them would leave the line dirty in
-// an XCD's L2.  Measured against an array per field (the check then read
+// votes) is in arrays of its own: atomics complete at the memory side, and a
+// plain store beside them would leave the line dirty in an XCD's L2.  Measured against an array per field (the check then read
 // three lines of a tet, a flip wrote three of each new tet): see
 // k_flip_decide_exec.
 struct __attribute__((aligned(64))) TetRec {
@@ -115,7 +114,7 @@ struct Mesh {
   const float4* pts;  // n + 5 points (n real, 4 super, 1 infinity)
   TetRec* rec;
   FlipMsg* tmsg;     // per slot destroyed by a flip this iteration
-  uint32_t* tqueue;  // queue tag, kFreed
+  uint32_t* tqueue;  // queue tag (kListed, kFreed)
   uint64_t* tvote;   // insertion vote (min key)
   uint64_t* fvote;   // flip vote (min key, iteration-tagged)
   uint32_t* ctr;     // Ctr counters
@@ -142,9 +141,7 @@ struct WgMesh : Mesh {};
 
 // atomics at the scope the mesh is shared at
 WT_HD void mesh_min(const Mesh&, uint64_t* p, uint64_t v) { at_min_u64(p, v); }
-WT_HD uint32_t mesh_max(const Mesh&, uint32_t* p, uint32_t v) { return at_max_u32(p, v); }
 WT_HD void mesh_min(const WgMesh&, uint64_t* p, uint64_t v) { wg_min_u64(p, v); }
-WT_HD uint32_t mesh_max(const WgMesh&, uint32_t* p, uint32_t v) { return wg_max_u32(p, v); }
 
 template <class MS>
 WT_HD uint4 TN(const MS& M, uint32_t t) {
@@ -310,7 +307,7 @@ WT_HD uint32_t child_slot(uint32_t t, uint32_t base, uint32_t j) {
 
 // c[0..3] receives the children's slots; returns which of them join the
 // active list of iteration `it` (bit j for child j; slot t only if the list
-// does not hold it yet).
+// does not hold it yet: the pick marked what it does).
 // The neighbours' split records are loaded before any store: this kernel
 // writes those of fresh slots only, never a neighbour's.
 template <class MS>
@@ -354,13 +351,13 @@ WT_HD uint32_t split_body(const MS& M, const uint2* wlist, uint32_t k, uint32_t 
     set_adj(M, c[j], no, nov);
     TVOTE(M, c[j]) = kVoteNone;
     if (j > 0) {  // fresh slot: initialise every per-slot field
-      TQUEUE(M, c[j]) = it;
+      TQUEUE(M, c[j]) = 0u;
       FVOTE(M, c[j]) = kVoteNone;
       TSPLIT(M, c[j]) = make_uint2(0u, 0u);
       FSTAMP(M, c[j]) = 0u;
     }
   }
-  return mesh_max(M, &TQUEUE(M, t), it) == it ? 0xEu : 0xFu;
+  return TQUEUE(M, t) == (kListed | it) ? 0xEu : 0xFu;
 }
 
 // ---------------------------------------------------------------------------
@@ -435,13 +432,15 @@ WT_HD void pick_xyz(const float (*P)[3], int k, float* out) {
 }
 
 // The proposal of tet t across face f (its kind, offending edge and third
-// tet as flip_check_lean finds them): votes for the tets it involves.
+// tet as flip_check_lean finds them): votes for the other tets it involves;
+// its tag is the vote for its own.  A vote is an atomic minimum on a random
+// line, 27 G/s on this card, a tag a store, 84 G/s.
 template <class MS>
 WT_HD uint4 flip_propose(const MS& M, uint32_t t, uint32_t f, uint32_t kind, uint32_t bad, uint32_t third,
                          uint32_t it) {
   uint32_t nt = opp_tet(*opp_word(M, t, f));
   uint64_t key = flip_key(it, t);
-  mesh_min(M, &FVOTE(M, t), key);
+  TQUEUE(M, t) = it;
   mesh_min(M, &FVOTE(M, nt), key);
   if (kind == 1u) mesh_min(M, &FVOTE(M, third), key);
   return make_uint4(t, f | kind << 2 | bad << 3, nt, third);
@@ -691,7 +690,7 @@ WT_HD void flip_exec_loaded(const MS& M, const uint4 pr, const FlipTets& F, uint
     FVOTE(M, s) = kVoteNone;
     TSPLIT(M, s) = make_uint2(0u, 0u);
     FSTAMP(M, s) = 0u;
-    TQUEUE(M, s) = it + 1u;  // fresh slot: queued by the caller
+    TQUEUE(M, s) = 0u;
     outk[0] = make_uint4(Txy, Tyz, Tzx, 0u);
     outk[1] = make_uint4(o, a, 0u, get4(to, pos[2]));
     outk[2] = make_uint4(get4(no, qz), get4(to, pos[0]), get4(no, qx), get4(to, pos[1]));
@@ -737,18 +736,15 @@ WT_HD void flip_exec_loaded(const MS& M, const uint4 pr, const FlipTets& F, uint
   }
 }
 
-// A proposal wins when it holds the vote of every tet it involves; the
+// A proposal wins when it holds the smallest vote of every tet it involves; the
 // winner executes at once (its tets belong to no other winner), losers go
 // back to the active list (src/shaders/mark_rejected_flips.wgsl:61-178 and
 // src/shaders/flip.wgsl:531-845, one pass here).
-// Decide proposal pr and claim the queue entries it needs: a winner's two
-// reused slots (and, for a 2-3 flip, the fresh slot, counted in *nslot), or a
-// loser's own tet.  qid[0..*nq) are the tets to append to the next active
-// list, that of iteration it + 1 (their queue tag is set here, so each tet is
-// appended once); for a 2-3 winner
-// the fresh slot is appended by the caller after qid.  A winner also loads
-// its flip's tets (into F), issued after its queue claims so that the loads
-// and the claims' round trips overlap.
+// Decide proposal pr.  qid[0..*nq) are the tets to append to the next active
+// list: the proposal's own, and for a winner its neighbour's slot unless that
+// proposed too and so appends itself (it lost: its vote is the winner's).  For
+// a 2-3 winner (*nslot = 1) the caller appends the fresh slot after qid.  A
+// winner also loads its flip's tets (into F).
 template <class MS>
 WT_HD bool flip_decide_load(const MS& M, const uint4& pr, uint32_t it, uint32_t qid[2],
                             uint32_t* nq, uint32_t* nslot, FlipTets& F) {
@@ -757,27 +753,40 @@ WT_HD bool flip_decide_load(const MS& M, const uint4& pr, uint32_t it, uint32_t 
   qid[0] = qid[1] = kInvalid;
   if (pr.x == kInvalid) return false;
   uint64_t key = flip_key(it, pr.x);
-  bool win = FVOTE(M, pr.x) == key && FVOTE(M, pr.z) == key;
-  if (((pr.y >> 2) & 1u) && FVOTE(M, pr.w) != key) win = false;
+  // a 2-3 flip reads its neighbour's words again for its third tet's: every
+  // load is issued before the first is used
+  const uint32_t m = ((pr.y >> 2) & 1u) ? pr.w : pr.z;
+  const uint64_t vx = FVOTE(M, pr.x), vz = FVOTE(M, pr.z), vm = FVOTE(M, m);
+  const uint32_t tag = TQUEUE(M, pr.z), tag_m = TQUEUE(M, m);
+  // votes of older iterations are larger than every one of this
+  const bool lost = (vx <= key) | (vz != key) | (vm != key) | ((tag == it) & (pr.z < pr.x)) |
+                    ((tag_m == it) & (m < pr.x));
+  const bool win = !lost;
+  qid[0] = pr.x;
+  qid[1] = pr.z;
+  *nq = 1;
   if (win) {
-    uint32_t o0 = mesh_max(M, &TQUEUE(M, pr.x), it + 1u);
-    uint32_t o1 = mesh_max(M, &TQUEUE(M, pr.z), it + 1u);
     flip_load(M, pr, F);
-    const bool q0 = o0 != it + 1u, q1 = o1 != it + 1u;
-    qid[0] = q0 ? pr.x : pr.z;
-    qid[1] = pr.z;
-    *nq = (uint32_t)q0 + (uint32_t)q1;
+    if ((tag & ~kWaits) != it) *nq = 2;
     if (((pr.y >> 2) & 1u) == 0u) *nslot = 1;
-  } else {
-    qid[0] = pr.x;
-    *nq = mesh_max(M, &TQUEUE(M, pr.x), it + 1u) != it + 1u ? 1u : 0u;
   }
   return win;
 }
 
 // The proposal of a tet that no kernel of this iteration decides: nobody
 // votes for it, so it loses and stays in the active list.
-WT_HD uint4 requeue_proposal(uint32_t t) { return make_uint4(t, 0u, t, kInvalid); }
+template <class MS>
+WT_HD uint4 requeue_proposal(const MS& M, uint32_t t, uint32_t it) {
+  TQUEUE(M, t) = kWaits | it;
+  return make_uint4(t, 0u, t, kInvalid);
+}
+
+// entry t of the list that iteration it begins with stays there over the
+// round's splits
+template <class MS>
+WT_HD void mark_listed(const MS& M, uint32_t t, uint32_t it) {
+  if (TQUEUE(M, t) != kFreed) TQUEUE(M, t) = kListed | it;
+}
 
 // src/shaders/update_opp.wgsl:73-220.  The flip's six external faces
 // (tet T, face e, T's vertex vT opposite e): a face whose neighbour q
