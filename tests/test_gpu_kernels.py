@@ -109,3 +109,16 @@ def test_flip_lists_left_over_rounds(ctx, oracle, n, iters, mode):
     r = ctx.delaunay(p, wtet_amd.Config(max_flip_iterations=iters, predicate_mode=mode))
     want = oracle.canonical_real(oracle.delaunay(oracle.normalize_points(p)[0]), n)
     assert np.array_equal(oracle.canonical_real(r.tets, n), want)
+
+
+@pytest.mark.parametrize("side,extra", [(12, 0), (13, 0), (20, 0), (20, 12000)])
+def test_lattices_that_take_the_full_predicates(ctx, oracle, side, extra):
+    """Inputs whose tets the filters leave: below and above the size of the
+    one-workgroup rounds, and mixed with points in general position."""
+    g = np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing="ij"), -1).reshape(-1, 3).astype(np.float32)
+    rng = np.random.default_rng(side + extra)
+    p = np.concatenate([g, rng.random((extra, 3)).astype(np.float32) * (side - 1) + np.float32(side)])
+    p = p[rng.permutation(len(p))].astype(np.float32)
+    want = oracle.canonical_real(oracle.delaunay(oracle.normalize_points(p)[0]), len(p))
+    for _ in range(3):  # launched, recorded and replayed
+        assert np.array_equal(oracle.canonical_real(ctx.delaunay(p).tets, len(p)), want)

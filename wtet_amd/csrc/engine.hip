@@ -391,14 +391,15 @@ FlipLists lists_of(wtet_ctx* c) {
 
 // The iterations of a batch of k, between launch_batch_begin and _end.
 // sparse: the full check of deferred tets runs in the first iteration only;
-// later ones leave such tets in the active list.
+// later ones leave such tets in the active list.  full: every tet takes the
+// full check.
 void enqueue_flip_iterations(wtet_ctx* c, const Mesh& M, const FlipLists& L, uint64_t* st, int k,
-                             uint32_t grid, uint32_t dgrid, bool sparse) {
+                             uint32_t grid, uint32_t dgrid, bool sparse, bool full) {
   hipStream_t s = c->stream;
   for (int i = 0; i < k; ++i) {
-    const bool requeue = sparse && i > 0;
-    timed(c, K_FLIP_CHECK, [&] { launch_flip_check(M, L, i, requeue, grid, st, s); });
-    if (!requeue) timed(c, K_FLIP_CHECK_DEFERRED, [&] { launch_flip_check_deferred(M, L, i, dgrid, st, s); });
+    const bool requeue = sparse && !full && i > 0;
+    timed(c, K_FLIP_CHECK, [&] { launch_flip_check(M, L, i, requeue, full, grid, st, s); });
+    if (!requeue && !full) timed(c, K_FLIP_CHECK_DEFERRED, [&] { launch_flip_check_deferred(M, L, i, dgrid, st, s); });
     timed(c, K_FLIP_EXEC, [&] { launch_flip_decide_exec(M, L, i, grid, s); });
     timed(c, K_FLIP_UPDATE, [&] { launch_flip_update(M, L, i, grid, s); });
   }
@@ -442,7 +443,7 @@ uint32_t deferred_grid(const wtet_ctx* c, uint64_t dper, uint32_t grid) {
 //             8,000 ms  6.60  6.50  6.49  6.96  7.65
 // The full predicates of the exact mode are work, four lanes per tet, and one
 // CU is slow at it.
-uint64_t small_list(int mode) { return mode == PRED_FILTERED ? 1024 : 128; }
+uint64_t small_list(bool full) { return full ? 128 : 1024; }
 constexpr uint32_t kSmallLimit = 2048;
 
 // Rounds of at most this many points whose flip lists begin with at most
@@ -456,7 +457,7 @@ constexpr uint32_t kSmallLimit = 2048;
 //             exact     0     512    2,048
 //             300 ms    3.31  3.08   3.01
 //             1,500 ms  4.29  4.26   5.22
-uint32_t small_points(int mode) { return mode == PRED_FILTERED ? 2048 : 512; }
+uint32_t small_points(bool full) { return full ? 512 : 2048; }
 
 // The device buffers a captured sequence reads: a graph of another buffer
 // set is stale.
@@ -527,11 +528,12 @@ void launch_cached_graph(wtet_ctx* c, std::vector<wtet_ctx::GraphEntry>& cache,
 // expected (from the previous round).  The deferred check runs the full
 // predicates, whose exact stage keeps a thread busy for microseconds, so its
 // grid follows the deferred count rather than the list.
+// full: the input's tets take the full predicates anyway (Run::full)
 void run_flip_batch(wtet_ctx* c, uint32_t inf, int mode, uint64_t* st, int k, uint64_t a_hint,
-                    uint64_t d_hint) {
+                    uint64_t d_hint, bool full) {
   Mesh M = mesh_of(c, inf, mode);
   FlipLists L = lists_of(c);
-  if (a_hint <= small_list(mode)) {
+  if (a_hint <= small_list(full || mode != PRED_FILTERED)) {
     timed(c, K_FLIP_SMALL, [&] {
       launch_flip_small(M, L, st, P<uint64_t>(c->isums), k, kSmallLimit, c->stream);
     });
@@ -542,7 +544,7 @@ void run_flip_batch(wtet_ctx* c, uint32_t inf, int mode, uint64_t* st, int k, ui
   uint32_t dgrid = deferred_grid(c, d_hint, grid);
   auto enqueue = [&] {
     launch_batch_begin(M.ctr, k, c->stream);
-    enqueue_flip_iterations(c, M, L, st, k, grid, dgrid, false);
+    enqueue_flip_iterations(c, M, L, st, k, grid, dgrid, false, full);
     launch_batch_end(M.ctr, P<uint64_t>(c->isums), k, c->stream);
   };
   if (!c->use_graphs || c->profiling) {
@@ -551,7 +553,7 @@ void run_flip_batch(wtet_ctx* c, uint32_t inf, int mode, uint64_t* st, int k, ui
     HIP_CHECK(hipGetLastError());
     return;
   }
-  launch_cached_graph(c, c->graphs, buffer_key(c, M, L, st), {(uint64_t)dgrid, (uint64_t)grid, (uint64_t)k}, enqueue);
+  launch_cached_graph(c, c->graphs, buffer_key(c, M, L, st), {(uint64_t)dgrid, (uint64_t)grid, (uint64_t)k, (uint64_t)full}, enqueue);
 }
 
 // tet slots after growth by `need`; the flip iterations read the capacity
@@ -590,7 +592,13 @@ struct Run {
   uint32_t round = 0;
   uint32_t U = 0;          // uninserted points
   uint32_t W = 0;          // insertions of the current round
-  uint64_t dsum_prev = 0;  // deferred-check total at the previous round
+  uint32_t dsum_prev = 0, csum_prev = 0;  // C_SLOW_SUM and C_CHECK_SUM at the previous round
+  // The filters have left most of a round's tets to the full predicates: from
+  // then on every tet takes them at once, and the one-workgroup kernels take
+  // the exact mode's lists.  48^3 lattice: device 18.4 -> 16.5 ms (an iteration's
+  // checks 40 -> 35 us, the last rounds 1.66 -> 0.61 ms).
+  bool full = false;
+  bool takes_full() const { return full || mode != PRED_FILTERED; }
   int max_fi = 10;
   uint32_t warmup = 0;     // rounds that insert one point per tet
   Counters K;
@@ -812,14 +820,22 @@ void dev_split_points(wtet_ctx* c, Run& R) {
   HIP_CHECK(hipGetLastError());
 }
 
+// Deferred tets per iteration to expect (twice the last round's average), from
+// the counters just read; also sets R.full.
+uint64_t deferred_per_iteration(wtet_ctx* c, Run& R) {
+  const uint32_t slow = c->h_ctr[C_SLOW_SUM] - R.dsum_prev, checked = c->h_ctr[C_CHECK_SUM] - R.csum_prev;
+  R.dsum_prev += slow;
+  R.csum_prev += checked;
+  if (R.mode == PRED_FILTERED && checked >= 1024u && slow > checked / 2u) R.full = true;
+  return (2ull * slow + R.max_fi - 1) / (uint64_t)R.max_fi;
+}
+
 // the round's flip iterations (src/phase1.rs, flip loop), from device counters
 void dev_round_flips(wtet_ctx* c, Run& R) {
   // the first list holds the entries carried over plus four per split;
   // the deferred count per iteration follows the previous round's
-  uint64_t dsum = c->h_ctr[C_SLOW_SUM];
-  uint64_t dper = (2 * (dsum - R.dsum_prev) + R.max_fi - 1) / (uint64_t)R.max_fi;
-  R.dsum_prev = dsum;
-  run_flip_batch(c, R.V, R.mode, R.st, R.max_fi, (uint64_t)c->h_ctr[C_LIST] + 4ull * R.W, dper);
+  const uint64_t dper = deferred_per_iteration(c, R);
+  run_flip_batch(c, R.V, R.mode, R.st, R.max_fi, (uint64_t)c->h_ctr[C_LIST] + 4ull * R.W, dper, R.full);
 }
 
 // uninserted points of flipped tets to their new tets (relocate_points_fast.wgsl)
@@ -849,11 +865,9 @@ void run_round(wtet_ctx* c, Run& R, bool last) {
   const uint32_t cur = R.cur, W = R.W, U = R.U;
   const int ring_next = R.round + 1 <= R.warmup ? 0 : c->ring;
   // the round's flips, sized as dev_round_flips sizes them
-  uint64_t dsum = c->h_ctr[C_SLOW_SUM];
-  uint64_t dper = (2 * (dsum - R.dsum_prev) + R.max_fi - 1) / (uint64_t)R.max_fi;
-  R.dsum_prev = dsum;
+  const uint64_t dper = deferred_per_iteration(c, R);
   const uint64_t a_hint = (uint64_t)c->h_ctr[C_LIST] + 4ull * W;
-  const int variant = !R.flipping ? 0 : (a_hint <= small_list(R.mode) ? 1 : 2);
+  const int variant = !R.flipping ? 0 : (a_hint <= small_list(R.takes_full()) ? 1 : 2);
   const uint32_t grid = variant == 2 ? grid_for(c, a_hint, 16) : 0u;
   const uint32_t dgrid = variant == 2 ? deferred_grid(c, dper, grid) : 0u;
   const int k = R.max_fi;
@@ -875,7 +889,7 @@ void run_round(wtet_ctx* c, Run& R, bool last) {
         timed(c, K_FLIP_SMALL, [&] { launch_flip_small(M, L, R.st, sums, k, kSmallLimit, s); });
       } else {
         if (!beside) launch_batch_begin(M.ctr, k, s);
-        enqueue_flip_iterations(c, M, L, R.st, k, grid, dgrid, sparse);
+        enqueue_flip_iterations(c, M, L, R.st, k, grid, dgrid, sparse, R.full);
         if (!beside) launch_batch_end(M.ctr, sums, k, s);
       }
       timed(c, K_RELOCATE, [&] { launch_relocate(M, uv, ut, U, R.st, slow_p, sums, beside, s); });
@@ -894,7 +908,7 @@ void run_round(wtet_ctx* c, Run& R, bool last) {
   } else {
     launch_cached_graph(c, c->round_graphs, buffer_key(c, M, L, R.st),
                         {(uint64_t)cur, (uint64_t)round_grid(W), (uint64_t)round_grid(U), (uint64_t)(U > 0),
-                         (uint64_t)variant, (uint64_t)grid, (uint64_t)dgrid, (uint64_t)sparse, (uint64_t)k, (uint64_t)last,
+                         (uint64_t)variant, (uint64_t)grid, (uint64_t)dgrid, (uint64_t)sparse, (uint64_t)R.full, (uint64_t)k, (uint64_t)last,
                          (uint64_t)ring_next},
                         enqueue);
   }
@@ -920,14 +934,15 @@ bool run_rounds_small(wtet_ctx* c, Run& R, bool voted) {
   J.ring = c->ring;
   J.warmup = (uint32_t)R.warmup;
   J.max_round = (uint32_t)R.cfg.max_insert_iterations;
-  J.list = (uint32_t)small_list(R.mode);
+  J.list = (uint32_t)small_list(R.takes_full());
+  J.list_full = (uint32_t)small_list(true);
   J.limit = kSmallLimit;
   if (c->profiling && c->evused > 4096) collect_times(c);
   timed(c, K_FLIP_SMALL, [&] { launch_rounds_small(M, lists_of(c), J, R.st, P<uint64_t>(c->isums), c->stream); });
   HIP_CHECK(hipGetLastError());
   read_ctr(c);
   const uint32_t* h = c->h_ctr;
-  R.dsum_prev = h[C_SLOW_SUM];
+  (void)deferred_per_iteration(c, R);
   R.round += (int)h[C_RUN_PICKS];
   R.cur ^= (int)(h[C_RUN_PICKS] & 1u);
   R.K.rounds += h[C_RUN_PICKS];
@@ -949,7 +964,7 @@ void dev_finish_flips(wtet_ctx* c, Run& R) {
     read_ctr(c);
     if (c->h_ctr[C_STOP]) grow_for(c, (uint64_t)c->h_ctr[C_TETS] + c->h_ctr[C_LIST] + 64);
     else if (c->h_ctr[C_LIST] == 0) break;
-    run_flip_batch(c, R.V, R.mode, R.st, 16, c->h_ctr[C_LIST], c->h_ctr[C_LIST] / 64);
+    run_flip_batch(c, R.V, R.mode, R.st, 16, c->h_ctr[C_LIST], c->h_ctr[C_LIST] / 64, R.full);
   }
 }
 
@@ -1102,11 +1117,11 @@ void run_device(wtet_ctx* c, const float* d_xyz, const std::vector<uint32_t>& of
   // rounds of few points run many to a launch (run_rounds_small).
   if (R.U > 0 && R.round < R.cfg.max_insert_iterations) {
     bool over = false;
-    if (R.flipping && R.U <= small_points(R.mode)) over = run_rounds_small(c, R, false);
+    if (R.flipping && R.U <= small_points(R.takes_full())) over = run_rounds_small(c, R, false);
     else dev_vote(c, R);
     while (!over) {
-      if (R.flipping && R.U + R.W <= small_points(R.mode) &&
-          (uint64_t)c->h_ctr[C_LIST] + 4ull * R.W <= small_list(R.mode)) {
+      if (R.flipping && R.U + R.W <= small_points(R.takes_full()) &&
+          (uint64_t)c->h_ctr[C_LIST] + 4ull * R.W <= small_list(R.takes_full())) {
         over = run_rounds_small(c, R, true);
         continue;
       }
@@ -2930,7 +2945,7 @@ wtet_status wtet_stage_flip(wtet_ctx* c, int predicate_mode, wtet_stage_info* in
     uint32_t a = c->h_ctr[C_LIST];
     uint64_t before[S_COUNT] = {}, after[S_COUNT] = {};
     HIP_CHECK(hipMemcpyAsync(before, c->isums.p, S_COUNT * 8, hipMemcpyDeviceToHost, c->stream));
-    if (a > 0) run_flip_batch(c, R.V, mode, R.st, 1, a, a / 8 + 1);
+    if (a > 0) run_flip_batch(c, R.V, mode, R.st, 1, a, a / 8 + 1, false);
     HIP_CHECK(hipMemcpyAsync(after, c->isums.p, S_COUNT * 8, hipMemcpyDeviceToHost, c->stream));
     HIP_CHECK(hipStreamSynchronize(c->stream));
     S->checked = (uint32_t)(after[0] - before[0]);

@@ -83,8 +83,8 @@ void launch_split_points(const Mesh& M, const uint32_t* uvert, uint32_t* utet, u
 void launch_batch_begin(uint32_t* ctr, int k, hipStream_t s);
 // filtered mode: the FP32-only check, deferring undecided tets to the full
 // check that follows or, with requeue, to a later iteration (none follows);
-// exact mode: the full check, nothing deferred
-void launch_flip_check(const Mesh& M, const FlipLists& L, int i, bool requeue, uint32_t grid, uint64_t* st,
+// exact mode, or with full: the full check, nothing deferred
+void launch_flip_check(const Mesh& M, const FlipLists& L, int i, bool requeue, bool full, uint32_t grid, uint64_t* st,
                        hipStream_t s);
 void launch_flip_check_deferred(const Mesh& M, const FlipLists& L, int i, uint32_t grid, uint64_t* st,
                                 hipStream_t s);
@@ -110,6 +110,8 @@ struct SmallRun {
   int ring;          // insertion ring after the warmup rounds
   uint32_t warmup, max_round;
   uint32_t list;     // longest flip list a round may begin with
+  uint32_t list_full;  // the same after a round that left more entries an
+                       // iteration to the full predicates
   uint32_t limit;    // and an iteration of it
 };
 void launch_rounds_small(const Mesh& M, const FlipLists& L, const SmallRun& J, uint64_t* st, uint64_t* sums,

@@ -470,6 +470,7 @@ __device__ __forceinline__ void batch_end(uint32_t* ctr, unsigned long long* sum
   sums[S_ITERS] += (unsigned long long)n;
   sums[S_FLIPS23] += ctr[C_TETS] - ctr[C_TETS_IT];
   ctr[C_SLOW_SUM] += sd;
+  ctr[C_CHECK_SUM] += (uint32_t)sa;
   ctr[C_SLOW_LAST] = last;
   if (peak > ctr[C_PEAKA]) ctr[C_PEAKA] = peak;
   if (n < k && left > 0u) ctr[C_STOP] = 1u;  // the tet slots could not hold the next one
@@ -727,6 +728,7 @@ __global__ void __launch_bounds__(kFlipSmallBlock) k_flip_small(WgMesh M, FlipLi
     sums[S_SMALL_FLIPS] += sf;
     ctr[C_TETS] = tets;
     ctr[C_SLOW_SUM] += slow;
+    ctr[C_CHECK_SUM] += sa;
     ctr[C_SLOW_LAST] = last;
     if (peak > ctr[C_PEAKA]) ctr[C_PEAKA] = peak;
     if (stop) ctr[C_STOP] = 1u;
@@ -758,6 +760,7 @@ __global__ void __launch_bounds__(kFlipSmallBlock) k_rounds_small(WgMesh M, Flip
   const uint32_t cap = ctr[C_CAP], tets0 = ctr[C_TETS];
   uint32_t U = ctr[C_SURV], W = ctr[C_WIN], A = ctr[C_LIST], par = ctr[C_PAR] & 1u, it = ctr[C_IT], it0 = ctr[C_IT0],
            round = ctr[C_ROUND], tets = tets0, cur = J.cur;
+  uint32_t round_slow = 0, round_it = 0;  // deferred entries and iterations of the last round
   uint32_t picks = 0, sumu = 0, sa = 0, sf = 0, peak = 0, slow = 0, last_slow = ctr[C_SLOW_LAST], done = 0, f23 = 0, iters = 0;
   bool stop = ctr[C_STOP] != 0u, voted = J.voted != 0;
   for (;;) {
@@ -799,7 +802,8 @@ __global__ void __launch_bounds__(kFlipSmallBlock) k_rounds_small(WgMesh M, Flip
       if (W == 0u) break;
     }
     voted = false;
-    if (stop || (uint64_t)tets + 3u * W + 64u > (uint64_t)cap || A + 4u * W > J.list) break;
+    const uint32_t bound = round_slow > J.list_full * round_it ? J.list_full : J.list;
+    if (stop || (uint64_t)tets + 3u * W + 64u > (uint64_t)cap || A + 4u * W > bound) break;
     // the splits; the children join the active list as in k_split
     const uint32_t* uv = cur ? J.uvert[1] : J.uvert[0];
     uint32_t* ut = cur ? J.utet[1] : J.utet[0];
@@ -849,6 +853,7 @@ __global__ void __launch_bounds__(kFlipSmallBlock) k_rounds_small(WgMesh M, Flip
     // the flips of the round, the last round's to the end of the list
     done = U == 0u || round >= J.max_round ? 1u : 0u;
     const uint32_t n_it = done ? 4096u : (uint32_t)J.k;
+    round_slow = round_it = 0u;
     for (uint32_t n = 0; n < n_it && A > 0u && A <= J.limit; ++n) {
       if ((uint64_t)tets + A + 64u > (uint64_t)cap) {
         stop = true;
@@ -862,6 +867,8 @@ __global__ void __launch_bounds__(kFlipSmallBlock) k_rounds_small(WgMesh M, Flip
       last_slow = c.slow;
       peak = max(peak, A);
       ++iters;
+      ++round_it;
+      round_slow += c.slow;
       f23 += c.slots - tets;
       A = c.act_next;
       tets = c.slots;
@@ -896,6 +903,7 @@ __global__ void __launch_bounds__(kFlipSmallBlock) k_rounds_small(WgMesh M, Flip
     sums[S_SMALL_FLIPS] += sf;
     ctr[C_TETS] = tets;
     ctr[C_SLOW_SUM] += slow;
+    ctr[C_CHECK_SUM] += sa;
     ctr[C_SLOW_LAST] = last_slow;
     if (peak > ctr[C_PEAKA]) ctr[C_PEAKA] = peak;
     if (stop) ctr[C_STOP] = 1u;
@@ -930,9 +938,9 @@ void launch_set_ctr(uint32_t* ctr, int idx, uint32_t v, int idx2, uint32_t v2, h
   k_set_ctr<<<1, 64, 0, s>>>(ctr, idx, v, idx2, v2);
 }
 
-void launch_flip_check(const Mesh& M, const FlipLists& L, int i, bool requeue, uint32_t grid, uint64_t* st,
+void launch_flip_check(const Mesh& M, const FlipLists& L, int i, bool requeue, bool full, uint32_t grid, uint64_t* st,
                        hipStream_t s) {
-  if (M.mode == PRED_FILTERED) k_flip_check<<<grid, kBlock, 0, s>>>(M, L, i, requeue ? 1 : 0, st);
+  if (M.mode == PRED_FILTERED && !full) k_flip_check<<<grid, kBlock, 0, s>>>(M, L, i, requeue ? 1 : 0, st);
   else k_flip_check_faces<true><<<std::min(4u * grid, 4096u), kBlock, 0, s>>>(M, L, i, st);
 }
 void launch_flip_check_deferred(const Mesh& M, const FlipLists& L, int i, uint32_t grid, uint64_t* st,
@@ -958,10 +966,10 @@ __global__ void __launch_bounds__(kBlock) k_relocate(Mesh M, const uint32_t* uve
   PredStats ls = {};
   if (FORM == SLOW) {
     uint32_t n = 4u * M.ctr[C_SLOW_R], stride = gridDim.x * blockDim.x;
-    for (uint32_t k = gid(); k < n; k += stride) relocate_faces(M, uvert, utet, slow[k >> 2], (int)(k & 3u), it0, &ls);
+    for (uint32_t k = gid(); k < n; k += stride) relocate_faces(M, uvert, utet, slow[k >> 2], (int)(k & 3u), it0, true, &ls);
   } else if (FORM == FULL) {
     uint32_t k = gid();
-    if (k < 4u * U) relocate_faces(M, uvert, utet, k >> 2, (int)(k & 3u), it0, &ls);
+    if (k < 4u * U) relocate_faces(M, uvert, utet, k >> 2, (int)(k & 3u), it0, false, &ls);
   } else {
     uint32_t i = gid();
     bool defer = false;

@@ -33,6 +33,7 @@ enum Ctr : int {
   C_NPTS = 13,      // points to insert (input minus exact duplicates)
   C_DUPSCAN = 14,   // duplicate scans that hit their length cap
   C_IT0 = 16,       // flip iterations before this round
+  C_CHECK_SUM = 20, // list entries checked in launched iterations, summed (wraps)
   C_RUN_PICKS = 17, // of k_rounds_small: rounds it picked,
   C_RUN_SUMU = 18,  // the points they chose from,
   C_RUN_DONE = 19,  // and whether the last round is over
@@ -891,7 +892,10 @@ WT_HD bool relocate_body_t(const MS& M, const uint32_t* uvert, uint32_t* utet, u
   if (!walk_start(M, it0, &t)) return false;
   int state = 0;
   t = walk_to_t<FAST>(M, t, uvert[i], walk_seed(i), st, &state);
-  if (state == 2) return true;  // the full walk restarts from utet[i]
+  if (state == 2) {  // the full walk goes on from here
+    utet[i] = t;
+    return true;
+  }
   if (state == 1) at_add_u32(&M.ctr[C_WALK_FAIL], 1u);
   utet[i] = t;
   return false;

@@ -533,17 +533,18 @@ constexpr int kNarrowSpan = 60;
   if (hi_ - lo_ + 1 <= kNarrowSpan) return fn<2>(P, lo_); \
   return fn<6>(P, lo_);
 
-// The difference tiers as leaf functions with their points passed by
-// value (in registers: no scratch traffic on the path degenerate inputs take
-// millions of times), returning 2 when neither applies; the wide
-// forms are separate calls for the rest.
+// The difference tiers, inline with their points passed by value: in registers,
+// no scratch traffic around a call on the path degenerate inputs take millions
+// of times (as calls, the checks of a 48^3 lattice took 28 to 35 us a launch,
+// inline 26 to 30, its walks 57 and 50).  They return 2 when neither applies; the
+// wide forms are calls for the rest.
 #define WT_P12(P) P[0], P[1], P[2], P[3], P[4], P[5], P[6], P[7], P[8], P[9], P[10], P[11]
 #define WT_P15(P) WT_P12(P), P[12], P[13], P[14]
 #define WT_ARGS12                                                                                                  \
   float p0, float p1, float p2, float p3, float p4, float p5, float p6, float p7, float p8, float p9, float p10, \
       float p11
 #define WT_LIST12 p0, p1, p2, p3, p4, p5, p6, p7, p8, p9, p10, p11
-WT_HDN int exact_orient3d_rel(WT_ARGS12) {
+WT_HD int exact_orient3d_rel(WT_ARGS12) {
   const float P[12] = {WT_LIST12};
   double v[3][3], top;
   if (!rel_diff<3>(P, v, &top)) return 2;
@@ -552,7 +553,7 @@ WT_HDN int exact_orient3d_rel(WT_ARGS12) {
   int64_t m[3][3];
   return rel_scale<3>(v, top, kMidSpan, m) ? sign_int(det3_int(m[0], m[1], m[2])) : 2;
 }
-WT_HDN int exact_insphere_rel(WT_ARGS12, float p12, float p13, float p14) {
+WT_HD int exact_insphere_rel(WT_ARGS12, float p12, float p13, float p14) {
   const float P[15] = {WT_LIST12, p12, p13, p14};
   double v[4][3], top;
   if (!rel_diff<4>(P, v, &top)) return 2;
@@ -1023,7 +1024,7 @@ WT_HD void sort2(Ranked& a, Ranked& b, int& parity) {
 // arrays indexed at run time and a loop over the depths kept them in scratch
 // memory.  Four distinct points that are not collinear end within the first
 // three.
-WT_HDN int orient3d_sos_only(WT_ARGS12, uint32_t ia, uint32_t ib, uint32_t ic, uint32_t id) {
+WT_HD int orient3d_sos_only(WT_ARGS12, uint32_t ia, uint32_t ib, uint32_t ic, uint32_t id) {
   Ranked a = {p0, p1, p2, ia}, b = {p3, p4, p5, ib}, c = {p6, p7, p8, ic}, d = {p9, p10, p11, id};
   int parity = 1;
   sort2(a, b, parity);
@@ -1140,15 +1141,16 @@ WT_HD int sos4_plane(const T (*v)[3]) {
   return r;
 }
 
-// The cascade's depths 1-5, 0 when they do not decide here.  Five distinct
+// The cascade's depths 1-8, 0 when they do not decide here.  Five distinct
 // cospherical points end here: depth 1 is zero only with points 1-4 coplanar;
-// depths 2-4 too only with those on a circle, three of which are not
-// collinear, and point 0 then lies off their plane (or the five are
-// coplanar), so depth 5 decides.  The depths share their differences and
-// minors, and nothing lies in scratch memory: a wave's insphere with the
-// cascade took 170 us through orient4d_sos_only, and the deferred flip checks of
-// a 48^3 lattice 97 us a launch with it, 38 us here.
-WT_HDN int orient4d_sos_short(WT_ARGS12, float p12, float p13, float p14, uint32_t ia, uint32_t ib, uint32_t ic,
+// depths 2-4 too only with those on a circle; depth 5 only with point 0 in
+// their plane; and of points 2-4, which are not collinear, one of the three
+// projections of depths 6-8 is not either.  The depths share their
+// differences and minors, and nothing lies in scratch memory: a wave's insphere
+// with the cascade took 170 us through orient4d_sos_only, and the deferred flip
+// checks of a 48^3 lattice, where flat tets reach depth 6, 97 us a launch with
+// it, 38 us with depths 1-5 here, 31 us.
+WT_HD int orient4d_sos_short(WT_ARGS12, float p12, float p13, float p14, uint32_t ia, uint32_t ib, uint32_t ic,
                               uint32_t id, uint32_t ie) {
   Ranked a = {p0, p1, p2, ia}, b = {p3, p4, p5, ib}, c = {p6, p7, p8, ic}, d = {p9, p10, p11, id},
          e = {p12, p13, p14, ie};
@@ -1180,6 +1182,11 @@ WT_HDN int orient4d_sos_short(WT_ARGS12, float p12, float p13, float p14, uint32
     else if (rel_scale<3>(v, top, kMidSpan, m)) r = pass ? sign_int(det3_int(m[0], m[1], m[2])) : sos4_plane(m);
     else return 0;
   }
+#define WT_O2(u, w) dsign(orient2d_plain(c.u, c.w, d.u, d.w, e.u, e.w))
+  if (r == 0) r = WT_O2(x, y);
+  if (r == 0) r = -WT_O2(x, z);
+  if (r == 0) r = WT_O2(y, z);
+#undef WT_O2
   return r * parity;
 }
 
