@@ -20,7 +20,9 @@ __global__ void k_fill_u32(uint32_t* p, uint32_t v, uint64_t n);
 // ---------------------------------------------------------------------------
 // helpers
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ uint32_t gid() { return blockIdx.x * blockDim.x + threadIdx.x; }
+// Thread of a grid of kBlock-thread blocks (blockDim.x is a load from the
+// dispatch's arguments, a memory round trip before anything else).
+__device__ __forceinline__ uint32_t gid() { return blockIdx.x * kBlock + threadIdx.x; }
 
 // exclusive rank of `flag` within the block; *total = block count.
 // Every thread of the block must call it.
@@ -150,7 +152,7 @@ __global__ void k_start_tets(Mesh M, StartTets S, Clouds K) {
 __global__ void __launch_bounds__(kBlock) k_minmax_single(const float* xyz, uint32_t n, uint32_t* mm) {
   __shared__ uint32_t red[6][kBlock / 64];
   uint32_t lo[3] = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu}, hi[3] = {0u, 0u, 0u};
-  uint32_t stride = gridDim.x * blockDim.x;
+  uint32_t stride = gridDim.x * kBlock;
   for (uint32_t i = gid(); i < n; i += stride)
     for (int k = 0; k < 3; ++k) {
       float v = xyz[3 * (size_t)i + k];
@@ -302,7 +304,7 @@ __global__ void __launch_bounds__(kBlock) k_pick_count(Mesh M, const uint32_t* u
                                                        FlipLists L) {
   const uint32_t U = M.ctr[C_SURV], A = M.ctr[C_LIST], it = M.ctr[C_IT] + 1u;
   const uint32_t* act = L.act[M.ctr[C_PAR] & 1u];
-  for (uint32_t j = gid(); j < A; j += gridDim.x * blockDim.x) mark_listed(M, act[j], it);
+  for (uint32_t j = gid(); j < A; j += gridDim.x * kBlock) mark_listed(M, act[j], it);
   uint32_t i = gid();
   if (i == 0) {
     M.ctr[C_ROUND] += 1u;
@@ -509,7 +511,7 @@ __global__ void __launch_bounds__(kBlock) k_split_points(Mesh M, const uint32_t*
   const uint32_t U = M.ctr[C_SURV], round = M.ctr[C_ROUND];
   PredStats ls = {};
   if (FORM == SLOW) {
-    uint32_t n = M.ctr[C_SLOW_P], stride = gridDim.x * blockDim.x;
+    uint32_t n = M.ctr[C_SLOW_P], stride = gridDim.x * kBlock;
     for (uint32_t k = gid(); k < n; k += stride)
       (void)split_points_body_t<false>(M, uvert, utet, slow[k], round, &ls);
   } else {
@@ -541,17 +543,36 @@ void launch_split_points(const Mesh& M, const uint32_t* uvert, uint32_t* utet, u
 // flips: iteration i of a batch.  The kernels are persistent: a fixed grid
 // strides over the current list.
 // ---------------------------------------------------------------------------
+// A kernel begins with its counters, and a load that only one side of a branch
+// uses is moved there by the compiler, behind the loads of the branch's
+// condition.  Here the values are complete: all of them come in one round trip.
+__device__ __forceinline__ void loaded(uint32_t& a, uint32_t& b, uint32_t& c) {
+  asm volatile("" : "+s"(a), "+s"(b), "+s"(c));
+}
+
+struct Iter {
+  uint32_t n;    // entries (flips) of the list, 0 when the iteration does not run
+  uint32_t it;   // tag
+  uint32_t par;  // which active list is current
+};
 // The first kernel of an iteration decides whether it runs (C_TETS changes in
 // decide_exec only) and says so to the others.
-__device__ __forceinline__ bool iter_runs(uint32_t* ctr, int i) {
-  const uint32_t A = *it_ctr(ctr, C_ITA, i);
+__device__ __forceinline__ Iter iter_first(uint32_t* ctr, int i) {
+  uint32_t A = *it_ctr(ctr, C_ITA, i), tets = ctr[C_TETS], stop = ctr[C_STOP], cap = ctr[C_CAP], it = ctr[C_IT],
+           par = ctr[C_PAR];
+  loaded(A, tets, stop);
+  loaded(cap, it, par);
   // worst case every proposal wins a 2-3 flip and takes a fresh slot
-  if (A == 0u || ctr[C_STOP] || (uint64_t)ctr[C_TETS] + A + 64u > (uint64_t)ctr[C_CAP]) return false;
-  if (gid() == 0) *it_ctr(ctr, C_ITR, i) = 1u;
-  return true;
+  const bool run = (A != 0u) & (stop == 0u) & ((uint64_t)tets + A + 64u <= (uint64_t)cap);
+  if (run && gid() == 0) *it_ctr(ctr, C_ITR, i) = 1u;
+  return Iter{run ? A : 0u, it + (uint32_t)i + 1u, (par + (uint32_t)i) & 1u};
 }
-__device__ __forceinline__ uint32_t iter_tag(const uint32_t* ctr, int i) { return ctr[C_IT] + (uint32_t)i + 1u; }
-__device__ __forceinline__ uint32_t iter_par(const uint32_t* ctr, int i) { return (ctr[C_PAR] + (uint32_t)i) & 1u; }
+// the others; which: the count (C_ITA, C_ITF, C_ITS) they run over
+__device__ __forceinline__ Iter iter_next(uint32_t* ctr, int which, int i) {
+  uint32_t run = *it_ctr(ctr, C_ITR, i), n = *it_ctr(ctr, which, i), it = ctr[C_IT], par = ctr[C_PAR];
+  loaded(run, n, it);
+  return Iter{run ? n : 0u, it + (uint32_t)i + 1u, (par + (uint32_t)i) & 1u};
+}
 
 // The filters of the flip check on every list entry, one thread per tet; the
 // entries they leave go to L.slow.  104 VGPRs, 4 waves per SIMD (at 96 and 5
@@ -559,21 +580,23 @@ __device__ __forceinline__ uint32_t iter_par(const uint32_t* ctr, int i) { retur
 // points: 6.68 ms of event time a triangulation with insphere_f32 and
 // insphere_f64 per face and three orient3d after each (158 VGPRs), 5.60 ms
 // with one set of cofactors per tet; 100k points 2.79 -> 2.05 ms.
+// The neighbours stay in registers with the record they came in (read again for
+// each proposal before): 1M points 21.1 -> 18.9 us a launch, on a sphere 8.7 -> 7.1.
 // requeue: no kernel of this iteration runs the full predicates; an entry that
 // needs them stays in the active list.
 __global__ void __launch_bounds__(kBlock) k_flip_check(Mesh M, FlipLists L, int i, int requeue, uint64_t* st) {
-  if (!iter_runs(M.ctr, i)) return;
-  const uint32_t it = iter_tag(M.ctr, i);
-  const uint32_t* cur = L.act[iter_par(M.ctr, i)];
-  uint32_t stride = gridDim.x * blockDim.x;
+  const Iter I = iter_first(M.ctr, i);
+  const uint32_t* cur = I.par ? L.act[1] : L.act[0];
+  const uint32_t stride = gridDim.x * kBlock;
   PredStats ls = {};
-  uint32_t A = *it_ctr(M.ctr, C_ITA, i);
-  for (uint32_t j = gid(); j < A; j += stride)
-    if (flip_check_lean(M, cur, L.prop, j, it, &ls)) {
+  for (uint32_t j = gid(); j < I.n; j += stride) {
+    const uint32_t t = cur[j];
+    if (flip_check_lean(M, t, L.prop, j, I.it, &ls)) {
       const uint32_t k = append_slot(it_ctr(M.ctr, C_ITS, i));
-      if (requeue) L.prop[j] = requeue_proposal(M, cur[j], it);
+      if (requeue) L.prop[j] = requeue_proposal(M, t, I.it);
       else L.slow[k] = j;
     }
+  }
   flush_stats(ls, st);
 }
 
@@ -584,10 +607,11 @@ __global__ void __launch_bounds__(kBlock) k_flip_check(Mesh M, FlipLists L, int 
 // lanes share a wave.
 template <bool ALL>
 __global__ void __launch_bounds__(kBlock) k_flip_check_faces(Mesh M, FlipLists L, int i, uint64_t* st) {
-  if (ALL ? !iter_runs(M.ctr, i) : !*it_ctr(M.ctr, C_ITR, i)) return;
-  const uint32_t it = iter_tag(M.ctr, i);
-  const uint32_t* cur = L.act[iter_par(M.ctr, i)];
-  const uint32_t n4 = 4u * *it_ctr(M.ctr, ALL ? C_ITA : C_ITS, i), stride = gridDim.x * blockDim.x;
+  const Iter I = ALL ? iter_first(M.ctr, i) : iter_next(M.ctr, C_ITS, i);
+  if (I.n == 0u) return;
+  const uint32_t it = I.it;
+  const uint32_t* cur = I.par ? L.act[1] : L.act[0];
+  const uint32_t n4 = 4u * I.n, stride = gridDim.x * kBlock;
   PredStats ls = {};
   for (uint32_t k = gid(); k < n4; k += stride)
     flip_check_faces(M, cur, L.prop, ALL ? k >> 2 : L.slow[k >> 2], (int)(k & 3u), it, &ls);
@@ -638,6 +662,11 @@ __device__ __forceinline__ uint32_t block_prefix3(uint32_t a, uint32_t b, uint32
 // slots and queue entries with one atomic per counter, and those
 // same-address atomics complete one at a time at the memory side; 512
 // halves them against 256 (1M uniform device 26.0-26.1 -> 25.7-26.0 ms).
+// Three lanes of one instruction make the three claims: from one lane the
+// compiler waited for each, up to three of the launch's round trips
+// (decide_exec at 100k points 10.7 -> 9.7 us, on a sphere 8.3 -> 7.7, at 1M 26.8
+// -> 26.1).  Tried beside it: every proposal loading its tets beside the votes,
+// instead of the winners after them (64 clouds 10.9 -> 11.2 us, 1M 26.9 -> 27.2).
 constexpr uint32_t kDecBlock = 512;
 static_assert(kDecBlock <= 512, "block_prefix3 packs totals of at most 512 threads");
 
@@ -645,9 +674,9 @@ __global__ void __launch_bounds__(kDecBlock) k_flip_decide_exec(Mesh M, FlipList
   constexpr uint32_t kBS = kDecBlock;
   __shared__ uint32_t wsum[kBS / 64];
   __shared__ uint32_t base[3];
-  if (!*it_ctr(M.ctr, C_ITR, i)) return;
-  const uint32_t A = *it_ctr(M.ctr, C_ITA, i), it = iter_tag(M.ctr, i);
-  uint32_t* act_next = L.act[iter_par(M.ctr, i) ^ 1u];
+  const Iter I = iter_next(M.ctr, C_ITA, i);
+  const uint32_t A = I.n, it = I.it;
+  uint32_t* act_next = I.par ? L.act[0] : L.act[1];
   for (uint32_t b0 = blockIdx.x * kBS; b0 < A; b0 += gridDim.x * kBS) {
     uint32_t j = b0 + threadIdx.x;
     uint4 pr = make_uint4(kInvalid, 0u, 0u, 0u);
@@ -660,10 +689,10 @@ __global__ void __launch_bounds__(kDecBlock) k_flip_decide_exec(Mesh M, FlipList
     uint32_t r = block_prefix3<kBS>(win ? 1u : 0u, nslot, nqa, &tot, wsum);
     uint32_t rf = r & 1023u, rs = (r >> 10) & 1023u, rq = r >> 20;
     uint32_t tf = tot & 1023u, ts = (tot >> 10) & 1023u, tq = tot >> 20;
-    if (threadIdx.x == 0) {
-      base[0] = tf ? atomicAdd(it_ctr(M.ctr, C_ITF, i), tf) : 0u;
-      base[1] = ts ? atomicAdd(&M.ctr[C_TETS], ts) : 0u;
-      base[2] = tq ? atomicAdd(it_ctr(M.ctr, C_ITA, i + 1), tq) : 0u;
+    if (threadIdx.x < 3u) {  // three lanes: one round trip, not one after another
+      const uint32_t l = threadIdx.x, v = l == 0u ? tf : (l == 1u ? ts : tq);
+      uint32_t* p = l == 0u ? it_ctr(M.ctr, C_ITF, i) : (l == 1u ? &M.ctr[C_TETS] : it_ctr(M.ctr, C_ITA, i + 1));
+      base[l] = v ? atomicAdd(p, v) : 0u;
     }
     __syncthreads();
     uint32_t q = base[2] + rq;
@@ -678,11 +707,14 @@ __global__ void __launch_bounds__(kDecBlock) k_flip_decide_exec(Mesh M, FlipList
   }
 }
 
+// Three round trips: records, stamps, messages.  With the messages behind a
+// branch each (loaded only where the neighbour flipped) the compiler waited for
+// each of the six; now a lane without one reads a line common to all: 1M points
+// 22.0 -> 20.0 us a launch, 64 clouds 6.8 -> 6.1, 2,048 clouds 70.6 -> 67.2.
 __global__ void __launch_bounds__(kBlock) k_flip_update(Mesh M, FlipLists L, int i) {
-  if (!*it_ctr(M.ctr, C_ITR, i)) return;
-  const uint32_t F = *it_ctr(M.ctr, C_ITF, i), it = iter_tag(M.ctr, i);
-  uint32_t stride = gridDim.x * blockDim.x;
-  for (uint32_t k = gid(); k < F; k += stride) flip_update_body(M, L.out, k, it);
+  const Iter I = iter_next(M.ctr, C_ITF, i);
+  const uint32_t stride = gridDim.x * kBlock;
+  for (uint32_t k = gid(); k < I.n; k += stride) flip_update_body(M, L.out, k, I.it);
 }
 
 // Up to k flip iterations of a short list in one workgroup
@@ -965,7 +997,7 @@ __global__ void __launch_bounds__(kBlock) k_relocate(Mesh M, const uint32_t* uve
   const uint32_t U = M.ctr[C_SURV], it0 = M.ctr[C_IT0];
   PredStats ls = {};
   if (FORM == SLOW) {
-    uint32_t n = 4u * M.ctr[C_SLOW_R], stride = gridDim.x * blockDim.x;
+    uint32_t n = 4u * M.ctr[C_SLOW_R], stride = gridDim.x * kBlock;
     for (uint32_t k = gid(); k < n; k += stride) relocate_faces(M, uvert, utet, slow[k >> 2], (int)(k & 3u), it0, true, &ls);
   } else if (FORM == FULL) {
     uint32_t k = gid();
@@ -1003,7 +1035,7 @@ __global__ void __launch_bounds__(kBlock) k_audit(MS M, uint32_t T, uint32_t* re
                                                   uint64_t* st, uint32_t* slow) {
   PredStats ls = {};
   if (FORM == SLOW) {
-    uint32_t n = M.ctr[C_SLOW_T], stride = gridDim.x * blockDim.x;
+    uint32_t n = M.ctr[C_SLOW_T], stride = gridDim.x * kBlock;
     for (uint32_t k = gid(); k < n; k += stride) (void)audit_body_t<false>(M, slow[k], rec, cap, &ls);
   } else {
     uint32_t t = gid();
@@ -1154,7 +1186,7 @@ __global__ void k_nbr_snap(const uint32_t* cnt, uint32_t* bounds, int k) {
 __global__ void k_nbr_ring(const uint32_t* adj, uint32_t M, uint32_t* mark, uint32_t* list,
                            uint32_t* cnt, const uint32_t* bounds, int k) {
   uint32_t b = bounds[k], e = bounds[k + 1];
-  uint32_t stride = gridDim.x * blockDim.x;
+  uint32_t stride = gridDim.x * kBlock;
   for (uint32_t i = b + gid(); i < e; i += stride) {
     uint32_t r = list[i];
     for (int f = 0; f < 4; ++f) {
@@ -1228,7 +1260,7 @@ __global__ void k_fill_u64(uint64_t* p, uint64_t v, uint64_t n) {
 }
 __global__ void k_copy16(uint4* dst, const uint4* src, uint64_t n) {
   uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+  uint64_t stride = (uint64_t)gridDim.x * kBlock;
   for (; i < n; i += stride) dst[i] = src[i];
 }
 void launch_copy16(uint4* dst, const uint4* src, uint64_t n, hipStream_t s) {

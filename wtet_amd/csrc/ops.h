@@ -282,19 +282,19 @@ WT_HD bool is_winner(const MS& M, const uint32_t* utet, uint32_t i, int ring) {
   uint64_t kt = TVOTE(M, t);
   if ((uint32_t)(kt & 0xFFFFFFFFull) != i) return false;
   if (ring <= 0) return true;
-  uint4 to = TN(M, t);
+  const uint4 to = TN(M, t);
+  // the four votes in one round trip
+  bool win = true;
+  for (int f = 0; f < 4; ++f) win &= TVOTE(M, opp_tet(get4(to, f))) >= kt;
+  if (!win || ring <= 1) return win;
   for (int f = 0; f < 4; ++f) {
-    uint32_t nt = opp_tet(get4(to, f));
-    if (TVOTE(M, nt) < kt) return false;
-    if (ring > 1) {
-      uint4 no = TN(M, nt);
-      for (int g = 0; g < 4; ++g) {
-        uint32_t n2 = opp_tet(get4(no, g));
-        if (n2 != t && TVOTE(M, n2) < kt) return false;
-      }
+    const uint4 no = TN(M, opp_tet(get4(to, f)));
+    for (int g = 0; g < 4; ++g) {
+      const uint32_t n2 = opp_tet(get4(no, g));
+      win &= n2 == t || TVOTE(M, n2) >= kt;
     }
   }
-  return true;
+  return win;
 }
 
 // ---------------------------------------------------------------------------
@@ -316,6 +316,7 @@ WT_HD uint32_t split_body(const MS& M, const uint2* wlist, uint32_t k, uint32_t 
                           uint32_t c[4]) {
   uint32_t t = wlist[k].x, p = wlist[k].y;
   uint32_t base = TSPLIT(M, t).y;
+  const uint32_t tag = TQUEUE(M, t);
   uint4 tv = TV(M, t);
   uint4 to = TN(M, t);
   uint4 tov = TOV(M, t);
@@ -358,7 +359,7 @@ WT_HD uint32_t split_body(const MS& M, const uint2* wlist, uint32_t k, uint32_t 
       FSTAMP(M, c[j]) = 0u;
     }
   }
-  return TQUEUE(M, t) == (kListed | it) ? 0xEu : 0xFu;
+  return tag == (kListed | it) ? 0xEu : 0xFu;
 }
 
 // ---------------------------------------------------------------------------
@@ -433,13 +434,12 @@ WT_HD void pick_xyz(const float (*P)[3], int k, float* out) {
 }
 
 // The proposal of tet t across face f (its kind, offending edge and third
-// tet as flip_check_lean finds them): votes for the other tets it involves;
+// tet as flip_check_lean finds them, nt the neighbour): votes for the other tets it involves;
 // its tag is the vote for its own.  A vote is an atomic minimum on a random
 // line, 27 G/s on this card, a tag a store, 84 G/s.
 template <class MS>
-WT_HD uint4 flip_propose(const MS& M, uint32_t t, uint32_t f, uint32_t kind, uint32_t bad, uint32_t third,
+WT_HD uint4 flip_propose(const MS& M, uint32_t t, uint32_t f, uint32_t nt, uint32_t kind, uint32_t bad, uint32_t third,
                          uint32_t it) {
-  uint32_t nt = opp_tet(*opp_word(M, t, f));
   uint64_t key = flip_key(it, t);
   TQUEUE(M, t) = it;
   mesh_min(M, &FVOTE(M, nt), key);
@@ -499,18 +499,17 @@ WT_HD int face_classify(const float* x, const float* y, const float* z, const fl
   return nbad == 1 && get4(tov, *pthird) == ov ? kFaceFlip : kFaceNo;
 }
 
-// Lean check of list entry j, one thread per tet: FP32 filters, and the FP64
+// Lean check of list entry j, tet t, one thread per tet: FP32 filters, and the FP64
 // filter for the faces whose insphere they leave.  The first face (in order)
 // that can flip is proposed; true (with no vote cast) when a
 // face before it is undecided, and the entry needs the full predicates.
 template <class MS>
-WT_HD bool flip_check_lean(const MS& M, const uint32_t* act, uint4* prop, uint32_t j, uint32_t it,
-                           PredStats* st) {
-  uint32_t t = act[j];
+WT_HD bool flip_check_lean(const MS& M, uint32_t t, uint4* prop, uint32_t j, uint32_t it, PredStats* st) {
   // Two memory round trips: the slot's record (vertices and opposite
   // vertices), then all eight points (the point array includes the infinity
   // vertex, so every id is loadable).
   uint4 tv = TV(M, t);
+  uint4 to = TN(M, t);
   uint4 tov = TOV(M, t);
   prop[j].x = kInvalid;
   if (tv.x == kInvalid) return false;  // freed since it was queued
@@ -566,8 +565,8 @@ WT_HD bool flip_check_lean(const MS& M, const uint32_t* act, uint4* prop, uint32
     const int v = face_classify(X, Y, Z, A, O, pos, tov, get4(tov, f), &kind, &bad, &pthird, st);
     if (v == kFaceUndecided) return true;
     if (v == kFaceNo) continue;
-    const uint32_t third = kind ? opp_tet(*opp_word(M, t, (uint32_t)pthird)) : kInvalid;
-    prop[j] = flip_propose(M, t, (uint32_t)f, kind, bad, third, it);
+    const uint32_t third = kind ? opp_tet(get4(to, pthird)) : kInvalid;
+    prop[j] = flip_propose(M, t, (uint32_t)f, opp_tet(get4(to, f)), kind, bad, third, it);
     return false;
   }
   return false;
@@ -814,9 +813,11 @@ WT_HD void flip_update_body(const MS& M, const uint4* out, uint32_t k, uint32_t 
   uint32_t ptr[6] = {w.w, p.x, p.y, p.z, p.w, out[4 * (size_t)k + 3].x}, fq[6];
   uint2 msg[6];
   for (int i = 0; i < 6; ++i) fq[i] = FSTAMP(M, opp_tet(ptr[i]));
+  // Every lane loads, from one common line where its neighbour did not flip:
+  // behind branches each of the six waited for itself.
   for (int i = 0; i < 6; ++i) {
-    msg[i] = make_uint2(0u, 0u);
-    if (fq[i] == it) msg[i] = reinterpret_cast<const uint2*>(&TMSG(M, opp_tet(ptr[i])))[opp_face(ptr[i])];
+    const uint32_t at = fq[i] == it ? ptr[i] : 0u;
+    msg[i] = reinterpret_cast<const uint2*>(&TMSG(M, opp_tet(at)))[opp_face(at)];
   }
   // one 8-byte store per face, its slot and value chosen without a branch
   for (int i = 0; i < 6; ++i) {

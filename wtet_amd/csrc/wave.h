@@ -162,7 +162,7 @@ __device__ __forceinline__ void flip_check_faces(const MS& M, const uint32_t* ac
   const uint32_t pk_c = (uint32_t)__shfl((int)pk, (int)(g0 + cf));
   const uint32_t third_c = (uint32_t)__shfl((int)third, (int)(g0 + cf));
   if (f == 0) {
-    if (grp) prop[j] = flip_propose(M, t, cf, (pk_c >> 2) & 1u, pk_c >> 3, third_c, it);
+    if (grp) prop[j] = flip_propose(M, t, cf, opp_tet(*opp_word(M, t, cf)), (pk_c >> 2) & 1u, pk_c >> 3, third_c, it);
     else prop[j].x = kInvalid;
   }
 }
@@ -300,7 +300,7 @@ __device__ __forceinline__ void wg_flip_iteration(const MS& M, WgCounters& c, co
   if (filtered) {
     PredStats ls = {};
     for (uint32_t j = tid; j < A; j += BS)
-      if (flip_check_lean(M, act, prop, j, it, &ls)) slow_t[lds_slot(&c.slow)] = j;
+      if (flip_check_lean(M, act[j], prop, j, it, &ls)) slow_t[lds_slot(&c.slow)] = j;
     flush_stats(ls, st);
     __syncthreads();
     ns = c.slow;
@@ -310,7 +310,7 @@ __device__ __forceinline__ void wg_flip_iteration(const MS& M, WgCounters& c, co
     __syncthreads();
   }
   // a wave claims its flips, fresh slots and queue entries with one LDS
-  // atomic each
+  // atomic of three lanes
   for (uint32_t b = 0; b < A; b += BS) {
     const uint32_t j = b + tid;
     uint4 pr = make_uint4(kInvalid, 0u, 0u, 0u);
@@ -320,15 +320,14 @@ __device__ __forceinline__ void wg_flip_iteration(const MS& M, WgCounters& c, co
     const bool win = flip_decide_load(M, pr, it, qid, &nq, &nslot, F);
     const uint32_t nqa = nq + nslot;
     const uint64_t bw = __ballot(win), bs = __ballot(nslot), q0 = __ballot(nqa & 1u), q1 = __ballot(nqa & 2u);
-    uint32_t cf = 0, cs = 0, cq = 0;
-    if (__lane_id() == 0) {
-      if (bw) cf = lds_add(&c.flips, __popcll(bw));
-      if (bs) cs = lds_add(&c.slots, __popcll(bs));
-      if (q0 | q1) cq = lds_add(&c.act_next, __popcll(q0) + 2u * __popcll(q1));
-    }
-    cf = __shfl(cf, 0) + __popcll(bw & lt);
-    cs = __shfl(cs, 0) + __popcll(bs & lt);
-    cq = __shfl(cq, 0) + __popcll(q0 & lt) + 2u * __popcll(q1 & lt);
+    const uint32_t l = __lane_id();
+    uint32_t* p = l == 0u ? &c.flips : (l == 1u ? &c.slots : &c.act_next);
+    const uint32_t v = l == 0u ? __popcll(bw) : (l == 1u ? __popcll(bs) : __popcll(q0) + 2u * __popcll(q1));
+    uint32_t claim = 0u;
+    if (l < 3u && v) claim = lds_add(p, v);
+    const uint32_t cf = __shfl(claim, 0) + __popcll(bw & lt);
+    const uint32_t cs = __shfl(claim, 1) + __popcll(bs & lt);
+    const uint32_t cq = __shfl(claim, 2) + __popcll(q0 & lt) + 2u * __popcll(q1 & lt);
     if (nq > 0u) next[cq] = qid[0];
     if (nq > 1u) next[cq + 1u] = qid[1];
     if (win) {
