@@ -21,16 +21,30 @@ __device__ __forceinline__ void flush_stats(const PredStats& ls, uint64_t* st) {
   }
 }
 
-__device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m) {
-  uint32_t lo = __shfl_xor((uint32_t)v, m), hi = __shfl_xor((uint32_t)(v >> 32), m);
-  return ((uint64_t)hi << 32) | lo;
+// The smallest of the wave's values, by lane shifts within the vector unit: rows
+// of 16 lanes (row_shr 1, 2, 4, 8), then row to row (row_bcast 15, 31) into lane
+// 63.  Every lane of the wave calls it.
+__device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
+#define WT_MIN_STEP(ctrl, rows) v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, ctrl, rows, 0xF, false))
+  WT_MIN_STEP(0x111, 0xF);
+  WT_MIN_STEP(0x112, 0xF);
+  WT_MIN_STEP(0x114, 0xF);
+  WT_MIN_STEP(0x118, 0xF);
+  WT_MIN_STEP(0x142, 0xA);
+  WT_MIN_STEP(0x143, 0xC);
+#undef WT_MIN_STEP
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
-// The votes of one wave (lane's point i, valid below U).  Lanes voting for
-// the same tet as the wave's first pending lane combine their keys with a
-// wave min first (a few passes), so early rounds -- when most points still
-// share a few tets -- issue one atomic per wave instead of one per point;
-// the remaining lanes vote directly.
+// The votes of one wave (lane's point i, valid below U; a higher lane's point is
+// a later one).  The lanes that vote for the tet of the wave's first pending lane
+// elect one vote: the smallest upper word of their keys, and the lowest lane that
+// has it, since the lower word is the point.  After kVotePasses such tets the
+// remaining lanes vote directly.  The atomics bound the vote (27 G/s on random
+// lines): with 4 passes, each a minimum of whole keys through LDS shuffles, 53.2 us
+// a launch at 1M points, 9.9 at 100k, 5.6 on a sphere of 50k, 74.1 for 2,048
+// clouds; now 48.2, 8.3, 5.4 and 61.5 (16 passes: 46.9, 9.6, 6.7, 55.7).
+constexpr int kVotePasses = 8;
 template <class MS>
 __device__ __forceinline__ void vote_wave(const MS& M, const uint32_t* uvert, const uint32_t* utet,
                                           uint32_t i, uint32_t U) {
@@ -41,19 +55,15 @@ __device__ __forceinline__ void vote_wave(const MS& M, const uint32_t* uvert, co
     key = vote_key(M, uvert, utet, i);
   }
   bool pending = key != kVoteNone;
-  for (int pass = 0; pass < 4; ++pass) {
-    uint64_t act = __ballot(pending);
+  const uint32_t hi = (uint32_t)(key >> 32);
+  for (int pass = 0; pass < kVotePasses; ++pass) {
+    const uint64_t act = __ballot(pending);
     if (!act) break;
-    int leader = __ffsll((unsigned long long)act) - 1;
-    uint32_t lt = __shfl(t, leader);
-    bool mine = pending && t == lt;
-    uint64_t k = mine ? key : kVoteNone;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      uint64_t o = shfl_xor_u64(k, off);
-      k = o < k ? o : k;
-    }
-    if (__lane_id() == leader) mesh_min(M, &TVOTE(M, lt), k);
+    const uint32_t lt = (uint32_t)__builtin_amdgcn_readlane((int)t, __ffsll((unsigned long long)act) - 1);
+    const bool mine = pending && t == lt;
+    const uint32_t least = wave_min_u32(mine ? hi : 0xFFFFFFFFu);
+    const uint64_t have = __ballot(mine && hi == least);
+    if (__lane_id() == __ffsll((unsigned long long)have) - 1) mesh_min(M, &TVOTE(M, lt), key);
     if (mine) pending = false;
   }
   if (pending) mesh_min(M, &TVOTE(M, t), key);
