@@ -122,3 +122,20 @@ def test_lattices_that_take_the_full_predicates(ctx, oracle, side, extra):
     want = oracle.canonical_real(oracle.delaunay(oracle.normalize_points(p)[0]), len(p))
     for _ in range(3):  # launched, recorded and replayed
         assert np.array_equal(oracle.canonical_real(ctx.delaunay(p).tets, len(p)), want)
+
+
+# around a wave, the one-workgroup rounds (2,048 points) and several workgroups
+@pytest.mark.parametrize("n", [4, 63, 64, 65, 2048, 2049, 30000])
+def test_first_vote_takes_the_deepest_point(ctx, oracle, n):
+    """All points lie in one tet: the round's one winner is the point deepest
+    inside its circumsphere.  Depths are compared in f32 on the device: two
+    roundings of 2^-24 (the f64 error is far below)."""
+    p = np.random.default_rng(n).random((n, 3)).astype(np.float32)
+    r = ctx.delaunay(p, wtet_amd.Config(max_insert_iterations=1, enable_splaying=False))
+    won = np.unique(r.tets[r.tets < n])
+    assert len(won) == 1 and r.stats["rounds"] == 1
+    V = oracle.extended_points(oracle.normalize_points(p)[0])
+    s = V[n:n + 4]
+    c = np.linalg.solve(2 * (s[1:] - s[0]), (s[1:] ** 2).sum(1) - (s[0] ** 2).sum())
+    depth = ((s[0] - c) ** 2).sum() - ((V[:n] - c) ** 2).sum(1)
+    assert depth[won[0]] >= depth.max() * (1 - 2 * 2.0 ** -24)
