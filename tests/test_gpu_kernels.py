@@ -139,3 +139,26 @@ def test_first_vote_takes_the_deepest_point(ctx, oracle, n):
     c = np.linalg.solve(2 * (s[1:] - s[0]), (s[1:] ** 2).sum(1) - (s[0] ** 2).sum())
     depth = ((s[0] - c) ** 2).sum() - ((V[:n] - c) ** 2).sum(1)
     assert depth[won[0]] >= depth.max() * (1 - 2 * 2.0 ** -24)
+
+
+# counts of 256 points or slots in one scan, four to a load
+@pytest.mark.parametrize("n", [255, 1023, 1025, 32769])
+def test_block_scan_remainders(ctx, oracle, n):
+    p = np.random.default_rng(n).random((n, 3)).astype(np.float32)
+    want = oracle.canonical_real(oracle.delaunay(oracle.normalize_points(p)[0]), n)
+    assert np.array_equal(oracle.canonical_real(ctx.delaunay(p).tets, n), want)
+
+
+def test_block_scan_of_several_steps(ctx):
+    """1.4M points have over the 32,768 blocks of slots that one step takes:
+    every point is a vertex and the adjacency is closed."""
+    n = 1400000
+    p = np.random.default_rng(9).random((n, 3)).astype(np.float32)
+    r = ctx.delaunay(p)
+    assert len(np.unique(r.tets[r.tets < n])) == n
+    t, f = r.adjacency >> 5, r.adjacency & 3
+    inner = r.adjacency != 0xFFFFFFFF
+    rows = np.repeat(np.arange(len(t), dtype=np.uint32)[:, None], 4, 1)
+    faces = np.tile(np.arange(4, dtype=np.uint32), (len(t), 1))
+    back = r.adjacency[t[inner], f[inner]]
+    assert np.array_equal(back >> 5, rows[inner]) and np.array_equal(back & 3, faces[inner])
