@@ -606,7 +606,7 @@ __device__ __forceinline__ Iter iter_next(uint32_t* ctr, int which, int i) {
 }
 
 // The filters of the flip check on every list entry, one thread per tet; the
-// entries they leave go to L.slow.  104 VGPRs, 4 waves per SIMD (at 96 and 5
+// entries they leave go to L.slow.  100 VGPRs, 4 waves per SIMD (at 96 and 5
 // waves, with two registers spilled, it took the same time).  1M uniform
 // points: 6.68 ms of event time a triangulation with insphere_f32 and
 // insphere_f64 per face and three orient3d after each (158 VGPRs), 5.60 ms
