@@ -299,10 +299,13 @@ __global__ void __launch_bounds__(512) k_radix_small(const K* kin, const uint32_
   }
 }
 
+// Enough for every smaller n too, since callers keep one workspace for lists
+// that shrink (the points left after duplicates).  The tiles do not grow with
+// n: 768 little ones just below kBigFrom, 192 big ones from there.
 template <typename K>
 size_t temp_bytes_t(uint32_t n, int end_bit) {
   (void)end_bit;
-  uint32_t tiles = std::max<uint32_t>(1u, tiles_of(n));
+  uint32_t tiles = std::max(1u, std::max(tiles_of(n), tiles_of(std::min(n, kBigFrom - 1u))));
   return align256((size_t)kMaxPasses * kRadix * 4) + align256((size_t)kRadix * tiles * 4) +
          align256((size_t)n * sizeof(K)) + align256((size_t)n * 4);
 }
