@@ -592,13 +592,20 @@ struct Run {
   uint32_t round = 0;
   uint32_t U = 0;          // uninserted points
   uint32_t W = 0;          // insertions of the current round
-  uint32_t dsum_prev = 0, csum_prev = 0;  // C_SLOW_SUM and C_CHECK_SUM at the previous round
+  uint32_t dsum_prev = 0, csum_prev = 0, it_prev = 0;  // C_SLOW_SUM, C_CHECK_SUM and C_IT at the previous round
+  uint64_t dper = 0;  // deferred tets per iteration to expect: twice the last round's average
   // The filters have left most of a round's tets to the full predicates: from
   // then on every tet takes them at once, and the one-workgroup kernels take
   // the exact mode's lists.  48^3 lattice: device 18.4 -> 16.5 ms (an iteration's
   // checks 40 -> 35 us, the last rounds 1.66 -> 0.61 ms).
   bool full = false;
   bool takes_full() const { return full || mode != PRED_FILTERED; }
+  // The last round left more entries an iteration to the full predicates than
+  // one workgroup takes of the exact mode's.  Device ms with the lists of such
+  // rounds kept in one workgroup and without: lattices of 8^3 4.17 and 3.75, 9^3
+  // 4.57 and 3.87, 10^3 5.22 and 4.85.
+  bool crowded = false;
+  uint64_t list_bound() const { return small_list(takes_full() || crowded); }
   int max_fi = 10;
   uint32_t warmup = 0;     // rounds that insert one point per tet
   Counters K;
@@ -762,12 +769,27 @@ void dev_prepare(wtet_ctx* c, Run& R, const float* d_xyz) {
   launch_set_ctr(P<uint32_t>(c->ctr), C_CAP, (uint32_t)c->cap_tets, -1, 0u, s);
 }
 
+// What the rounds since the last call left to the full predicates, from the
+// counters just read: sets R.dper, R.full and R.crowded.
+void note_deferred(wtet_ctx* c, Run& R) {
+  const uint32_t slow = c->h_ctr[C_SLOW_SUM] - R.dsum_prev, checked = c->h_ctr[C_CHECK_SUM] - R.csum_prev,
+                 its = c->h_ctr[C_IT] - R.it_prev;
+  R.dsum_prev += slow;
+  R.csum_prev += checked;
+  R.it_prev += its;
+  if (R.mode == PRED_FILTERED && checked >= 1024u && slow > checked / 2u) R.full = true;
+  const uint64_t per = std::max((uint32_t)R.max_fi, its);
+  R.dper = (2ull * slow + per - 1) / per;
+  R.crowded = slow > small_list(true) * its;
+}
+
 // After a round's pick, on the host: the one read of the round (winners,
 // reserved slots, and whether the previous round's flips stopped for
 // capacity), its checks and the growth of the tet slots.  U: the round's
 // uninserted count before the pick.
 void after_pick(wtet_ctx* c, Run& R, uint32_t U) {
   read_ctr(c);
+  note_deferred(c, R);
   uint32_t W = c->h_ctr[C_WIN];
   if (c->h_ctr[C_BADTET]) throw Fail{WTET_ERR_INTERNAL, "a point was located outside the super tet"};
   if (W == 0) throw Fail{WTET_ERR_INTERNAL, "no insertion possible in a round"};
@@ -820,24 +842,6 @@ void dev_split_points(wtet_ctx* c, Run& R) {
   HIP_CHECK(hipGetLastError());
 }
 
-// Deferred tets per iteration to expect (twice the last round's average), from
-// the counters just read; also sets R.full.
-uint64_t deferred_per_iteration(wtet_ctx* c, Run& R) {
-  const uint32_t slow = c->h_ctr[C_SLOW_SUM] - R.dsum_prev, checked = c->h_ctr[C_CHECK_SUM] - R.csum_prev;
-  R.dsum_prev += slow;
-  R.csum_prev += checked;
-  if (R.mode == PRED_FILTERED && checked >= 1024u && slow > checked / 2u) R.full = true;
-  return (2ull * slow + R.max_fi - 1) / (uint64_t)R.max_fi;
-}
-
-// the round's flip iterations (src/phase1.rs, flip loop), from device counters
-void dev_round_flips(wtet_ctx* c, Run& R) {
-  // the first list holds the entries carried over plus four per split;
-  // the deferred count per iteration follows the previous round's
-  const uint64_t dper = deferred_per_iteration(c, R);
-  run_flip_batch(c, R.V, R.mode, R.st, R.max_fi, (uint64_t)c->h_ctr[C_LIST] + 4ull * R.W, dper, R.full);
-}
-
 // uninserted points of flipped tets to their new tets (relocate_points_fast.wgsl)
 void dev_relocate(wtet_ctx* c, Run& R) {
   if (R.U == 0) return;
@@ -864,10 +868,11 @@ void run_round(wtet_ctx* c, Run& R, bool last) {
   FlipLists L = lists_of(c);
   const uint32_t cur = R.cur, W = R.W, U = R.U;
   const int ring_next = R.round + 1 <= R.warmup ? 0 : c->ring;
-  // the round's flips, sized as dev_round_flips sizes them
-  const uint64_t dper = deferred_per_iteration(c, R);
+  // the first list holds the entries carried over plus four per split;
+  // the deferred count per iteration follows the previous round's
+  const uint64_t dper = R.dper;
   const uint64_t a_hint = (uint64_t)c->h_ctr[C_LIST] + 4ull * W;
-  const int variant = !R.flipping ? 0 : (a_hint <= small_list(R.takes_full()) ? 1 : 2);
+  const int variant = !R.flipping ? 0 : (a_hint <= R.list_bound() ? 1 : 2);
   const uint32_t grid = variant == 2 ? grid_for(c, a_hint, 16) : 0u;
   const uint32_t dgrid = variant == 2 ? deferred_grid(c, dper, grid) : 0u;
   const int k = R.max_fi;
@@ -934,7 +939,7 @@ bool run_rounds_small(wtet_ctx* c, Run& R, bool voted) {
   J.ring = c->ring;
   J.warmup = (uint32_t)R.warmup;
   J.max_round = (uint32_t)R.cfg.max_insert_iterations;
-  J.list = (uint32_t)small_list(R.takes_full());
+  J.list = (uint32_t)R.list_bound();
   J.list_full = (uint32_t)small_list(true);
   J.limit = kSmallLimit;
   if (c->profiling && c->evused > 4096) collect_times(c);
@@ -942,7 +947,8 @@ bool run_rounds_small(wtet_ctx* c, Run& R, bool voted) {
   HIP_CHECK(hipGetLastError());
   read_ctr(c);
   const uint32_t* h = c->h_ctr;
-  (void)deferred_per_iteration(c, R);
+  note_deferred(c, R);
+  R.crowded = h[C_RUN_CROWDED] != 0u;  // of its last round alone
   R.round += (int)h[C_RUN_PICKS];
   R.cur ^= (int)(h[C_RUN_PICKS] & 1u);
   R.K.rounds += h[C_RUN_PICKS];
@@ -1121,7 +1127,7 @@ void run_device(wtet_ctx* c, const float* d_xyz, const std::vector<uint32_t>& of
     else dev_vote(c, R);
     while (!over) {
       if (R.flipping && R.U + R.W <= small_points(R.takes_full()) &&
-          (uint64_t)c->h_ctr[C_LIST] + 4ull * R.W <= small_list(R.takes_full())) {
+          (uint64_t)c->h_ctr[C_LIST] + 4ull * R.W <= R.list_bound()) {
         over = run_rounds_small(c, R, true);
         continue;
       }

@@ -823,7 +823,7 @@ __global__ void __launch_bounds__(kFlipSmallBlock) k_rounds_small(WgMesh M, Flip
   const uint32_t cap = ctr[C_CAP], tets0 = ctr[C_TETS];
   uint32_t U = ctr[C_SURV], W = ctr[C_WIN], A = ctr[C_LIST], par = ctr[C_PAR] & 1u, it = ctr[C_IT], it0 = ctr[C_IT0],
            round = ctr[C_ROUND], tets = tets0, cur = J.cur;
-  uint32_t round_slow = 0, round_it = 0;  // deferred entries and iterations of the last round
+  bool crowded = false;
   uint32_t picks = 0, sumu = 0, sa = 0, sf = 0, peak = 0, slow = 0, last_slow = ctr[C_SLOW_LAST], done = 0, f23 = 0, iters = 0;
   bool stop = ctr[C_STOP] != 0u, voted = J.voted != 0;
   for (;;) {
@@ -865,7 +865,7 @@ __global__ void __launch_bounds__(kFlipSmallBlock) k_rounds_small(WgMesh M, Flip
       if (W == 0u) break;
     }
     voted = false;
-    const uint32_t bound = round_slow > J.list_full * round_it ? J.list_full : J.list;
+    const uint32_t bound = crowded ? J.list_full : J.list;
     if (stop || (uint64_t)tets + 3u * W + 64u > (uint64_t)cap || A + 4u * W > bound) break;
     // the splits; the children join the active list as in k_split
     const uint32_t* uv = cur ? J.uvert[1] : J.uvert[0];
@@ -916,7 +916,7 @@ __global__ void __launch_bounds__(kFlipSmallBlock) k_rounds_small(WgMesh M, Flip
     // the flips of the round, the last round's to the end of the list
     done = U == 0u || round >= J.max_round ? 1u : 0u;
     const uint32_t n_it = done ? 4096u : (uint32_t)J.k;
-    round_slow = round_it = 0u;
+    uint32_t round_slow = 0, round_it = 0;
     for (uint32_t n = 0; n < n_it && A > 0u && A <= J.limit; ++n) {
       if ((uint64_t)tets + A + 64u > (uint64_t)cap) {
         stop = true;
@@ -938,6 +938,7 @@ __global__ void __launch_bounds__(kFlipSmallBlock) k_rounds_small(WgMesh M, Flip
       par ^= 1u;
       __syncthreads();  // the counters are read before the next iteration resets them
     }
+    crowded = round_slow > J.list_full * round_it;
     if (U > 0u) {
       // points of flipped tets to the tets now holding them
       if (tid == 0) c.slow = 0u;
@@ -982,6 +983,7 @@ __global__ void __launch_bounds__(kFlipSmallBlock) k_rounds_small(WgMesh M, Flip
     ctr[C_RUN_PICKS] = picks;
     ctr[C_RUN_SUMU] = sumu;
     ctr[C_RUN_DONE] = done;
+    ctr[C_RUN_CROWDED] = crowded;
   }
 }
 

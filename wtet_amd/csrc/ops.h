@@ -36,7 +36,8 @@ enum Ctr : int {
   C_CHECK_SUM = 20, // list entries checked in launched iterations, summed (wraps)
   C_RUN_PICKS = 17, // of k_rounds_small: rounds it picked,
   C_RUN_SUMU = 18,  // the points they chose from,
-  C_RUN_DONE = 19,  // and whether the last round is over
+  C_RUN_DONE = 19,  // whether the last round is over,
+  C_RUN_CROWDED = 21,  // and whether its last round left too many to the full predicates (SmallRun::list_full)
   C_SURV = 15,      // uninserted points (the pick's winners leave at the split)
   C_TETS = 256,     // next free tet slot (the winners' at the split)
   C_LIST = 512,     // length of the active list between batches of iterations
