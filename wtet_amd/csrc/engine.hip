@@ -594,10 +594,17 @@ struct Run {
   uint32_t W = 0;          // insertions of the current round
   uint32_t dsum_prev = 0, csum_prev = 0, it_prev = 0;  // C_SLOW_SUM, C_CHECK_SUM and C_IT at the previous round
   uint64_t dper = 0;  // deferred tets per iteration to expect: twice the last round's average
-  // The filters have left most of a round's tets to the full predicates: from
-  // then on every tet takes them at once, and the one-workgroup kernels take
-  // the exact mode's lists.  48^3 lattice: device 18.4 -> 16.5 ms (an iteration's
-  // checks 40 -> 35 us, the last rounds 1.66 -> 0.61 ms).
+  // The filters leave, or with full would have left, over a quarter of the last
+  // round's list entries: every tet takes the full predicates at once, and the
+  // one-workgroup kernels take the exact mode's lists.  48^3 lattice: device 18.4
+  // -> 16.5 ms (an iteration's checks 40 -> 35 us, the last rounds 1.66 -> 0.61
+  // ms).  Device ms by the share, the last column half and never back:
+  //                                           1/8    1/4    1/3    1/2    1/2..
+  //  48^3 lattice                             14.2   14.2   14.2   14.4   14.4
+  //  48^3 lattice, 300,000 points beside it   18.4   17.6   17.7   17.5   17.6
+  //  64 lattices of 8^3, a cloud of 200,000   11.0   11.2   11.1   11.2   11.9
+  //  64 lattices of 16^3, a cloud of 100,000  19.0   19.3   19.2   19.4   18.7
+  //  200 lattices of 8^3, 200 clouds of 2,000 16.7   15.9   15.8   15.9   15.9
   bool full = false;
   bool takes_full() const { return full || mode != PRED_FILTERED; }
   // The last round left more entries an iteration to the full predicates than
@@ -777,7 +784,7 @@ void note_deferred(wtet_ctx* c, Run& R) {
   R.dsum_prev += slow;
   R.csum_prev += checked;
   R.it_prev += its;
-  if (R.mode == PRED_FILTERED && checked >= 1024u && slow > checked / 2u) R.full = true;
+  if (R.mode == PRED_FILTERED && checked >= 1024u) R.full = slow > checked / 4u;
   const uint64_t per = std::max((uint32_t)R.max_fi, its);
   R.dper = (2ull * slow + per - 1) / per;
   R.crowded = slow > small_list(true) * its;

@@ -635,7 +635,8 @@ __global__ void __launch_bounds__(kBlock) k_flip_check(Mesh M, FlipLists L, int 
 // the filters left or, with ALL, on every entry of the list (exact mode: one
 // thread per tet and its faces in turn took 159 us a launch at 10,000 points,
 // four lanes 41 us).  A wave's first k is a multiple of 64, so a tet's four
-// lanes share a wave.
+// lanes share a wave.  Where ALL runs beside filters (Run::full) it counts the
+// tets that those would have left, one atomic a block.
 template <bool ALL>
 __global__ void __launch_bounds__(kBlock) k_flip_check_faces(Mesh M, FlipLists L, int i, uint64_t* st) {
   const Iter I = ALL ? iter_first(M.ctr, i) : iter_next(M.ctr, C_ITS, i);
@@ -644,9 +645,24 @@ __global__ void __launch_bounds__(kBlock) k_flip_check_faces(Mesh M, FlipLists L
   const uint32_t* cur = I.par ? L.act[1] : L.act[0];
   const uint32_t n4 = 4u * I.n, stride = gridDim.x * kBlock;
   PredStats ls = {};
-  for (uint32_t k = gid(); k < n4; k += stride)
+  uint32_t left = 0u;
+  for (uint32_t k = gid(); k < n4; k += stride) {
+    const uint32_t before = ls.c[6] + ls.c[7];
     flip_check_faces(M, cur, L.prop, ALL ? k >> 2 : L.slow[k >> 2], (int)(k & 3u), it, &ls);
+    uint64_t b = __ballot(ls.c[6] + ls.c[7] != before);  // lanes whose face took the exact insphere
+    b |= b >> 1;
+    b |= b >> 2;
+    left += (uint32_t)__popcll(b & 0x1111111111111111ull);
+  }
   flush_stats(ls, st);
+  if (!ALL || M.mode != PRED_FILTERED) return;
+  // a wave's active lanes are its first: lane 0 has counted them all
+  __shared__ uint32_t part[kBlock / 64];
+  if (__lane_id() == 0) part[threadIdx.x >> 6] = left;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  for (int w = 1; w < kBlock / 64; ++w) left += part[w];
+  if (left) atomicAdd(it_ctr(M.ctr, C_ITS, i), left);
 }
 
 // Exclusive prefixes of three small counts in one pass (a, b in {0, 1},
