@@ -2357,9 +2357,20 @@ static void predict_impl(void* a_) {
   (void)hipFree(o.p);
 }
 
-// device buffers of one training / gradient call
-// Device memory of one training call, in the context's arena (kept between
-// calls; a call's data does not outlive it)
+// Device memory of one training or gradient call, in the context's arena (a
+// call's data does not outlive it).  Up to kMlpKeep bytes are kept between calls:
+// any batch (at most 4,096 rows, 32 MB) with a training set of some 15,000 rows.
+// A larger arena is given back when the call ends.
+constexpr size_t kMlpKeep = (size_t)64 << 20;
+struct MlpArena {
+  wtet_ctx* c;
+  ~MlpArena() {
+    if (c->mlp.bytes <= kMlpKeep) return;
+    (void)hipFree(c->mlp.p);  // waits for the kernels that use it
+    c->mlp.p = nullptr;
+    c->mlp.bytes = 0;
+  }
+};
 struct MlpDev {
   MlpWork w;
   float *params, *grad, *m, *v, *feat, *tgt, *loss;
@@ -2412,6 +2423,7 @@ static void grad_impl(void* a_) {
   wtet_ctx* c = a.c;
   HIP_CHECK(hipSetDevice(c->device));
   hipStream_t s = c->stream;
+  const MlpArena arena{c};
   const MlpDev d = mlp_alloc(c, a.rows, a.rows, 1);
   HIP_CHECK(hipMemcpyAsync(d.params, a.params, kParamCount * 4, hipMemcpyHostToDevice, s));
   HIP_CHECK(hipMemcpyAsync(d.feat, a.feat, (size_t)a.rows * kFeat * 4, hipMemcpyHostToDevice, s));
@@ -2442,6 +2454,7 @@ static void train_impl(void* a_) {
   HIP_CHECK(hipSetDevice(c->device));
   hipStream_t s = c->stream;
   const uint32_t nb = a.rows / a.batch;
+  const MlpArena arena{c};
   const MlpDev d = mlp_alloc(c, a.rows, a.batch, std::max<uint32_t>(nb, 1));
   HIP_CHECK(hipMemcpyAsync(d.params, a.params, kParamCount * 4, hipMemcpyHostToDevice, s));
   HIP_CHECK(hipMemcpyAsync(d.feat, a.feat, (size_t)a.rows * kFeat * 4, hipMemcpyHostToDevice, s));
