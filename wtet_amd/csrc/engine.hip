@@ -810,13 +810,17 @@ void after_pick(wtet_ctx* c, Run& R, uint32_t U) {
   R.cur ^= 1;
 }
 
+void next_rounds(Run& R, uint32_t k) {
+  R.round += k;
+  if (R.round > (1u << 16)) throw Fail{WTET_ERR_NOT_CONVERGED, "insertion did not finish"};
+}
+
 // One insertion round's vote, winner pick and compaction of the survivors
 // (vote.wgsl:89-344, compact_vertex_arrays_*.wgsl), launched one by one:
 // returns the round's insertions; the survivors become the uninserted list.
 uint32_t dev_vote(wtet_ctx* c, Run& R) {
   hipStream_t s = c->stream;
-  ++R.round;
-  if (R.round > (1u << 16)) throw Fail{WTET_ERR_NOT_CONVERGED, "insertion did not finish"};
+  next_rounds(R, 1);
   Mesh M = mesh_of(c, R.V, R.mode);
   const uint32_t U = R.U, cur = R.cur, round = R.round;
   launch_set_ctr(M.ctr, C_SURV, U, C_ROUND, round - 1u, s);  // the pick begins the round
@@ -956,7 +960,7 @@ bool run_rounds_small(wtet_ctx* c, Run& R, bool voted) {
   const uint32_t* h = c->h_ctr;
   note_deferred(c, R);
   R.crowded = h[C_RUN_CROWDED] != 0u;  // of its last round alone
-  R.round += (int)h[C_RUN_PICKS];
+  next_rounds(R, h[C_RUN_PICKS]);
   R.cur ^= (int)(h[C_RUN_PICKS] & 1u);
   R.K.rounds += h[C_RUN_PICKS];
   R.K.sumU += h[C_RUN_SUMU];
@@ -1142,8 +1146,7 @@ void run_device(wtet_ctx* c, const float* d_xyz, const std::vector<uint32_t>& of
       const uint32_t U = R.U;
       run_round(c, R, last);
       if (last) break;
-      ++R.round;  // the device counted it too (launch_round_next)
-      if (R.round > (1u << 16)) throw Fail{WTET_ERR_NOT_CONVERGED, "insertion did not finish"};
+      next_rounds(R, 1);  // the device counted it too (k_pick_count)
       after_pick(c, R, U);
     }
   }
