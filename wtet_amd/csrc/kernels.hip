@@ -1079,8 +1079,8 @@ void launch_relocate(const Mesh& M, const uint32_t* uvert, uint32_t* utet, uint3
 
 // LEAN: every slot, FP32 filter, undecided tets to slow[ctr[C_SLOW_T]];
 // SLOW: the full predicates on those; FULL: the full predicates on every slot
-template <int FORM, class MS>
-__global__ void __launch_bounds__(kBlock) k_audit(MS M, uint32_t T, uint32_t* rec, uint32_t cap,
+template <int FORM>
+__global__ void __launch_bounds__(kBlock) k_audit(Mesh M, uint32_t T, uint32_t* rec, uint32_t cap,
                                                   uint64_t* st, uint32_t* slow) {
   PredStats ls = {};
   if (FORM == SLOW) {
@@ -1094,9 +1094,8 @@ __global__ void __launch_bounds__(kBlock) k_audit(MS M, uint32_t T, uint32_t* re
   flush_stats(ls, st);
 }
 
-template <class MS>
-static void audit_t(const MS& M, uint32_t T, uint32_t* rec, uint32_t cap, uint64_t* st, uint32_t* slow,
-                    hipStream_t s) {
+void launch_audit(const Mesh& M, uint32_t T, uint32_t* rec, uint32_t cap, uint64_t* st, uint32_t* slow,
+                  hipStream_t s) {
   if (!T) return;
   if (M.mode == PRED_FILTERED) {
     k_set_ctr<<<1, 64, 0, s>>>(M.ctr, C_SLOW_T, 0u, -1, 0u);
@@ -1107,16 +1106,10 @@ static void audit_t(const MS& M, uint32_t T, uint32_t* rec, uint32_t cap, uint64
   }
 }
 
-void launch_audit(const Mesh& M, uint32_t T, uint32_t* rec, uint32_t cap, uint64_t* st, uint32_t* slow,
-                  hipStream_t s) {
-  audit_t(M, T, rec, cap, st, slow, s);
-}
-
 // ---------------------------------------------------------------------------
 // output
 // ---------------------------------------------------------------------------
-template <class MS>
-__global__ void k_alive_count(MS M, uint32_t T, uint32_t* blk) {
+__global__ void k_alive_count(Mesh M, uint32_t T, uint32_t* blk) {
   uint32_t t = gid();
   bool a = t < T && slot_alive(M, t);
   uint32_t tot;
@@ -1160,8 +1153,7 @@ __global__ void k_cstart_tail(uint32_t* cstart, uint32_t C, const uint32_t* ctr)
   if (threadIdx.x == 0) cstart[C] = ctr[C_ALIVE];
 }
 
-template <class MS>
-__global__ void k_output_rows(MS M, uint32_t T, const uint32_t* olist, const uint32_t* okey,
+__global__ void k_output_rows(Mesh M, uint32_t T, const uint32_t* olist, const uint32_t* okey,
                               const uint32_t* cstart, const uint32_t* slot2pos, const uint32_t* vrank,
                               Clouds K, uint32_t* out_tets, uint32_t* out_adj) {
   uint32_t j = gid();

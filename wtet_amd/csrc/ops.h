@@ -162,30 +162,12 @@ WT_HD void set_adj(const MS& M, uint32_t t, uint4 n, uint4 ov) {
   ADJ(M, t).hi = make_uint4(n.z, ov.z, n.w, ov.w);
 }
 template <class MS>
-WT_HD float3 P3(const MS& M, uint32_t v) {
-  float4 p = M.pts[v];
-  return make_float3(p.x, p.y, p.z);
-}
-
-template <class MS>
 WT_HD void load_pt(const MS& M, uint32_t v, float* out, uint32_t* rank) {
   float4 p = M.pts[v];
   out[0] = p.x;
   out[1] = p.y;
   out[2] = p.z;
   *rank = pt_rank(p);
-}
-
-// orient3d_sos on four vertex ids
-template <class MS>
-WT_HD int o3(const MS& M, uint32_t a, uint32_t b, uint32_t c, uint32_t d, PredStats* st) {
-  float A[3], B[3], C[3], D[3];
-  uint32_t ra, rb, rc, rd;
-  load_pt(M, a, A, &ra);
-  load_pt(M, b, B, &rb);
-  load_pt(M, c, C, &rc);
-  load_pt(M, d, D, &rd);
-  return orient3d_sos(A, B, C, D, ra, rb, rc, rd, M.mode, st);
 }
 
 // Predicates of the lean (FAST) and full bodies.  FAST runs the FP32 filter
@@ -207,25 +189,9 @@ WT_HD int o4s(const MS& M, const float* a, const float* b, const float* c, const
   return orient4d(a, b, c, d, e, ra, rb, rc, rd, re, M.mode, st);
 }
 
-template <bool FAST, class MS>
-WT_HD int o3v(const MS& M, uint32_t a, uint32_t b, uint32_t c, uint32_t d, PredStats* st) {
-  float A[3], B[3], C[3], D[3];
-  uint32_t ra, rb, rc, rd;
-  load_pt(M, a, A, &ra);
-  load_pt(M, b, B, &rb);
-  load_pt(M, c, C, &rc);
-  load_pt(M, d, D, &rd);
-  return o3s<FAST>(M, A, B, C, D, ra, rb, rc, rd, st);
-}
-
 template <class MS>
 WT_HD uint32_t* opp_word(const MS& M, uint32_t t, uint32_t f) {
   return reinterpret_cast<uint32_t*>(&ADJ(M, t)) + 2 * f;
-}
-
-template <class MS>
-WT_HD uint32_t* oppv_word(const MS& M, uint32_t t, uint32_t f) {
-  return reinterpret_cast<uint32_t*>(&ADJ(M, t)) + 2 * f + 1;
 }
 
 // face f of slot t: neighbour pointer and opposite vertex in one store
@@ -263,12 +229,6 @@ WT_HD uint64_t vote_key(const MS& M, const uint32_t* uvert, const uint32_t* utet
   bool bad = tv.x == M.inf || tv.y == M.inf || tv.z == M.inf || tv.w == M.inf;
   if (bad) at_add_u32(&M.ctr[C_BADTET], 1u);
   return bad ? kVoteNone : key;
-}
-
-template <class MS>
-WT_HD void vote_body(const MS& M, const uint32_t* uvert, const uint32_t* utet, uint32_t i) {
-  uint64_t key = vote_key(M, uvert, utet, i);
-  if (key != kVoteNone) mesh_min(M, &TVOTE(M, utet[i]), key);
 }
 
 // Point i is inserted this round when it holds its tet's vote and no tet
@@ -411,12 +371,6 @@ WT_HD bool split_points_body_t(const MS& M, const uint32_t* uvert, uint32_t* ute
   int child = s > 0 ? a : b;
   utet[i] = child_slot(t, base, (uint32_t)child);
   return false;
-}
-
-template <class MS>
-WT_HD void split_points_body(const MS& M, const uint32_t* uvert, uint32_t* utet, uint32_t i,
-                             uint32_t round, PredStats* st) {
-  (void)split_points_body_t<false>(M, uvert, utet, i, round, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -910,8 +864,8 @@ WT_HD bool relocate_body_t(const MS& M, const uint32_t* uvert, uint32_t* utet, u
 // returns true (nothing recorded) when a face is undecided, for the full
 // pass to redo the tet.
 // ---------------------------------------------------------------------------
-template <bool FAST, class MS>
-WT_HD bool audit_body_t(const MS& M, uint32_t t, uint32_t* rec, uint32_t cap, PredStats* st) {
+template <bool FAST>
+WT_HD bool audit_body_t(const Mesh& M, uint32_t t, uint32_t* rec, uint32_t cap, PredStats* st) {
   if (!slot_alive(M, t)) return false;
   uint4 tv = TV(M, t);
   if (tv.x == M.inf || tv.y == M.inf || tv.z == M.inf || tv.w == M.inf) return false;
@@ -940,11 +894,6 @@ WT_HD bool audit_body_t(const MS& M, uint32_t t, uint32_t* rec, uint32_t cap, Pr
       if (k < cap) rec[k] = (t << 2) | (uint32_t)f;
     }
   return false;
-}
-
-template <class MS>
-WT_HD void audit_body(const MS& M, uint32_t t, uint32_t* rec, uint32_t cap, PredStats* st) {
-  (void)audit_body_t<false>(M, t, rec, cap, st);
 }
 
 }  // namespace wtet

@@ -273,17 +273,16 @@ inline StartTets make_start_tets() {
   return S;
 }
 
-// start tet t (0..4) of cloud c, the cloud's five in slots base..base + 4
-template <class MS>
-WT_HD void start_tet_at(const MS& M, const StartTets& S, uint32_t c, uint32_t t, uint32_t base,
-                        const Clouds& K) {
-  uint32_t sb = super_base(K.off, c), g = base + t;
+// g in [0, 5C): start tet g % 5 of cloud g / 5, in slot g
+WT_HD void start_tet_body(const Mesh& M, const StartTets& S, uint32_t g, const Clouds& K) {
+  uint32_t c = g / 5u, t = g - 5u * c;
+  uint32_t sb = super_base(K.off, c);
   uint4 tv, to, tov;
   for (int k = 0; k < 4; ++k) {
     uint32_t code = S.tv[4 * t + k];
     set4(tv, k, code == 4u ? K.V : sb + code);
     uint32_t e = S.to[4 * t + k];
-    set4(to, k, enc_opp(base + opp_tet(e), opp_face(e)));
+    set4(to, k, enc_opp(5u * c + opp_tet(e), opp_face(e)));
     uint32_t ocode = S.tv[4 * opp_tet(e) + opp_face(e)];  // the neighbour's vertex opposite
     set4(tov, k, ocode == 4u ? K.V : sb + ocode);
   }
@@ -294,13 +293,6 @@ WT_HD void start_tet_at(const MS& M, const StartTets& S, uint32_t c, uint32_t t,
   FVOTE(M, g) = kVoteNone;
   TSPLIT(M, g) = make_uint2(0u, 0u);
   FSTAMP(M, g) = 0u;
-}
-
-// g in [0, 5C): start tet g % 5 of cloud g / 5, in slot g
-template <class MS>
-WT_HD void start_tet_body(const MS& M, const StartTets& S, uint32_t g, const Clouds& K) {
-  uint32_t c = g / 5u;
-  start_tet_at(M, S, c, g - 5u * c, 5u * c, K);
 }
 
 // Exact duplicates (equal normalized coordinates in one cloud) share a key,
@@ -329,8 +321,7 @@ WT_HD bool redundant_dup(const float4* cpts, const uint64_t* keys, uint32_t n, u
 }
 
 // output: cloud of a live tet = cloud of its smallest vertex (never V)
-template <class MS>
-WT_HD uint32_t cloud_of_tet(const MS& M, uint32_t t, const Clouds& K) {
+WT_HD uint32_t cloud_of_tet(const Mesh& M, uint32_t t, const Clouds& K) {
   if (K.C <= 1) return 0u;
   uint4 v = TV(M, t);
   uint32_t m = v.x < v.y ? v.x : v.y;
@@ -344,8 +335,7 @@ WT_HD uint32_t cloud_of_tet(const MS& M, uint32_t t, const Clouds& K) {
 // n_c + 4), adjacency (local row << 5) | face.  slot2pos: slot -> row.
 // vrank[v]: vertex v's rank (its input id within its cloud), one word per
 // vertex so that the four lookups of a row stay in a small array
-template <class MS>
-WT_HD void output_body(const MS& M, uint32_t j, const uint32_t* olist, const uint32_t* ocloud,
+WT_HD void output_body(const Mesh& M, uint32_t j, const uint32_t* olist, const uint32_t* ocloud,
                        const uint32_t* cstart, const uint32_t* slot2pos, const uint32_t* vrank,
                        const Clouds& K, uint32_t* out_tets, uint32_t* out_adj) {
   uint32_t t = olist[j];
