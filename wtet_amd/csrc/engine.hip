@@ -885,13 +885,15 @@ void run_round(wtet_ctx* c, Run& R, bool last) {
   const uint64_t a_hint = (uint64_t)c->h_ctr[C_LIST] + 4ull * W;
   const int variant = !R.flipping ? 0 : (a_hint <= R.list_bound() ? 1 : 2);
   const uint32_t grid = variant == 2 ? grid_for(c, a_hint, 16) : 0u;
-  const uint32_t dgrid = variant == 2 ? deferred_grid(c, dper, grid) : 0u;
+  // the deferred check runs beside the filters only: a round without them has
+  // one graph whatever it would defer
+  const uint32_t dgrid = variant == 2 && !R.full ? deferred_grid(c, dper, grid) : 0u;
   const int k = R.max_fi;
   uint32_t* uv = P<uint32_t>(c->uvert[cur]);
   uint32_t* ut = P<uint32_t>(c->utet[cur]);
   uint32_t* slow_p = P<uint32_t>(c->slow_p);
   uint64_t* sums = P<uint64_t>(c->isums);
-  const bool sparse = dper <= kSparseDeferred;
+  const bool sparse = !R.full && dper <= kSparseDeferred;
   auto enqueue = [&] {
     // the batch of iterations begins and ends in the point kernels beside
     // it, unless there are no points left
