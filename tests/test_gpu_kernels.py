@@ -162,3 +162,19 @@ def test_block_scan_of_several_steps(ctx):
     faces = np.tile(np.arange(4, dtype=np.uint32), (len(t), 1))
     back = r.adjacency[t[inner], f[inner]]
     assert np.array_equal(back >> 5, rows[inner]) and np.array_equal(back & 3, faces[inner])
+
+
+# a histogram block for 8,192 keys, from 256 to 1,024 of them; digits that all
+# lanes of a wave share, and that few do
+@pytest.mark.parametrize("n", [257 * 8192 - 1, 257 * 8192, 1025 * 8192 + 1])
+@pytest.mark.parametrize("distinct", [1, 3, 4096])
+def test_sort_histogram_blocks_and_ties(ctx, n, distinct):
+    keys = np.random.default_rng(n + distinct).integers(0, distinct, n).astype(np.uint32) + np.uint32(7)
+    d = [ctx.upload(a) for a in (keys, np.arange(n, dtype=np.uint32), np.zeros_like(keys), np.zeros(n, np.uint32))]
+    try:
+        ctx.sort_pairs(d[0], d[1], d[2], d[3], n, 32, 13)
+        got = ctx.download(d[3], (n,), np.uint32)
+    finally:
+        for p in d:
+            ctx.free(p)
+    assert np.array_equal(got, np.argsort(keys, kind="stable").astype(np.uint32))
