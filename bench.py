@@ -26,18 +26,19 @@ HBM_PEAK_GBS = 8000.0  # MI355X HBM3E
 
 # Algorithmic bytes of each kernel group over one call, from the run's own
 # counters (minimal SoA traffic per unit):
-#   flip_check (FP32-only check): per tet checked -- own quad + adjacency 32,
+#   flip_check (the filters): per tet checked -- own quad + adjacency 32,
 #     four neighbour quads 64, eight vertex xyz 96, vote atomic 8 = 200
 #   flip_decide_exec: per tet checked 24 (its vote word, the face's vote
-#     word, info) + per executed flip 208 (read/write <= 3 tets 192, flip
+#     word, queue tags) + per executed flip 208 (read/write <= 3 tets 192, flip
 #     record 16)
 #   flip_update: per executed flip 48 (six external back-pointers 24 and
 #     their messages 24); decide_exec + update = 24 per check + 256 per flip
-#   flip_small: the three above for the short-list iterations
+#   flip_small: the three above for the one-workgroup iterations (its time
+#     holds the votes, splits and walks of whole rounds too)
 #   split: per insertion 224; output: per tet 32
-#   audit: per live tet 124 (quad 16, adjacency 32, info 4, its four points
+#   audit: per live tet 124 (quad 16, adjacency 32, tag 4, its four points
 #     48, the opposite points of the two faces it owns 24); per slot a 3-2
-#     flip freed, its info word 4
+#     flip freed, its tag 4
 def kernel_bytes(st):
     a_big = st["sum_active"] - st["small_checked"]
     f_big = st["sum_flips"] - st["small_flips"]
@@ -54,13 +55,13 @@ def kernel_bytes(st):
 
 
 KERNEL_NAMES = {
-    "flip_check": "k_flip_check<LEAN> (FP32-only flip check)",
+    "flip_check": "k_flip_check (filters of the flip check)",
     "flip_decide_exec": "k_flip_decide_exec (flip vote, claim and 2-3 / 3-2 execution)",
     "flip_update": "k_flip_update (external adjacency through flip messages)",
-    "flip_small": "k_flip_small (one-workgroup iterations of short lists)",
+    "flip_small": "k_flip_small, k_rounds_small (one-workgroup iterations and rounds)",
     "split": "k_split (1-4 split)",
     "audit": "k_audit<LEAN> (exact audit of every finite face)",
-    "output": "k_output (compaction and id remap)",
+    "output": "k_output_rows (compaction and id remap)",
 }
 
 

@@ -100,8 +100,8 @@ typedef struct wtet_stats {
                                      and failed_verts lists them                */
   uint64_t flips_23;              /* executed 2-3 flips (of sum_flips)         */
   uint64_t flips_32;              /* executed 3-2 flips (of sum_flips)         */
-  uint64_t small_checked;         /* of sum_active: checked in the one-workgroup
-                                     iterations of short lists              */
+  uint64_t small_checked;         /* of sum_active: checked in one-workgroup
+                                     kernels (short lists, few points)      */
   uint64_t small_flips;           /* of sum_flips: executed in those iterations */
 } wtet_stats;
 
@@ -341,10 +341,12 @@ wtet_status wtet_mlp_train(wtet_ctx *ctx, float *params, const float *feat, cons
 /* Per-kernel-group timing with HIP events on the context's stream (the
  * reference's GpuProfiler/CpuProfiler scopes, src/profiler.rs:5-224).
  * wtet_set_profiling resets the totals; kinds 0..12 are prepare_points,
- * vote, pick, split, split_points, flip_check (the FP32-only check),
+ * vote, pick, split, split_points, flip_check (the filters, or the full
+ * predicates on every tet),
  * flip_check_deferred (full predicates on the tets it deferred),
  * flip_decide_exec, flip_update, relocate, audit, output, flip_small (the
- * one-workgroup iterations of short lists).  Totals
+ * one-workgroup iterations of short lists, and the whole rounds of few
+ * points).  Totals
  * accumulate over calls. */
 wtet_status wtet_set_profiling(wtet_ctx *ctx, int on);
 wtet_status wtet_kernel_times(const wtet_ctx *ctx, uint32_t kind, const char **name,

@@ -391,7 +391,7 @@ WT_HD void pick_xyz(const float (*P)[3], int k, float* out) {
 // The proposal of tet t across face f (its kind, offending edge and third
 // tet as flip_check_lean finds them, nt the neighbour): votes for the other tets it involves;
 // its tag is the vote for its own.  A vote is an atomic minimum on a random
-// line, 27 G/s on this card, a tag a store, 84 G/s.
+// line, 27 G/s on this card, a tag a store, 89 G/s.
 template <class MS>
 WT_HD uint4 flip_propose(const MS& M, uint32_t t, uint32_t f, uint32_t nt, uint32_t kind, uint32_t bad, uint32_t third,
                          uint32_t it) {
